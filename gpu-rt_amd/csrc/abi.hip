@@ -1,5 +1,6 @@
 // abi.hip -- the extern "C" entry points of include/gpurt.h: argument checks, device
 // selection, ownership, and dispatch to the builder / traversal / backward launchers.
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -100,14 +101,103 @@ void wait_uses(gpurt_bvh_s* b, hipStream_t s) {
         }
 }
 
-// frees a BVH's buffers in order on stream s (all come from the stream-ordered pool)
+// gives a BVH's memory back in order on stream s
 static void free_bvh_buffers(gpurt_bvh_s* b, hipStream_t s) {
-    for (void* p : {b->nodes, b->qnodes, (void*)b->tris, (void*)b->tri_idx, (void*)b->verts, (void*)b->leaf_order})
-        if (p) (void)hipFreeAsync(p, s);
-    b->nodes = b->qnodes = nullptr;
+    for (void* p : {b->mesh_mem, b->node_mem})
+        if (p) pool_free(b->ctx, p, s);
+    b->mesh_mem = b->node_mem = b->nodes = b->qnodes = nullptr;
     b->tris = nullptr;
-    b->tri_idx = b->leaf_order = nullptr;
+    b->tri_idx = b->leaf_order = b->refit_tmp = nullptr;
     b->verts = nullptr;
+}
+
+// frees idle pool blocks, the longest idle first, until at most `keep` idle bytes are left
+// (the caller holds pool_mu)
+static void pool_trim(gpurt_ctx_s* c, size_t keep) {
+    while (c->pool_idle > keep) {
+        size_t k = c->pool.size();
+        for (size_t i = 0; i < c->pool.size(); i++)
+            if (!c->pool[i].used && (k == c->pool.size() || c->pool[i].when < c->pool[k].when)) k = i;
+        if (k == c->pool.size()) return;
+        gpurt_ctx_s::PoolBlock& e = c->pool[k];
+        (void)hipEventSynchronize(e.freed);
+        (void)hipFree(e.mem);
+        (void)hipEventDestroy(e.freed);
+        (void)hipGetLastError();
+        c->pool_idle -= e.bytes;
+        c->pool.erase(c->pool.begin() + (ptrdiff_t)k);
+    }
+}
+
+int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
+    *p = nullptr;
+    // sizes in steps of an eighth of their power of two (at least 64 KiB), so that the
+    // slightly different node counts of similar meshes share blocks
+    size_t step = size_t(1) << 16;
+    while (step * 16 <= bytes) step *= 2;
+    bytes = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+    std::lock_guard<std::mutex> lk(c->pool_mu);
+    // the smallest idle block that fits without wasting half of it; of equals the one
+    // given back first
+    gpurt_ctx_s::PoolBlock* best = nullptr;
+    for (auto& e : c->pool)
+        if (!e.used && e.bytes >= bytes && e.bytes <= 2 * bytes &&
+            (!best || e.bytes < best->bytes || (e.bytes == best->bytes && e.when < best->when)))
+            best = &e;
+    if (best && hipStreamWaitEvent(s, best->freed, 0) == hipSuccess) {
+        best->used = true;
+        c->pool_idle -= best->bytes;
+        *p = best->mem;
+        return GPURT_OK;
+    }
+    gpurt_ctx_s::PoolBlock e;
+    e.bytes = bytes;
+    e.used = true;
+    if (hipMalloc(&e.mem, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        e.mem = nullptr;
+        pool_trim(c, 0);
+        if (hipMalloc(&e.mem, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return set_error(GPURT_E_OOM, "allocation of " + std::to_string(bytes) + " bytes failed");
+        }
+    }
+    if (hipEventCreateWithFlags(&e.freed, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(e.mem);
+        return set_error(GPURT_E_DEVICE, "event creation failed");
+    }
+    c->pool.push_back(e);
+    *p = e.mem;
+    return GPURT_OK;
+}
+
+void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(c->pool_mu);
+    for (auto& e : c->pool)
+        if (e.mem == p) {
+            if (hipEventRecord(e.freed, s) != hipSuccess) {
+                // the stream cannot say when its work is done: wait for the device
+                (void)hipGetLastError();
+                (void)hipDeviceSynchronize();
+            }
+            e.used = false;
+            e.when = ++c->pool_clock;
+            c->pool_idle += e.bytes;
+            break;
+        }
+    pool_trim(c, c->pool_limit);
+}
+
+void pool_release(gpurt_ctx_s* c) {
+    std::lock_guard<std::mutex> lk(c->pool_mu);
+    for (auto& e : c->pool) {
+        (void)hipFree(e.mem);
+        (void)hipEventDestroy(e.freed);
+    }
+    c->pool.clear();
+    c->pool_idle = 0;
 }
 
 int compact_verts(const float* verts, size_t stride_floats, size_t n, float* out, hipStream_t s) {
@@ -273,7 +363,10 @@ int gpurt_ctx_create(int device, gpurt_ctx* out) {
             return rc;
         }
     }
-    // keep freed stream-ordered allocations (traversal spill stacks) in the pool
+    size_t mem_free = 0, mem_total = 0;
+    if (hipMemGetInfo(&mem_free, &mem_total) == hipSuccess) c->pool_limit = std::max(c->pool_limit, mem_total / 16);
+    // keep freed stream-ordered allocations (scratch of captured or concurrent calls) in
+    // HIP's pool
     hipMemPool_t pool;
     if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) {
         uint64_t thr = ~0ull;
@@ -301,7 +394,9 @@ void gpurt_ctx_destroy(gpurt_ctx ctx) {
         }
         ctx->bvhs.clear();
     }
+    if (ctx->release) (void)hipStreamSynchronize(ctx->release);
     ctx_scratch_release(ctx);
+    pool_release(ctx);
     if (ctx->release) (void)hipStreamSynchronize(ctx->release);
     (void)hipGetLastError();
     if (ctx->release) (void)hipStreamDestroy(ctx->release);
@@ -370,18 +465,24 @@ int gpurt_bvh_build(gpurt_ctx ctx, const float* verts, size_t vstride_bytes, siz
         delete b;
         return code;
     };
-    rc = build_segments(ctx, &sd, 1, bp.width, bp.leaf_size, bp.treelet_size, bp.treelet_rounds, bp.format, s, b);
-    if (rc) return fail(rc);
-    // keep the index buffer and compact positions for the backward passes and refit
-    if (hipMallocAsync((void**)&b->tri_idx, sizeof(uint32_t) * 3 * n_tris, s) != hipSuccess ||
-        hipMallocAsync((void**)&b->verts, sizeof(float) * 3 * n_verts, s) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(set_error(GPURT_E_OOM, "allocation of the mesh copy failed"));
-    }
+    // the mesh copy of the backward passes and refit, and the triangles that the build
+    // leaves here
+    auto carve = [&](Carver c) {
+        c.take(b->tri_idx, 3 * n_tris);
+        c.take(b->verts, 3 * n_verts);
+        c.take(b->tris, 3 * n_tris);
+        c.take(b->leaf_order, n_tris);
+        c.take(b->refit_tmp, 2);
+        return c.off;
+    };
+    if ((rc = pool_alloc(ctx, &b->mesh_mem, carve(Carver{}), s))) return fail(rc);
+    carve(Carver{0, static_cast<char*>(b->mesh_mem)});
     if (hipMemcpyAsync(b->tri_idx, tri_idx, sizeof(uint32_t) * 3 * n_tris, hipMemcpyDeviceToDevice, s) !=
         hipSuccess)
         return fail(hip_error(hipGetLastError(), "copying indices"));
     if ((rc = compact_verts(verts, vstride_bytes / 4, n_verts, b->verts, s)) != GPURT_OK) return fail(rc);
+    rc = build_segments(ctx, &sd, 1, bp.width, bp.leaf_size, bp.treelet_size, bp.treelet_rounds, bp.format, s, b);
+    if (rc) return fail(rc);
     // the handle is complete when this returns, so queries on any stream may follow
     if (hipStreamSynchronize(s) != hipSuccess) return fail(hip_error(hipGetLastError(), "build"));
     {

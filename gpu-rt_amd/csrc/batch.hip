@@ -375,8 +375,7 @@ struct DevGuard {
 int enqueue_batch(gpurt_batch_s* b, int treelet_size, int treelet_rounds, hipStream_t s) {
     int rc;
     if ((rc = build_enqueue_binary(b->build, treelet_size, treelet_rounds, s))) return rc;
-    // all levels: empty levels exit at once, and the tree cannot be deeper (kMaxLevels)
-    if ((rc = build_enqueue_levels(b->build, b->leaf_size, 0, kMaxLevels, s))) return rc;
+    if ((rc = build_enqueue_collapse(b->build, b->leaf_size, s))) return rc;
     if (has_qnodes(b->format)) {
         // counters[0] holds the wide-node count the levels produced
         launch_quantize(b->width, b->build.nodes, b->qnodes, 0, b->build.capacity, b->build.counters, s);

@@ -5,17 +5,18 @@
 //
 // Pipeline (every stage is one launch over ALL meshes of the build; a plain build is a
 // batch of one mesh):
-//   k_prep         triangle AABBs, centroid bounds and coordinate scale per mesh
-//                  (wave-reduced, ordered-uint atomics)
-//   k_morton       key = mesh_id << 30 | 30-bit Morton code of the AABB centre over the
+//   k_prep         centroid bounds and coordinate scale per mesh (wave-reduced,
+//                  ordered-uint atomics), triangle box centres
+//   k_morton       key = mesh_id << 30 | 30-bit Morton code of the box centre over the
 //                  mesh's centroid bounds; value = triangle index
 //   radix sort     LSD, 8-bit digits, LDS histograms + LDS ranking by wave ballots
-//                  (stable, so equal codes stay in triangle order)
-//   k_pack         triangles and AABBs gathered into sorted (leaf) order
+//                  (stable, so equal codes stay in triangle order); one block up to 8192
+//   k_pack         triangles and boxes gathered into sorted (leaf) order
 //   k_karras       Karras (HPG 2012) binary radix tree over the sorted keys; because the
 //                  mesh id is in the high key bits every mesh is one subtree, whose root
 //                  is recorded
-//   k_boxes_level  node AABBs bottom-up, one launch per common-prefix length (no atomics)
+//   k_boxes_*      node boxes: those inside a chunk of 256 leaves bottom-up by one block,
+//                  the others as unions over their leaf range (no atomics, no order)
 //   k_treelet      optional SAH treelet restructuring (treelet.hip)
 //   k_collapse     one launch per wide level: a node opens the child with the largest
 //                  surface area until it has W children; subtrees of <= leaf_size
@@ -69,15 +70,11 @@ __device__ __forceinline__ int find_seg(const SegDesc* segs, int n_seg, uint32_t
 }
 
 
-__global__ void k_fill_u32(uint32_t* p, size_t n, uint32_t v) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = v;
-}
-
-__global__ void k_init_build(const SegDesc* segs, int n_seg, uint32_t* segstat_rep, uint32_t* seg_root,
-                             uint32_t* lvl_cnt, uint32_t* counters) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Clears what the build accumulates into.  A plain build hands its one mesh over as an
+// argument (no copy to the device to wait for).
+__global__ void k_init_build(SegDesc* segs, int n_seg, SegDesc one, int has_one, uint32_t* segstat_rep, uint32_t* seg_root,
+                             uint32_t* report, uint32_t* lvl_hist) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n_seg * kRep) {
         uint32_t* st = segstat_rep + (size_t)i * kStat;
         for (int k = 0; k < 3; k++) {
@@ -87,9 +84,12 @@ __global__ void k_init_build(const SegDesc* segs, int n_seg, uint32_t* segstat_r
         st[6] = 0u;
         st[7] = 0u;
     }
-    if (i < n_seg) seg_root[i] = kLeafBit | segs[i].tri_offset;  // single-triangle mesh: leaf root
-    if (i <= kMaxLevels) lvl_cnt[i] = (i == 0) ? (uint32_t)n_seg : 0u;
-    if (i < 4) counters[i] = (i == 0) ? (uint32_t)n_seg : 0u;  // [0] wide nodes, [1] error
+    if (i == 0 && has_one) segs[0] = one;
+    // single-triangle mesh: leaf root
+    if (i < n_seg) seg_root[i] = kLeafBit | (has_one ? one.tri_offset : segs[i].tri_offset);
+    // level 0 and the wide nodes start with one node per mesh; everything else is zero
+    if (i < kReportWords) report[i] = (i == kReportLvl || i == kReportCounters) ? (uint32_t)n_seg : 0u;
+    if (i < (int)kLevelBuckets) lvl_hist[i] = 0u;
 }
 
 // folds the kRep replicas of every mesh's statistics into segstat
@@ -100,6 +100,7 @@ __global__ void k_reduce_stats(int n_seg, const uint32_t* __restrict__ segstat_r
     const int sgi = i / kStat, k = i % kStat;
     const bool is_min = k < 3;
     uint32_t v = is_min ? 0xFFFFFFFFu : 0u;
+#pragma unroll 16
     for (int r = 0; r < kRep; r++) {
         uint32_t x = segstat_rep[((size_t)r * n_seg + sgi) * kStat + k];
         v = is_min ? min(v, x) : max(v, x);
@@ -108,96 +109,130 @@ __global__ void k_reduce_stats(int n_seg, const uint32_t* __restrict__ segstat_r
 }
 
 // ------------------------------------------------------------------------------------
-// k_prep: AABBs + per-mesh centroid bounds
+// k_prep: box centres + per-mesh centroid bounds
 // ------------------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kBlock) void k_prep(const SegDesc* __restrict__ segs, int n_seg,
-                                                 uint32_t N, float4* __restrict__ aabb_lo,
-                                                 float4* __restrict__ aabb_hi,
-                                                 uint32_t* __restrict__ segstat,
-                                                 uint32_t* __restrict__ counters) {
-    uint32_t g = blockIdx.x * kBlock + threadIdx.x;
-    bool valid = g < N;
-    int s = valid ? find_seg(segs, n_seg, g) : 0;
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    float cen[3] = {INFINITY, INFINITY, INFINITY}, cenx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    float amax = 0.0f;
-    if (valid) {
-        const SegDesc sd = segs[s];
-        uint32_t t = g - sd.tri_offset;
-        uint32_t vi[3];
-        bool bad = false;
-        for (int k = 0; k < 3; k++) {
-            vi[k] = sd.idx[3 * (size_t)t + k];
-            if (vi[k] >= sd.n_verts) { bad = true; vi[k] = 0; }
-        }
-        if (bad) atomicOr(&counters[1], 1u);
-        float v[3][3];
-        bool finite = true;
-        for (int k = 0; k < 3; k++) {
-            const float* p = sd.verts + (size_t)vi[k] * sd.vstride;
-            v[k][0] = p[0]; v[k][1] = p[1]; v[k][2] = p[2];
-            finite = finite && isfinite(v[k][0]) && isfinite(v[k][1]) && isfinite(v[k][2]);
-        }
-        // a non-finite position is reported (the build fails with GPURT_E_INVALID); the
-        // triangle's box is then the origin so every later stage works on finite boxes
-        if (!finite) atomicOr(&counters[1], 4u);
-        for (int a = 0; a < 3; a++) {
-            for (int k = 0; k < 3; k++) {
-                const float x = finite ? v[k][a] : 0.0f;
-                lo[a] = fminf(lo[a], x);
-                hi[a] = fmaxf(hi[a], x);
-                amax = fmaxf(amax, fabsf(x));
-            }
-            cen[a] = (lo[a] + hi[a]) * 0.5f;
-            cenx[a] = cen[a];
-        }
-        aabb_lo[g] = make_float4(lo[0], lo[1], lo[2], __uint_as_float((uint32_t)s));
-        aabb_hi[g] = make_float4(hi[0], hi[1], hi[2], 0.0f);
-    }
-    // reduce over the wave when it covers one mesh, else per lane; this block's replica
-    segstat += (size_t)(blockIdx.x % kRep) * n_seg * kStat;
-    int s0 = __shfl(s, 0);
-    bool uniform = __all(s == s0 || !valid);
+// A mesh's running bounds in the lanes of a wave (ordered uints): centroid minimum and
+// maximum, largest |coordinate|.
+struct WaveStats {
     uint32_t o[7];
-    for (int a = 0; a < 3; a++) {
-        o[a] = valid ? f2o(cen[a]) : 0xFFFFFFFFu;
-        o[3 + a] = valid ? f2o(cenx[a]) : 0u;
+    __device__ __forceinline__ void reset() {
+        for (int a = 0; a < 3; a++) {
+            o[a] = 0xFFFFFFFFu;
+            o[3 + a] = 0u;
+        }
+        o[6] = 0u;
     }
-    o[6] = valid ? f2o(amax) : 0u;
-    if (uniform) {
+    // wave-reduced into mesh s of a replica, one atomic per word (all lanes call it)
+    __device__ __forceinline__ void flush(uint32_t* segstat, int s) {
         for (int a = 0; a < 3; a++) {
             o[a] = wave_min_u32(o[a]);
             o[3 + a] = wave_max_u32(o[3 + a]);
         }
         o[6] = wave_max_u32(o[6]);
-        if ((threadIdx.x & 63) == 0 && __any(valid)) {
+        if ((threadIdx.x & 63) == 0) {
             for (int a = 0; a < 3; a++) {
-                atomicMin(&segstat[s0 * kStat + a], o[a]);
-                atomicMax(&segstat[s0 * kStat + 3 + a], o[3 + a]);
+                atomicMin(&segstat[s * kStat + a], o[a]);
+                atomicMax(&segstat[s * kStat + 3 + a], o[3 + a]);
             }
-            atomicMax(&segstat[s0 * kStat + 6], o[6]);
+            atomicMax(&segstat[s * kStat + 6], o[6]);
         }
-    } else if (valid) {
-        for (int a = 0; a < 3; a++) {
-            atomicMin(&segstat[s * kStat + a], o[a]);
-            atomicMax(&segstat[s * kStat + 3 + a], o[3 + a]);
-        }
-        atomicMax(&segstat[s * kStat + 6], o[6]);
+        reset();
     }
+};
+
+// Each wave takes `rounds` x 64 consecutive triangles and keeps its mesh's bounds in
+// registers until the mesh ends: one set of atomics per wave and mesh.  (With a set per 64
+// triangles the same-address atomics were most of the kernel: 182 us for 2.3 M triangles.)
+__global__ __launch_bounds__(kBlock) void k_prep(const SegDesc* __restrict__ segs, int n_seg,
+                                                 uint32_t N, int rounds, float4* __restrict__ cen,
+                                                 uint32_t* __restrict__ segstat,
+                                                 uint32_t* __restrict__ counters) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    const uint32_t beg = wave * (uint32_t)rounds * 64u;
+    if (beg >= N) return;
+    segstat += (size_t)(wave % kRep) * n_seg * kStat;
+    WaveStats ws;
+    ws.reset();
+    int s = find_seg(segs, n_seg, beg);  // mesh of the wave's running bounds
+    SegDesc sd = segs[s];
+    for (int r = 0; r < rounds; r++) {
+        const uint32_t g0 = beg + (uint32_t)r * 64u, g = g0 + lane;
+        if (g0 >= N) break;
+        const bool valid = g < N;
+        const uint32_t last = min(g0 + 63u, N - 1u);
+        // most rounds lie in one mesh; the others search per lane
+        if (g0 >= sd.tri_offset + sd.n_tris) {
+            ws.flush(segstat, s);
+            s = find_seg(segs, n_seg, g0);
+            sd = segs[s];
+        }
+        const bool uniform = last < sd.tri_offset + sd.n_tris;
+        const int sl = uniform || !valid ? s : find_seg(segs, n_seg, g);
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        float c[3] = {0.f, 0.f, 0.f};
+        float amax = 0.0f;
+        if (valid) {
+            const SegDesc d = uniform ? sd : segs[sl];
+            const uint32_t t = g - d.tri_offset;
+            uint32_t vi[3];
+            bool bad = false;
+            for (int k = 0; k < 3; k++) {
+                vi[k] = d.idx[3 * (size_t)t + k];
+                if (vi[k] >= d.n_verts) { bad = true; vi[k] = 0; }
+            }
+            if (bad) atomicOr(&counters[1], 1u);
+            float v[3][3];
+            bool finite = true;
+            for (int k = 0; k < 3; k++) {
+                const float* p = d.verts + (size_t)vi[k] * d.vstride;
+                v[k][0] = p[0]; v[k][1] = p[1]; v[k][2] = p[2];
+                finite = finite && isfinite(v[k][0]) && isfinite(v[k][1]) && isfinite(v[k][2]);
+            }
+            // a non-finite position is reported (the build fails with GPURT_E_INVALID); the
+            // triangle's box is then the origin so every later stage works on finite boxes
+            if (!finite) atomicOr(&counters[1], 4u);
+            for (int a = 0; a < 3; a++) {
+                for (int k = 0; k < 3; k++) {
+                    const float x = finite ? v[k][a] : 0.0f;
+                    lo[a] = fminf(lo[a], x);
+                    hi[a] = fmaxf(hi[a], x);
+                    amax = fmaxf(amax, fabsf(x));
+                }
+                c[a] = (lo[a] + hi[a]) * 0.5f;
+            }
+            cen[g] = make_float4(c[0], c[1], c[2], __uint_as_float((uint32_t)sl));
+        }
+        if (uniform) {
+            if (valid) {
+                for (int a = 0; a < 3; a++) {
+                    ws.o[a] = min(ws.o[a], f2o(c[a]));
+                    ws.o[3 + a] = max(ws.o[3 + a], f2o(c[a]));
+                }
+                ws.o[6] = max(ws.o[6], f2o(amax));
+            }
+        } else if (valid) {
+            for (int a = 0; a < 3; a++) {
+                atomicMin(&segstat[sl * kStat + a], f2o(c[a]));
+                atomicMax(&segstat[sl * kStat + 3 + a], f2o(c[a]));
+            }
+            atomicMax(&segstat[sl * kStat + 6], f2o(amax));
+        }
+    }
+    ws.flush(segstat, s);
 }
 
-__global__ __launch_bounds__(kBlock) void k_morton(uint32_t N, const float4* __restrict__ aabb_lo,
-                                                   const float4* __restrict__ aabb_hi,
+__global__ __launch_bounds__(kBlock) void k_morton(uint32_t N, const float4* __restrict__ cen,
                                                    const uint32_t* __restrict__ segstat,
                                                    uint64_t* __restrict__ keys,
                                                    uint32_t* __restrict__ vals) {
     uint32_t g = blockIdx.x * kBlock + threadIdx.x;
     if (g >= N) return;
-    float4 lo = aabb_lo[g], hi = aabb_hi[g];
-    uint32_t s = __float_as_uint(lo.w);
+    const float4 c4 = cen[g];
+    const uint32_t s = __float_as_uint(c4.w);
     const uint32_t* st = segstat + s * kStat;
-    float c[3] = {(lo.x + hi.x) * 0.5f, (lo.y + hi.y) * 0.5f, (lo.z + hi.z) * 0.5f};
+    const float c[3] = {c4.x, c4.y, c4.z};
     uint32_t q[3];
     for (int a = 0; a < 3; a++) {
         float l = o2f(st[a]), h = o2f(st[3 + a]);
@@ -232,77 +267,38 @@ __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint64_t* __restric
     hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-// Exclusive scan of `total` counts in three launches: per-tile sums, one block scanning
-// the tile sums, then per-tile scans offset by their tile's prefix.
-constexpr int kScanTile = 4096;
-
-__global__ __launch_bounds__(kBlock) void k_scan_tiles(const uint32_t* __restrict__ a, uint32_t total,
-                                                       uint32_t* __restrict__ tile_sum) {
-    __shared__ uint32_t red[kBlock];
-    const uint32_t base = blockIdx.x * kScanTile;
-    uint32_t s = 0;
-    for (int k = 0; k < kScanTile / kBlock; k++) {
-        uint32_t i = base + k * kBlock + threadIdx.x;
-        if (i < total) s += a[i];
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) tile_sum[blockIdx.x] = red[0];
-}
-
-__global__ __launch_bounds__(1024) void k_scan_sums(uint32_t* __restrict__ t, uint32_t n) {
-    __shared__ uint32_t part[1024];
-    uint32_t chunk = (n + 1023) / 1024;
-    uint32_t beg = threadIdx.x * chunk, end = min(beg + chunk, n);
-    uint32_t s = 0;
-    for (uint32_t i = beg; i < end; i++) s += t[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        uint32_t v = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off] : 0u;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint32_t run = part[threadIdx.x] - s;
-    for (uint32_t i = beg; i < end; i++) {
-        uint32_t x = t[i];
-        t[i] = run;
-        run += x;
-    }
-}
-
-// one tile of kScanTile entries per block: 16 consecutive entries per thread
-__global__ __launch_bounds__(kBlock) void k_scan_apply(uint32_t* __restrict__ a, uint32_t total,
-                                                       const uint32_t* __restrict__ tile_off) {
-    __shared__ uint32_t part[kBlock];
-    constexpr int kPer = kScanTile / kBlock;
-    const uint32_t beg = blockIdx.x * kScanTile + threadIdx.x * kPer;
-    uint32_t v[kPer];
-    uint32_t s = 0;
+// Exclusive scan of each digit's counts over the blocks (block d scans row d); the row's
+// total goes to row_total[d].  The scatter adds the digits before its own from the 256
+// totals, so the counts need one launch between histogram and scatter (tile sums, a scan
+// of the sums and their application were three: 16 us of a pass on 2.3 M pairs, all
+// launch and round trip).
+__global__ __launch_bounds__(kBlock) void k_scan_rows(uint32_t* __restrict__ hist, uint32_t nblocks,
+                                                      uint32_t* __restrict__ row_total) {
+    __shared__ uint32_t wsum[kBlock / 64];
+    uint32_t* row = hist + (size_t)blockIdx.x * nblocks;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint32_t run = 0;
+    for (uint32_t b0 = 0; b0 < nblocks; b0 += kBlock) {
+        const uint32_t b = b0 + tid;
+        const uint32_t v = b < nblocks ? row[b] : 0u;
+        uint32_t x = v;
 #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        v[k] = (beg + k < total) ? a[beg + k] : 0u;
-        s += v[k];
-    }
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 1; off < kBlock; off <<= 1) {
-        uint32_t x = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off] : 0u;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d);
+            if (lane >= (uint32_t)d) x += y;
+        }
+        __syncthreads();  // the last round's sums have been read
+        if (lane == 63u) wsum[wave] = x;
         __syncthreads();
-        part[threadIdx.x] += x;
-        __syncthreads();
-    }
-    uint32_t run = tile_off[blockIdx.x] + part[threadIdx.x] - s;
+        uint32_t before = run;
 #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        if (beg + k < total) a[beg + k] = run;
-        run += v[k];
+        for (uint32_t w = 0; w < kBlock / 64; w++) {
+            if (w < wave) before += wsum[w];
+            run += wsum[w];
+        }
+        if (b < nblocks) row[b] = before + x - v;
     }
+    if (tid == 0) row_total[blockIdx.x] = run;
 }
 
 // Scatter of one radix pass.  The block's tile (kSortTile pairs) is first ordered by
@@ -320,6 +316,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
                                                           uint32_t* __restrict__ vout, uint32_t n,
                                                           int shift,
                                                           const uint32_t* __restrict__ offs,
+                                                          const uint32_t* __restrict__ row_total,
                                                           uint32_t nblocks) {
     constexpr int kWaves = kBlock / 64;
     constexpr uint32_t kWaveItems = kSortTile / kWaves;  // consecutive pairs per wave
@@ -333,9 +330,22 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x * kSortTile;
     const uint32_t m = min((uint32_t)kSortTile, n - tile);
-    gbase[tid] = offs[(size_t)tid * nblocks + blockIdx.x];
+    // this block's first output slot of digit tid: the digits before it, then its row
+    const uint32_t dtot = row_total[tid];
+    uint32_t dincl = dtot;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t x = __shfl_up(dincl, off);
+        if (lane >= off) dincl += x;
+    }
+    if (lane == 63) wsum[wave] = dincl;
     for (int w = 0; w < kWaves; w++) wcnt[w][tid] = 0;
     __syncthreads();
+    {
+        uint32_t base = dincl - dtot + offs[(size_t)tid * nblocks + blockIdx.x];
+        for (int w = 0; w < wave; w++) base += wsum[w];
+        gbase[tid] = base;
+    }
     uint32_t* const mycnt = wcnt[wave];
     const uint32_t wbase = (uint32_t)wave * kWaveItems;
     const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
@@ -404,28 +414,124 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
     }
 }
 
+// Up to kSmallSort pairs are sorted by one block in LDS, all passes in one launch: a pass
+// over two tiles is five launches' latency (108 us of a 5 K triangle build for its four).
+// Wave w holds pairs [512 w, 512 w + 512), 8 per lane, and ranks them as k_radix_scatter.
+constexpr uint32_t kSmallSort = 8192;
+constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64, kSmallItems = kSmallSort / kSmallThreads;
+
+__global__ __launch_bounds__(kSmallThreads) void k_sort_small(const uint64_t* __restrict__ kin,
+                                                              const uint32_t* __restrict__ vin,
+                                                              uint64_t* __restrict__ kout,
+                                                              uint32_t* __restrict__ vout, uint32_t n,
+                                                              int key_bits) {
+    __shared__ uint64_t skey[kSmallSort];
+    __shared__ uint32_t sval[kSmallSort];
+    __shared__ uint32_t wcnt[kSmallWaves][256];
+    __shared__ uint32_t wsum[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+    const uint32_t wbase = (uint32_t)wave * 64u * kSmallItems;
+    uint64_t key[kSmallItems];
+    uint32_t val[kSmallItems], rank[kSmallItems];
+#pragma unroll
+    for (int r = 0; r < kSmallItems; r++) {
+        const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
+        key[r] = i < n ? kin[i] : 0ull;
+        val[r] = i < n ? vin[i] : 0u;
+    }
+    for (int shift = 0; shift < key_bits; shift += 8) {
+        for (int k = tid; k < kSmallWaves * 256; k += kSmallThreads) wcnt[k >> 8][k & 255] = 0;
+        __syncthreads();
+        uint32_t* const mycnt = wcnt[wave];
+#pragma unroll
+        for (int r = 0; r < kSmallItems; r++) {
+            const bool valid = wbase + (uint32_t)r * 64u + (uint32_t)lane < n;
+            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+            uint64_t peers = __ballot(valid);
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const uint64_t bb = __ballot((d >> b) & 1u);
+                peers &= ((d >> b) & 1u) ? bb : ~bb;
+            }
+            const uint32_t rk = (uint32_t)__popcll(peers & lt_mask);
+            const uint32_t before = mycnt[d];
+            rank[r] = before + rk;
+            if (valid && rk == 0) mycnt[d] = before + (uint32_t)__popcll(peers);
+        }
+        __syncthreads();
+        // first slot of every (digit, wave): scan over the digits by the first 256 threads
+        uint32_t tot = 0, incl = 0;
+        if (tid < 256) {
+            for (int w = 0; w < kSmallWaves; w++) tot += wcnt[w][tid];
+            incl = tot;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t x = __shfl_up(incl, off);
+                if (lane >= off) incl += x;
+            }
+            if (lane == 63) wsum[wave] = incl;
+        }
+        __syncthreads();
+        if (tid < 256) {
+            uint32_t start = incl - tot;
+            for (int w = 0; w < wave; w++) start += wsum[w];
+            for (int w = 0; w < kSmallWaves; w++) {
+                const uint32_t c = wcnt[w][tid];
+                wcnt[w][tid] = start;
+                start += c;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSmallItems; r++) {
+            if (wbase + (uint32_t)r * 64u + (uint32_t)lane < n) {
+                const uint32_t pos = mycnt[(uint32_t)(key[r] >> shift) & 255u] + rank[r];
+                skey[pos] = key[r];
+                sval[pos] = val[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSmallItems; r++) {
+            const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
+            if (i < n) {
+                key[r] = skey[i];
+                val[r] = sval[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kSmallItems; r++) {
+        const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
+        if (i < n) {
+            kout[i] = key[r];
+            vout[i] = val[r];
+        }
+    }
+}
+
 size_t radix_sort_scratch_words(uint32_t n) {
-    const uint32_t nblocks = cdiv(n, kSortTile);
-    return 256 * (size_t)nblocks + cdiv(256 * (size_t)nblocks, kScanTile);
+    return 256 * (size_t)cdiv(n, kSortTile) + 256;
 }
 
 bool radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint32_t n, int key_bits,
                       uint32_t* scratch, hipStream_t s) {
+    if (n <= kSmallSort) {
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kSmallThreads), 0, s, k0, v0, k1, v1, n, key_bits);
+        return true;
+    }
     const uint32_t nblocks = cdiv(n, kSortTile);
     uint32_t* hist = scratch;  // 256 digit counts per block, digit-major
-    uint32_t* scan_tmp = scratch + 256 * (size_t)nblocks;
-    const uint32_t hist_n = 256u * nblocks;
-    const unsigned scan_tiles = cdiv(hist_n, kScanTile);
+    uint32_t* totals = scratch + 256 * (size_t)nblocks;
     uint64_t *kin = k0, *kout = k1;
     uint32_t *vin = v0, *vout = v1;
     bool in1 = false;
     for (int shift = 0; shift < key_bits; shift += 8) {
         hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kBlock), 0, s, kin, n, shift, hist, nblocks);
-        hipLaunchKernelGGL(k_scan_tiles, dim3(scan_tiles), dim3(kBlock), 0, s, hist, hist_n, scan_tmp);
-        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, scan_tmp, scan_tiles);
-        hipLaunchKernelGGL(k_scan_apply, dim3(scan_tiles), dim3(kBlock), 0, s, hist, hist_n, scan_tmp);
+        hipLaunchKernelGGL(k_scan_rows, dim3(256), dim3(kBlock), 0, s, hist, nblocks, totals);
         hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kBlock), 0, s, kin, vin, kout, vout, n, shift, hist,
-                           nblocks);
+                           totals, nblocks);
         std::swap(kin, kout);
         std::swap(vin, vout);
         in1 = !in1;
@@ -493,15 +599,9 @@ __device__ __forceinline__ int kdelta(const uint64_t* __restrict__ k, int n, int
 // binary references: internal node i -> i; leaf (sorted primitive p) -> kLeafBit | p
 __global__ __launch_bounds__(kBlock) void k_karras(int N, const uint64_t* __restrict__ keys,
                                                    const SegDesc* __restrict__ segs,
-                                                   uint32_t* __restrict__ left,
-                                                   uint32_t* __restrict__ right,
-                                                   uint2* __restrict__ range,
-                                                   uint32_t* __restrict__ node_parent,
-                                                   uint32_t* __restrict__ leaf_parent,
+                                                   uint2* __restrict__ kids, uint2* __restrict__ range,
                                                    uint32_t* __restrict__ seg_root,
-                                                   uint8_t* __restrict__ is_root,
-                                                   uint8_t* __restrict__ dlev,
-                                                   uint32_t* __restrict__ cnt) {
+                                                   uint8_t* __restrict__ dlev) {
     int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= N - 1) return;
     int d = (kdelta(keys, N, i, i + 1) - kdelta(keys, N, i, i - 1)) >= 0 ? 1 : -1;
@@ -522,22 +622,14 @@ __global__ __launch_bounds__(kBlock) void k_karras(int N, const uint64_t* __rest
     int first = min(i, j), last = max(i, j);
     uint32_t L = (first == split) ? (kLeafBit | (uint32_t)split) : (uint32_t)split;
     uint32_t R = (last == split + 1) ? (kLeafBit | (uint32_t)(split + 1)) : (uint32_t)(split + 1);
-    left[i] = L;
-    right[i] = R;
+    kids[i] = make_uint2(L, R);
     range[i] = make_uint2((uint32_t)first, (uint32_t)last);
-    cnt[i] = (uint32_t)(last - first + 1);
-    if (L & kLeafBit) leaf_parent[split] = (uint32_t)i;
-    else node_parent[split] = (uint32_t)i;
-    if (R & kLeafBit) leaf_parent[split + 1] = (uint32_t)i;
-    else node_parent[split + 1] = (uint32_t)i;
     uint32_t sf = (uint32_t)(keys[first] >> 30), sl = (uint32_t)(keys[last] >> 30);
-    bool root = false;
     if (sf == sl) {
         const SegDesc sd = segs[sf];
-        root = (uint32_t)first == sd.tri_offset && (uint32_t)last == sd.tri_offset + sd.n_tris - 1u;
+        if ((uint32_t)first == sd.tri_offset && (uint32_t)last == sd.tri_offset + sd.n_tris - 1u)
+            seg_root[sf] = (uint32_t)i;
     }
-    is_root[i] = root ? 1 : 0;
-    if (root) seg_root[sf] = (uint32_t)i;
     // nodes above the mesh roots (their range spans several meshes) belong to no BVH:
     // prefix length 0xFF keeps the box and treelet passes away from them
     dlev[i] = (sf == sl) ? (uint8_t)dnode : (uint8_t)0xFF;
@@ -547,21 +639,14 @@ __global__ __launch_bounds__(kBlock) void k_karras(int N, const uint64_t* __rest
 // internal node boxes and SAH costs
 // ------------------------------------------------------------------------------------
 
-// Internal nodes bucketed by prefix length l (a counting sort, order within a bucket
-// arbitrary), each length split in two: bucket 2l holds the nodes with more than
-// 2 leaf_size triangles, which are the treelet roots, and 2l + 1 the others, so the box
-// pass reads buckets 2l and 2l + 1 and the treelet pass only 2l (it used to load and
-// skip the small roots: two dependent loads per node, which made up most of a launch on
-// the deep levels).  lvl_hist[512] counts, lvl_begin[513] prefix sums, lvl_order the
-// nodes.  Each block counts a contiguous range of nodes in LDS and adds to the global
-// counts once per bucket it saw: with one block per 256 nodes, the same-address device
-// atomics alone took over 1 ms per pass for a 25 M-node batch.  Within a block's range a
-// bucket keeps roughly node order, so the per-level passes read neighbouring nodes.
+// Treelet builds: the internal nodes of more than 2 leaf_size triangles, which are the
+// treelet roots, bucketed by prefix length (a counting sort, order within a bucket
+// arbitrary).  lvl_hist[256] counts, lvl_begin[257] prefix sums, lvl_order the nodes.  Each
+// block counts a contiguous range of nodes in LDS and adds to the global counts once per
+// bucket it saw: with one block per 256 nodes, the same-address device atomics alone took
+// over 1 ms per pass for a 25 M-node batch.  Within a block's range a bucket keeps roughly
+// node order, so the per-level passes read neighbouring nodes.
 constexpr unsigned kLevelBlocks = 1024;
-
-__device__ __forceinline__ uint32_t level_bucket(uint8_t dlev, uint32_t cnt, uint32_t small_max) {
-    return 2u * dlev + (cnt <= small_max ? 1u : 0u);
-}
 
 __device__ __forceinline__ void level_range(int n_int, uint32_t& lo, uint32_t& hi) {
     const uint32_t per = (((uint32_t)n_int + gridDim.x - 1) / gridDim.x + kBlock - 1) / kBlock * kBlock;
@@ -569,61 +654,73 @@ __device__ __forceinline__ void level_range(int n_int, uint32_t& lo, uint32_t& h
     hi = min((uint32_t)n_int, lo + per);
 }
 
-static_assert(kLevelBuckets == 2 * kBlock, "two buckets per thread in the level kernels");
+static_assert(kLevelBuckets == kBlock, "one bucket per thread in the level kernels");
+constexpr uint32_t kNoBucket = 255;  // small nodes and nodes above the mesh roots (0xFF)
+
+__device__ __forceinline__ uint32_t level_bucket(uint8_t dlev, uint2 range, uint32_t small_max) {
+    return range.y - range.x + 1u > small_max ? dlev : kNoBucket;
+}
 
 __global__ __launch_bounds__(kBlock) void k_level_hist(int n_int, const uint8_t* __restrict__ dlev,
-                                                       const uint32_t* __restrict__ cnt, uint32_t small_max,
+                                                       const uint2* __restrict__ range, uint32_t small_max,
                                                        uint32_t* __restrict__ hist) {
     __shared__ uint32_t h[kLevelBuckets];
     h[threadIdx.x] = 0;
-    h[threadIdx.x + kBlock] = 0;
     __syncthreads();
     uint32_t lo, hi;
     level_range(n_int, lo, hi);
-    for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) atomicAdd(&h[level_bucket(dlev[i], cnt[i], small_max)], 1u);
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) {
+        const uint32_t l = level_bucket(dlev[i], range[i], small_max);
+        if (l != kNoBucket) atomicAdd(&h[l], 1u);
+    }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < kLevelBuckets; k += kBlock)
-        if (h[k]) gatomic_add(&hist[k], h[k]);
+    if (h[threadIdx.x]) gatomic_add(&hist[threadIdx.x], h[threadIdx.x]);
 }
 
-__global__ void k_level_scan(const uint32_t* __restrict__ hist, uint32_t* __restrict__ begin,
-                             uint32_t* __restrict__ fill) {
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (uint32_t k = 0; k < kLevelBuckets; k++) {
-            begin[k] = run;
-            fill[k] = run;
-            run += hist[k];
-        }
-        begin[kLevelBuckets] = run;
+__global__ __launch_bounds__(kBlock) void k_level_scan(const uint32_t* __restrict__ hist, uint32_t* __restrict__ begin,
+                                                       uint32_t* __restrict__ fill) {
+    __shared__ uint32_t wsum[kBlock / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t v = hist[tid];
+    uint32_t x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d);
+        if (lane >= (uint32_t)d) x += y;
     }
+    if (lane == 63u) wsum[wave] = x;
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; w++) x += wsum[w];
+    begin[tid] = x - v;
+    fill[tid] = x - v;
+    if (tid == kBlock - 1) begin[kBlock] = x;
 }
 
 __global__ __launch_bounds__(kBlock) void k_level_scatter(int n_int, const uint8_t* __restrict__ dlev,
-                                                          const uint32_t* __restrict__ cnt, uint32_t small_max,
+                                                          const uint2* __restrict__ range, uint32_t small_max,
                                                           uint32_t* __restrict__ fill,
                                                           uint32_t* __restrict__ order) {
     __shared__ uint32_t h[kLevelBuckets], base[kLevelBuckets];
     h[threadIdx.x] = 0;
-    h[threadIdx.x + kBlock] = 0;
     __syncthreads();
     uint32_t lo, hi;
     level_range(n_int, lo, hi);
-    for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) atomicAdd(&h[level_bucket(dlev[i], cnt[i], small_max)], 1u);
-    __syncthreads();
-    // reserve this block's part of every bucket, then place its nodes there
-    for (uint32_t k = threadIdx.x; k < kLevelBuckets; k += kBlock) {
-        base[k] = h[k] ? gatomic_add(&fill[k], h[k]) : 0u;
-        h[k] = 0;
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) {
+        const uint32_t l = level_bucket(dlev[i], range[i], small_max);
+        if (l != kNoBucket) atomicAdd(&h[l], 1u);
     }
     __syncthreads();
+    // reserve this block's part of every bucket, then place its nodes there
+    base[threadIdx.x] = h[threadIdx.x] ? gatomic_add(&fill[threadIdx.x], h[threadIdx.x]) : 0u;
+    h[threadIdx.x] = 0;
+    __syncthreads();
     for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) {
-        const uint32_t l = level_bucket(dlev[i], cnt[i], small_max);
-        order[base[l] + atomicAdd(&h[l], 1u)] = i;
+        const uint32_t l = level_bucket(dlev[i], range[i], small_max);
+        if (l != kNoBucket) order[base[l] + atomicAdd(&h[l], 1u)] = i;
     }
 }
 
-// Node boxes without atomics or fences, in two parts.
+// Node boxes without atomics, fences or an order between launches.
 //
 // k_boxes_local: block c owns internal nodes [256c, 256c + 256).  A node whose leaf range
 // lies in one such chunk has its whole subtree there (a Karras node's index is an end of
@@ -632,105 +729,229 @@ __global__ __launch_bounds__(kBlock) void k_level_scatter(int n_int, const uint8
 // merges their boxes, with the chunk's boxes and costs kept in LDS (its own global writes
 // are not read back, so no cache can hand a lane a stale box) until no node is left.  A
 // round always finishes the deepest pending node, so the loop ends.  This covers ~90% of
-// the nodes in one launch.
+// the nodes.
+//
+// The others (ranges across chunks) are unions over their leaf range.  The leaves' boxes
+// are merged in aligned blocks of 4, 16, 64, ... leaves (rbox, level after level: the
+// local pass makes the blocks up to its chunk, k_range_top the rest), and k_boxes_cross
+// covers a node's range with at most 6 blocks per level.  Minima and maxima are exact, so
+// the boxes are the ones a bottom-up pass gives; one launch per prefix length in use (43 to
+// 61 of them) gave them before: 110 us of GPU time and 40 launches' gaps in a 5 K triangle
+// build, 235 us at 2.3 M, 390 us in a 7 M triangle batch.
 __device__ __forceinline__ bool box_in_chunk(uint2 r) { return (r.x >> 8) == (r.y >> 8); }
 static_assert(kBlock == 256, "k_boxes_local chunks are 256 nodes");
 
-__global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, const uint2* __restrict__ range,
-                                                        const uint32_t* __restrict__ left,
-                                                        const uint32_t* __restrict__ right,
-                                                        const uint32_t* __restrict__ cnt,
+__device__ __forceinline__ void write_bnode(float4* __restrict__ bnode, uint32_t i, float4 lo, float4 hi, uint2 kid,
+                                            uint2 range, float cost) {
+    lo.w = __uint_as_float(kid.x);
+    hi.w = __uint_as_float(kid.y);
+    bnode[3 * (size_t)i] = lo;
+    bnode[3 * (size_t)i + 1] = hi;
+    bnode[3 * (size_t)i + 2] = make_float4(__uint_as_float(range.y - range.x + 1u), cost, __uint_as_float(range.x), 0.0f);
+}
+
+__device__ __forceinline__ float4 min4(float4 a, float4 b) {
+    return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.0f);
+}
+__device__ __forceinline__ float4 max4(float4 a, float4 b) {
+    return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z), 0.0f);
+}
+__device__ __forceinline__ float4 shfl_xor4(float4 v, int o) {
+    return make_float4(__shfl_xor(v.x, o), __shfl_xor(v.y, o), __shfl_xor(v.z, o), 0.0f);
+}
+
+__global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t N, const uint2* __restrict__ range,
+                                                        const uint2* __restrict__ kids,
                                                         const uint8_t* __restrict__ dlev,
                                                         const float4* __restrict__ saabb,
-                                                        float4* __restrict__ nbox, float* __restrict__ cost,
+                                                        float4* __restrict__ bnode, float4* __restrict__ rbox,
                                                         int leaf_size) {
+    __shared__ float4 slo[kBlock], shi[kBlock];  // the chunk's leaf boxes
     __shared__ float4 blo[kBlock], bhi[kBlock];
     __shared__ float bcost[kBlock];
     __shared__ uint8_t done[kBlock];
-    const uint32_t c0 = blockIdx.x * kBlock;
-    const uint32_t i = c0 + threadIdx.x;
+    const uint32_t c0 = blockIdx.x * kBlock, tid = threadIdx.x;
+    const uint32_t i = c0 + tid;
     bool todo = false;
     uint32_t L = 0, R = 0;
+    uint2 rg = make_uint2(0u, 0u);
     if (i < n_int && dlev[i] != 0xFF) {
-        todo = box_in_chunk(range[i]);
-        L = left[i];
-        R = right[i];
+        rg = range[i];
+        todo = box_in_chunk(rg);
+        const uint2 k = kids[i];
+        L = k.x;
+        R = k.y;
     }
-    done[threadIdx.x] = 0;
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    if (i < N) {
+        lo = saabb[2 * (size_t)i];
+        hi = saabb[2 * (size_t)i + 1];
+    }
+    slo[tid] = lo;
+    shi[tid] = hi;
+    done[tid] = 0;
+    // aligned blocks of 4, 16, 64 leaves and the chunk
+    if (rbox) {
+        float4* at = rbox;
+        uint32_t cnt = N;
+        for (int lvl = 1; lvl <= 3; lvl++) {
+            const int o = 1 << (2 * (lvl - 1));
+            lo = min4(lo, shfl_xor4(lo, o));
+            hi = max4(hi, shfl_xor4(hi, o));
+            lo = min4(lo, shfl_xor4(lo, 2 * o));
+            hi = max4(hi, shfl_xor4(hi, 2 * o));
+            cnt = (cnt + 3) / 4;
+            const uint32_t e = i >> (2 * lvl);
+            if ((tid & (4u * o - 1u)) == 0 && e < cnt) {
+                at[2 * (size_t)e] = lo;
+                at[2 * (size_t)e + 1] = hi;
+            }
+            at += 2 * (size_t)cnt;
+        }
+        if ((tid & 63u) == 0) {
+            blo[tid >> 6] = lo;
+            bhi[tid >> 6] = hi;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            at[2 * (size_t)blockIdx.x] = min4(min4(blo[0], blo[1]), min4(blo[2], blo[3]));
+            at[2 * (size_t)blockIdx.x + 1] = max4(max4(bhi[0], bhi[1]), max4(bhi[2], bhi[3]));
+        }
+    }
     __syncthreads();
     while (__syncthreads_or(todo)) {
         const bool ready = todo && ((L & kLeafBit) || done[L - c0]) && ((R & kLeafBit) || done[R - c0]);
-        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
         float c = 0.f;
         if (ready) {
-            float4 al, ah, bl, bh;
-            float cl, cr;
-            if (L & kLeafBit) {
-                const size_t p = L & ~kLeafBit;
-                al = saabb[2 * p];
-                ah = saabb[2 * p + 1];
-                cl = kCt * box_area(al, ah);
-            } else {
-                al = blo[L - c0];
-                ah = bhi[L - c0];
-                cl = bcost[L - c0];
-            }
-            if (R & kLeafBit) {
-                const size_t p = R & ~kLeafBit;
-                bl = saabb[2 * p];
-                bh = saabb[2 * p + 1];
-                cr = kCt * box_area(bl, bh);
-            } else {
-                bl = blo[R - c0];
-                bh = bhi[R - c0];
-                cr = bcost[R - c0];
-            }
-            lo = make_float4(fminf(al.x, bl.x), fminf(al.y, bl.y), fminf(al.z, bl.z), 0.0f);
-            hi = make_float4(fmaxf(ah.x, bh.x), fmaxf(ah.y, bh.y), fmaxf(ah.z, bh.z), 0.0f);
-            c = sah_node_cost(lo, hi, cnt[i], cl, cr, leaf_size);
+            // a leaf of an in-chunk node lies in the chunk
+            const uint32_t l = (L & ~kLeafBit) - c0, r = (R & ~kLeafBit) - c0;
+            const bool ll = (L & kLeafBit) != 0u, rl = (R & kLeafBit) != 0u;
+            const float4 al = ll ? slo[l] : blo[l], ah = ll ? shi[l] : bhi[l];
+            const float4 bl = rl ? slo[r] : blo[r], bh = rl ? shi[r] : bhi[r];
+            const float cl = ll ? kCt * box_area(al, ah) : bcost[l], cr = rl ? kCt * box_area(bl, bh) : bcost[r];
+            lo = min4(al, bl);
+            hi = max4(ah, bh);
+            c = sah_node_cost(lo, hi, rg.y - rg.x + 1u, cl, cr, leaf_size);
         }
         __syncthreads();  // every read of this round before any write
         if (ready) {
-            blo[threadIdx.x] = lo;
-            bhi[threadIdx.x] = hi;
-            bcost[threadIdx.x] = c;
-            done[threadIdx.x] = 1;
-            nbox[2 * (size_t)i] = lo;
-            nbox[2 * (size_t)i + 1] = hi;
-            cost[i] = c;
+            blo[tid] = lo;
+            bhi[tid] = hi;
+            bcost[tid] = c;
+            done[tid] = 1;
+            write_bnode(bnode, i, lo, hi, make_uint2(L, R), rg, c);
             todo = false;
         }
     }
 }
 
-// k_boxes_level: the remaining nodes (ranges across chunks).  A child's common-prefix
-// length (Karras' delta of its range) is strictly greater than its parent's, so
-// launching once per delta value from the largest down makes every child box final
-// before its parent reads it.
-__global__ __launch_bounds__(kBlock) void k_boxes_level(int level, const uint32_t* __restrict__ lvl_begin,
-                                                        const uint32_t* __restrict__ lvl_order,
-                                                        const uint2* __restrict__ range,
-                                                        const uint32_t* __restrict__ left,
-                                                        const uint32_t* __restrict__ right,
-                                                        const uint32_t* __restrict__ cnt,
-                                                        const float4* __restrict__ saabb,
-                                                        float4* __restrict__ nbox, float* __restrict__ cost,
-                                                        int leaf_size) {
-    const uint32_t beg = lvl_begin[2 * level], end = lvl_begin[2 * level + 2];  // both size buckets
-    const uint32_t stride = gridDim.x * kBlock;
-    for (uint32_t k = beg + blockIdx.x * kBlock + threadIdx.x; k < end; k += stride) {
-        const uint32_t i = lvl_order[k];
-        if (box_in_chunk(range[i])) continue;  // done by k_boxes_local
-        float4 al, ah, bl, bh;
-        const uint32_t L = left[i], R = right[i];
-        ref_box(L, saabb, nbox, al, ah);
-        ref_box(R, saabb, nbox, bl, bh);
-        const float4 lo = make_float4(fminf(al.x, bl.x), fminf(al.y, bl.y), fminf(al.z, bl.z), 0.0f);
-        const float4 hi = make_float4(fmaxf(ah.x, bh.x), fmaxf(ah.y, bh.y), fmaxf(ah.z, bh.z), 0.0f);
-        nbox[2 * (size_t)i] = lo;
-        nbox[2 * (size_t)i + 1] = hi;
-        cost[i] = sah_node_cost(lo, hi, cnt[i], ref_cost(L, saabb, cost), ref_cost(R, saabb, cost), leaf_size);
+// The aligned blocks above the chunks, level by level: one block of threads for all levels
+// (they hold a 768th of the leaf count in all), so no launch per level.  The level below is
+// read back from this block's own writes.
+__global__ __launch_bounds__(1024) void k_range_top(uint32_t N, float4* rbox) {
+    uint32_t cnt = N;
+    size_t off = 0;
+    for (int lvl = 1; lvl < 4; lvl++) {
+        cnt = (cnt + 3) / 4;
+        off += cnt;
     }
+    cnt = (cnt + 3) / 4;  // the chunks
+    while (cnt > 1) {
+        const uint32_t up = (cnt + 3) / 4;
+        float4* src = rbox + 2 * off;
+        float4* dst = src + 2 * (size_t)cnt;
+        for (uint32_t e = threadIdx.x; e < up; e += 1024) {
+            float4 lo = src[8 * (size_t)e], hi = src[8 * (size_t)e + 1];
+            for (uint32_t k = 1; k < 4 && 4 * e + k < cnt; k++) {
+                lo = min4(lo, src[2 * (4 * (size_t)e + k)]);
+                hi = max4(hi, src[2 * (4 * (size_t)e + k) + 1]);
+            }
+            dst[2 * (size_t)e] = lo;
+            dst[2 * (size_t)e + 1] = hi;
+        }
+        __threadfence_block();
+        __syncthreads();
+        off += cnt;
+        cnt = up;
+    }
+}
+
+// entries (boxes) of all levels of rbox for N leaves: four levels up to the chunks and
+// those above down to one entry
+static size_t range_boxes(uint32_t N) {
+    size_t total = 0;
+    uint32_t cnt = N;
+    for (int lvl = 1; lvl <= 4 || cnt > 1; lvl++) {
+        cnt = (cnt + 3) / 4;
+        total += cnt;
+    }
+    return total;
+}
+
+// A subtree of at most 2 leaf_size triangles that crosses a chunk: its SAH cost, by a walk
+// (larger nodes' costs are formed by the treelet pass, from their children's).
+__device__ float small_cost(uint32_t root, const uint2* __restrict__ kids, const uint2* __restrict__ range,
+                            const float4* __restrict__ saabb, int leaf_size) {
+    float c = 0.0f;
+    uint32_t stack[16];
+    int sp = 0;
+    stack[sp++] = root;
+    while (sp > 0) {
+        const uint32_t r = stack[--sp];
+        const bool leaf = (r & kLeafBit) != 0u;
+        const uint2 rg = leaf ? make_uint2(r & ~kLeafBit, r & ~kLeafBit) : range[r];
+        float4 lo = saabb[2 * (size_t)rg.x], hi = saabb[2 * (size_t)rg.x + 1];
+        for (uint32_t p = rg.x + 1; p <= rg.y; p++) {
+            lo = min4(lo, saabb[2 * (size_t)p]);
+            hi = max4(hi, saabb[2 * (size_t)p + 1]);
+        }
+        const uint32_t n = rg.y - rg.x + 1u;
+        if (n <= (uint32_t)leaf_size) {
+            c += kCt * box_area(lo, hi) * (float)n;
+        } else {
+            c += kCi * box_area(lo, hi);
+            if (sp + 2 <= 16) {
+                const uint2 k = kids[r];
+                stack[sp++] = k.y;
+                stack[sp++] = k.x;
+            }
+        }
+    }
+    return c;
+}
+
+__global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t n_int, uint32_t N, const uint2* __restrict__ range,
+                                                        const uint2* __restrict__ kids,
+                                                        const uint8_t* __restrict__ dlev,
+                                                        const float4* __restrict__ saabb,
+                                                        const float4* __restrict__ rbox, float4* __restrict__ bnode,
+                                                        int leaf_size, int costs) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n_int || dlev[i] == 0xFF) return;
+    const uint2 rg = range[i];
+    if (box_in_chunk(rg)) return;  // done by k_boxes_local
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    const float4* at = saabb;  // the level's boxes
+    uint32_t l = rg.x, r = rg.y + 1u, cnt = N;
+    while (l < r) {
+        // the blocks left and right of the next level's
+        const uint32_t l4 = min((l + 3u) & ~3u, r), r4 = max(r & ~3u, l4);
+        for (uint32_t k = l; k < l4; k++) {
+            lo = min4(lo, at[2 * (size_t)k]);
+            hi = max4(hi, at[2 * (size_t)k + 1]);
+        }
+        for (uint32_t k = r4; k < r; k++) {
+            lo = min4(lo, at[2 * (size_t)k]);
+            hi = max4(hi, at[2 * (size_t)k + 1]);
+        }
+        at = at == saabb ? rbox : at + 2 * (size_t)cnt;
+        cnt = (cnt + 3) / 4;
+        l = l4 / 4;
+        r = r4 / 4;
+    }
+    float c = 0.0f;
+    if (costs && rg.y - rg.x + 1u <= 2u * (uint32_t)leaf_size) c = small_cost(i, kids, range, saabb, leaf_size);
+    write_bnode(bnode, i, lo, hi, kids[i], rg, c);
 }
 
 // ------------------------------------------------------------------------------------
@@ -738,58 +959,55 @@ __global__ __launch_bounds__(kBlock) void k_boxes_level(int level, const uint32_
 // ------------------------------------------------------------------------------------
 
 struct CollapseArgs {
-    const uint32_t* left;
-    const uint32_t* right;
-    const uint2* range;
-    const uint32_t* cnt;  // triangles under each internal node
+    const float4* bnode;  // binary nodes (build_common.h)
     const float4* saabb;
-    const float4* nbox;
     const uint32_t* segstat;
     uint32_t* wsrc;  // wide node -> binary ref
     uint32_t* wseg;  // wide node -> mesh
+    uint32_t* wfirst;  // wide node -> first packed triangle of its range
     uint32_t* lvl_cnt;
-    uint32_t* counters;  // [0] wide nodes allocated, [1] error bits, [2] triangles re-packed
+    uint32_t* counters;  // [0] wide nodes allocated, [1] error bits
     void* nodes;
     uint32_t capacity;
     int leaf_size;
     int level;
     // re-pack (after treelet restructuring a leaf's triangles are no longer one sorted
-    // range): leaves get fresh contiguous slots and their triangles are copied there
+    // range): a node's range is dealt to its children in slot order, so every subtree's
+    // triangles are contiguous again; perm[slot] = sorted position, gathered by k_repack
     int repack;
-    const float4* tris_in;
-    const uint32_t* order_in;
-    float4* tris_out;
-    uint32_t* order_out;
+    uint32_t* perm;
 };
 
-__device__ __forceinline__ uint32_t ref_count(uint32_t r, const uint32_t* cnt) {
-    return (r & kLeafBit) ? 1u : cnt[r];
-}
-__device__ __forceinline__ uint32_t ref_first(uint32_t r, const uint2* range) {
-    if (r & kLeafBit) return r & ~kLeafBit;
-    return range[r].x;
-}
-
-// Copies the <= leaf_size triangles under binary ref r to the slots from `base`.
-__device__ void repack_leaf(const CollapseArgs& a, uint32_t r, uint32_t base) {
+// The sorted positions of the <= leaf_size triangles under binary ref r, to slots from `out`.
+__device__ void list_leaf(const CollapseArgs& a, uint32_t r, uint32_t out) {
     uint32_t stack[8];
     int sp = 0;
-    uint32_t out = base;
     stack[sp++] = r;
     while (sp > 0) {
         const uint32_t x = stack[--sp];
         if (x & kLeafBit) {
-            const size_t p = x & ~kLeafBit;
-            a.tris_out[3 * (size_t)out] = a.tris_in[3 * p];
-            a.tris_out[3 * (size_t)out + 1] = a.tris_in[3 * p + 1];
-            a.tris_out[3 * (size_t)out + 2] = a.tris_in[3 * p + 2];
-            a.order_out[out] = a.order_in[p];
-            out++;
+            a.perm[out++] = x & ~kLeafBit;
         } else if (sp + 2 <= 8) {
-            stack[sp++] = a.right[x];
-            stack[sp++] = a.left[x];
+            stack[sp++] = __float_as_uint(a.bnode[3 * (size_t)x + 1].w);
+            stack[sp++] = __float_as_uint(a.bnode[3 * (size_t)x].w);
         }
     }
+}
+
+// Triangles copied to their slots after all leaves have theirs: a thread per float4, so the
+// writes are contiguous (copied inside the collapse, a node's 16 triangles one after the
+// other were most of its 730 us on 2.3 M triangles).
+__global__ __launch_bounds__(kBlock) void k_repack(uint32_t N, const uint32_t* __restrict__ perm,
+                                                   const float4* __restrict__ tris_in,
+                                                   const uint32_t* __restrict__ order_in,
+                                                   float4* __restrict__ tris_out,
+                                                   uint32_t* __restrict__ order_out) {
+    const size_t k = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (k >= 3 * (size_t)N) return;
+    const uint32_t out = (uint32_t)(k / 3), v = (uint32_t)(k - 3 * (size_t)out);
+    const uint32_t in = perm[out];
+    tris_out[k] = tris_in[3 * (size_t)in + v];
+    if (v == 0) order_out[out] = order_in[in];
 }
 
 // Wave-aggregated allocation: each lane asks for n slots of *counter (any lane may ask
@@ -811,59 +1029,70 @@ __device__ __forceinline__ uint32_t wave_alloc(uint32_t* counter, uint32_t n, ui
     return base + x - n;
 }
 
+// Collapses nodes [begin, begin + cnt) of level `level`, dealt to the grid's threads; all
+// 64 lanes of a wave call it together.
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
-    // the graph of a batch launches every possible level: most are empty or small, so
-    // surplus blocks leave before anything else
-    const uint32_t cnt = a.lvl_cnt[a.level];
-    if (blockIdx.x * kBlock >= cnt) return;
-    uint32_t begin = 0;
-    for (int l = 0; l < a.level; l++) begin += a.lvl_cnt[l];
+__device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level, uint32_t begin, uint32_t cnt) {
     WNode<W>* nodes = reinterpret_cast<WNode<W>*>(a.nodes);
     // every lane runs every iteration (slot allocation is wave-wide); lanes past the
     // level's end take part with nothing to allocate
-    for (uint32_t k0 = blockIdx.x * kBlock; k0 < cnt; k0 += gridDim.x * kBlock) {
+    for (uint32_t k0 = blockIdx.x * blockDim.x; k0 < cnt; k0 += gridDim.x * blockDim.x) {
         const uint32_t k = k0 + threadIdx.x;
         const bool act = k < cnt;
         uint32_t wi = begin + (act ? k : 0u);
         uint32_t bref = a.wsrc[wi];
         uint32_t seg = a.wseg[wi];
+        uint32_t run = a.wfirst[wi];
         float pad = o2f(a.segstat[seg * kStat + 6]) * 0x1p-18f;
         // The wide node's children, kept in registers with their triangle counts and
-        // boxes: a child is loaded once, together with its own children when it is an
-        // internal node, so opening it (the child with the largest area among those with
-        // more than leaf_size triangles, the lowest slot on ties) costs one round of
-        // loads instead of re-reading every child's count and box.  Slots are addressed
-        // with compile-time indices only, so nothing spills to scratch.
-        uint32_t refs[W], rc[W], rl[W], rr[W];
+        // boxes: a child is loaded once, with its own children when it is an internal
+        // node (one 48-byte record), so opening it (the child with the largest area among
+        // those with more than leaf_size triangles, the lowest slot on ties) costs one
+        // round of loads instead of re-reading every child's count and box.  Slots are
+        // addressed with compile-time indices only, so nothing spills to scratch.
+        uint32_t refs[W], rc[W], rf[W], rl[W], rr[W];
         float4 rlo[W], rhi[W];
         float rar[W];
-        auto load_child = [&](uint32_t r, uint32_t& ref, uint32_t& c, uint32_t& l, uint32_t& rgt, float4& lo,
-                              float4& hi, float& ar) {
+        auto load_child = [&](uint32_t r, uint32_t& ref, uint32_t& c, uint32_t& first, uint32_t& l, uint32_t& rgt,
+                              float4& lo, float4& hi, float& ar) {
             ref = r;
-            c = ref_count(r, a.cnt);
-            ref_box(r, a.saabb, a.nbox, lo, hi);
             const bool internal = !(r & kLeafBit);
-            l = internal ? a.left[r] : 0u;
-            rgt = internal ? a.right[r] : 0u;
+            if (internal) {
+                const float4* p = a.bnode + 3 * (size_t)r;
+                lo = p[0];
+                hi = p[1];
+                const float4 x = p[2];
+                l = __float_as_uint(lo.w);
+                rgt = __float_as_uint(hi.w);
+                c = __float_as_uint(x.x);
+                first = __float_as_uint(x.z);
+            } else {
+                const size_t p = r & ~kLeafBit;
+                lo = a.saabb[2 * p];
+                hi = a.saabb[2 * p + 1];
+                l = rgt = 0u;
+                c = 1u;
+                first = (uint32_t)p;
+            }
             ar = c > (uint32_t)a.leaf_size ? box_area(lo, hi) : -1.0f;
         };
         int n = 0;
         if (!act) {
             // nothing: n stays 0
         } else {
-            uint32_t bc, bl, br;
+            uint32_t bc, bf, bl, br;
             float4 blo, bhi;
             float bar;
-            load_child(bref, refs[0], bc, bl, br, blo, bhi, bar);
+            load_child(bref, refs[0], bc, bf, bl, br, blo, bhi, bar);
             if (bc <= (uint32_t)a.leaf_size) {
                 rc[0] = bc;
+                rf[0] = bf;
                 rlo[0] = blo;
                 rhi[0] = bhi;
                 n = 1;
             } else {
-                load_child(bl, refs[0], rc[0], rl[0], rr[0], rlo[0], rhi[0], rar[0]);
-                load_child(br, refs[1], rc[1], rl[1], rr[1], rlo[1], rhi[1], rar[1]);
+                load_child(bl, refs[0], rc[0], rf[0], rl[0], rr[0], rlo[0], rhi[0], rar[0]);
+                load_child(br, refs[1], rc[1], rf[1], rl[1], rr[1], rlo[1], rhi[1], rar[1]);
                 n = 2;
                 while (n < W) {
                     int best = -1;
@@ -886,44 +1115,31 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
                     }
 #pragma unroll
                     for (int j = 0; j < W; j++) {
-                        if (j == best) load_child(ol, refs[j], rc[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
-                        if (j == n) load_child(orr, refs[j], rc[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
+                        if (j == best) load_child(ol, refs[j], rc[j], rf[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
+                        if (j == n) load_child(orr, refs[j], rc[j], rf[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
                     }
                     n++;
                 }
             }
         }
         WNode<W> out;
-        uint32_t n_internal = 0, n_repack = 0;
+        uint32_t n_internal = 0;
+#pragma unroll
+        for (int j = 0; j < W; j++)
+            if (j < n && rc[j] > (uint32_t)a.leaf_size) n_internal++;
 #pragma unroll
         for (int j = 0; j < W; j++) {
             if (j < n) {
-                const uint32_t c = rc[j];
-                if (c <= (uint32_t)a.leaf_size) n_repack += c;
-                else n_internal++;
-            }
-        }
-        uint32_t wave_total = 0;
-        uint32_t rp = a.repack ? wave_alloc(&a.counters[2], n_repack, wave_total) : 0u;
-#pragma unroll
-        for (int j = 0; j < W; j++) {
-            if (j < n) {
-                const uint32_t r = refs[j];
                 const float4 lo = rlo[j], hi = rhi[j];
                 out.lox[j] = lo.x - pad; out.loy[j] = lo.y - pad; out.loz[j] = lo.z - pad;
                 out.hix[j] = hi.x + pad; out.hiy[j] = hi.y + pad; out.hiz[j] = hi.z + pad;
                 const uint32_t c = rc[j];
                 out.aux[j] = c;
+                if (a.repack) rf[j] = run;
+                run += c;
                 if (c <= (uint32_t)a.leaf_size) {
-                    uint32_t first;
-                    if (a.repack) {
-                        repack_leaf(a, r, rp);
-                        first = rp;
-                        rp += c;
-                    } else {
-                        first = ref_first(r, a.range);
-                    }
-                    out.child[j] = make_leaf(first, c);
+                    if (a.repack) list_leaf(a, refs[j], rf[j]);
+                    out.child[j] = make_leaf(rf[j], c);
                 }
             } else {
                 out.lox[j] = out.loy[j] = out.loz[j] = INFINITY;
@@ -932,8 +1148,9 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
                 out.aux[j] = 0;
             }
         }
+        uint32_t wave_total = 0;
         const uint32_t base = wave_alloc(&a.counters[0], n_internal, wave_total);
-        if ((threadIdx.x & 63u) == 63u && wave_total) gatomic_add(&a.lvl_cnt[a.level + 1], wave_total);
+        if ((threadIdx.x & 63u) == 63u && wave_total) gatomic_add(&a.lvl_cnt[level + 1], wave_total);
         if (n_internal) {
             uint32_t m = 0;
 #pragma unroll
@@ -943,6 +1160,7 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
                     if (idx < a.capacity) {
                         a.wsrc[idx] = refs[j];
                         a.wseg[idx] = seg;
+                        a.wfirst[idx] = rf[j];
                         out.child[j] = idx;
                     } else {
                         gatomic_or(&a.counters[1], 2u);
@@ -955,14 +1173,51 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
     }
 }
 
-// SAH cost of a finished wide tree: sum over nodes of kCi * area for internal children
-// and kCt * count * area for leaves, accumulated in double per wave then atomically.
+// One wide level per launch: each reads the nodes that the one before it allocated.
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_sah_cost(uint32_t n_nodes, const WNode<W>* __restrict__ nodes,
-                                                     double* acc) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
+    // launches past the tree's depth find an empty level, and surplus blocks leave before
+    // anything else
+    const uint32_t cnt = a.lvl_cnt[a.level];
+    if (blockIdx.x * kBlock >= cnt) return;
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t begin = lane < (uint32_t)a.level ? a.lvl_cnt[lane] : 0u;
+    for (int o = 32; o > 0; o >>= 1) begin += __shfl_xor(begin, o);
+    collapse_level<W>(a, a.level, begin, cnt);
+}
+static_assert(kMaxLevels <= 64, "k_collapse sums the levels before its own with one wave");
+
+// The levels from a.level on, by one block: the few nodes of levels that trees of ordinary
+// depth do not reach (a launch each would be 40 empty launches per batch replay).  The
+// counts are read past the L1, where the atomics left them.
+template <int W>
+__global__ __launch_bounds__(1024) void k_collapse_tail(CollapseArgs a) {
+    auto count = [&](int l) {
+        return __hip_atomic_load((global_u32*)(a.lvl_cnt + l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    uint32_t begin = 0;
+    for (int l = 0; l < a.level; l++) begin += count(l);
+    for (int l = a.level; l < kMaxLevels; l++) {
+        const uint32_t cnt = count(l);
+        if (cnt == 0) break;
+        collapse_level<W>(a, l, begin, cnt);
+        begin += cnt;
+        __threadfence_block();
+        __syncthreads();
+    }
+}
+
+// SAH cost of a finished wide tree: sum over nodes of kCi * area for internal children
+// and kCt * count * area for leaves, accumulated in double per block, then atomically (one
+// atomic per block: one per wave was 88 us on 400 K nodes); with it the mesh's scale and
+// the root's box go to the build's report.
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_sah_cost(const WNode<W>* __restrict__ nodes, const float4* __restrict__ bnode,
+                                                     const uint32_t* __restrict__ segstat, uint32_t* report) {
+    __shared__ double part[kBlock / 64];
+    const uint32_t n_nodes = report[kReportCounters];
     double c = 0.0;
-    if (k < n_nodes) {
+    for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < n_nodes; k += gridDim.x * kBlock) {
         const WNode<W>& nd = nodes[k];
 #pragma unroll
         for (int j = 0; j < W; j++) {
@@ -973,16 +1228,29 @@ __global__ __launch_bounds__(kBlock) void k_sah_cost(uint32_t n_nodes, const WNo
         }
     }
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-    if ((threadIdx.x & 63) == 0 && c != 0.0) atomicAdd(acc, c);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        c = 0.0;
+        for (int w = 0; w < kBlock / 64; w++) c += part[w];
+        if (c != 0.0) atomicAdd(reinterpret_cast<double*>(report + kReportSah), c);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 7) {
+        const float* root = reinterpret_cast<const float*>(bnode);  // node 0: lo, left, hi, right
+        report[kReportRoot + threadIdx.x] =
+            threadIdx.x < 6 ? __float_as_uint(root[threadIdx.x < 3 ? threadIdx.x : threadIdx.x + 1]) : segstat[6];
+    }
 }
 
 // level 0 of the wide tree: one node per mesh root
-__global__ void k_init_levels(int n_seg, const uint32_t* __restrict__ seg_root, uint32_t* __restrict__ wsrc,
-                              uint32_t* __restrict__ wseg) {
+__global__ void k_init_levels(int n_seg, const SegDesc* __restrict__ segs, const uint32_t* __restrict__ seg_root,
+                              uint32_t* __restrict__ wsrc, uint32_t* __restrict__ wseg,
+                              uint32_t* __restrict__ wfirst) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n_seg) {
         wsrc[i] = seg_root[i];
         wseg[i] = (uint32_t)i;
+        wfirst[i] = segs[i].tri_offset;
     }
 }
 
@@ -991,63 +1259,58 @@ __global__ void k_init_levels(int n_seg, const uint32_t* __restrict__ seg_root, 
 // ------------------------------------------------------------------------------------
 
 BuildBufs::~BuildBufs() {
-    for (void* p : allocs)
-        if (p) (void)(pooled ? hipFreeAsync(p, pool_stream) : hipFree(p));
-}
-
-void* BuildBufs::release(void* p) {
-    for (auto& a : allocs)
-        if (a == p) a = nullptr;
-    return p;
-}
-
-// All scratch of a build lives in one allocation carved into 256-byte aligned pieces
-// (one hipMalloc instead of ~25); the products handed to a BVH are separate.
-struct Carver {
-    size_t off = 0;
-    char* base = nullptr;
-    template <typename T>
-    void take(T*& p, size_t count) {
-        size_t bytes = std::max<size_t>(count * sizeof(T), 256);
-        off = (off + 255) & ~size_t(255);
-        p = base ? reinterpret_cast<T*>(base + off) : nullptr;
-        off += bytes;
+    for (void* p : allocs) {
+        if (ctx) pool_free(ctx, p, pool_stream);
+        else (void)hipFree(p);
     }
-};
+}
 
+hipError_t BuildBufs::alloc(void** p, size_t bytes) {
+    *p = nullptr;
+    const hipError_t e = ctx ? (pool_alloc(ctx, p, bytes, pool_stream) ? hipErrorOutOfMemory : hipSuccess)
+                             : hipMalloc(p, bytes);
+    if (e == hipSuccess) allocs.push_back(*p);
+    return e;
+}
+
+// All scratch of a build lives in one allocation.
 static void carve_all(BuildBufs& b, Carver& c, size_t NI) {
     const uint32_t N = b.N;
     const int n_seg = b.n_seg;
+    c.take(b.report, kReportWords);
     c.take(b.segs, n_seg);
-    c.take(b.aabb_lo, N);
-    c.take(b.aabb_hi, N);
+    c.take(b.cen, N);
     c.take(b.segstat_rep, (size_t)kStat * n_seg * kRep);
     c.take(b.segstat, (size_t)kStat * n_seg);
     c.take(b.keys0, N);
     c.take(b.keys1, N);
     c.take(b.vals0, N);
     c.take(b.vals1, N);
-    c.take(b.hist, radix_sort_scratch_words(N));  // the sort's digit counts and scan partials
+    c.take(b.hist, radix_sort_scratch_words(N));  // the sort's digit counts and totals
     c.take(b.saabb, 2 * (size_t)N);
-    c.take(b.left, NI);
-    c.take(b.right, NI);
+    c.take(b.rbox, 2 * range_boxes(N));
+    c.take(b.kids, NI);
     c.take(b.range, NI);
-    c.take(b.nparent, NI);
-    c.take(b.lparent, N);
     c.take(b.seg_root, n_seg);
-    c.take(b.is_root, NI);
     c.take(b.dlev, NI);
-    c.take(b.cnt, NI);
-    c.take(b.cost, NI);
-    c.take(b.lvl_order, NI);
+    c.take(b.lvl_order, b.treelets ? NI : 1);
     c.take(b.lvl_hist, kLevelBuckets);
     c.take(b.lvl_begin, kLevelBuckets + 1);
     c.take(b.lvl_fill, kLevelBuckets);
-    c.take(b.nbox, 2 * NI);
+    c.take(b.bnode, 3 * NI);
     c.take(b.wsrc, b.capacity);
     c.take(b.wseg, b.capacity);
-    c.take(b.lvl, kMaxLevels + 1);
-    c.take(b.counters, 4);
+    c.take(b.wfirst, b.capacity);
+    c.take(b.perm, b.treelets ? N : 1);
+    char* nodes = nullptr;  // (a plain build copies the nodes in use to the BVH)
+    c.take(nodes, node_bytes(b.width) * b.capacity);
+    b.nodes = nodes;
+    if (b.treelets) {  // the sorted triangles, re-packed into the final ones
+        c.take(b.tris, 3 * (size_t)N);
+        c.take(b.leaf_order, N);
+    }
+    b.lvl = b.report ? b.report + kReportLvl : nullptr;
+    b.counters = b.report ? b.report + kReportCounters : nullptr;
 }
 
 int build_alloc(const SegDesc* host_segs, int n_seg, int W, int leaf_size, int treelet_size, BuildBufs& b) {
@@ -1063,7 +1326,7 @@ int build_alloc(const SegDesc* host_segs, int n_seg, int W, int leaf_size, int t
     b.n_seg = n_seg;
     b.width = W;
     b.leaf_size = leaf_size;
-    b.nblocks_sort = cdiv(N, kSortTile);
+    b.treelets = treelet_size > 0;
     const size_t NI = N > 1 ? N - 1 : 1;
     b.capacity = (uint32_t)(NI + n_seg);
     Carver sizing;
@@ -1076,33 +1339,27 @@ int build_alloc(const SegDesc* host_segs, int n_seg, int W, int leaf_size, int t
     Carver c;
     c.base = static_cast<char*>(scratch);
     carve_all(b, c, NI);
-    void* nodes = nullptr;
-    void* tris = nullptr;
-    void* order = nullptr;
-    if (b.alloc(&nodes, node_bytes(W) * b.capacity) != hipSuccess ||
-        b.alloc(&tris, sizeof(float4) * 3 * (size_t)N) != hipSuccess ||
-        b.alloc(&order, sizeof(uint32_t) * (size_t)N) != hipSuccess) {
-        (void)hipGetLastError();
-        return set_error(GPURT_E_OOM, "allocation of BVH storage failed");  // b frees what it holds
-    }
-    b.nodes = nodes;
-    b.tris = static_cast<float4*>(tris);
-    b.leaf_order = static_cast<uint32_t*>(order);
-    if (treelet_size > 0) {
-        void* t2 = nullptr;
-        void* o2 = nullptr;
-        if (b.alloc(&t2, sizeof(float4) * 3 * (size_t)N) != hipSuccess ||
-            b.alloc(&o2, sizeof(uint32_t) * (size_t)N) != hipSuccess) {
+    float4*& tris = b.treelets ? b.tris2 : b.tris;
+    uint32_t*& order = b.treelets ? b.leaf_order2 : b.leaf_order;
+    tris = b.own_tris;
+    order = b.own_order;
+    if (!tris || !order) {
+        void *t = nullptr, *o = nullptr;
+        if (b.alloc(&t, sizeof(float4) * 3 * (size_t)N) != hipSuccess ||
+            b.alloc(&o, sizeof(uint32_t) * (size_t)N) != hipSuccess) {
             (void)hipGetLastError();
-            return set_error(GPURT_E_OOM, "allocation of re-pack buffers failed");
+            return set_error(GPURT_E_OOM, "allocation of BVH storage failed");  // b frees what it holds
         }
-        b.tris2 = static_cast<float4*>(t2);
-        b.leaf_order2 = static_cast<uint32_t*>(o2);
+        tris = static_cast<float4*>(t);
+        order = static_cast<uint32_t*>(o);
     }
-    if (b.pooled) {
-        GPURT_HIP(hipMemcpyAsync(b.segs, host_segs, sizeof(SegDesc) * n_seg, hipMemcpyHostToDevice, b.pool_stream));
-    } else {
-        GPURT_HIP(hipMemcpy(b.segs, host_segs, sizeof(SegDesc) * n_seg, hipMemcpyHostToDevice));
+    b.one = n_seg == 1 ? host_segs[0] : SegDesc{};
+    if (n_seg > 1) {  // (a single mesh is handed over by k_init_build)
+        if (b.ctx) {
+            GPURT_HIP(hipMemcpyAsync(b.segs, host_segs, sizeof(SegDesc) * n_seg, hipMemcpyHostToDevice, b.pool_stream));
+        } else {
+            GPURT_HIP(hipMemcpy(b.segs, host_segs, sizeof(SegDesc) * n_seg, hipMemcpyHostToDevice));
+        }
     }
     return GPURT_OK;
 }
@@ -1112,20 +1369,17 @@ int build_alloc(const SegDesc* host_segs, int n_seg, int W, int leaf_size, int t
 int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hipStream_t s) {
     const uint32_t N = b.N;
     const int n_seg = b.n_seg;
-    const size_t NI = N > 1 ? N - 1 : 1;
     const unsigned gN = cdiv(N, kBlock);
-    hipLaunchKernelGGL(k_init_build, dim3(cdiv(std::max(n_seg * kRep, kMaxLevels + 1), kBlock)),
-                       dim3(kBlock), 0, s, b.segs, n_seg, b.segstat_rep, b.seg_root, b.lvl, b.counters);
-    hipLaunchKernelGGL(k_fill_u32, dim3(std::min(gN, 4096u)), dim3(kBlock), 0, s, b.lparent, (size_t)N,
-                       kEmpty);
-    hipLaunchKernelGGL(k_fill_u32, dim3(std::min(cdiv(NI, kBlock), 4096u)), dim3(kBlock), 0, s,
-                       b.nparent, NI, kEmpty);
-    hipLaunchKernelGGL(k_prep, dim3(gN), dim3(kBlock), 0, s, b.segs, n_seg, N, b.aabb_lo, b.aabb_hi,
-                       b.segstat_rep, b.counters);
+    hipLaunchKernelGGL(k_init_build, dim3(cdiv(std::max(n_seg * kRep, (int)kLevelBuckets), kBlock)), dim3(kBlock), 0, s,
+                       b.segs, n_seg, b.one, n_seg == 1 ? 1 : 0, b.segstat_rep, b.seg_root, b.report, b.lvl_hist);
+    // rounds of 64 triangles per wave: enough waves to fill the chip first, then fewer
+    // atomics (up to 16 rounds)
+    const int rounds = (int)std::min<uint32_t>(16u, std::max<uint32_t>(1u, N / (64u * 4096u)));
+    hipLaunchKernelGGL(k_prep, dim3(cdiv(N, kBlock * (size_t)rounds)), dim3(kBlock), 0, s, b.segs, n_seg, N, rounds,
+                       b.cen, b.segstat_rep, b.counters);
     hipLaunchKernelGGL(k_reduce_stats, dim3(cdiv((size_t)n_seg * kStat, kBlock)), dim3(kBlock), 0, s, n_seg,
                        b.segstat_rep, b.segstat);
-    hipLaunchKernelGGL(k_morton, dim3(gN), dim3(kBlock), 0, s, N, b.aabb_lo, b.aabb_hi, b.segstat,
-                       b.keys0, b.vals0);
+    hipLaunchKernelGGL(k_morton, dim3(gN), dim3(kBlock), 0, s, N, b.cen, b.segstat, b.keys0, b.vals0);
     // radix sort over the bits in use: 30 Morton bits + mesh-id bits
     int seg_bits = 0;
     while ((1u << seg_bits) < (uint32_t)n_seg) seg_bits++;
@@ -1138,169 +1392,151 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
     }
     hipLaunchKernelGGL(k_pack, dim3(gN), dim3(kBlock), 0, s, N, kin, vin, b.segs, b.saabb, b.tris, b.leaf_order);
     if (N > 1) {
-        const int n_int = (int)(N - 1);
-        hipLaunchKernelGGL(k_karras, dim3(cdiv(N - 1, kBlock)), dim3(kBlock), 0, s, (int)N, kin, b.segs,
-                           b.left, b.right, b.range, b.nparent, b.lparent, b.seg_root, b.is_root, b.dlev,
-                           b.cnt);
-        // bucket the internal nodes by prefix length, then one launch per length in use,
-        // longest first; distinct keys give [64 - key_bits, 63], equal keys give
-        // 64 + clz32(i ^ j) with i, j < N, i.e. [96 - ceil(log2 N), 95]
-        int nbits = 0;
-        while ((1u << nbits) < N) nbits++;
+        const uint32_t n_int = N - 1;
         const unsigned gI = cdiv(n_int, kBlock);
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, s, b.lvl_hist, (size_t)kLevelBuckets, 0u);
-        const unsigned gL = std::min(gI, kLevelBlocks);
-        const uint32_t small_max = 2u * (uint32_t)b.leaf_size;  // subtrees no treelet restructures
-        hipLaunchKernelGGL(k_level_hist, dim3(gL), dim3(kBlock), 0, s, n_int, b.dlev, b.cnt, small_max, b.lvl_hist);
-        hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(64), 0, s, b.lvl_hist, b.lvl_begin, b.lvl_fill);
-        hipLaunchKernelGGL(k_level_scatter, dim3(gL), dim3(kBlock), 0, s, n_int, b.dlev, b.cnt, small_max, b.lvl_fill,
-                           b.lvl_order);
-        hipLaunchKernelGGL(k_boxes_local, dim3(gI), dim3(kBlock), 0, s, (uint32_t)n_int, b.range, b.left, b.right,
-                           b.cnt, b.dlev, b.saabb, b.nbox, b.cost, b.leaf_size);
-        const unsigned lgrid = std::min(gI, 1024u);
-        for (int level = 95; level >= 64 - key_bits; level--) {
-            if (level >= 64 && level < 96 - nbits) continue;
-            hipLaunchKernelGGL(k_boxes_level, dim3(lgrid), dim3(kBlock), 0, s, level, b.lvl_begin, b.lvl_order,
-                               b.range, b.left, b.right, b.cnt, b.saabb, b.nbox, b.cost, b.leaf_size);
+        hipLaunchKernelGGL(k_karras, dim3(gI), dim3(kBlock), 0, s, (int)N, kin, b.segs, b.kids, b.range, b.seg_root,
+                           b.dlev);
+        const bool cross = N > kBlock;  // more than one chunk
+        hipLaunchKernelGGL(k_boxes_local, dim3(gN), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
+                           b.bnode, cross ? b.rbox : nullptr, b.leaf_size);
+        if (cross) {
+            hipLaunchKernelGGL(k_range_top, dim3(1), dim3(1024), 0, s, N, b.rbox);
+            hipLaunchKernelGGL(k_boxes_cross, dim3(gI), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
+                               b.rbox, b.bnode, b.leaf_size, b.treelets ? 1 : 0);
         }
         if (treelet_size > 0) {
+            // bucket the treelet roots by prefix length; distinct keys give
+            // [64 - key_bits, 63], equal keys give 64 + clz32(i ^ j) with i, j < N, i.e.
+            // [96 - ceil(log2 N), 95]
+            int nbits = 0;
+            while ((1u << nbits) < N) nbits++;
+            const unsigned gL = std::min(gI, kLevelBlocks);
+            const uint32_t small_max = 2u * (uint32_t)b.leaf_size;  // subtrees no treelet restructures
+            hipLaunchKernelGGL(k_level_hist, dim3(gL), dim3(kBlock), 0, s, (int)n_int, b.dlev, b.range, small_max,
+                               b.lvl_hist);
+            hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(kBlock), 0, s, b.lvl_hist, b.lvl_begin, b.lvl_fill);
+            hipLaunchKernelGGL(k_level_scatter, dim3(gL), dim3(kBlock), 0, s, (int)n_int, b.dlev, b.range, small_max,
+                               b.lvl_fill, b.lvl_order);
             int trc = run_treelets(b, treelet_size, treelet_rounds, key_bits, nbits, s);
             if (trc != GPURT_OK) return trc;
             b.repacked = true;
         }
     }
-    hipLaunchKernelGGL(k_init_levels, dim3(cdiv(n_seg, kBlock)), dim3(kBlock), 0, s, n_seg, b.seg_root,
-                       b.wsrc, b.wseg);
+    hipLaunchKernelGGL(k_init_levels, dim3(cdiv(n_seg, kBlock)), dim3(kBlock), 0, s, n_seg, b.segs, b.seg_root,
+                       b.wsrc, b.wseg, b.wfirst);
     GPURT_HIP(hipGetLastError());
     return GPURT_OK;
 }
 
 template <int W>
-static void launch_collapse_level(const CollapseArgs& a, unsigned grid, hipStream_t s) {
-    hipLaunchKernelGGL(k_collapse<W>, dim3(grid), dim3(kBlock), 0, s, a);
+static void launch_collapse(CollapseArgs a, int levels, unsigned grid, hipStream_t s) {
+    for (int level = 0; level < levels; level++) {
+        a.level = level;
+        hipLaunchKernelGGL(k_collapse<W>, dim3(grid), dim3(kBlock), 0, s, a);
+    }
+    a.level = levels;
+    hipLaunchKernelGGL(k_collapse_tail<W>, dim3(1), dim3(1024), 0, s, a);
 }
 
-static void collapse_level(int W, const CollapseArgs& a, unsigned grid, hipStream_t s) {
-    if (W == 2) launch_collapse_level<2>(a, grid, s);
-    else if (W == 4) launch_collapse_level<4>(a, grid, s);
-    else launch_collapse_level<8>(a, grid, s);
-}
-
-int build_enqueue_levels(BuildBufs& b, int leaf_size, int level_begin, int level_end, hipStream_t s) {
-    CollapseArgs ca;
-    ca.left = b.left;
-    ca.right = b.right;
-    ca.range = b.range;
-    ca.cnt = b.cnt;
+// Enqueues the wide collapse (every level: no host synchronisation) and the re-pack.
+int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s) {
+    CollapseArgs ca{};
+    ca.bnode = b.bnode;
     ca.saabb = b.saabb;
-    ca.nbox = b.nbox;
     ca.segstat = b.segstat;
     ca.wsrc = b.wsrc;
     ca.wseg = b.wseg;
+    ca.wfirst = b.wfirst;
     ca.lvl_cnt = b.lvl;
     ca.counters = b.counters;
     ca.nodes = b.nodes;
     ca.capacity = b.capacity;
     ca.leaf_size = leaf_size;
     ca.repack = b.repacked ? 1 : 0;
-    ca.tris_in = b.tris;
-    ca.order_in = b.leaf_order;
-    ca.tris_out = b.tris2;
-    ca.order_out = b.leaf_order2;
-    const unsigned cgrid = std::min(cdiv(b.capacity, kBlock), 2048u);
-    for (int level = level_begin; level < level_end; level++) {
-        ca.level = level;
-        collapse_level(b.width, ca, cgrid, s);
-    }
+    ca.perm = b.perm;
+    // Launches for the depth that trees of this size have (5 K triangles: 8 wide levels at
+    // W = 4, 2.3 M: 16; a W-wide level takes about log2(W) binary ones on the way down the
+    // larger side) and some; a deeper tree's last levels, with few nodes, are the tail's.
+    int nbits = 1;
+    while ((1u << nbits) < b.N) nbits++;
+    const int per = b.width == 2 ? 10 : (b.width == 4 ? 8 : 5);
+    const int levels = std::min(kMaxLevels - 1, 2 + nbits * per / 10);
+    const unsigned grid = std::min(cdiv(b.capacity, kBlock), 2048u);
+    if (b.width == 2) launch_collapse<2>(ca, levels, grid, s);
+    else if (b.width == 4) launch_collapse<4>(ca, levels, grid, s);
+    else launch_collapse<8>(ca, levels, grid, s);
+    if (b.repacked)
+        hipLaunchKernelGGL(k_repack, dim3(cdiv(3 * (size_t)b.N, kBlock)), dim3(kBlock), 0, s, b.N, b.perm, b.tris,
+                           b.leaf_order, b.tris2, b.leaf_order2);
     GPURT_HIP(hipGetLastError());
     return GPURT_OK;
 }
 
-// Plain (single-mesh) build: enqueue, run the collapse in groups of levels until the
-// tree ends (host checks between groups), then hand the products to *out.
+// Plain (single-mesh) build: everything is enqueued, then one read of the report gives the
+// node count, the levels and the errors, and the products are handed to *out.
 int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, int leaf_size,
                    int treelet_size, int treelet_rounds, int format, hipStream_t s, gpurt_bvh_s* out) {
-    (void)ctx;
-    // every buffer from the stream-ordered pool on the build stream: the products become
-    // the BVH's (freed in stream order by gpurt_bvh_destroy), the scratch is freed on the
-    // stream when b goes out of scope
-    BuildBufs b;
-    b.pooled = true;
+    BuildBufs b;  // its scratch goes back to the pool, in stream order, with it
+    b.ctx = ctx;
     b.pool_stream = s;
+    b.own_tris = out->tris;
+    b.own_order = out->leaf_order;
     int rc;
     if ((rc = build_alloc(host_segs, n_seg, W, leaf_size, treelet_size, b))) return rc;
     if ((rc = build_enqueue_binary(b, treelet_size, treelet_rounds, s))) return rc;
-    std::vector<uint32_t> h_lvl(kMaxLevels + 1, 0);
-    int level = 0;
-    bool done = false;
-    while (!done && level < kMaxLevels) {
-        int group_end = std::min(level + 8, kMaxLevels);
-        if ((rc = build_enqueue_levels(b, leaf_size, level, group_end, s))) return rc;
-        level = group_end;
-        GPURT_HIP(hipMemcpyAsync(h_lvl.data(), b.lvl, sizeof(uint32_t) * (kMaxLevels + 1),
-                                 hipMemcpyDeviceToHost, s));
-        GPURT_HIP(hipStreamSynchronize(s));
-        done = h_lvl[level] == 0;
-    }
-    uint32_t h_counters[4] = {0, 0, 0, 0};
-    GPURT_HIP(hipMemcpyAsync(h_counters, b.counters, sizeof(h_counters), hipMemcpyDeviceToHost, s));
-    uint32_t st[kStat];
-    GPURT_HIP(hipMemcpyAsync(st, b.segstat, sizeof(st), hipMemcpyDeviceToHost, s));
+    if ((rc = build_enqueue_collapse(b, leaf_size, s))) return rc;
+    const unsigned gsah = std::min(cdiv(b.capacity, kBlock), 512u);
+    if (W == 2) hipLaunchKernelGGL(k_sah_cost<2>, dim3(gsah), dim3(kBlock), 0, s, (const WNode<2>*)b.nodes, b.bnode, b.segstat, b.report);
+    else if (W == 4) hipLaunchKernelGGL(k_sah_cost<4>, dim3(gsah), dim3(kBlock), 0, s, (const WNode<4>*)b.nodes, b.bnode, b.segstat, b.report);
+    else hipLaunchKernelGGL(k_sah_cost<8>, dim3(gsah), dim3(kBlock), 0, s, (const WNode<8>*)b.nodes, b.bnode, b.segstat, b.report);
+    GPURT_HIP(hipGetLastError());
+    uint32_t rep[kReportWords];
+    GPURT_HIP(hipMemcpyAsync(rep, b.report, sizeof(rep), hipMemcpyDeviceToHost, s));
     GPURT_HIP(hipStreamSynchronize(s));
-    if (!done) return set_error(GPURT_E_UNSUPPORTED, "BVH deeper than the supported level count");
+    const uint32_t* h_lvl = rep + kReportLvl;
+    const uint32_t* h_counters = rep + kReportCounters;
+    if (h_lvl[kMaxLevels]) return set_error(GPURT_E_UNSUPPORTED, "BVH deeper than the supported level count");
     if (h_counters[1] & 1u) return set_error(GPURT_E_INVALID, "triangle index >= n_verts");
     if (h_counters[1] & 4u) return set_error(GPURT_E_INVALID, "non-finite vertex position");
     if (h_counters[1] & 2u) return set_error(GPURT_E_DEVICE, "wide-node capacity exceeded");
     int depth = 0;
     while (depth <= kMaxLevels && h_lvl[depth] > 0) depth++;
-    // shrink the node array to the nodes in use
+    // the nodes in use go to the BVH's own memory
     const uint32_t n_nodes = h_counters[0];
-    void* nodes = b.nodes;
-    void* tight = nullptr;
-    if (hipMallocAsync(&tight, node_bytes(W) * n_nodes, s) == hipSuccess) {
-        if (hipMemcpyAsync(tight, nodes, node_bytes(W) * n_nodes, hipMemcpyDeviceToDevice, s) == hipSuccess) {
-            nodes = tight;  // b frees the large array (after the copy, in stream order)
-        } else {
-            (void)hipFreeAsync(tight, s);
-            (void)hipGetLastError();
-            b.release(nodes);
-        }
-    } else {
-        (void)hipGetLastError();
-        b.release(nodes);
-    }
-    out->nodes = nodes;  // the caller frees the products on failure from here on
-    uint32_t u = st[6];
+    auto carve = [&](Carver c) {
+        char *nodes = nullptr, *q = nullptr;
+        c.take(nodes, node_bytes(W) * n_nodes);
+        out->nodes = nodes;
+        if (has_qnodes(format)) c.take(q, qnode_bytes(W) * n_nodes);
+        out->qnodes = q;
+        return c.off;
+    };
+    if ((rc = pool_alloc(ctx, &out->node_mem, carve(Carver{}), s))) return rc;  // the caller frees the products
+    carve(Carver{0, static_cast<char*>(out->node_mem)});
+    GPURT_HIP(hipMemcpyAsync(out->nodes, b.nodes, node_bytes(W) * n_nodes, hipMemcpyDeviceToDevice, s));
+    uint32_t u = rep[kReportRoot + 6];
     u = (u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u;
     float scale;
     std::memcpy(&scale, &u, 4);
     // SAH cost relative to the root box area
     double sah = 0.0;
     {
-        double* acc = reinterpret_cast<double*>(b.hist);  // scratch no longer needed
-        GPURT_HIP(hipMemsetAsync(acc, 0, sizeof(double), s));
-        if (W == 2) hipLaunchKernelGGL(k_sah_cost<2>, dim3(cdiv(n_nodes, kBlock)), dim3(kBlock), 0, s, n_nodes, (const WNode<2>*)nodes, acc);
-        else if (W == 4) hipLaunchKernelGGL(k_sah_cost<4>, dim3(cdiv(n_nodes, kBlock)), dim3(kBlock), 0, s, n_nodes, (const WNode<4>*)nodes, acc);
-        else hipLaunchKernelGGL(k_sah_cost<8>, dim3(cdiv(n_nodes, kBlock)), dim3(kBlock), 0, s, n_nodes, (const WNode<8>*)nodes, acc);
-        float rl[4], rh[4];
-        GPURT_HIP(hipMemcpyAsync(&sah, acc, sizeof(double), hipMemcpyDeviceToHost, s));
-        GPURT_HIP(hipMemcpyAsync(rl, b.nbox, sizeof(rl), hipMemcpyDeviceToHost, s));
-        GPURT_HIP(hipMemcpyAsync(rh, b.nbox + 1, sizeof(rh), hipMemcpyDeviceToHost, s));
-        GPURT_HIP(hipStreamSynchronize(s));
-        const float ex = rh[0] - rl[0], ey = rh[1] - rl[1], ez = rh[2] - rl[2];
+        float r[6];
+        std::memcpy(&sah, rep + kReportSah, sizeof(sah));
+        std::memcpy(r, rep + kReportRoot, sizeof(r));
+        const float ex = r[3] - r[0], ey = r[4] - r[1], ez = r[5] - r[2];
         const double root_area = 2.0 * ((double)ex * ez + (double)ex * ey + (double)ey * ez);
         sah = (b.N > 1 && root_area > 0.0) ? sah / root_area : 0.0;
     }
-    out->nodes = nodes;
     out->format = format;
     if (has_qnodes(format)) {
-        GPURT_HIP(hipMallocAsync(&out->qnodes, qnode_bytes(W) * std::max<uint32_t>(n_nodes, 1u), s));
-        launch_quantize(W, nodes, out->qnodes, n_nodes, n_nodes, nullptr, s);
+        launch_quantize(W, out->nodes, out->qnodes, n_nodes, n_nodes, nullptr, s);
         GPURT_HIP(hipGetLastError());
     }
-    if (b.repacked && h_counters[2] != b.N) return set_error(GPURT_E_DEVICE, "leaf re-pack lost triangles");
-    out->tris = (float4*)b.release(b.final_tris());
-    out->leaf_order = (uint32_t*)b.release(b.final_order());
+    if (!b.repacked && b.treelets) {  // (a single triangle) the sorted ones are final
+        GPURT_HIP(hipMemcpyAsync(out->tris, b.tris, sizeof(float4) * 3 * (size_t)b.N, hipMemcpyDeviceToDevice, s));
+        GPURT_HIP(hipMemcpyAsync(out->leaf_order, b.leaf_order, sizeof(uint32_t) * (size_t)b.N, hipMemcpyDeviceToDevice, s));
+    }
     out->n_nodes = n_nodes;
     out->node_capacity = n_nodes;
     out->depth = depth;
@@ -1310,7 +1546,7 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
     out->scale = scale;
     out->pad = scale * 0x1p-18f;
     out->sah_cost = (float)sah;
-    out->level_cnt.assign(h_lvl.begin(), h_lvl.begin() + depth);
+    out->level_cnt.assign(h_lvl, h_lvl + depth);
     return GPURT_OK;
 }
 

@@ -23,16 +23,14 @@ __device__ __forceinline__ float o2f(uint32_t u) {
 }
 
 // Binary references: internal node i -> i; leaf (sorted primitive p) -> kLeafBit | p.
+// An internal node is a 48-byte record of three float4: (lo.xyz, left), (hi.xyz, right),
+// (triangles under it, SAH cost, first sorted primitive under it, -), the integers as bits,
+// so that a pass that visits a node has all of it from one or two cache lines.
 __device__ __forceinline__ void ref_box(uint32_t r, const float4* __restrict__ saabb,
-                                        const float4* __restrict__ nbox, float4& lo, float4& hi) {
-    if (r & kLeafBit) {
-        size_t p = r & ~kLeafBit;
-        lo = saabb[2 * p];
-        hi = saabb[2 * p + 1];
-    } else {
-        lo = nbox[2 * (size_t)r];
-        hi = nbox[2 * (size_t)r + 1];
-    }
+                                        const float4* bnode, float4& lo, float4& hi) {
+    const float4* p = (r & kLeafBit) ? saabb + 2 * (size_t)(r & ~kLeafBit) : bnode + 3 * (size_t)r;
+    lo = p[0];
+    hi = p[1];
 }
 
 __device__ __forceinline__ float box_area(float4 lo, float4 hi) {
@@ -45,15 +43,6 @@ __device__ __forceinline__ float box_area(float4 lo, float4 hi) {
 // always collapsed into one leaf by the wide collapse, so they are priced as leaves.
 constexpr float kCi = 1.2f;
 constexpr float kCt = 1.0f;
-
-__device__ __forceinline__ float ref_cost(uint32_t r, const float4* __restrict__ saabb,
-                                          const float* __restrict__ cost) {
-    if (r & kLeafBit) {
-        size_t p = r & ~kLeafBit;
-        return kCt * box_area(saabb[2 * p], saabb[2 * p + 1]);
-    }
-    return cost[r];
-}
 
 __device__ __forceinline__ float sah_node_cost(float4 lo, float4 hi, uint32_t count, float cl, float cr,
                                                int leaf_size) {

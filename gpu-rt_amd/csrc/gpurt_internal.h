@@ -39,8 +39,11 @@ constexpr uint32_t kMaxLeafFirst = 0x0FFFFFFFu;  // 2^28 - 1 packed triangles ma
 // at least one binary level, so 64 launches always finish the tree.
 constexpr int kMaxLevels = 64;
 constexpr int kBlock = 256;
-// buckets of the per-prefix-length build passes: two per length (0..255)
-constexpr uint32_t kLevelBuckets = 512;
+// buckets of the treelet pass, one per prefix length
+constexpr uint32_t kLevelBuckets = 256;
+// words of a build's report: wide nodes per level, counters ([0] wide nodes, [1] error
+// bits), SAH sum (double), root box and coordinate scale
+constexpr int kReportLvl = 0, kReportCounters = 72, kReportSah = 80, kReportRoot = 82, kReportWords = 96;
 
 __host__ __device__ inline uint32_t make_leaf(uint32_t first, uint32_t count) {
     return kLeafBit | ((count - 1u) << 28) | first;
@@ -155,6 +158,18 @@ struct gpurt_ctx_s {
     };
     std::mutex scratch_mu;
     std::vector<StreamBuf> scratch;
+    // device memory of builds and BVHs (pool_alloc)
+    struct PoolBlock {
+        void* mem = nullptr;
+        size_t bytes = 0;
+        bool used = false;
+        hipEvent_t freed = nullptr;  // recorded where the block was given back
+        uint64_t when = 0;           // order of giving back
+    };
+    std::mutex pool_mu;
+    std::vector<PoolBlock> pool;
+    size_t pool_idle = 0, pool_limit = size_t(1) << 30;
+    uint64_t pool_clock = 0;
 };
 
 namespace gpurt_impl {
@@ -184,6 +199,9 @@ struct gpurt_bvh_s {
     float scale = 0.f;
     float pad = 0.f;
     float sah_cost = 0.f;
+    // two blocks of the context's pool hold all of these: the mesh copy, triangles and leaf
+    // order, and the nodes
+    void *mesh_mem = nullptr, *node_mem = nullptr;
     void* nodes = nullptr;        // WNode<W>[node_capacity] (boxes in FP32; refit updates these)
     void* qnodes = nullptr;       // QNode<W>[n_nodes] when has_qnodes(format)
     int format = 1;
@@ -191,10 +209,10 @@ struct gpurt_bvh_s {
     uint32_t* tri_idx = nullptr;  // 3 * n_tris, original order (for backward / refit)
     float* verts = nullptr;       // 3 * n_verts compact positions, original order
     uint32_t* leaf_order = nullptr;  // packed position -> original triangle (refit)
+    uint32_t* refit_tmp = nullptr;   // two words of a refit
     std::vector<uint32_t> level_cnt;  // wide nodes per level (level l starts at sum of previous)
-    // Every buffer above comes from the stream-ordered pool (hipMallocAsync on the build
-    // stream), so gpurt_bvh_destroy frees it with hipFreeAsync on ctx->release after
-    // waiting for the last use recorded on each stream that used the handle.
+    // gpurt_bvh_destroy gives the blocks back on ctx->release after waiting for the last
+    // use recorded on each stream that used the handle.
     std::mutex use_mu;
     std::vector<std::pair<hipStream_t, hipEvent_t>> uses;
     bool uses_lost = false;  // an event could not be recorded: destroy waits for the device
@@ -211,6 +229,31 @@ int hip_error(hipError_t e, const char* what);
 // makes stream `s` wait for every recorded use
 void note_use(gpurt_bvh_s* b, hipStream_t s);
 void wait_uses(gpurt_bvh_s* b, hipStream_t s);
+
+// Device memory of builds and BVHs, kept by the context: a block given back on a stream is
+// handed out again after a wait (on the device) for that point of the stream, so any
+// stream and thread may take it.  Idle blocks are bounded (1/16 of the device's memory; the
+// longest idle go first) and all are freed with the context.  hipMallocAsync and
+// hipFreeAsync, used before, cost a small build about 100 us for its ten buffers, and after
+// a hundred builds of 2.3 M triangles each hipFreeAsync took 10 ms (a build 27 ms instead
+// of 8).
+int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s);
+void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s);
+void pool_release(gpurt_ctx_s* c);  // after the device is idle (context destroy)
+
+// Lays buffers out in one allocation, 256-byte aligned: a first pass without a base gives
+// the size.
+struct Carver {
+    size_t off = 0;
+    char* base = nullptr;
+    template <typename T>
+    void take(T*& p, size_t count) {
+        const size_t bytes = count * sizeof(T) < 256 ? 256 : count * sizeof(T);
+        off = (off + 255) & ~size_t(255);
+        p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+        off += bytes;
+    }
+};
 
 #define GPURT_HIP(call)                                            \
     do {                                                           \
@@ -231,30 +274,33 @@ struct BuildBufs {
     int width = 4;
     int leaf_size = 4;
     bool repacked = false;  // treelets changed the tree: leaves re-packed into tris2
-    uint32_t nblocks_sort = 0;
     uint32_t capacity = 0;  // wide nodes the node array can hold
     SegDesc* segs = nullptr;
-    float4 *aabb_lo = nullptr, *aabb_hi = nullptr;
+    SegDesc one{};       // the mesh of a plain build
+    bool treelets = false;
+    float4* cen = nullptr;  // triangle box centres; w: mesh (bits)
     uint32_t* segstat_rep = nullptr;  // per-mesh statistics, replicated for atomics
     uint32_t* segstat = nullptr;      // per-mesh statistics, reduced
     uint64_t *keys0 = nullptr, *keys1 = nullptr;
     uint32_t *vals0 = nullptr, *vals1 = nullptr, *hist = nullptr;
     float4* saabb = nullptr;  // sorted triangle boxes (lo, hi)
-    uint32_t *left = nullptr, *right = nullptr;
-    uint2* range = nullptr;
-    uint32_t *nparent = nullptr, *lparent = nullptr, *seg_root = nullptr;
-    uint8_t* is_root = nullptr;
+    float4* rbox = nullptr;   // boxes of aligned blocks of 4, 16, ... sorted triangles
+    uint2 *kids = nullptr, *range = nullptr;  // binary tree: children, leaf range
+    uint32_t* seg_root = nullptr;
     uint8_t* dlev = nullptr;  // common-prefix length (Karras delta) of each internal node
-    uint32_t* cnt = nullptr;  // triangles under each internal node
-    float* cost = nullptr;    // SAH cost of each internal node's subtree
-    // internal nodes bucketed by prefix length l and size: bucket 2l holds those with
-    // more than 2 leaf_size triangles (the treelet roots), 2l + 1 the others
+    // treelet roots bucketed by prefix length
     uint32_t* lvl_order = nullptr;
     uint32_t* lvl_hist = nullptr;   // kLevelBuckets counts
     uint32_t* lvl_begin = nullptr;  // bucket k = lvl_order[lvl_begin[k] .. lvl_begin[k+1])
     uint32_t* lvl_fill = nullptr;
-    float4* nbox = nullptr;   // binary node boxes (lo, hi)
-    uint32_t *wsrc = nullptr, *wseg = nullptr, *lvl = nullptr, *counters = nullptr;
+    float4* bnode = nullptr;  // binary node records, 3 float4 each (build_common.h)
+    uint32_t *wsrc = nullptr, *wseg = nullptr;
+    uint32_t* wfirst = nullptr;  // wide node -> first packed triangle of its (contiguous) range
+    uint32_t* perm = nullptr;    // re-packed slot -> sorted position (treelet builds)
+    // What the host reads of a build, in one piece (kReportWords); lvl and counters point
+    // into it
+    uint32_t* report = nullptr;
+    uint32_t *lvl = nullptr, *counters = nullptr;
     void* nodes = nullptr;
     float4* tris = nullptr;          // triangles in sorted (Morton) order
     uint32_t* leaf_order = nullptr;  // sorted position -> triangle
@@ -262,27 +308,24 @@ struct BuildBufs {
     uint32_t* leaf_order2 = nullptr;
     float4* final_tris() const { return repacked ? tris2 : tris; }
     uint32_t* final_order() const { return repacked ? leaf_order2 : leaf_order; }
-    std::vector<void*> allocs;  // freed with the object unless release()d
-    // stream-ordered allocations (hipMallocAsync / hipFreeAsync on pool_stream) when set,
-    // else hipMalloc / hipFree (the batch keeps its buffers for its lifetime)
+    // Plain builds: scratch from the context's pool, and the BVH's own buffers for the
+    // triangles and their order.  Without a context everything is hipMalloc'ed and kept
+    // (the batch).
+    gpurt_ctx_s* ctx = nullptr;
     hipStream_t pool_stream = nullptr;
-    bool pooled = false;
-    hipError_t alloc(void** p, size_t bytes) {
-        *p = nullptr;
-        const hipError_t e = pooled ? hipMallocAsync(p, bytes, pool_stream) : hipMalloc(p, bytes);
-        if (e == hipSuccess) allocs.push_back(*p);
-        return e;
-    }
+    float4* own_tris = nullptr;
+    uint32_t* own_order = nullptr;
+    std::vector<void*> allocs;  // freed with the object
+    hipError_t alloc(void** p, size_t bytes);
     BuildBufs() = default;
     BuildBufs(const BuildBufs&) = delete;
     BuildBufs& operator=(const BuildBufs&) = delete;
     ~BuildBufs();
-    void* release(void* p);  // hands ownership of one allocation to the caller
 };
 int build_alloc(const SegDesc* host_segs, int n_seg, int width, int leaf_size, int treelet_size,
                 BuildBufs& b);
 int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hipStream_t s);
-int build_enqueue_levels(BuildBufs& b, int leaf_size, int level_begin, int level_end, hipStream_t s);
+int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s);
 int run_treelets(BuildBufs& b, int treelet_size, int rounds, int key_bits, int nbits, hipStream_t s);
 // Stable LSD radix sort (build.hip) of n (uint64 key, uint32 value) pairs on the low
 // key_bits bits, 8 bits per pass, ping-ponging between (k0, v0) and (k1, v1); returns

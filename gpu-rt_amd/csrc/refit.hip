@@ -133,9 +133,7 @@ static void refit_levels(gpurt_bvh_s* b, const uint32_t* scale, hipStream_t s) {
 
 int launch_refit(gpurt_bvh_s* b, const float* verts, size_t vstride_floats, hipStream_t s) {
     if (!b->leaf_order || !b->tri_idx || !b->verts) return set_error(GPURT_E_INVALID, "bvh has no mesh copy");
-    void* tmp = nullptr;
-    GPURT_HIP(hipMallocAsync(&tmp, 256, s));
-    uint32_t* scale = static_cast<uint32_t*>(tmp);
+    uint32_t* scale = b->refit_tmp;
     hipLaunchKernelGGL(k_refit_init, dim3(1), dim3(64), 0, s, scale);
     // every new position must be finite; the tree is left as it was otherwise
     hipLaunchKernelGGL(k_refit_check, dim3(cdiv(b->n_verts, kBlock)), dim3(kBlock), 0, s, (uint32_t)b->n_verts,
@@ -144,7 +142,6 @@ int launch_refit(gpurt_bvh_s* b, const float* verts, size_t vstride_floats, hipS
     hipError_t ce = hipMemcpyAsync(&bad, scale + 1, sizeof(bad), hipMemcpyDeviceToHost, s);
     if (ce == hipSuccess) ce = hipStreamSynchronize(s);
     if (ce != hipSuccess || bad) {
-        (void)hipFreeAsync(tmp, s);
         if (ce != hipSuccess) return hip_error(ce, "refit check");
         return set_error(GPURT_E_INVALID, "non-finite vertex position");
     }
@@ -160,7 +157,6 @@ int launch_refit(gpurt_bvh_s* b, const float* verts, size_t vstride_floats, hipS
     if (has_qnodes(b->format)) launch_quantize(b->width, b->nodes, b->qnodes, (uint32_t)b->n_nodes,
                                                 (uint32_t)b->n_nodes, nullptr, s);
     hipError_t e = hipGetLastError();
-    (void)hipFreeAsync(tmp, s);
     if (e != hipSuccess) return hip_error(e, "refit launch");
     return GPURT_OK;
 }

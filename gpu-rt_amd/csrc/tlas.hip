@@ -530,8 +530,16 @@ struct gpurt_tlas_s {
     // a TLAS whose context is gone (tlas_orphan) holds no device memory
     ~gpurt_tlas_s() {
         if (inst_d && ctx) {
-            if (top) wait_uses(top, ctx->release);
-            (void)hipFreeAsync(inst_d, ctx->release);
+            if (top) {
+                wait_uses(top, ctx->release);
+                bool lost;
+                {
+                    std::lock_guard<std::mutex> lk(top->use_mu);
+                    lost = top->uses_lost;
+                }
+                if (lost) (void)hipDeviceSynchronize();  // uses that no event marks
+            }
+            pool_free(ctx, inst_d, ctx->release);
         }
         if (top) gpurt_bvh_destroy(top);
     }
@@ -688,16 +696,14 @@ int gpurt_tlas_build(gpurt_ctx ctx, const gpurt_instance* instances, size_t n, c
         T->custom[i] = instances[i].custom_index;
         T->blas[i] = instances[i].blas;
     }
-    // stream-ordered allocations on the build stream; the instance table lives with the
-    // TLAS and is freed in stream order by gpurt_tlas_destroy
+    // memory from the context's pool; the instance table lives with the TLAS and is given
+    // back in stream order by gpurt_tlas_destroy
     float* vd = nullptr;
     uint32_t* id = nullptr;
-    rc = GPURT_OK;
-    if (hipMallocAsync((void**)&vd, sizeof(float) * verts.size(), s) != hipSuccess ||
-        hipMallocAsync((void**)&id, sizeof(uint32_t) * idx.size(), s) != hipSuccess ||
-        hipMallocAsync((void**)&T->inst_d, sizeof(InstDev) * n, s) != hipSuccess) {
-        (void)hipGetLastError();
-        rc = set_error(GPURT_E_OOM, "TLAS allocation failed");
+    if ((rc = pool_alloc(ctx, (void**)&vd, sizeof(float) * verts.size(), s)) ||
+        (rc = pool_alloc(ctx, (void**)&id, sizeof(uint32_t) * idx.size(), s)) ||
+        (rc = pool_alloc(ctx, (void**)&T->inst_d, sizeof(InstDev) * n, s))) {
+        // reported below
     } else if (hipMemcpyAsync(vd, verts.data(), sizeof(float) * verts.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
                hipMemcpyAsync(id, idx.data(), sizeof(uint32_t) * idx.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
                hipMemcpyAsync(T->inst_d, dev.data(), sizeof(InstDev) * n, hipMemcpyHostToDevice, s) != hipSuccess) {
@@ -712,8 +718,8 @@ int gpurt_tlas_build(gpurt_ctx ctx, const gpurt_instance* instances, size_t n, c
         to.node_format = q8 ? kFormatQ8 : kFormatF32;
         rc = gpurt_bvh_build(ctx, vd, 12, 3 * n, id, n, &to, stream, &T->top);
     }
-    if (vd) (void)hipFreeAsync(vd, s);
-    if (id) (void)hipFreeAsync(id, s);
+    pool_free(ctx, vd, s);
+    pool_free(ctx, id, s);
     // the host arrays above feed asynchronous copies: wait for them on every path
     if (hipStreamSynchronize(s) != hipSuccess && rc == GPURT_OK) rc = hip_error(hipGetLastError(), "TLAS build");
     if (rc) {
@@ -809,7 +815,7 @@ void tlas_note_use(gpurt_tlas t, hipStream_t s) {
 }
 
 void tlas_orphan(gpurt_tlas t) {
-    if (t->inst_d) (void)hipFreeAsync(t->inst_d, t->ctx->release);
+    pool_free(t->ctx, t->inst_d, t->ctx->release);
     t->inst_d = nullptr;
     t->ctx = nullptr;
 }

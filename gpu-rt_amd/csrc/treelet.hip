@@ -38,8 +38,7 @@ __device__ __forceinline__ int nth_submask(int s, int mask) {
 template <int N>
 __global__ __launch_bounds__(64) void k_treelet(int level, const uint32_t* __restrict__ lvl_begin,
                                                 const uint32_t* __restrict__ lvl_order, int leaf_size,
-                                                uint32_t* left, uint32_t* right, uint32_t* cnt, float* cost,
-                                                float4* nbox, const float4* __restrict__ saabb) {
+                                                float4* bnode, const float4* __restrict__ saabb) {
     constexpr int NS = 1 << N;
     __shared__ uint32_t s_leaf[N], s_int[N];
     __shared__ float4 s_llo[N], s_lhi[N];
@@ -54,11 +53,11 @@ __global__ __launch_bounds__(64) void k_treelet(int level, const uint32_t* __res
     __shared__ float s_cur;
     const int lane = threadIdx.x;
     // one wave per treelet root of this prefix length: the roots with more than
-    // 2 leaf_size triangles (bucket 2 * level; the others become at most two leaves of one
+    // 2 leaf_size triangles (the others become at most two leaves of one
     // wide node, where a new topology gains nothing measurable -- rays_scene: skipping them
     // builds in 10.7 instead of 13.4 ms with the same ray times; skipping up to 16 or 32
     // triangles builds faster still but costs 2-5% in ray time)
-    const uint32_t beg = lvl_begin[2 * level], end = lvl_begin[2 * level + 1];
+    const uint32_t beg = lvl_begin[level], end = lvl_begin[level + 1];
     for (uint32_t k = beg + blockIdx.x; k < end; k += gridDim.x) {
         const int r = (int)lvl_order[k];
         {
@@ -73,34 +72,31 @@ __global__ __launch_bounds__(64) void k_treelet(int level, const uint32_t* __res
             float xcost = 0.0f, xarea = -1.0f;
             auto take = [&](uint32_t ref) {
                 x = ref;
-                ref_box(ref, saabb, nbox, xlo, xhi);
+                ref_box(ref, saabb, bnode, xlo, xhi);
                 if (ref & kLeafBit) {
                     xc = 1u;
                     xcost = kCt * box_area(xlo, xhi);
                     xarea = -1.0f;  // not openable
                 } else {
-                    xc = cnt[ref];
-                    xcost = cost[ref];
-                    xl = left[ref];
-                    xr = right[ref];
+                    const float4 y = bnode[3 * (size_t)ref + 2];
+                    xc = __float_as_uint(y.x);
+                    xcost = y.y;
+                    xl = __float_as_uint(xlo.w);
+                    xr = __float_as_uint(xhi.w);
                     const float a = box_area(xlo, xhi);
                     xarea = a > -1.0f ? a : -1.0f;  // (a NaN area is never opened)
                 }
             };
-            float4 rlo = xlo, rhi = xhi;
-            uint32_t rc = 0;
-            if (lane == 0) {
-                rlo = nbox[2 * (size_t)r];
-                rhi = nbox[2 * (size_t)r + 1];
-                rc = cnt[r];
-            }
-            if (lane < 2) take(lane ? right[r] : left[r]);
+            const float4 rlo = bnode[3 * (size_t)r], rhi = bnode[3 * (size_t)r + 1];
+            const float4 rx = bnode[3 * (size_t)r + 2];
+            const uint32_t rc = __float_as_uint(rx.x);
+            if (lane < 2) take(__float_as_uint(lane ? rhi.w : rlo.w));
             // the root's cost, refreshed from its (finished) children, the first two
             // candidates
             const float c_right = __shfl(xcost, 1);
             if (lane == 0) {
                 s_cur = sah_node_cost(rlo, rhi, rc, xcost, c_right, leaf_size);
-                cost[r] = s_cur;
+                bnode[3 * (size_t)r + 2].y = s_cur;
                 s_int[0] = (uint32_t)r;
             }
             int nl = 2, ni = 1;
@@ -261,12 +257,12 @@ __global__ __launch_bounds__(64) void k_treelet(int level, const uint32_t* __res
                             sp++;
                         }
                     }
-                    left[node] = ref[0];
-                    right[node] = ref[1];
-                    nbox[2 * (size_t)node] = s_lo[sub];
-                    nbox[2 * (size_t)node + 1] = s_hi[sub];
-                    cnt[node] = s_cnt[sub];
-                    cost[node] = s_copt[sub];
+                    // (a rewritten node's sorted primitives are no longer one range: its
+                    // first field is unused, the leaves are re-packed)
+                    const float4 lo = s_lo[sub], hi = s_hi[sub];
+                    bnode[3 * (size_t)node] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(ref[0]));
+                    bnode[3 * (size_t)node + 1] = make_float4(hi.x, hi.y, hi.z, __uint_as_float(ref[1]));
+                    bnode[3 * (size_t)node + 2] = make_float4(__uint_as_float(s_cnt[sub]), s_copt[sub], 0.0f, 0.0f);
                 }
             }
             __syncthreads();
@@ -280,7 +276,7 @@ static void launch_treelet_levels(BuildBufs& b, int key_bits, int nbits, hipStre
     for (int level = 95; level >= 64 - key_bits; level--) {
         if (level >= 64 && level < 96 - nbits) continue;
         hipLaunchKernelGGL(k_treelet<N>, dim3(grid), dim3(64), 0, s, level, b.lvl_begin, b.lvl_order, b.leaf_size,
-                           b.left, b.right, b.cnt, b.cost, b.nbox, b.saabb);
+                           b.bnode, b.saabb);
     }
 }
 

@@ -235,13 +235,10 @@ int gpurt_tune_queries(gpurt_ctx ctx, const float* verts, size_t vstride_bytes, 
     if (sp && sp->cache_path && gpurt_tune_cache_load(sp->cache_path, key.c_str(), out) == GPURT_OK) return GPURT_OK;
     const int reps = sp && sp->reps ? sp->reps : 3;
     hipStream_t s = (hipStream_t)stream;
-    // outputs of the trial queries (stream-ordered, freed on the stream at the end)
+    // outputs of the trial queries (given back in stream order at the end)
     void* mem = nullptr;
     const size_t qbytes = n_q * (4 + 12 + 4), rbytes = n_r * (4 + 4 + 8);
-    if (hipMallocAsync(&mem, std::max<size_t>(qbytes + rbytes, 256), s) != hipSuccess) {
-        (void)hipGetLastError();
-        return set_error(GPURT_E_OOM, "tuner output allocation failed");
-    }
+    if (const int rc0 = pool_alloc(ctx, &mem, qbytes + rbytes, s)) return rc0;
     char* p = static_cast<char*>(mem);
     int32_t* qp = reinterpret_cast<int32_t*>(p);
     float* qpt = reinterpret_cast<float*>(p + 4 * n_q);
@@ -293,7 +290,7 @@ int gpurt_tune_queries(gpurt_ctx ctx, const float* verts, size_t vstride_bytes, 
         }
         gpurt_bvh_destroy(b);
     }
-    (void)hipFreeAsync(mem, s);
+    pool_free(ctx, mem, s);
     if (rc) return rc;
     set_key(&r, key);
     if (sp && sp->cache_path && (rc = gpurt_tune_cache_store(sp->cache_path, &r))) return rc;
