@@ -107,7 +107,7 @@ static void free_bvh_buffers(gpurt_bvh_s* b, hipStream_t s) {
         if (p) pool_free(b->ctx, p, s);
     b->mesh_mem = b->node_mem = b->nodes = b->qnodes = nullptr;
     b->tris = nullptr;
-    b->tri_idx = b->leaf_order = b->refit_tmp = nullptr;
+    b->tri_idx = b->leaf_order = b->refit_tmp = b->node_first = nullptr;
     b->verts = nullptr;
 }
 

@@ -750,16 +750,6 @@ __device__ __forceinline__ void write_bnode(float4* __restrict__ bnode, uint32_t
     bnode[3 * (size_t)i + 2] = make_float4(__uint_as_float(range.y - range.x + 1u), cost, __uint_as_float(range.x), 0.0f);
 }
 
-__device__ __forceinline__ float4 min4(float4 a, float4 b) {
-    return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.0f);
-}
-__device__ __forceinline__ float4 max4(float4 a, float4 b) {
-    return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z), 0.0f);
-}
-__device__ __forceinline__ float4 shfl_xor4(float4 v, int o) {
-    return make_float4(__shfl_xor(v.x, o), __shfl_xor(v.y, o), __shfl_xor(v.z, o), 0.0f);
-}
-
 __global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t N, const uint2* __restrict__ range,
                                                         const uint2* __restrict__ kids,
                                                         const uint8_t* __restrict__ dlev,
@@ -790,34 +780,7 @@ __global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t
     slo[tid] = lo;
     shi[tid] = hi;
     done[tid] = 0;
-    // aligned blocks of 4, 16, 64 leaves and the chunk
-    if (rbox) {
-        float4* at = rbox;
-        uint32_t cnt = N;
-        for (int lvl = 1; lvl <= 3; lvl++) {
-            const int o = 1 << (2 * (lvl - 1));
-            lo = min4(lo, shfl_xor4(lo, o));
-            hi = max4(hi, shfl_xor4(hi, o));
-            lo = min4(lo, shfl_xor4(lo, 2 * o));
-            hi = max4(hi, shfl_xor4(hi, 2 * o));
-            cnt = (cnt + 3) / 4;
-            const uint32_t e = i >> (2 * lvl);
-            if ((tid & (4u * o - 1u)) == 0 && e < cnt) {
-                at[2 * (size_t)e] = lo;
-                at[2 * (size_t)e + 1] = hi;
-            }
-            at += 2 * (size_t)cnt;
-        }
-        if ((tid & 63u) == 0) {
-            blo[tid >> 6] = lo;
-            bhi[tid >> 6] = hi;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            at[2 * (size_t)blockIdx.x] = min4(min4(blo[0], blo[1]), min4(blo[2], blo[3]));
-            at[2 * (size_t)blockIdx.x + 1] = max4(max4(bhi[0], bhi[1]), max4(bhi[2], bhi[3]));
-        }
-    }
+    if (rbox) write_range_blocks(N, i, lo, hi, rbox, blo);  // (blo is not in use yet)
     __syncthreads();
     while (__syncthreads_or(todo)) {
         const bool ready = todo && ((L & kLeafBit) || done[L - c0]) && ((R & kLeafBit) || done[R - c0]);
@@ -876,9 +839,8 @@ __global__ __launch_bounds__(1024) void k_range_top(uint32_t N, float4* rbox) {
     }
 }
 
-// entries (boxes) of all levels of rbox for N leaves: four levels up to the chunks and
-// those above down to one entry
-static size_t range_boxes(uint32_t N) {
+// four levels up to the chunks and those above down to one entry
+size_t range_boxes(uint32_t N) {
     size_t total = 0;
     uint32_t cnt = N;
     for (int lvl = 1; lvl <= 4 || cnt > 1; lvl++) {
@@ -886,6 +848,10 @@ static size_t range_boxes(uint32_t N) {
         total += cnt;
     }
     return total;
+}
+
+void launch_range_top(uint32_t N, float4* rbox, hipStream_t s) {
+    hipLaunchKernelGGL(k_range_top, dim3(1), dim3(1024), 0, s, N, rbox);
 }
 
 // A subtree of at most 2 leaf_size triangles that crosses a chunk: its SAH cost, by a walk
@@ -930,25 +896,14 @@ __global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t n_int, uint32_t
     if (i >= n_int || dlev[i] == 0xFF) return;
     const uint2 rg = range[i];
     if (box_in_chunk(rg)) return;  // done by k_boxes_local
-    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-    const float4* at = saabb;  // the level's boxes
-    uint32_t l = rg.x, r = rg.y + 1u, cnt = N;
-    while (l < r) {
-        // the blocks left and right of the next level's
-        const uint32_t l4 = min((l + 3u) & ~3u, r), r4 = max(r & ~3u, l4);
-        for (uint32_t k = l; k < l4; k++) {
-            lo = min4(lo, at[2 * (size_t)k]);
-            hi = max4(hi, at[2 * (size_t)k + 1]);
-        }
-        for (uint32_t k = r4; k < r; k++) {
-            lo = min4(lo, at[2 * (size_t)k]);
-            hi = max4(hi, at[2 * (size_t)k + 1]);
-        }
-        at = at == saabb ? rbox : at + 2 * (size_t)cnt;
-        cnt = (cnt + 3) / 4;
-        l = l4 / 4;
-        r = r4 / 4;
-    }
+    float4 lo, hi;
+    range_union(
+        rg.x, rg.y + 1u, N, rbox,
+        [&](uint32_t k, float4& l, float4& h) {
+            l = min4(l, saabb[2 * (size_t)k]);
+            h = max4(h, saabb[2 * (size_t)k + 1]);
+        },
+        lo, hi);
     float c = 0.0f;
     if (costs && rg.y - rg.x + 1u <= 2u * (uint32_t)leaf_size) c = small_cost(i, kids, range, saabb, leaf_size);
     write_bnode(bnode, i, lo, hi, kids[i], rg, c);
@@ -1400,7 +1355,7 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
         hipLaunchKernelGGL(k_boxes_local, dim3(gN), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
                            b.bnode, cross ? b.rbox : nullptr, b.leaf_size);
         if (cross) {
-            hipLaunchKernelGGL(k_range_top, dim3(1), dim3(1024), 0, s, N, b.rbox);
+            launch_range_top(N, b.rbox, s);
             hipLaunchKernelGGL(k_boxes_cross, dim3(gI), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
                                b.rbox, b.bnode, b.leaf_size, b.treelets ? 1 : 0);
         }
@@ -1509,6 +1464,7 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
         out->nodes = nodes;
         if (has_qnodes(format)) c.take(q, qnode_bytes(W) * n_nodes);
         out->qnodes = q;
+        c.take(out->node_first, n_nodes);
         return c.off;
     };
     if ((rc = pool_alloc(ctx, &out->node_mem, carve(Carver{}), s))) return rc;  // the caller frees the products
@@ -1537,6 +1493,7 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
         GPURT_HIP(hipMemcpyAsync(out->tris, b.tris, sizeof(float4) * 3 * (size_t)b.N, hipMemcpyDeviceToDevice, s));
         GPURT_HIP(hipMemcpyAsync(out->leaf_order, b.leaf_order, sizeof(uint32_t) * (size_t)b.N, hipMemcpyDeviceToDevice, s));
     }
+    GPURT_HIP(hipMemcpyAsync(out->node_first, b.wfirst, sizeof(uint32_t) * n_nodes, hipMemcpyDeviceToDevice, s));
     out->n_nodes = n_nodes;
     out->node_capacity = n_nodes;
     out->depth = depth;
@@ -1546,7 +1503,6 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
     out->scale = scale;
     out->pad = scale * 0x1p-18f;
     out->sah_cost = (float)sah;
-    out->level_cnt.assign(h_lvl, h_lvl + depth);
     return GPURT_OK;
 }
 

@@ -98,7 +98,6 @@ constexpr int kFormatMixed = 3;  // 8-bit boxes for rays, FP32 boxes for closest
 inline bool has_qnodes(int f) { return f != kFormatF32; }
 inline bool rays_use_q8(int f) { return f == kFormatQ8 || f == kFormatMixed; }
 inline bool cpq_use_q8(int f) { return f == kFormatQ8; }
-
 // Atomics on global memory through a global-address-space pointer: no flat-address
 // (LDS / scratch aperture) checks are generated around them.
 typedef __attribute__((address_space(1))) uint32_t global_u32;
@@ -204,13 +203,13 @@ struct gpurt_bvh_s {
     void *mesh_mem = nullptr, *node_mem = nullptr;
     void* nodes = nullptr;        // WNode<W>[node_capacity] (boxes in FP32; refit updates these)
     void* qnodes = nullptr;       // QNode<W>[n_nodes] when has_qnodes(format)
+    uint32_t* node_first = nullptr;  // first packed triangle of each node's (contiguous) range
     int format = 1;
     float4* tris = nullptr;       // 3 * n_tris
     uint32_t* tri_idx = nullptr;  // 3 * n_tris, original order (for backward / refit)
     float* verts = nullptr;       // 3 * n_verts compact positions, original order
     uint32_t* leaf_order = nullptr;  // packed position -> original triangle (refit)
     uint32_t* refit_tmp = nullptr;   // two words of a refit
-    std::vector<uint32_t> level_cnt;  // wide nodes per level (level l starts at sum of previous)
     // gpurt_bvh_destroy gives the blocks back on ctx->release after waiting for the last
     // use recorded on each stream that used the handle.
     std::mutex use_mu;
@@ -336,6 +335,11 @@ bool radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, ui
 size_t radix_sort_scratch_words(uint32_t n);
 int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int width, int leaf_size,
                    int treelet_size, int treelet_rounds, int format, hipStream_t stream, gpurt_bvh_s* out);
+
+// boxes of aligned blocks of primitives (build_common.h): how many for N, and the levels
+// above 256 from the ones below
+size_t range_boxes(uint32_t N);
+void launch_range_top(uint32_t N, float4* rbox, hipStream_t s);
 
 // quantized node copies (quantize.hip): nodes [0, n) with n = *n_dev when n_dev is given
 // (then `capacity` threads are launched), else n_host
