@@ -11,9 +11,8 @@ The same JSON line carries:
                 mean duration (HIP events on the launch stream), against the 8 TB/s HBM3E
                 peak.  Algorithmic bytes, the same formula for every traversal leg:
                   query I/O + node_bytes per wide node visited + 36 per triangle tested
-                (node_bytes = the traversed node encoding: 64 for the 8-bit 4-wide nodes
-                rays use, 128 for the FP32 4-wide nodes closest points use; 36 = three
-                float3 vertices), visits counted by the kernel's counting variant on the
+                (node_bytes = the traversed node encoding: 64 for the 8-bit 4-wide nodes of
+                rays and the oriented ones of closest points; 36 = three float3 vertices), visits counted by the kernel's counting variant on the
                 same BVH and inputs.  I/O: closest hit 32 in + 16 out, any hit 32 + 1,
                 closest point 12 in + 20 out + 12 barycentrics.  Backward: 144 B per
                 closest-point query, 180 B per ray.
@@ -67,8 +66,10 @@ def ray_bytes(n, nodes, tris, node_bytes, any_hit=False):
 def build_bytes(info):
     """The least a BVH build must move: read each triangle's indices and vertices (12 +
     36 B), write its packed record and leaf-order entry (48 + 4 B) and every wide node in
-    each encoding kept (cpq_node_bytes, plus node_bytes when rays use 8-bit nodes)."""
-    per_node = info["cpq_node_bytes"] + (info["node_bytes"] if info["node_bytes"] != info["cpq_node_bytes"] else 0)
+    each encoding kept (32 B per child FP32; the 8-bit nodes of rays; the oriented nodes of
+    closest points)."""
+    fmt, w = info["node_format"], info["node_width"]
+    per_node = 32 * w + (info["node_bytes"] if fmt != 1 else 0) + (info["cpq_node_bytes"] if fmt == 3 and w == 4 else 0)
     return info["n_tris"] * (12 + 36 + 48 + 4) + info["n_nodes"] * per_node
 
 
@@ -145,8 +146,11 @@ def fp64_cpq(O, V, F, Q, prim, dist, every):
 
 def roof_kernel(args, info, kind):
     q8 = info["node_format"] in (2, 3) if kind != "cpq" else info["node_format"] == 2
+    enc = "q8" if q8 else "f32"
+    if kind == "cpq" and info["node_format"] == 3 and args.width == 4:
+        enc = "oriented"
     name = {"closest": "k_ray<W=%d,%s,closest>", "any": "k_ray<W=%d,%s,any>", "cpq": "k_cpq<W=%d,%s>+k_cpq_finish"}[kind]
-    return name % (args.width, "q8" if q8 else "f32")
+    return name % (args.width, enc)
 
 
 def ray_bench(args, torch, gpurt, W, O, dev, ctx):

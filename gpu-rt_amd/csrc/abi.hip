@@ -105,7 +105,7 @@ void wait_uses(gpurt_bvh_s* b, hipStream_t s) {
 static void free_bvh_buffers(gpurt_bvh_s* b, hipStream_t s) {
     for (void* p : {b->mesh_mem, b->node_mem})
         if (p) pool_free(b->ctx, p, s);
-    b->mesh_mem = b->node_mem = b->nodes = b->qnodes = nullptr;
+    b->mesh_mem = b->node_mem = b->nodes = b->qnodes = b->onodes = nullptr;
     b->tris = nullptr;
     b->tri_idx = b->leaf_order = b->refit_tmp = b->node_first = nullptr;
     b->verts = nullptr;
@@ -535,7 +535,9 @@ int gpurt_bvh_get_info(gpurt_bvh b, gpurt_bvh_info* out) {
     out->n_verts = b->n_verts;
     out->n_nodes = b->n_nodes;
     out->node_bytes = (int64_t)(rays_use_q8(b->format) ? qnode_bytes(b->width) : node_bytes(b->width));
-    out->cpq_node_bytes = (int32_t)(cpq_use_q8(b->format) ? qnode_bytes(b->width) : node_bytes(b->width));
+    out->cpq_node_bytes = (int32_t)(cpq_use_oriented(b->format, b->width) ? sizeof(ONode)
+                                    : cpq_use_q8(b->format)               ? qnode_bytes(b->width)
+                                                                          : node_bytes(b->width));
     out->tri_bytes = 48;
     out->depth = b->depth;
     out->node_width = b->width;

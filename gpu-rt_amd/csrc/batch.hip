@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "backward.h"
+#include "build_common.h"
 #include "traverse.h"
 
 namespace gpurt_impl {
@@ -124,10 +125,10 @@ struct BatchArgs {
     uint32_t leaf_trigger;
 };
 
-template <int W, bool Q, int S, int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, Q>::value))) void k_batch_cpq(
+template <int W, int E, int S, int BS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, E>::value))) void k_batch_cpq(
     BatchArgs a) {
-    const NodeOf<W, Q>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, Q>*>(a.nodes);
+    const NodeOf<W, E>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, E>*>(a.nodes);
     LaneStack<S, BS> st;
     st.init(a.spill, a.spill_slots, blockIdx.x * BS + threadIdx.x, gridDim.x * BS);
     ChunkSource src{a.meshes, a.chunks, a.n_chunks, a.counter, false};
@@ -135,13 +136,13 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W,
         a.meshes[h.m].q_prim[h.i] = id == 0xFFFFFFFFu ? -1 : (int32_t)id;
     };
     unsigned long long dn = 0, dt = 0;
-    if (!cpq_stream<NodeOf<W, Q>, S, BS, false>(nodes, a.tris, src, a.leaf_trigger, st, out, dn, dt)) gatomic_or(a.err, 1u);
+    if (!cpq_stream<NodeOf<W, E>, S, BS, false>(nodes, a.tris, src, a.leaf_trigger, st, out, dn, dt)) gatomic_or(a.err, 1u);
 }
 
-template <int W, bool Q, int S, int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, Q>::value))) void k_batch_ray(
+template <int W, int E, int S, int BS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, E>::value))) void k_batch_ray(
     BatchArgs a) {
-    const NodeOf<W, Q>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, Q>*>(a.nodes);
+    const NodeOf<W, E>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, E>*>(a.nodes);
     LaneStack<S, BS> st;
     st.init(a.spill, a.spill_slots, blockIdx.x * BS + threadIdx.x, gridDim.x * BS);
     ChunkSource src{a.meshes, a.chunks, a.n_chunks, a.counter, true};
@@ -157,36 +158,40 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W,
         }
     };
     unsigned long long dn = 0, dt = 0;
-    if (!ray_stream<NodeOf<W, Q>, S, BS, false, false>(nodes, a.tris, src, a.leaf_trigger, st, out, dn, dt)) gatomic_or(a.err, 1u);
+    if (!ray_stream<NodeOf<W, E>, S, BS, false, false>(nodes, a.tris, src, a.leaf_trigger, st, out, dn, dt)) gatomic_or(a.err, 1u);
 }
 
-template <int W, bool Q, int S, int BS>
+template <int W, int E, int S, int BS>
 static void launch_batch_kind(bool rays, unsigned grid, hipStream_t s, const BatchArgs& a) {
-    if (rays)
-        hipLaunchKernelGGL((k_batch_ray<W, Q, S, BS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
-    else
-        hipLaunchKernelGGL((k_batch_cpq<W, Q, S, BS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+    if constexpr (E != kEncOriented) {
+        if (rays) {
+            hipLaunchKernelGGL((k_batch_ray<W, E, S, BS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_batch_cpq<W, E, S, BS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
 }
 
-template <int W, bool Q>
+template <int W, int E>
 static int launch_batch_w(int S, bool rays, unsigned grid, hipStream_t s, const BatchArgs& a) {
     switch (S) {
-        case 8: launch_batch_kind<W, Q, 8, 256>(rays, grid, s, a); return 256;
-        case 16: launch_batch_kind<W, Q, 16, 256>(rays, grid, s, a); return 256;
-        case 32: launch_batch_kind<W, Q, 32, 128>(rays, grid, s, a); return 128;
-        case 64: launch_batch_kind<W, Q, 64, 64>(rays, grid, s, a); return 64;
+        case 8: launch_batch_kind<W, E, 8, 256>(rays, grid, s, a); return 256;
+        case 16: launch_batch_kind<W, E, 16, 256>(rays, grid, s, a); return 256;
+        case 32: launch_batch_kind<W, E, 32, 128>(rays, grid, s, a); return 128;
+        case 64: launch_batch_kind<W, E, 64, 64>(rays, grid, s, a); return 64;
     }
     return 0;
 }
 
-static int launch_batch(int W, bool q8, int S, bool rays, unsigned grid, hipStream_t s, const BatchArgs& a) {
-    switch (W * 2 + (q8 ? 1 : 0)) {
-        case 4: return launch_batch_w<2, false>(S, rays, grid, s, a);
-        case 5: return launch_batch_w<2, true>(S, rays, grid, s, a);
-        case 8: return launch_batch_w<4, false>(S, rays, grid, s, a);
-        case 9: return launch_batch_w<4, true>(S, rays, grid, s, a);
-        case 16: return launch_batch_w<8, false>(S, rays, grid, s, a);
-        case 17: return launch_batch_w<8, true>(S, rays, grid, s, a);
+static int launch_batch(int W, int enc, int S, bool rays, unsigned grid, hipStream_t s, const BatchArgs& a) {
+    switch (W * 4 + enc) {
+        case 8 + kEncF32: return launch_batch_w<2, kEncF32>(S, rays, grid, s, a);
+        case 8 + kEncQ8: return launch_batch_w<2, kEncQ8>(S, rays, grid, s, a);
+        case 16 + kEncF32: return launch_batch_w<4, kEncF32>(S, rays, grid, s, a);
+        case 16 + kEncQ8: return launch_batch_w<4, kEncQ8>(S, rays, grid, s, a);
+        case 16 + kEncOriented: return launch_batch_w<4, kEncOriented>(S, rays, grid, s, a);
+        case 32 + kEncF32: return launch_batch_w<8, kEncF32>(S, rays, grid, s, a);
+        case 32 + kEncQ8: return launch_batch_w<8, kEncQ8>(S, rays, grid, s, a);
     }
     return 0;
 }
@@ -316,6 +321,7 @@ struct gpurt_batch_s {
     uint32_t leaf_trigger = 32;
     BuildBufs build;
     void* qnodes = nullptr;  // QNode<W>[build.capacity] when has_qnodes(format)
+    void* onodes = nullptr;  // ONode[build.capacity] when the batch uses oriented nodes
     BatchMeshDev* meshes_d = nullptr;
     uint2* chunks_d = nullptr;    // closest-point chunks, then ray chunks
     uint32_t n_cpq_chunks = 0, n_ray_chunks = 0;
@@ -355,6 +361,7 @@ struct gpurt_batch_s {
         if (counter_d) (void)hipFree(counter_d);
         if (spill) (void)hipFree(spill);
         if (qnodes) (void)hipFree(qnodes);
+        if (onodes) (void)hipFree(onodes);
     }
 };
 
@@ -380,6 +387,9 @@ int enqueue_batch(gpurt_batch_s* b, int treelet_size, int treelet_rounds, hipStr
         // counters[0] holds the wide-node count the levels produced
         launch_quantize(b->width, b->build.nodes, b->qnodes, 0, b->build.capacity, b->build.counters, s);
     }
+    if (b->onodes)
+        launch_orient(b->build.nodes, b->build.wfirst, b->build.final_tris(), b->onodes, 0, b->build.capacity,
+                      b->build.counters, b->build.segstat + 6, kStat, b->build.wseg, nullptr, s);
     hipLaunchKernelGGL(k_reset_counters, dim3(cdiv(2 * kQueues, 256)), dim3(256), 0, s, b->counter_d);
     BatchArgs a{};
     a.tris = b->build.final_tris();
@@ -391,13 +401,14 @@ int enqueue_batch(gpurt_batch_s* b, int treelet_size, int treelet_rounds, hipStr
     for (int rays = 0; rays < 2; rays++) {
         const uint32_t n = rays ? b->n_ray_chunks : b->n_cpq_chunks;
         if (n == 0) continue;
-        const bool q8 = rays ? rays_use_q8(b->format) : cpq_use_q8(b->format);
-        a.nodes = q8 ? b->qnodes : b->build.nodes;
+        const int enc = rays ? (rays_use_q8(b->format) ? kEncQ8 : kEncF32)
+                             : (b->onodes ? kEncOriented : (cpq_use_q8(b->format) ? kEncQ8 : kEncF32));
+        a.nodes = enc == kEncOriented ? b->onodes : (enc == kEncQ8 ? b->qnodes : b->build.nodes);
         a.chunks = b->chunks_d + (rays ? b->n_cpq_chunks : 0u);
         a.n_chunks = n;
         a.counter = b->counter_d + (size_t)rays * kQueues * kQueueStride;
         const unsigned grid = std::max<size_t>(1, std::min<size_t>(b->grid, (size_t)n * 64 / b->block + 1));
-        if (!launch_batch(b->width, q8, b->stack, rays != 0, grid, s, a))
+        if (!launch_batch(b->width, enc, b->stack, rays != 0, grid, s, a))
             return set_error(GPURT_E_UNSUPPORTED, "batch stack/width");
         if (!rays)
             hipLaunchKernelGGL(k_batch_cpq_finish, dim3(cdiv(n, 4)), dim3(256), 0, s, b->meshes_d, b->chunks_d, n);
@@ -494,14 +505,21 @@ int gpurt_batch_create(gpurt_ctx ctx, const gpurt_batch_mesh* meshes, size_t n_m
     for (uint32_t m : order)
         for (uint32_t st = 0; st < md[m].n_r; st += 64) chunks.push_back(make_uint2(m, st));
     b->n_ray_chunks = (uint32_t)chunks.size() - b->n_cpq_chunks;
+    // Oriented nodes are remade with every replay's trees, which only enough closest-point
+    // queries pay for: 7.1 M triangles and 3.0 M queries (256 meshes): the nodes cost 500
+    // us and the queries take 1.63 instead of 2.42 ms, so the line lies at a query for
+    // every four triangles; below it the queries use the FP32 nodes.
+    uint64_t total_q = 0;
+    for (size_t m = 0; m < n_meshes; m++) total_q += md[m].n_q;
+    const bool oriented = cpq_use_oriented(bp.format, W) && 4 * total_q >= off;
     const int BS = block_for_stack_b(S);
     b->block = BS;
     const int waves_per_block = BS / 64;
     // register-limited waves: the larger of the two kernels' needs (FP32 8-wide nodes
     // need the most registers)
     const bool any_f32 = !rays_use_q8(bp.format) || !cpq_use_q8(bp.format);
-    const int hint = W == 8 ? (any_f32 ? WavesHint<8, false>::value : WavesHint<8, true>::value)
-                            : WavesHint<4, false>::value;
+    const int hint = W == 8 ? (any_f32 ? WavesHint<8>::value : WavesHint<8, kEncQ8>::value)
+                            : WavesHint<4>::value;
     int blocks_per_cu = std::min(ctx->lds_per_cu / ((S * 8 + kGroupKeyBytes) * BS), std::min(32, 4 * hint) / waves_per_block);
     // default 4 waves/SIMD, as the single-mesh closest-point kernels, which dominate a
     // batch (256-mesh batch: 36.1 -> 34.9 ms per replay against every slot registers allow)
@@ -519,6 +537,8 @@ int gpurt_batch_create(gpurt_ctx ctx, const gpurt_batch_mesh* meshes, size_t n_m
                 hipMalloc((void**)&b->chunks_d, sizeof(uint2) * std::max<size_t>(1, chunks.size())) != hipSuccess ||
                 hipMalloc((void**)&b->counter_d, sizeof(uint32_t) * 2 * kQueues * kQueueStride) != hipSuccess ||
                 (has_qnodes(bp.format) && hipMalloc(&b->qnodes, qnode_bytes(W) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
+                (oriented &&
+                 hipMalloc(&b->onodes, sizeof(ONode) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
                 (b->spill_slots &&
                  hipMalloc((void**)&b->spill, (size_t)b->spill_slots * b->grid * BS * sizeof(uint2)) != hipSuccess);
     if (fail) {

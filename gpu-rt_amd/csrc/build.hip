@@ -1464,6 +1464,11 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
         out->nodes = nodes;
         if (has_qnodes(format)) c.take(q, qnode_bytes(W) * n_nodes);
         out->qnodes = q;
+        if (cpq_use_oriented(format, W)) {
+            ONode* o = nullptr;
+            c.take(o, n_nodes);
+            out->onodes = o;
+        }
         c.take(out->node_first, n_nodes);
         return c.off;
     };
@@ -1494,6 +1499,11 @@ int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int W, in
         GPURT_HIP(hipMemcpyAsync(out->leaf_order, b.leaf_order, sizeof(uint32_t) * (size_t)b.N, hipMemcpyDeviceToDevice, s));
     }
     GPURT_HIP(hipMemcpyAsync(out->node_first, b.wfirst, sizeof(uint32_t) * n_nodes, hipMemcpyDeviceToDevice, s));
+    if (cpq_use_oriented(format, W)) {
+        launch_orient(out->nodes, out->node_first, out->tris, out->onodes, n_nodes, n_nodes, nullptr, b.segstat + 6, 0,
+                      nullptr, nullptr, s);
+        GPURT_HIP(hipGetLastError());
+    }
     out->n_nodes = n_nodes;
     out->node_capacity = n_nodes;
     out->depth = depth;

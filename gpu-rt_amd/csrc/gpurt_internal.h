@@ -91,13 +91,47 @@ static_assert(sizeof(QNode<8>) == 96, "node size");
 
 inline size_t qnode_bytes(int W) { return W == 2 ? 48 : (W == 4 ? 64 : 96); }
 
+// Oriented 4-wide node of closest-point queries (oriented.hip), as 32-bit words.  The
+// frame R (oriented.h) follows from n.x and n.y; a point p lies at Y = R (p - c) / s + 128
+// per axis, in the units of the byte planes, with s_a = 2^(e_a - 127) and e_a byte a of
+// word 3.
+//   words 0..2    c (float)
+//   word 3        exponent bytes
+//   words 4, 5    n.x, n.y (float; 0, 0: axis-aligned boxes)
+//   words 6..9    child[4]
+//   words 10..15  q[6][4] bytes: qlo x, y, z, then qhi x, y, z (255 and 0 in an empty slot)
+struct alignas(64) ONode {
+    static constexpr int kWidth = 4;
+    uint32_t w[16];
+};
+static_assert(sizeof(ONode) == 64, "node size");
+
 // Node formats of gpurt_build_opts::node_format (0 selects the library default, mixed).
 constexpr int kFormatF32 = 1;    // FP32 boxes for every query
 constexpr int kFormatQ8 = 2;     // 8-bit boxes for every query
-constexpr int kFormatMixed = 3;  // 8-bit boxes for rays, FP32 boxes for closest points
+constexpr int kFormatMixed = 3;  // 8-bit boxes for rays; for closest points oriented 8-bit
+                                 // boxes (4-wide nodes) or FP32 boxes (2- and 8-wide nodes)
 inline bool has_qnodes(int f) { return f != kFormatF32; }
 inline bool rays_use_q8(int f) { return f == kFormatQ8 || f == kFormatMixed; }
 inline bool cpq_use_q8(int f) { return f == kFormatQ8; }
+inline bool cpq_use_oriented(int f, int width) { return f == kFormatMixed && width == 4; }
+// node encodings that a traversal kernel is compiled for (NodeOf)
+constexpr int kEncF32 = 0, kEncQ8 = 1, kEncOriented = 2;
+
+// position of the n-th (from 0) set bit of m; n < popcount(m)
+__device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t n) {
+    uint32_t pos = 0;
+#pragma unroll
+    for (uint32_t w = 32; w >= 1; w >>= 1) {
+        const uint32_t c = (uint32_t)__popcll((m >> pos) & ((1ull << w) - 1ull));
+        if (n >= c) {
+            n -= c;
+            pos += w;
+        }
+    }
+    return pos;
+}
+
 // Atomics on global memory through a global-address-space pointer: no flat-address
 // (LDS / scratch aperture) checks are generated around them.
 typedef __attribute__((address_space(1))) uint32_t global_u32;
@@ -203,6 +237,7 @@ struct gpurt_bvh_s {
     void *mesh_mem = nullptr, *node_mem = nullptr;
     void* nodes = nullptr;        // WNode<W>[node_capacity] (boxes in FP32; refit updates these)
     void* qnodes = nullptr;       // QNode<W>[n_nodes] when has_qnodes(format)
+    void* onodes = nullptr;       // ONode[n_nodes] when cpq_use_oriented(format, width)
     uint32_t* node_first = nullptr;  // first packed triangle of each node's (contiguous) range
     int format = 1;
     float4* tris = nullptr;       // 3 * n_tris
@@ -345,6 +380,15 @@ void launch_range_top(uint32_t N, float4* rbox, hipStream_t s);
 // (then `capacity` threads are launched), else n_host
 void launch_quantize(int width, const void* nodes, void* qnodes, uint32_t n_host, uint32_t capacity,
                      const uint32_t* n_dev, hipStream_t s);
+
+// oriented copies of 4-wide nodes (oriented.hip): nodes [0, n) with n = *n_dev when n_dev is
+// given (at most capacity), else n_host.  first: each node's first packed triangle (its
+// triangles are contiguous); scale: each mesh's largest coordinate as an ordered uint,
+// scale_stride words apart, of mesh seg[node] (0 without seg); skip (or null): a device
+// word that, when set, leaves everything as it is
+void launch_orient(const void* nodes, const uint32_t* first, const float4* tris, void* onodes, uint32_t n_host,
+                   uint32_t capacity, const uint32_t* n_dev, const uint32_t* scale, uint32_t scale_stride,
+                   const uint32_t* seg, const uint32_t* skip, hipStream_t s);
 
 // traversal launch planning (query.hip): stack depth, block size, grid, spill slots and
 // leaf trigger for one launch of a query kind, and the per-call scratch (queue counters

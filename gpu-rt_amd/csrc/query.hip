@@ -33,10 +33,10 @@ struct TravArgs {
     uint32_t leaf_trigger;  // 1..64, see leaf_step_now
 };
 
-template <int W, bool Q, int S, int BS, bool STATS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, Q>::value))) void k_cpq(
+template <int W, int E, int S, int BS, bool STATS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, E>::value))) void k_cpq(
     TravArgs a) {
-    const NodeOf<W, Q>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, Q>*>(a.nodes);
+    const NodeOf<W, E>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, E>*>(a.nodes);
     const uint32_t total = gridDim.x * BS;
     const uint32_t gid = blockIdx.x * BS + threadIdx.x;
     LaneStack<S, BS> st;
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W,
     unsigned long long n_nodes = 0, n_tris = 0;
     QueueSource src{nullptr, a.q, a.n, first_query(gid, total), total, a.counter};
     auto out = [&](uint32_t qi, uint32_t id) { a.prim[qi] = id == 0xFFFFFFFFu ? -1 : (int32_t)id; };
-    if (!cpq_stream<NodeOf<W, Q>, S, BS, STATS>(nodes, a.tris, src, a.leaf_trigger, st, out, n_nodes, n_tris))
+    if (!cpq_stream<NodeOf<W, E>, S, BS, STATS>(nodes, a.tris, src, a.leaf_trigger, st, out, n_nodes, n_tris))
         gatomic_or(a.err, 1u);
     if (STATS) {
         atomicAdd(&a.stats[0], n_nodes);
@@ -53,10 +53,10 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W,
     }
 }
 
-template <int W, bool Q, int S, int BS, bool ANY, bool STATS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, Q>::value))) void k_ray(
+template <int W, int E, int S, int BS, bool ANY, bool STATS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W, E>::value))) void k_ray(
     TravArgs a) {
-    const NodeOf<W, Q>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, Q>*>(a.nodes);
+    const NodeOf<W, E>* __restrict__ nodes = reinterpret_cast<const NodeOf<W, E>*>(a.nodes);
     const uint32_t total = gridDim.x * BS;
     const uint32_t gid = blockIdx.x * BS + threadIdx.x;
     LaneStack<S, BS> st;
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WavesHint<W,
             }
         }
     };
-    if (!ray_stream<NodeOf<W, Q>, S, BS, ANY, STATS>(nodes, a.tris, src, a.leaf_trigger, st, out, n_nodes, n_tris))
+    if (!ray_stream<NodeOf<W, E>, S, BS, ANY, STATS>(nodes, a.tris, src, a.leaf_trigger, st, out, n_nodes, n_tris))
         gatomic_or(a.err, 1u);
     if (STATS) {
         atomicAdd(&a.stats[0], n_nodes);
@@ -93,29 +93,31 @@ __global__ void k_clear_counters(uint32_t* c) {
 // launch plumbing
 // ------------------------------------------------------------------------------------
 
-template <int W, bool Q, int S, int BS, bool STATS>
+template <int W, int E, int S, int BS, bool STATS>
 static void launch_kind(QKind kind, const TravArgs& a, unsigned grid, hipStream_t s) {
-    switch (kind) {
+    if constexpr (E == kEncOriented) {
+        hipLaunchKernelGGL((k_cpq<W, E, S, BS, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+    } else switch (kind) {
         case QKind::Cpq:
-            hipLaunchKernelGGL((k_cpq<W, Q, S, BS, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+            hipLaunchKernelGGL((k_cpq<W, E, S, BS, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
             break;
         case QKind::Closest:
-            hipLaunchKernelGGL((k_ray<W, Q, S, BS, false, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+            hipLaunchKernelGGL((k_ray<W, E, S, BS, false, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
             break;
         case QKind::Any:
-            hipLaunchKernelGGL((k_ray<W, Q, S, BS, true, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
+            hipLaunchKernelGGL((k_ray<W, E, S, BS, true, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kGroupKeyBytes) * BS, s, a);
             break;
     }
 }
 
 // LDS per block is S * BS * 8 bytes: 16 KB for S = 8, 32 KB for the others.
-template <int W, bool Q, bool STATS>
+template <int W, int E, bool STATS>
 static int dispatch_stack(int S, QKind kind, const TravArgs& a, unsigned grid, hipStream_t s) {
     switch (S) {
-        case 8: launch_kind<W, Q, 8, 256, STATS>(kind, a, grid, s); return 256;
-        case 16: launch_kind<W, Q, 16, 256, STATS>(kind, a, grid, s); return 256;
-        case 32: launch_kind<W, Q, 32, 128, STATS>(kind, a, grid, s); return 128;
-        case 64: launch_kind<W, Q, 64, 64, STATS>(kind, a, grid, s); return 64;
+        case 8: launch_kind<W, E, 8, 256, STATS>(kind, a, grid, s); return 256;
+        case 16: launch_kind<W, E, 16, 256, STATS>(kind, a, grid, s); return 256;
+        case 32: launch_kind<W, E, 32, 128, STATS>(kind, a, grid, s); return 128;
+        case 64: launch_kind<W, E, 64, 64, STATS>(kind, a, grid, s); return 64;
     }
     return 0;
 }
@@ -154,8 +156,8 @@ int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need
     // and by registers (WavesHint waves per SIMD), unless the caller asks for waves/CU
     const int waves_per_block = p.BS / 64;
     const int hint = waves_per_simd > 0 ? waves_per_simd
-                     : width == 8 ? (q8 ? WavesHint<8, true>::value : WavesHint<8, false>::value)
-                                  : (q8 ? WavesHint<4, true>::value : WavesHint<4, false>::value);
+                     : width == 8 ? (q8 ? WavesHint<8, kEncQ8>::value : WavesHint<8>::value)
+                                  : (q8 ? WavesHint<4, kEncQ8>::value : WavesHint<4>::value);
     int blocks_per_cu = std::min(ctx->lds_per_cu / ((p.S * 8 + lds_extra) * p.BS), std::min(32, 4 * hint) / waves_per_block);
     if (opts && opts->waves_per_cu > 0)
         blocks_per_cu = std::max(1, opts->waves_per_cu / waves_per_block);
@@ -289,20 +291,24 @@ static int run_query(gpurt_bvh_s* b, QKind kind, TravArgs a, size_t n, const gpu
     a.leaf_trigger = p.leaf_trigger;
     const bool stats = a.stats != nullptr;
     int bs = 0;
-    a.nodes = q8 ? b->qnodes : b->nodes;
-    switch (b->width * 4 + (q8 ? 2 : 0) + (stats ? 1 : 0)) {
-        case 8: bs = dispatch_stack<2, false, false>(p.S, kind, a, p.grid, s); break;
-        case 9: bs = dispatch_stack<2, false, true>(p.S, kind, a, p.grid, s); break;
-        case 10: bs = dispatch_stack<2, true, false>(p.S, kind, a, p.grid, s); break;
-        case 11: bs = dispatch_stack<2, true, true>(p.S, kind, a, p.grid, s); break;
-        case 16: bs = dispatch_stack<4, false, false>(p.S, kind, a, p.grid, s); break;
-        case 17: bs = dispatch_stack<4, false, true>(p.S, kind, a, p.grid, s); break;
-        case 18: bs = dispatch_stack<4, true, false>(p.S, kind, a, p.grid, s); break;
-        case 19: bs = dispatch_stack<4, true, true>(p.S, kind, a, p.grid, s); break;
-        case 32: bs = dispatch_stack<8, false, false>(p.S, kind, a, p.grid, s); break;
-        case 33: bs = dispatch_stack<8, false, true>(p.S, kind, a, p.grid, s); break;
-        case 34: bs = dispatch_stack<8, true, false>(p.S, kind, a, p.grid, s); break;
-        case 35: bs = dispatch_stack<8, true, true>(p.S, kind, a, p.grid, s); break;
+    const bool oriented = kind == QKind::Cpq && cpq_use_oriented(b->format, b->width);
+    a.nodes = oriented ? b->onodes : (q8 ? b->qnodes : b->nodes);
+    if (oriented)
+        bs = stats ? dispatch_stack<4, kEncOriented, true>(p.S, kind, a, p.grid, s)
+                   : dispatch_stack<4, kEncOriented, false>(p.S, kind, a, p.grid, s);
+    else switch (b->width * 4 + (q8 ? 2 : 0) + (stats ? 1 : 0)) {
+        case 8: bs = dispatch_stack<2, kEncF32, false>(p.S, kind, a, p.grid, s); break;
+        case 9: bs = dispatch_stack<2, kEncF32, true>(p.S, kind, a, p.grid, s); break;
+        case 10: bs = dispatch_stack<2, kEncQ8, false>(p.S, kind, a, p.grid, s); break;
+        case 11: bs = dispatch_stack<2, kEncQ8, true>(p.S, kind, a, p.grid, s); break;
+        case 16: bs = dispatch_stack<4, kEncF32, false>(p.S, kind, a, p.grid, s); break;
+        case 17: bs = dispatch_stack<4, kEncF32, true>(p.S, kind, a, p.grid, s); break;
+        case 18: bs = dispatch_stack<4, kEncQ8, false>(p.S, kind, a, p.grid, s); break;
+        case 19: bs = dispatch_stack<4, kEncQ8, true>(p.S, kind, a, p.grid, s); break;
+        case 32: bs = dispatch_stack<8, kEncF32, false>(p.S, kind, a, p.grid, s); break;
+        case 33: bs = dispatch_stack<8, kEncF32, true>(p.S, kind, a, p.grid, s); break;
+        case 34: bs = dispatch_stack<8, kEncQ8, false>(p.S, kind, a, p.grid, s); break;
+        case 35: bs = dispatch_stack<8, kEncQ8, true>(p.S, kind, a, p.grid, s); break;
         default: break;
     }
     hipError_t le = hipGetLastError();

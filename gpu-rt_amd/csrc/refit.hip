@@ -141,6 +141,9 @@ int launch_refit(gpurt_bvh_s* b, const float* verts, size_t vstride_floats, hipS
     // (unchanged boxes give the same copies)
     if (has_qnodes(b->format)) launch_quantize(b->width, b->nodes, b->qnodes, (uint32_t)b->n_nodes,
                                                 (uint32_t)b->n_nodes, nullptr, s);
+    if (b->onodes)
+        launch_orient(b->nodes, b->node_first, b->tris, b->onodes, (uint32_t)b->n_nodes, (uint32_t)b->n_nodes, nullptr,
+                      tmp, 0, nullptr, tmp + 1, s);
     const hipError_t e = hipGetLastError();
     uint32_t bad = 0;
     hipError_t ce = hipMemcpyAsync(&bad, tmp + 1, sizeof(bad), hipMemcpyDeviceToHost, s);

@@ -16,6 +16,7 @@
 #pragma once
 
 #include "gpurt_internal.h"
+#include "oriented.h"
 #include "tri_math.h"
 
 #include <type_traits>
@@ -244,8 +245,10 @@ __device__ __forceinline__ void fetch_node(const QNode<W>* __restrict__ nodes, u
     }
 }
 
-template <int W, bool Q>
-using NodeOf = typename std::conditional<Q, QNode<W>, WNode<W>>::type;
+// node type of an encoding (kEncOriented: 4-wide, closest points only)
+template <int W, int E>
+using NodeOf = typename std::conditional<
+    E == kEncF32, WNode<W>, typename std::conditional<E == kEncQ8, QNode<W>, ONode>::type>::type;
 
 // Ray / child-box slab tests of one wide node: tn[j] = entry distance of child j and c[j]
 // its child word, or INFINITY / kEmpty when the ray's [tmin, best] misses the box.  The
@@ -361,6 +364,63 @@ __device__ __forceinline__ void ray_children(const QNode<W>* __restrict__ nodes,
 // closest point
 // ------------------------------------------------------------------------------------
 
+// Squared distances dd[j] of a point to the child boxes of one wide node (INFINITY for an
+// empty slot) and the child words c[j].
+template <int W, typename NodeT>
+__device__ __forceinline__ void point_children(const NodeT* __restrict__ nodes, uint32_t i, V3 q, float (&dd)[W],
+                                               uint32_t (&c)[W]) {
+    ChildBoxes<W> nd;
+    fetch_node(nodes, i, nd);
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        const float dx = fmaxf(fmaxf(nd.lox[j] - q.x, q.x - nd.hix[j]), 0.0f);
+        const float dy = fmaxf(fmaxf(nd.loy[j] - q.y, q.y - nd.hiy[j]), 0.0f);
+        const float dz = fmaxf(fmaxf(nd.loz[j] - q.z, q.z - nd.hiz[j]), 0.0f);
+        c[j] = nd.child[j];
+        dd[j] = (c[j] == kEmpty) ? INFINITY : fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    }
+}
+
+// Oriented node: the point goes into the node's frame and into the units of its byte
+// planes once (so no plane is decoded), and its offset from a child's box on an axis is
+// what a median-of-three clamp leaves over.  The clamp of q - c keeps every term finite;
+// it moves only points whose squared distance overflows.
+template <int W>
+__device__ __forceinline__ void point_children(const ONode* __restrict__ nodes, uint32_t i, V3 q, float (&dd)[W],
+                                               uint32_t (&c)[W]) {
+    static_assert(W == 4, "oriented nodes are 4-wide");
+    const uint4* p = reinterpret_cast<const uint4*>(nodes + i);
+    uint32_t w[16];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint4 v = p[k];
+        w[4 * k] = v.x;
+        w[4 * k + 1] = v.y;
+        w[4 * k + 2] = v.z;
+        w[4 * k + 3] = v.w;
+    }
+    const Frame R(__uint_as_float(w[4]), __uint_as_float(w[5]));
+    constexpr float kFar = 5e37f;
+    const V3 y = R.to_local(v3(__builtin_amdgcn_fmed3f(q.x - __uint_as_float(w[0]), -kFar, kFar),
+                               __builtin_amdgcn_fmed3f(q.y - __uint_as_float(w[1]), -kFar, kFar),
+                               __builtin_amdgcn_fmed3f(q.z - __uint_as_float(w[2]), -kFar, kFar)));
+    const uint32_t e = w[3], ei = 0x00FEFEFEu - e;  // exponents of the steps and of their inverses
+    const float sx = __uint_as_float((e & 0xFFu) << 23), sy = __uint_as_float((e & 0xFF00u) << 15),
+                sz = __uint_as_float((e & 0xFF0000u) << 7);
+    const float X = fmaf(y.x, __uint_as_float((ei & 0xFFu) << 23), 128.0f);
+    const float Y = fmaf(y.y, __uint_as_float((ei & 0xFF00u) << 15), 128.0f);
+    const float Z = fmaf(y.z, __uint_as_float((ei & 0xFF0000u) << 7), 128.0f);
+    auto qb = [&](int row, int j) -> float { return (float)((w[10 + row] >> (8 * j)) & 0xFFu); };
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float dx = (X - __builtin_amdgcn_fmed3f(X, qb(0, j), qb(3, j))) * sx;
+        const float dy = (Y - __builtin_amdgcn_fmed3f(Y, qb(1, j), qb(4, j))) * sy;
+        const float dz = (Z - __builtin_amdgcn_fmed3f(Z, qb(2, j), qb(5, j))) * sz;
+        c[j] = w[6 + j];
+        dd[j] = (c[j] == kEmpty) ? INFINITY : fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    }
+}
+
 // Resident waves per SIMD the register allocator targets: 7 (<= 72 VGPRs) for 2- and
 // 4-wide nodes.  At 8 (64 VGPRs) the 4-wide closest-hit kernel spilled 5 VGPRs to
 // scratch and 20 SGPRs to VGPR lanes, reloading them with v_readlane in the loop; at 7
@@ -370,7 +430,7 @@ __device__ __forceinline__ void ray_children(const QNode<W>* __restrict__ nodes,
 // waves per CU each (the two-stream ray step) still run side by side as fast as before.
 // 8-wide nodes need more live registers for the child boxes and sort keys, so they get
 // what they need (5-7 waves).
-template <int W, bool Q = false>
+template <int W, int E = kEncF32>
 struct WavesHint {
     static constexpr int value = W == 8 ? 4 : 7;
 };
@@ -523,20 +583,6 @@ struct QueueSource {
 // every lane culls only against a value that some primitive (or the query's own limit)
 // reached, so the answer is the one a single lane finds.
 // ------------------------------------------------------------------------------------
-
-// position of the n-th (from 0) set bit of m; n < popcount(m)
-__device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t n) {
-    uint32_t pos = 0;
-#pragma unroll
-    for (uint32_t w = 32; w >= 1; w >>= 1) {
-        const uint32_t c = (uint32_t)__popcll((m >> pos) & ((1ull << w) - 1ull));
-        if (n >= c) {
-            n -= c;
-            pos += w;
-        }
-    }
-    return pos;
-}
 
 __device__ __forceinline__ uint64_t lanes_below() {
     const uint32_t lane = __lane_id();
@@ -1023,18 +1069,9 @@ __device__ __forceinline__ bool cpq_stream(const NodeT* __restrict__ nodes, cons
         }
         if (!node_ready) continue;
         if (STATS) n_nodes++;
-        ChildBoxes<W> nd;
-        fetch_node(nodes, cur, nd);
         float dd[W];
         uint32_t c[W];
-#pragma unroll
-        for (int j = 0; j < W; j++) {
-            const float dx = fmaxf(fmaxf(nd.lox[j] - q.x, q.x - nd.hix[j]), 0.0f);
-            const float dy = fmaxf(fmaxf(nd.loy[j] - q.y, q.y - nd.hiy[j]), 0.0f);
-            const float dz = fmaxf(fmaxf(nd.loz[j] - q.z, q.z - nd.hiz[j]), 0.0f);
-            c[j] = nd.child[j];
-            dd[j] = (c[j] == kEmpty) ? INFINITY : fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-        }
+        point_children<W>(nodes, cur, q, dd, c);
         sort_children<W>(dd, c);
         have = false;
         bool hit[W];

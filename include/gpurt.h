@@ -84,7 +84,9 @@ typedef struct gpurt_build_opts {
                                1 = FP32 child boxes (32*W bytes per node),
                                2 = 8-bit child boxes relative to the node's box
                                    (48/64/96 bytes for W = 2/4/8),
-                               3 = both: 8-bit for rays, FP32 for closest points,
+                               3 = 8-bit for rays; for closest points 8-bit boxes in a
+                                   frame of each node's own (W = 4, 64 bytes) or FP32
+                                   boxes (W = 2, 8),
                                0 = library default (3)                                */
 } gpurt_build_opts;
 
