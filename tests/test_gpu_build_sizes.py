@@ -142,3 +142,43 @@ def test_memory_of_closed_bvhs_is_reused_in_order(dev):
     for k, p in enumerate(got):
         assert np.array_equal(p.cpu().numpy(), exp[k % 4]), k
     ctx.close()
+
+
+def _best_sah(V, F):
+    """Least SAH cost of any binary tree over the triangles, one per leaf, without the
+    root's own term and over the root's area (1.2 per unit of inner area, 1 per leaf's)."""
+    n = F.shape[0]
+    t = V[F].astype(np.float64)
+    area, cost = np.zeros(1 << n), np.zeros(1 << n)
+    for s in range(1, 1 << n):
+        p = t[[j for j in range(n) if s >> j & 1]].reshape(-1, 3)
+        e = p.max(0) - p.min(0)
+        area[s] = 2 * (e[0] * e[1] + e[1] * e[2] + e[0] * e[2])
+    for s in range(1, 1 << n):
+        low = s & -s
+        if s == low:
+            cost[s] = area[s]
+            continue
+        best, p = np.inf, (s - 1) & s
+        while p:
+            if p & low:
+                best = min(best, cost[p] + cost[s ^ p])
+            p = (p - 1) & s
+        cost[s] = 1.2 * area[s] + best
+    full = (1 << n) - 1
+    return (cost[full] - 1.2 * area[full]) / area[full]
+
+
+@pytest.mark.parametrize("tsize", [5, 6, 7])
+@pytest.mark.parametrize("n", [3, 4, 5, 6, 7])
+def test_treelet_of_the_whole_mesh_is_optimal(ctx, dev, n, tsize):
+    """With at most tsize triangles the root's treelet is the whole tree: its topology is the
+    best of all (boxes carry an inflation of 2^-18 of the coordinates, under 1e-3 of the
+    cost of boxes of about 0.05)."""
+    if n > tsize:
+        pytest.skip("more triangles than a treelet has leaves")
+    for seed in range(4):
+        V, F = _soup(n, 100 * n + seed)
+        bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev), node_width=2, leaf_size=1, treelet_size=tsize)
+        want = _best_sah(V, F)
+        assert abs(bvh.info()["sah_cost"] - want) <= 2e-3 * want, (seed, bvh.info()["sah_cost"], want)
