@@ -398,6 +398,7 @@ struct TravPlan {
     int S = 8, BS = 256;
     unsigned grid = 1;
     uint32_t total = 256, spill_slots = 0, leaf_trigger = 32;
+    size_t n = 0;  // queries of the launch
 };
 // Device scratch of one query or backward call.  Outside graph capture it is the
 // context's buffer for the call's stream: grown when a call needs more (hipMalloc, after
@@ -435,7 +436,7 @@ void free_traversal_scratch(gpurt_ctx_s* c, TravScratch& t);
 // the same scratch in memory the caller holds
 size_t traversal_scratch_bytes(const TravPlan& p);
 void carve_traversal_scratch(const TravPlan& p, void* mem, TravScratch& t);
-void clear_traversal_counters(const TravScratch& t, hipStream_t s);
+void clear_traversal_counters(const TravPlan& p, const TravScratch& t, hipStream_t s);
 
 // traversal launchers (query.hip)
 int launch_cpq(gpurt_bvh_s* b, const float* q, size_t n, int32_t* prim, float* pt, float* dist,

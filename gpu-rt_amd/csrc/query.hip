@@ -139,6 +139,9 @@ static uint32_t default_leaf_trigger(QKind) { return 32u; }
 static uint32_t default_refill_trigger(QKind kind) { return kind == QKind::Closest ? 24u : 16u; }
 static int default_waves_per_cu(QKind kind) { return kind == QKind::Cpq ? 16 : 28; }
 
+// waves per CU up to which a small set gets a wave per query (plan_traversal)
+constexpr size_t kWidePoints = 16, kWideRays = 8;
+
 static int block_for_stack(int S) { return S <= 16 ? 256 : (S == 32 ? 128 : 64); }
 
 int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need, const gpurt_query_opts* opts,
@@ -164,12 +167,22 @@ int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need
     else if (default_waves_per_cu(kind) > 0)
         blocks_per_cu = std::min(blocks_per_cu, std::max(1, default_waves_per_cu(kind) / waves_per_block));
     blocks_per_cu = std::max(blocks_per_cu, 1);
-    // up to kSpread lanes per query: a small set is spread over more waves (first_query),
-    // whose idle lanes take work from the busy ones once the queues are empty
-    constexpr size_t kSpread = 4;
-    p.grid = (unsigned)std::min<size_t>(cdiv(n * kSpread, p.BS), (size_t)ctx->n_cu * blocks_per_cu);
+    // A small set is spread over more lanes than it has queries (first_query); the idle
+    // ones take work from the busy ones once the queues are empty.  A launch of few queries
+    // is one chain of visits, so it gets a wave per query -- until the launch holds kWide
+    // waves per CU, all that run at once for points; for rays fewer, since a wave with
+    // less than 16 rays starts its donation late (65,536 rays on rays_scene 119 us with 8
+    // waves per CU, 137 us with the 28 a launch may hold) -- and 4 lanes per query beyond
+    // that.  Against 4 lanes for every set, us: 100 points on 1,200 triangles 58 -> 46,
+    // 1,000 near 252,000 triangles 91 -> 57, 20,000 on 1.3 M 261 -> 220; 100 rays on 2.3 M
+    // triangles 70 -> 65, 1,000 on 236,000 66 -> 55, 100 on the same scene as instances
+    // 88 -> 73.
+    const size_t wide = (size_t)ctx->n_cu * (kind == QKind::Cpq ? kWidePoints : kWideRays) * 64;
+    const size_t lanes = std::max(n * 4, std::min(n * 64, wide));
+    p.grid = (unsigned)std::min<size_t>(cdiv(lanes, p.BS), (size_t)ctx->n_cu * blocks_per_cu);
     if (p.grid == 0) p.grid = 1;
     p.total = p.grid * p.BS;
+    p.n = n;
     // the part of the worst-case stack beyond the LDS slots spills to device memory
     p.spill_slots = stack_need > p.S ? (uint32_t)(stack_need - p.S) : 0u;
     p.leaf_trigger = opts && opts->leaf_trigger ? (uint32_t)opts->leaf_trigger : default_leaf_trigger(kind);
@@ -191,7 +204,11 @@ void carve_traversal_scratch(const TravPlan& p, void* mem, TravScratch& t) {
     t.spill = p.spill_slots ? (uint2*)((char*)mem + kCounterBytes) : nullptr;
 }
 
-void clear_traversal_counters(const TravScratch& t, hipStream_t s) {
+// Lanes read the counters only for the queries beyond their first ones, so a set with no
+// more queries than lanes does without the clearing launch (3-5 us of a call that takes
+// 45-70 us in all).
+void clear_traversal_counters(const TravPlan& p, const TravScratch& t, hipStream_t s) {
+    if (p.n <= p.total) return;
     hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(kQueues), 0, s, t.counters);
 }
 
@@ -204,7 +221,7 @@ int alloc_traversal_scratch(gpurt_ctx_s* c, const TravPlan& p, hipStream_t s, Tr
     }
     carve_traversal_scratch(p, cs.mem, t);
     t.cs = cs;
-    clear_traversal_counters(t, s);
+    clear_traversal_counters(p, t, s);
     return GPURT_OK;
 }
 
@@ -275,7 +292,7 @@ static int run_query(gpurt_bvh_s* b, QKind kind, TravArgs a, size_t n, const gpu
     if (fixed_scratch) {
         if ((rc = fit_plan_to_scratch(p, fixed_bytes))) return rc;
         carve_traversal_scratch(p, fixed_scratch, t);
-        clear_traversal_counters(t, s);
+        clear_traversal_counters(p, t, s);
         t.mem = nullptr;  // not freed below
     } else if ((rc = alloc_traversal_scratch(b->ctx, p, s, t))) {
         return rc;

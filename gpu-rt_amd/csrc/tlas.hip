@@ -842,7 +842,7 @@ int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t*
         if (scratch_bytes < traversal_scratch_bytes(p))
             return set_error(GPURT_E_INVALID, "traversal scratch buffer too small");
         carve_traversal_scratch(p, scratch, sc);
-        clear_traversal_counters(sc, s);
+        clear_traversal_counters(p, sc, s);
     } else if ((rc = alloc_traversal_scratch(T->ctx, p, s, sc))) {
         return rc;
     }
