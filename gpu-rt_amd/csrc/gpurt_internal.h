@@ -398,8 +398,19 @@ struct TravPlan {
     int S = 8, BS = 256;
     unsigned grid = 1;
     uint32_t total = 256, spill_slots = 0, leaf_trigger = 32;
-    size_t n = 0;  // queries of the launch
+    size_t n = 0;     // queries of the launch
+    size_t wide = 0;  // lanes up to which each query gets a wave (spread_lanes)
 };
+// work queues of a launch: counters at the start of the traversal scratch, kQueueStride
+// words apart (traverse.h)
+constexpr uint32_t kQueues = 256;
+constexpr uint32_t kQueueStride = 64;
+// lanes that a set of n queries is spread over: a wave per query up to `wide` lanes, 4
+// lanes per query beyond (plan_traversal)
+__host__ __device__ inline size_t spread_lanes(size_t n, size_t wide) {
+    const size_t w = n * 64 < wide ? n * 64 : wide;
+    return n * 4 > w ? n * 4 : w;
+}
 // Device scratch of one query or backward call.  Outside graph capture it is the
 // context's buffer for the call's stream: grown when a call needs more (hipMalloc, after
 // a device wait to free the old one), reused by the next call on that stream without an
@@ -466,12 +477,20 @@ int launch_refit(gpurt_bvh_s* b, const float* verts, size_t vstride_floats, hipS
 // and the BLAS
 int tlas_host_info(gpurt_tlas t, gpurt_ctx* ctx, const std::vector<uint32_t>** custom,
                    const std::vector<gpurt_bvh_s*>** blas);
+// A second ray list of a closest-hit launch, in the caller's scratch: only the object hit
+// is written (-1: none).  The caller has cleared the queue counters of the scratch.
+struct TlasSecond {
+    const gpurt_ray* rays;
+    size_t n;               // capacity of the list
+    const uint32_t* n_dev;  // its length in device memory; nullptr: no list
+    int32_t* obj;
+};
 // TLAS traversal for wavefront callers (tlas.hip): the ray count may be read from device
 // memory at launch (n_dev, at most n) and the traversal scratch may be the caller's
-// (scratch of >= tlas_scratch_bytes(T, n) bytes; nullptr: allocated per call)
+// (scratch of >= tlas_scratch_bytes(T, n + second's n) bytes; nullptr: allocated per call)
 int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t* n_dev, int32_t* obj,
                   int32_t* prim, float* t, float* uv, uint8_t* occ, bool any, const gpurt_query_opts* opts,
-                  hipStream_t s, void* scratch, size_t scratch_bytes);
+                  hipStream_t s, void* scratch, size_t scratch_bytes, const TlasSecond* second = nullptr);
 size_t tlas_scratch_bytes(gpurt_tlas T, size_t n);
 // records a use of the TLAS (and through it of its BLASes) on stream s (tlas.hip)
 void tlas_note_use(gpurt_tlas t, hipStream_t s);

@@ -177,9 +177,8 @@ int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need
     // 1,000 near 252,000 triangles 91 -> 57, 20,000 on 1.3 M 261 -> 220; 100 rays on 2.3 M
     // triangles 70 -> 65, 1,000 on 236,000 66 -> 55, 100 on the same scene as instances
     // 88 -> 73.
-    const size_t wide = (size_t)ctx->n_cu * (kind == QKind::Cpq ? kWidePoints : kWideRays) * 64;
-    const size_t lanes = std::max(n * 4, std::min(n * 64, wide));
-    p.grid = (unsigned)std::min<size_t>(cdiv(lanes, p.BS), (size_t)ctx->n_cu * blocks_per_cu);
+    p.wide = (size_t)ctx->n_cu * (kind == QKind::Cpq ? kWidePoints : kWideRays) * 64;
+    p.grid = (unsigned)std::min<size_t>(cdiv(spread_lanes(n, p.wide), p.BS), (size_t)ctx->n_cu * blocks_per_cu);
     if (p.grid == 0) p.grid = 1;
     p.total = p.grid * p.BS;
     p.n = n;

@@ -411,6 +411,17 @@ __device__ __forceinline__ bool tlas_ray_stream(const NodeT* __restrict__ top_no
 template <int W>
 constexpr int kTlasWaves = W == 8 ? 4 : 6;
 
+// Two ray lists as one set: rays [0, n1) of the first, then the second list's.
+struct PairSource : QueueSource {
+    const float4* rays2;
+    uint32_t n1;
+    __device__ __forceinline__ void ray(Handle h, float4& r0, float4& r1) const {
+        const float4* const p = h < n1 ? rays + 2 * (size_t)h : rays2 + 2 * (size_t)(h - n1);
+        r0 = p[0];
+        r1 = p[1];
+    }
+};
+
 struct TlasArgs {
     const void* top_nodes;
     const float4* top_tris;
@@ -418,6 +429,11 @@ struct TlasArgs {
     const float4* rays;
     uint32_t n;             // rays (or, with n_dev, the capacity of the ray array)
     const uint32_t* n_dev;  // nullable: the ray count, read from device memory at launch
+    const float4* rays2;    // the second list: capacity, length in device memory (nullable),
+    uint32_t n2;            // object of each hit
+    const uint32_t* n2_dev;
+    int32_t* obj2;
+    uint32_t wide;  // of spread_lanes
     int32_t* obj;
     int32_t* prim;
     float* t;
@@ -435,15 +451,28 @@ struct TlasArgs {
 template <int W, bool Q, int S, int BS, bool ANY, bool STATS>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kTlasWaves<W>))) void k_tlas_ray(
     TlasArgs a) {
-    const uint32_t total = gridDim.x * BS;
+    const uint32_t n1 = a.n_dev ? min(*a.n_dev, a.n) : a.n;
+    const uint32_t n2 = a.n2_dev ? min(*a.n2_dev, a.n2) : 0u;
+    // A launch sized for a list's capacity takes as many of its blocks as the list's true
+    // length would be given (they are fewer than the grid only when every query is some
+    // lane's first, so the queues' share by grid stays right): the late bounces of a
+    // frame hold a few thousand of 460,000 rays, and waves with a ray or two each find no
+    // idle lanes to help them.
+    uint32_t blocks = gridDim.x;
+    if (a.n_dev) {
+        blocks = (uint32_t)min((size_t)blocks, (spread_lanes((size_t)n1 + n2, a.wide) + BS - 1) / BS);
+        if (blockIdx.x >= blocks) return;
+    }
+    const uint32_t total = blocks * BS;
     const uint32_t gid = blockIdx.x * BS + threadIdx.x;
     LaneStack<S, BS> st;
     st.init(a.spill, a.spill_slots, gid, total);
-    const uint32_t n = a.n_dev ? min(*a.n_dev, a.n) : a.n;
-    QueueSource src{a.rays, nullptr, n, first_query(gid, total), total, a.counter};
+    PairSource src{{a.rays, nullptr, n1 + n2, first_query(gid, total), total, a.counter}, a.rays2, n1};
     auto out = [&](uint32_t ri, uint32_t obj, uint32_t id, float t, float u, float v, bool any) {
         if (ANY) {
             a.occ[ri] = any ? 1 : 0;
+        } else if (ri >= n1) {
+            a.obj2[ri - n1] = id != 0xFFFFFFFFu ? (int32_t)obj : -1;
         } else {
             const bool hit = id != 0xFFFFFFFFu;
             a.obj[ri] = hit ? (int32_t)obj : -1;
@@ -822,7 +851,7 @@ void tlas_orphan(gpurt_tlas t) {
 
 int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t* n_dev, int32_t* obj,
                   int32_t* prim, float* t, float* uv, uint8_t* occ, bool any, const gpurt_query_opts* opts,
-                  hipStream_t stream, void* scratch, size_t scratch_bytes) {
+                  hipStream_t stream, void* scratch, size_t scratch_bytes, const TlasSecond* second) {
     if (!T) return set_error(GPURT_E_INVALID, "null tlas");
     if (n == 0) return GPURT_OK;
     if (!rays || (any ? !occ : (!obj || !prim || !t))) return set_error(GPURT_E_INVALID, "null ray/output pointer");
@@ -835,14 +864,15 @@ int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t*
     hipStream_t s = stream;
     const int W = T->width;
     TravPlan p;
-    int rc = tlas_plan(T, n, any, opts, p);
+    const size_t n2 = second && second->n_dev ? second->n : 0;
+    int rc = tlas_plan(T, n + n2, any, opts, p);
     if (rc) return rc;
     TravScratch sc;
     if (scratch) {  // the caller's buffer: clear the queue counters, keep the memory
         if (scratch_bytes < traversal_scratch_bytes(p))
             return set_error(GPURT_E_INVALID, "traversal scratch buffer too small");
         carve_traversal_scratch(p, scratch, sc);
-        clear_traversal_counters(p, sc, s);
+        if (!second) clear_traversal_counters(p, sc, s);
     } else if ((rc = alloc_traversal_scratch(T->ctx, p, s, sc))) {
         return rc;
     }
@@ -853,6 +883,13 @@ int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t*
     a.rays = reinterpret_cast<const float4*>(rays);
     a.n = (uint32_t)n;
     a.n_dev = n_dev;
+    if (n2) {
+        a.rays2 = reinterpret_cast<const float4*>(second->rays);
+        a.n2 = (uint32_t)n2;
+        a.n2_dev = second->n_dev;
+        a.obj2 = second->obj;
+    }
+    a.wide = (uint32_t)p.wide;
     a.obj = obj;
     a.prim = prim;
     a.t = t;

@@ -502,9 +502,6 @@ __device__ __forceinline__ uint32_t first_query(uint32_t g, uint32_t total) {
 // atomics from serializing on one address (one shared counter costs ~0.1 ms per
 // million queries).  refill is called by all lanes together, so the pool stays
 // wave-uniform.
-constexpr uint32_t kQueues = 256;
-constexpr uint32_t kQueueStride = 64;  // uint32 words between counters
-
 struct QueueSource {
     using Handle = uint32_t;
     const float4* rays;

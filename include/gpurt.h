@@ -503,7 +503,7 @@ typedef struct gpurt_render_params {
     uint64_t* ray_counts; /* host, nullable: [0] += camera / bounce rays traced (closest hit),
                              [1] += shadow (any hit) or light (closest hit) rays traced */
     int32_t concurrency;  /* pixel groups rendered concurrently on their own streams, 1..8
-                             (0 = library default: 2 / 4 / 1 for integrators 0 / 1 / 2);
+                             (0 = library default: 1);
                              results do not depend on it */
     int32_t reserved;
 } gpurt_render_params;

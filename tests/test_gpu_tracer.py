@@ -262,3 +262,20 @@ def test_render_independent_of_pixel_groups(box, integrator):
     for img, g in imgs[1:]:
         assert torch.equal(img, imgs[0][0])
         assert all(torch.equal(x, y) for x, y in zip(g, imgs[0][1]))
+
+
+@pytest.mark.parametrize("samples,depth", [(1, 1), (1, 2), (2, 1), (2, 3), (3, 2), (5, 1)])
+@pytest.mark.parametrize("integrator", [1, 2])
+def test_few_samples_and_bounces(box, integrator, samples, depth):
+    """Light rays are traced with the next bounce's, or the next sample's camera rays, or in
+    a last launch of their own, and sums are added two samples late: the shortest chains."""
+    sc, scene = box
+    p = _params(sc, 37, 23, integrator=integrator, samples=samples, max_depth=depth, env_light=(0.1, 0.2, 0.05),
+                use_rr=0, seed=5)
+    print("render integrator", integrator, "samples", samples, "depth", depth, flush=True)
+    for conc in (1, 3):
+        img = scene.render(p["width"], p["height"], p["inv_view"], p["inv_proj"], concurrency=conc,
+                           **{k: p[k] for k in ("samples", "max_depth", "integrator", "brdf", "use_rr", "clear_col",
+                                                "env_light", "seed")})
+        torch.cuda.synchronize()
+        _agree(img.cpu().numpy(), O.render(sc["objects"], p))
