@@ -164,14 +164,14 @@ __device__ __forceinline__ void scatter_terms(const CornerTerms& t, float* g_ver
 //                  the sum of that key's terms in the wave (partial[p])
 //   k_run_sum      the first term of each key's run adds the partials of the waves the
 //                  run spans (one per 64 terms) and hands the total to the sink
-template <int BS>
-__global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const uint64_t* __restrict__ keys,
+template <int BS, typename K>
+__global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const K* __restrict__ keys,
                                                     const uint32_t* __restrict__ vals, const float* __restrict__ terms,
                                                     float* __restrict__ partial) {
     const uint32_t p = blockIdx.x * BS + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
     const bool in = p < m;
-    const uint64_t key = in ? keys[p] : ~0ull;
+    const K key = in ? keys[p] : ~(K)0;
     const bool head = in && (lane == 0 || keys[p - 1] != key);
     float x = 0.f, y = 0.f, z = 0.f;
     if (in) {
@@ -200,12 +200,12 @@ __global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const uint64_t* 
     }
 }
 
-template <int BS, typename Sink>
-__global__ __launch_bounds__(BS) void k_run_sum(uint32_t m, const uint64_t* __restrict__ keys,
+template <int BS, typename K, typename Sink>
+__global__ __launch_bounds__(BS) void k_run_sum(uint32_t m, const K* __restrict__ keys,
                                                 const float* __restrict__ partial, uint64_t none, Sink sink) {
     const uint32_t p = blockIdx.x * BS + threadIdx.x;
     if (p >= m) return;
-    const uint64_t key = keys[p];
+    const K key = keys[p];
     if (key >= none || (p > 0 && keys[p - 1] == key)) return;
     float x = partial[3 * (size_t)p], y = partial[3 * (size_t)p + 1], z = partial[3 * (size_t)p + 2];
     for (uint32_t q = (p | 63u) + 1u; q < m && keys[q] == key; q += 64u) {

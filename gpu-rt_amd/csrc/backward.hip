@@ -19,14 +19,13 @@
 namespace gpurt_impl {
 
 // term k = 3 * item + corner: key = its vertex (n_verts when there is none, sorted last),
-// value = k, terms[3k .. 3k+2] = the float3 to add
-__device__ __forceinline__ void write_terms(size_t i, const CornerTerms& t, uint32_t n_verts, uint64_t* __restrict__ keys,
-                                            uint32_t* __restrict__ vals, float* __restrict__ terms) {
+// terms[3k .. 3k+2] = the float3 to add
+__device__ __forceinline__ void write_terms(size_t i, const CornerTerms& t, uint32_t n_verts, uint32_t* __restrict__ keys,
+                                            float* __restrict__ terms) {
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         const size_t k = 3 * i + j;
         keys[k] = t.v[j] == kNoVertex ? n_verts : t.v[j];
-        vals[k] = (uint32_t)k;
         terms[3 * k] = t.c[j][0];
         terms[3 * k + 1] = t.c[j][1];
         terms[3 * k + 2] = t.c[j][2];
@@ -38,11 +37,11 @@ __global__ __launch_bounds__(kBlock) void k_cpq_bwd_terms(uint32_t n, const floa
                                                           const float* __restrict__ g,
                                                           const uint32_t* __restrict__ tri_idx, uint32_t n_tris,
                                                           const float* __restrict__ verts, uint32_t n_verts,
-                                                          float* __restrict__ g_q, uint64_t* __restrict__ keys,
-                                                          uint32_t* __restrict__ vals, float* __restrict__ terms) {
+                                                          float* __restrict__ g_q, uint32_t* __restrict__ keys,
+                                                          float* __restrict__ terms) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    write_terms(i, cpq_bwd_terms(i, q, prim, g, tri_idx, n_tris, verts, 3, g_q), n_verts, keys, vals, terms);
+    write_terms(i, cpq_bwd_terms(i, q, prim, g, tri_idx, n_tris, verts, 3, g_q), n_verts, keys, terms);
 }
 
 __global__ __launch_bounds__(kBlock) void k_ray_bwd_terms(uint32_t n, const float4* __restrict__ rays,
@@ -53,12 +52,10 @@ __global__ __launch_bounds__(kBlock) void k_ray_bwd_terms(uint32_t n, const floa
                                                           const uint32_t* __restrict__ tri_idx, uint32_t n_tris,
                                                           const float* __restrict__ verts, uint32_t n_verts,
                                                           float* __restrict__ g_o, float* __restrict__ g_d,
-                                                          uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                          float* __restrict__ terms) {
+                                                          uint32_t* __restrict__ keys, float* __restrict__ terms) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    write_terms(i, ray_bwd_terms(i, rays, prim, t, uv, g, tri_idx, n_tris, verts, 3, g_o, g_d), n_verts, keys, vals,
-                terms);
+    write_terms(i, ray_bwd_terms(i, rays, prim, t, uv, g, tri_idx, n_tris, verts, 3, g_o, g_d), n_verts, keys, terms);
 }
 
 __global__ __launch_bounds__(kBlock) void k_cpq_bwd(uint32_t n, const float* __restrict__ q,
@@ -98,8 +95,7 @@ namespace {
 struct TermScratch {
     void* mem = nullptr;
     CallScratch cs;
-    uint64_t *k0 = nullptr, *k1 = nullptr;
-    uint32_t *v0 = nullptr, *v1 = nullptr, *sort = nullptr;
+    uint32_t *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr, *sort = nullptr;
     float *terms = nullptr, *partial = nullptr;
 };
 
@@ -108,15 +104,15 @@ int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
     const size_t m = 3 * n;
     const size_t words = radix_sort_scratch_words((uint32_t)m);
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t bytes = 2 * up(8 * m) + 2 * up(4 * m) + 2 * up(12 * m) + up(4 * words) + 256;
+    const size_t bytes = 4 * up(4 * m) + 2 * up(12 * m) + up(4 * words) + 256;
     const int rc = ctx_scratch(c, s, bytes, t.cs);
     if (rc) return rc;
     t.mem = t.cs.mem;
     char* p = static_cast<char*>(t.mem);
-    t.k0 = reinterpret_cast<uint64_t*>(p);
-    p += up(8 * m);
-    t.k1 = reinterpret_cast<uint64_t*>(p);
-    p += up(8 * m);
+    t.k0 = reinterpret_cast<uint32_t*>(p);
+    p += up(4 * m);
+    t.k1 = reinterpret_cast<uint32_t*>(p);
+    p += up(4 * m);
     t.v0 = reinterpret_cast<uint32_t*>(p);
     p += up(4 * m);
     t.v1 = reinterpret_cast<uint32_t*>(p);
@@ -138,14 +134,14 @@ int bits_for(uint32_t n_verts) {
 // sort the terms by vertex and add each vertex's run to g_verts
 void sum_terms(TermScratch& t, size_t n, uint32_t n_verts, float* g_verts, hipStream_t s) {
     const uint32_t m = (uint32_t)(3 * n);
-    uint64_t* k = t.k0;
+    uint32_t* k = t.k0;
     uint32_t* v = t.v0;
     if (radix_sort_pairs(t.k0, t.v0, t.k1, t.v1, m, bits_for(n_verts), t.sort, s)) {
         k = t.k1;
         v = t.v1;
     }
-    hipLaunchKernelGGL(k_wave_segsum<kBlock>, dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, v, t.terms, t.partial);
-    hipLaunchKernelGGL((k_run_sum<kBlock, VertexSink>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, t.partial,
+    hipLaunchKernelGGL((k_wave_segsum<kBlock, uint32_t>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, v, t.terms, t.partial);
+    hipLaunchKernelGGL((k_run_sum<kBlock, uint32_t, VertexSink>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, t.partial,
                        (uint64_t)n_verts, VertexSink{g_verts});
 }
 
@@ -164,7 +160,7 @@ int launch_cpq_bwd(gpurt_bvh_s* b, const float* q, size_t n, const int32_t* prim
     int rc = alloc_terms(b->ctx, n, s, t);
     if (rc) return rc;
     hipLaunchKernelGGL(k_cpq_bwd_terms, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n, q, prim, g,
-                       b->tri_idx, (uint32_t)b->n_tris, b->verts, (uint32_t)b->n_verts, g_q, t.k0, t.v0, t.terms);
+                       b->tri_idx, (uint32_t)b->n_tris, b->verts, (uint32_t)b->n_verts, g_q, t.k0, t.terms);
     sum_terms(t, n, (uint32_t)b->n_verts, g_verts, s);
     const hipError_t e = hipGetLastError();
     ctx_scratch_done(b->ctx, t.cs);
@@ -189,7 +185,7 @@ int launch_ray_bwd(gpurt_bvh_s* b, const gpurt_ray* rays, size_t n, const int32_
     if (rc) return rc;
     hipLaunchKernelGGL(k_ray_bwd_terms, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n,
                        reinterpret_cast<const float4*>(rays), prim, t, uv, g, b->tri_idx, (uint32_t)b->n_tris,
-                       b->verts, (uint32_t)b->n_verts, g_o, g_d, ts.k0, ts.v0, ts.terms);
+                       b->verts, (uint32_t)b->n_verts, g_o, g_d, ts.k0, ts.terms);
     sum_terms(ts, n, (uint32_t)b->n_verts, g_verts, s);
     const hipError_t e = hipGetLastError();
     ctx_scratch_done(b->ctx, ts.cs);

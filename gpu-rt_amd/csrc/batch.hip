@@ -249,12 +249,12 @@ __global__ __launch_bounds__(256) void k_batch_cpq_finish(const BatchMeshDev* __
 // writes them to term slots 3 (64 c + l) .. + 2, keyed by the vertex's batch-wide index
 // (the mesh's voff + its vertex), or `none` when it adds nothing (no such item, no vertex
 // gradient requested), for the fixed-order sum.
-template <bool RAYS>
+template <bool RAYS, typename K>
 __global__ __launch_bounds__(256) void k_batch_bwd(const BatchMeshDev* __restrict__ meshes,
                                                    const BatchGradDev* __restrict__ grads,
                                                    const uint2* __restrict__ chunks, uint32_t n_chunks,
                                                    uint32_t first_chunk, uint64_t none,
-                                                   uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                   K* __restrict__ keys,
                                                    float* __restrict__ terms) {
     const uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6);
     if (c >= n_chunks) return;
@@ -279,8 +279,7 @@ __global__ __launch_bounds__(256) void k_batch_bwd(const BatchMeshDev* __restric
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         const size_t k = k0 + j;
-        keys[k] = (t.v[j] == kNoVertex || !gd.g_verts) ? none : gd.voff + t.v[j];
-        vals[k] = (uint32_t)k;
+        keys[k] = (K)((t.v[j] == kNoVertex || !gd.g_verts) ? none : gd.voff + t.v[j]);
         terms[3 * k] = t.c[j][0];
         terms[3 * k + 1] = t.c[j][1];
         terms[3 * k + 2] = t.c[j][2];
@@ -296,12 +295,18 @@ struct MeshVertexSink {
     const uint64_t* voff;
     uint32_t n_meshes;
     __device__ void operator()(uint64_t key, float x, float y, float z) const {
-        uint32_t lo = 0, hi = n_meshes;  // voff[lo] <= key < voff[hi]
+        // Sorted keys: the first active lane's mesh by a search with one value for the wave,
+        // then the few meshes up to this lane's.  (A search per lane is a chain of ~8
+        // dependent loads each: k_run_sum of the 256-mesh batch 228 -> 158 us.)
+        const uint64_t key0 = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(key >> 32)) << 32 |
+                              __builtin_amdgcn_readfirstlane((uint32_t)key);
+        uint32_t lo = 0, hi = n_meshes;  // voff[lo] <= key0 < voff[hi]
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) / 2;
-            if (voff[mid] <= key) lo = mid;
+            if (voff[mid] <= key0) lo = mid;
             else hi = mid;
         }
+        while (voff[lo + 1] <= key) lo++;  // ends: key < voff[n_meshes]
         float* g = grads[lo].g_verts;
         const size_t v = key - voff[lo];
         g[3 * v] += x;
@@ -415,6 +420,42 @@ int enqueue_batch(gpurt_batch_s* b, int treelet_size, int treelet_rounds, hipStr
     }
     GPURT_HIP(hipGetLastError());
     return GPURT_OK;
+}
+
+}  // namespace
+
+namespace {
+
+// term memory of a recorded backward pass: keys of 32 bits where they number every vertex
+struct BatchTerms {
+    void *k0, *k1;
+    uint32_t *v0, *v1, *sort;
+    float *terms, *partial;
+    const uint64_t* voff;
+    uint64_t none;
+    uint32_t m;
+    int kbits;
+};
+
+template <typename K>
+void record_batch_bwd(gpurt_batch b, const BatchTerms& t, uint32_t n_meshes) {
+    K *k0 = static_cast<K*>(t.k0), *k1 = static_cast<K*>(t.k1);
+    hipStream_t s = b->cap;
+    if (b->n_cpq_chunks)
+        hipLaunchKernelGGL((k_batch_bwd<false, K>), dim3(cdiv(b->n_cpq_chunks, 4)), dim3(256), 0, s, b->meshes_d,
+                           b->grads_d, b->chunks_d, b->n_cpq_chunks, 0u, t.none, k0, t.terms);
+    if (b->n_ray_chunks)
+        hipLaunchKernelGGL((k_batch_bwd<true, K>), dim3(cdiv(b->n_ray_chunks, 4)), dim3(256), 0, s, b->meshes_d,
+                           b->grads_d, b->chunks_d + b->n_cpq_chunks, b->n_ray_chunks, b->n_cpq_chunks, t.none, k0,
+                           t.terms);
+    if (!t.m) return;
+    // each (mesh, vertex)'s terms in chunk order, summed in a fixed order
+    const bool in1 = radix_sort_pairs(k0, t.v0, k1, t.v1, t.m, t.kbits, t.sort, s);
+    const K* k = in1 ? k1 : k0;
+    hipLaunchKernelGGL((k_wave_segsum<kBlock, K>), dim3(cdiv(t.m, kBlock)), dim3(kBlock), 0, s, t.m, k,
+                       in1 ? t.v1 : t.v0, t.terms, t.partial);
+    hipLaunchKernelGGL((k_run_sum<kBlock, K, MeshVertexSink>), dim3(cdiv(t.m, kBlock)), dim3(kBlock), 0, s, t.m, k,
+                       t.partial, t.none, MeshVertexSink{b->grads_d, t.voff, n_meshes});
 }
 
 }  // namespace
@@ -636,7 +677,8 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     int kbits = 1;
     while (kbits < 64 && (none >> kbits)) kbits++;
     auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
-    const size_t tbytes = 2 * up(8 * (size_t)m) + 2 * up(4 * (size_t)m) + 2 * up(12 * (size_t)m) +
+    const size_t ksize = kbits <= 32 ? 4 : 8;
+    const size_t tbytes = 2 * up(ksize * m) + 2 * up(4 * (size_t)m) + 2 * up(12 * (size_t)m) +
                           up(4 * radix_sort_scratch_words(std::max<uint32_t>(m, 1))) + up(8 * (n_meshes + 1));
     DevGuard dg(b->ctx->device);
     if (!dg.ok) return set_error(GPURT_E_DEVICE, "hipSetDevice failed");
@@ -648,21 +690,21 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
         b->drop_backward();
         return set_error(GPURT_E_OOM, "batch gradient allocation failed");
     }
-    uint64_t *k0 = nullptr, *k1 = nullptr;
+    void *k0 = nullptr, *k1 = nullptr;
     uint32_t *v0 = nullptr, *v1 = nullptr, *sort_scratch = nullptr;
     float *terms = nullptr, *partial = nullptr;
     uint64_t* voff_d = nullptr;
     if (m) {
         char* tp = static_cast<char*>(b->terms_mem);
-        const size_t m8 = up(8 * (size_t)m), m4 = up(4 * (size_t)m), m12 = up(12 * (size_t)m);
-        k0 = reinterpret_cast<uint64_t*>(tp);
-        k1 = reinterpret_cast<uint64_t*>(tp + m8);
-        v0 = reinterpret_cast<uint32_t*>(tp + 2 * m8);
-        v1 = reinterpret_cast<uint32_t*>(tp + 2 * m8 + m4);
-        terms = reinterpret_cast<float*>(tp + 2 * m8 + 2 * m4);
-        partial = reinterpret_cast<float*>(tp + 2 * m8 + 2 * m4 + m12);
-        sort_scratch = reinterpret_cast<uint32_t*>(tp + 2 * m8 + 2 * m4 + 2 * m12);
-        voff_d = reinterpret_cast<uint64_t*>(tp + 2 * m8 + 2 * m4 + 2 * m12 +
+        const size_t mk = up(ksize * m), m4 = up(4 * (size_t)m), m12 = up(12 * (size_t)m);
+        k0 = tp;
+        k1 = tp + mk;
+        v0 = reinterpret_cast<uint32_t*>(tp + 2 * mk);
+        v1 = reinterpret_cast<uint32_t*>(tp + 2 * mk + m4);
+        terms = reinterpret_cast<float*>(tp + 2 * mk + 2 * m4);
+        partial = reinterpret_cast<float*>(tp + 2 * mk + 2 * m4 + m12);
+        sort_scratch = reinterpret_cast<uint32_t*>(tp + 2 * mk + 2 * m4 + 2 * m12);
+        voff_d = reinterpret_cast<uint64_t*>(tp + 2 * mk + 2 * m4 + 2 * m12 +
                                              up(4 * radix_sort_scratch_words(std::max<uint32_t>(m, 1))));
     }
     if (hipMemcpy(b->grads_d, gd.data(), sizeof(BatchGradDev) * n_meshes, hipMemcpyHostToDevice) != hipSuccess ||
@@ -681,21 +723,11 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     if (!segs.empty())
         hipLaunchKernelGGL(k_batch_zero_vgrads, dim3((unsigned)segs.size()), dim3(256), 0, b->cap, b->grads_d,
                            b->zero_segs_d);
-    if (b->n_cpq_chunks)
-        hipLaunchKernelGGL(k_batch_bwd<false>, dim3(cdiv(b->n_cpq_chunks, 4)), dim3(256), 0, b->cap, b->meshes_d,
-                           b->grads_d, b->chunks_d, b->n_cpq_chunks, 0u, none, k0, v0, terms);
-    if (b->n_ray_chunks)
-        hipLaunchKernelGGL(k_batch_bwd<true>, dim3(cdiv(b->n_ray_chunks, 4)), dim3(256), 0, b->cap, b->meshes_d,
-                           b->grads_d, b->chunks_d + b->n_cpq_chunks, b->n_ray_chunks, b->n_cpq_chunks, none,
-                           k0, v0, terms);
-    if (m) {
-        // each (mesh, vertex)'s terms in chunk order, summed in a fixed order
-        const bool in1 = radix_sort_pairs(k0, v0, k1, v1, m, kbits, sort_scratch, b->cap);
-        hipLaunchKernelGGL(k_wave_segsum<kBlock>, dim3(cdiv(m, kBlock)), dim3(kBlock), 0, b->cap, m, in1 ? k1 : k0,
-                           in1 ? v1 : v0, terms, partial);
-        hipLaunchKernelGGL((k_run_sum<kBlock, MeshVertexSink>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, b->cap, m,
-                           in1 ? k1 : k0, partial, none, MeshVertexSink{b->grads_d, voff_d, (uint32_t)n_meshes});
-    }
+    const BatchTerms bt{k0, k1, v0, v1, sort_scratch, terms, partial, voff_d, none, m, kbits};
+    if (kbits <= 32)
+        record_batch_bwd<uint32_t>(b, bt, (uint32_t)n_meshes);
+    else
+        record_batch_bwd<uint64_t>(b, bt, (uint32_t)n_meshes);
     hipError_t el = hipGetLastError();
     hipGraph_t g = nullptr;
     hipError_t ec = hipStreamEndCapture(b->cap, &g);

@@ -225,8 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(const SegDesc* __restrict__ seg
 
 __global__ __launch_bounds__(kBlock) void k_morton(uint32_t N, const float4* __restrict__ cen,
                                                    const uint32_t* __restrict__ segstat,
-                                                   uint64_t* __restrict__ keys,
-                                                   uint32_t* __restrict__ vals) {
+                                                   uint64_t* __restrict__ keys) {
     uint32_t g = blockIdx.x * kBlock + threadIdx.x;
     if (g >= N) return;
     const float4 c4 = cen[g];
@@ -241,24 +240,25 @@ __global__ __launch_bounds__(kBlock) void k_morton(uint32_t N, const float4* __r
     }
     uint32_t code = (expand_bits10(q[0]) << 2) | (expand_bits10(q[1]) << 1) | expand_bits10(q[2]);
     keys[g] = ((uint64_t)s << 30) | code;
-    vals[g] = g;
 }
 
 // ------------------------------------------------------------------------------------
-// LSD radix sort of (uint64 key, uint32 value), 8-bit digits, stable
+// LSD radix sort of (uint64 or uint32 key, uint32 index), 8-bit digits, stable
 // ------------------------------------------------------------------------------------
 
 constexpr int kSortItems = 16;
 constexpr int kSortTile = kBlock * kSortItems;
+constexpr int kSortThreads = 512;  // of the scatter
 
-__global__ __launch_bounds__(kBlock) void k_radix_hist(const uint64_t* __restrict__ keys, uint32_t n,
+template <typename K>
+__global__ __launch_bounds__(kBlock) void k_radix_hist(const K* __restrict__ keys, uint32_t n,
                                                        int shift, uint32_t* __restrict__ hist,
                                                        uint32_t nblocks) {
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
     uint32_t base = blockIdx.x * kSortTile;
-#pragma unroll 4
+#pragma unroll
     for (int r = 0; r < kSortItems; r++) {
         uint32_t i = base + r * kBlock + threadIdx.x;
         if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & 255u], 1u);
@@ -304,59 +304,63 @@ __global__ __launch_bounds__(kBlock) void k_scan_rows(uint32_t* __restrict__ his
 // Scatter of one radix pass.  The block's tile (kSortTile pairs) is first ordered by
 // digit in LDS, stably, and then written out in that order, so each digit's run of the
 // tile (16 pairs on average) leaves as one contiguous stretch of the output instead of
-// one isolated 12-byte write per pair.  Each wave ranks its own 1024 consecutive pairs:
-// per round of 64, an 8-ballot multisplit ranks the lanes of equal digit, and a
-// wave-private LDS counter per digit (read by all lanes, advanced by each group's first
-// lane; a wave's LDS operations complete in order) carries the rank across rounds, so the
-// rounds need no block barrier.  One scan over (digit, wave) counts then gives every
-// wave's first slot per digit.
-__global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __restrict__ kin,
-                                                          const uint32_t* __restrict__ vin,
-                                                          uint64_t* __restrict__ kout,
-                                                          uint32_t* __restrict__ vout, uint32_t n,
-                                                          int shift,
-                                                          const uint32_t* __restrict__ offs,
-                                                          const uint32_t* __restrict__ row_total,
-                                                          uint32_t nblocks) {
-    constexpr int kWaves = kBlock / 64;
-    constexpr uint32_t kWaveItems = kSortTile / kWaves;  // consecutive pairs per wave
-    static_assert(kWaveItems == 64 * kSortItems, "one pair per lane and round");
-    __shared__ uint64_t skey[kSortTile];
-    __shared__ uint32_t sval[kSortTile];
-    __shared__ uint32_t gbase[256];          // this block's first output slot of digit d
-    __shared__ uint32_t lstart[256];         // the tile's first LDS slot of digit d
-    __shared__ uint32_t wcnt[kWaves][256];   // a wave's pairs of digit d, then its first slot
-    __shared__ uint32_t wsum[kWaves];
+// one isolated write per pair.  Each wave ranks its own 512 consecutive pairs: per round
+// of 64, an 8-ballot multisplit ranks the lanes of equal digit, and a wave-private LDS
+// counter per digit (read by all lanes, advanced by each group's first lane; a wave's LDS
+// operations complete in order) carries the rank across rounds, so the rounds need no
+// block barrier.  One scan over (digit, wave) counts then gives every wave's first slot
+// per digit.  Bound by the latency of that chain, not by memory, so what counts is waves in
+// flight: the values pass through the LDS that the keys have left, and with 16-bit counts
+// a CU holds 3-4 blocks of 8 waves (2 of 4 waves with keys and values side by side): 2.3 M
+// pairs of 12 bytes 30.5 -> 16.5 us a pass, 3.1 M of 8 bytes (33 us as 12) 17 us, 3.5 TB/s.
+template <typename K>
+__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const K* __restrict__ kin,
+                                                                const uint32_t* __restrict__ vin,
+                                                                K* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                                uint32_t n, int shift,
+                                                                const uint32_t* __restrict__ offs,
+                                                                const uint32_t* __restrict__ row_total,
+                                                                uint32_t nblocks) {
+    constexpr int kWaves = kSortThreads / 64;
+    constexpr int kItems = kSortTile / kSortThreads;
+    constexpr uint32_t kWaveItems = 64 * kItems;  // consecutive pairs per wave
+    static_assert(kSortTile <= 65535, "16-bit slots");
+    __shared__ K skey[kSortTile];            // keys in slot order, then the values
+    __shared__ uint32_t gofs[256];           // output slot of digit d less its first LDS slot
+    __shared__ uint16_t wcnt[kWaves][256];   // a wave's pairs of digit d, then its first slot
+    __shared__ uint32_t wsum[2][4];
+    uint32_t* const sval = reinterpret_cast<uint32_t*>(skey);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x * kSortTile;
     const uint32_t m = min((uint32_t)kSortTile, n - tile);
+    const uint32_t wbase = (uint32_t)wave * kWaveItems + (uint32_t)lane;
+    K key[kItems];
+    uint32_t val[kItems], rank[kItems];
+#pragma unroll
+    for (int r = 0; r < kItems; r++) {
+        const uint32_t i = wbase + (uint32_t)r * 64u;
+        key[r] = i < m ? kin[tile + i] : (K)0;
+        val[r] = !vin ? tile + i : i < m ? vin[tile + i] : 0u;
+    }
     // this block's first output slot of digit tid: the digits before it, then its row
-    const uint32_t dtot = row_total[tid];
-    uint32_t dincl = dtot;
+    uint32_t dtot = 0, dincl = 0, row = 0;
+    if (tid < 256) {
+        dtot = dincl = row_total[tid];
+        row = offs[(size_t)tid * nblocks + blockIdx.x];
+    }
+    for (int k = tid; k < kWaves * 256; k += kSortThreads) wcnt[k >> 8][k & 255] = 0;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
         const uint32_t x = __shfl_up(dincl, off);
         if (lane >= off) dincl += x;
     }
-    if (lane == 63) wsum[wave] = dincl;
-    for (int w = 0; w < kWaves; w++) wcnt[w][tid] = 0;
+    if (tid < 256 && lane == 63) wsum[0][wave] = dincl;
     __syncthreads();
-    {
-        uint32_t base = dincl - dtot + offs[(size_t)tid * nblocks + blockIdx.x];
-        for (int w = 0; w < wave; w++) base += wsum[w];
-        gbase[tid] = base;
-    }
-    uint32_t* const mycnt = wcnt[wave];
-    const uint32_t wbase = (uint32_t)wave * kWaveItems;
+    uint16_t* const mycnt = wcnt[wave];
     const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-    uint64_t key[kSortItems];
-    uint32_t val[kSortItems], rank[kSortItems];
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
-        const bool valid = i < m;
-        key[r] = valid ? kin[tile + i] : 0ull;
-        val[r] = valid ? vin[tile + i] : 0u;
+    for (int r = 0; r < kItems; r++) {
+        const bool valid = wbase + (uint32_t)r * 64u < m;
         const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -367,50 +371,64 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
         const uint32_t rk = (uint32_t)__popcll(peers & lt_mask);
         const uint32_t before = mycnt[d];
         rank[r] = before + rk;
-        if (valid && rk == 0) mycnt[d] = before + (uint32_t)__popcll(peers);
+        if (valid && rk == 0) mycnt[d] = (uint16_t)(before + (uint32_t)__popcll(peers));
     }
     __syncthreads();
-    // digit tid: the tile's count and every wave's offset inside the digit's run
-    uint32_t c[kWaves], tot = 0;
+    // digit tid: the tile's count and every wave's first slot inside the digit's run, from
+    // an exclusive scan of the 256 totals within each wave by shuffles, then across
+    uint32_t tot = 0, incl = 0;
+    if (tid < 256) {
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-        c[w] = wcnt[w][tid];
-        tot += c[w];
-    }
-    // exclusive scan of the 256 digit totals: within each wave by shuffles, then across
-    uint32_t incl = tot;
+        for (int w = 0; w < kWaves; w++) tot += wcnt[w][tid];
+        incl = tot;
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t x = __shfl_up(incl, off);
-        if (lane >= off) incl += x;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    uint32_t start = incl - tot;
-    for (int w = 0; w < wave; w++) start += wsum[w];
-    lstart[tid] = start;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-        wcnt[w][tid] = start;
-        start += c[w];
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t x = __shfl_up(incl, off);
+            if (lane >= off) incl += x;
+        }
+        if (lane == 63) wsum[1][wave] = incl;
     }
     __syncthreads();
+    if (tid < 256) {
+        uint32_t start = incl - tot, base = dincl - dtot + row;
+        for (int w = 0; w < wave; w++) {
+            start += wsum[1][w];
+            base += wsum[0][w];
+        }
+        gofs[tid] = base - start;
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        if (wbase + (uint32_t)r * 64u + (uint32_t)lane < m) {
-            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
-            const uint32_t pos = mycnt[d] + rank[r];
-            skey[pos] = key[r];
-            sval[pos] = val[r];
+        for (int w = 0; w < kWaves; w++) {
+            const uint32_t c = wcnt[w][tid];
+            wcnt[w][tid] = (uint16_t)start;
+            start += c;
         }
     }
     __syncthreads();
-    for (uint32_t j = tid; j < m; j += kBlock) {
-        const uint64_t k = skey[j];
-        const uint32_t d = (uint32_t)(k >> shift) & 255u;
-        const uint32_t o = gbase[d] + (j - lstart[d]);
-        kout[o] = k;
-        vout[o] = sval[j];
+#pragma unroll
+    for (int r = 0; r < kItems; r++) {
+        rank[r] += mycnt[(uint32_t)(key[r] >> shift) & 255u];  // the pair's slot
+        if (wbase + (uint32_t)r * 64u < m) skey[rank[r]] = key[r];
+    }
+    __syncthreads();
+    uint32_t out[kItems];
+#pragma unroll
+    for (int r = 0; r < kItems; r++) {
+        const uint32_t j = (uint32_t)tid + (uint32_t)r * kSortThreads;
+        if (j < m) {
+            const K k = skey[j];
+            out[r] = gofs[(uint32_t)(k >> shift) & 255u] + j;
+            kout[out[r]] = k;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; r++)
+        if (wbase + (uint32_t)r * 64u < m) sval[rank[r]] = val[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; r++) {
+        const uint32_t j = (uint32_t)tid + (uint32_t)r * kSortThreads;
+        if (j < m) vout[out[r]] = sval[j];
     }
 }
 
@@ -420,25 +438,25 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
 constexpr uint32_t kSmallSort = 8192;
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64, kSmallItems = kSmallSort / kSmallThreads;
 
-__global__ __launch_bounds__(kSmallThreads) void k_sort_small(const uint64_t* __restrict__ kin,
-                                                              const uint32_t* __restrict__ vin,
-                                                              uint64_t* __restrict__ kout,
+template <typename K>
+__global__ __launch_bounds__(kSmallThreads) void k_sort_small(const K* __restrict__ kin,
+                                                              K* __restrict__ kout,
                                                               uint32_t* __restrict__ vout, uint32_t n,
                                                               int key_bits) {
-    __shared__ uint64_t skey[kSmallSort];
+    __shared__ K skey[kSmallSort];
     __shared__ uint32_t sval[kSmallSort];
     __shared__ uint32_t wcnt[kSmallWaves][256];
     __shared__ uint32_t wsum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
     const uint32_t wbase = (uint32_t)wave * 64u * kSmallItems;
-    uint64_t key[kSmallItems];
+    K key[kSmallItems];
     uint32_t val[kSmallItems], rank[kSmallItems];
 #pragma unroll
     for (int r = 0; r < kSmallItems; r++) {
         const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
-        key[r] = i < n ? kin[i] : 0ull;
-        val[r] = i < n ? vin[i] : 0u;
+        key[r] = i < n ? kin[i] : (K)0;
+        val[r] = i;
     }
     for (int shift = 0; shift < key_bits; shift += 8) {
         for (int k = tid; k < kSmallWaves * 256; k += kSmallThreads) wcnt[k >> 8][k & 255] = 0;
@@ -515,29 +533,35 @@ size_t radix_sort_scratch_words(uint32_t n) {
     return 256 * (size_t)cdiv(n, kSortTile) + 256;
 }
 
-bool radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint32_t n, int key_bits,
+template <typename K>
+bool radix_sort_pairs(K* k0, uint32_t* v0, K* k1, uint32_t* v1, uint32_t n, int key_bits,
                       uint32_t* scratch, hipStream_t s) {
     if (n <= kSmallSort) {
-        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kSmallThreads), 0, s, k0, v0, k1, v1, n, key_bits);
+        hipLaunchKernelGGL((k_sort_small<K>), dim3(1), dim3(kSmallThreads), 0, s, k0, k1, v1, n, key_bits);
         return true;
     }
     const uint32_t nblocks = cdiv(n, kSortTile);
     uint32_t* hist = scratch;  // 256 digit counts per block, digit-major
     uint32_t* totals = scratch + 256 * (size_t)nblocks;
-    uint64_t *kin = k0, *kout = k1;
-    uint32_t *vin = v0, *vout = v1;
+    K *kin = k0, *kout = k1;
+    uint32_t *vin = nullptr, *vout = v1;  // the first pass's values are the indices
     bool in1 = false;
     for (int shift = 0; shift < key_bits; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kBlock), 0, s, kin, n, shift, hist, nblocks);
+        hipLaunchKernelGGL((k_radix_hist<K>), dim3(nblocks), dim3(kBlock), 0, s, kin, n, shift, hist, nblocks);
         hipLaunchKernelGGL(k_scan_rows, dim3(256), dim3(kBlock), 0, s, hist, nblocks, totals);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kBlock), 0, s, kin, vin, kout, vout, n, shift, hist,
+        hipLaunchKernelGGL((k_radix_scatter<K>), dim3(nblocks), dim3(kSortThreads), 0, s, kin, vin, kout, vout, n, shift, hist,
                            totals, nblocks);
         std::swap(kin, kout);
-        std::swap(vin, vout);
+        vin = vout;
+        vout = in1 ? v1 : v0;
         in1 = !in1;
     }
     return in1;
 }
+template bool radix_sort_pairs<uint64_t>(uint64_t*, uint32_t*, uint64_t*, uint32_t*, uint32_t, int, uint32_t*,
+                                         hipStream_t);
+template bool radix_sort_pairs<uint32_t>(uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t, int, uint32_t*,
+                                         hipStream_t);
 
 // ------------------------------------------------------------------------------------
 // k_pack: gather triangles and AABBs into sorted order
@@ -1334,7 +1358,7 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
                        b.cen, b.segstat_rep, b.counters);
     hipLaunchKernelGGL(k_reduce_stats, dim3(cdiv((size_t)n_seg * kStat, kBlock)), dim3(kBlock), 0, s, n_seg,
                        b.segstat_rep, b.segstat);
-    hipLaunchKernelGGL(k_morton, dim3(gN), dim3(kBlock), 0, s, N, b.cen, b.segstat, b.keys0, b.vals0);
+    hipLaunchKernelGGL(k_morton, dim3(gN), dim3(kBlock), 0, s, N, b.cen, b.segstat, b.keys0);
     // radix sort over the bits in use: 30 Morton bits + mesh-id bits
     int seg_bits = 0;
     while ((1u << seg_bits) < (uint32_t)n_seg) seg_bits++;

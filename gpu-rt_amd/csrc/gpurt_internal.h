@@ -361,12 +361,13 @@ int build_alloc(const SegDesc* host_segs, int n_seg, int width, int leaf_size, i
 int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hipStream_t s);
 int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s);
 int run_treelets(BuildBufs& b, int treelet_size, int rounds, int key_bits, int nbits, hipStream_t s);
-// Stable LSD radix sort (build.hip) of n (uint64 key, uint32 value) pairs on the low
-// key_bits bits, 8 bits per pass, ping-ponging between (k0, v0) and (k1, v1); returns
-// true when the sorted pairs end in (k1, v1).  scratch: radix_sort_scratch_words(n)
+// Stable LSD radix sort (build.hip) of n uint64 or uint32 keys k0, each with its index as
+// value, on the low key_bits bits, 8 bits per pass, ping-ponging between (k0, v0) and
+// (k1, v1) (v0 need not be set); returns true when the sorted pairs end in (k1, v1).  scratch: radix_sort_scratch_words(n)
 // words.
-bool radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint32_t n, int key_bits,
-                      uint32_t* scratch, hipStream_t s);
+template <typename K>
+bool radix_sort_pairs(K* k0, uint32_t* v0, K* k1, uint32_t* v1, uint32_t n, int key_bits, uint32_t* scratch,
+                      hipStream_t s);
 size_t radix_sort_scratch_words(uint32_t n);
 int build_segments(gpurt_ctx ctx, const SegDesc* host_segs, int n_seg, int width, int leaf_size,
                    int treelet_size, int treelet_rounds, int format, hipStream_t stream, gpurt_bvh_s* out);

@@ -250,3 +250,36 @@ def test_auto_vertex_sums_pick_the_fixed_order_for_large_calls(dev):
     assert np.array_equal(out["auto"], out["fixed"])
     scale = np.abs(out["fixed"]).max()
     np.testing.assert_allclose(out["atomic"], out["fixed"], atol=1e-5 * scale, rtol=1e-4)
+
+
+@pytest.mark.parametrize("level", [1, 4, 7])
+@pytest.mark.parametrize("n", [1, 85, 1365, 1366, 2730, 2731, 4096, 5461, 5462, 21845, 21846, 90001])
+def test_fixed_order_sums_at_sort_edges(dev, level, n):
+    """Fixed-order sums of 3 n terms around the sizes at which the sort changes (one block up
+    to 8192 pairs, tiles of 4096) and for vertex numbers of 6, 12 and 18 bits (one to three
+    passes), against the FP64 sum.  A vertex's sum of c FP32 terms of total magnitude S is
+    off by at most (c + 4) 2^-24 S."""
+    ctx = gpurt.Context(0, vertex_sums="fixed")
+    V, F = _sphere(level, 3)
+    rng = np.random.default_rng(n)
+    Q = W.surface_samples(V.astype(np.float64), F, rng, n, 0.05).astype(np.float32)
+    tq, g = _t(Q, dev), torch.from_numpy(rng.normal(size=n).astype(np.float32)).to(dev)
+    bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev))
+    prim, pt, dist, bary = bvh.closest_point(tq)
+    runs = []
+    for _ in range(2):
+        gv = torch.zeros((V.shape[0], 3), device=dev)
+        bvh.closest_point_bwd(tq, prim, bary, pt, dist, g, None, gv)
+        runs.append(gv.cpu().numpy())
+    assert np.array_equal(*runs)
+    p, gn = prim.cpu().numpy(), g.cpu().numpy().astype(np.float64)
+    ev, total, count = np.zeros(V.shape), np.zeros(len(V)), np.zeros(len(V))
+    gq, _ = O.cpq_grad_f64(V.astype(np.float64), F, Q.astype(np.float64), p)
+    b = bary.cpu().numpy().astype(np.float64)
+    for j in range(3):
+        np.add.at(ev, F[p, j], -(b[:, j] * gn)[:, None] * gq)
+        np.add.at(total, F[p, j], np.abs(b[:, j] * gn))
+        np.add.at(count, F[p, j], 1)
+    assert (np.abs(runs[0] - ev) <= ((count + 4) * 2.0**-24 * total)[:, None] + 1e-30).all()
+    bvh.close()
+    ctx.close()
