@@ -941,11 +941,11 @@ struct CollapseArgs {
     const float4* bnode;  // binary nodes (build_common.h)
     const float4* saabb;
     const uint32_t* segstat;
-    uint32_t* wsrc;  // wide node -> binary ref
+    uint2* wsrc;     // wide node -> the two binary refs it starts from (root_kids)
     uint32_t* wseg;  // wide node -> mesh
     uint32_t* wfirst;  // wide node -> first packed triangle of its range
     uint32_t* lvl_cnt;
-    uint32_t* counters;  // [0] wide nodes allocated, [1] error bits
+    uint32_t* counters;  // [0] wide nodes (set at the end), [1] error bits
     void* nodes;
     uint32_t capacity;
     int leaf_size;
@@ -989,29 +989,63 @@ __global__ __launch_bounds__(kBlock) void k_repack(uint32_t N, const uint32_t* _
     if (v == 0) order_out[out] = order_in[in];
 }
 
-// Wave-aggregated allocation: each lane asks for n slots of *counter (any lane may ask
-// for 0; all 64 lanes take part), one device atomic per wave returns the wave's block
-// and the lane gets its part in lane order.  Many same-address device atomics, one per
-// node, serialise at the memory side.
-__device__ __forceinline__ uint32_t wave_alloc(uint32_t* counter, uint32_t n, uint32_t& total) {
-    const uint32_t lane = threadIdx.x & 63u;
+constexpr int kBlockLevelThreads = 512;  // of the one-block kernels: 8-wide nodes need 217 VGPRs
+
+// Block-wide allocation: each thread asks for n slots of a counter (any may ask for 0; all
+// threads of the block take part), one atomic per block (add) returns the block's slots and
+// a thread gets its part in thread order.  Device atomics on one address go one after another
+// at the memory side: with one per wave on the node counter and one on the level's count, the
+// atomics were most of a large level (the collapse of a 256-mesh batch, 6.9 M triangles:
+// 494 us with them, 315 with one per block of 256 threads).
+template <typename Add>
+__device__ __forceinline__ uint32_t block_alloc(Add add, uint32_t n) {
+    __shared__ uint32_t wsum[kBlockLevelThreads / 64], first;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     uint32_t x = n;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         const uint32_t y = __shfl_up(x, d);
         if (lane >= (uint32_t)d) x += y;
     }
-    total = __shfl(x, 63);
-    uint32_t base = 0;
-    if (lane == 63u && total) base = gatomic_add(counter, total);
-    base = __shfl(base, 63);
-    return base + x - n;
+    __syncthreads();  // the last call's sums have been read
+    if (lane == 63u) wsum[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    for (uint32_t w = 0; w < blockDim.x / 64; w++) {
+        if (w < wave) before += wsum[w];
+        total += wsum[w];
+    }
+    if (threadIdx.x == 0) first = total ? add(total) : 0u;
+    __syncthreads();
+    return first + before + x - n;
 }
 
-// Collapses nodes [begin, begin + cnt) of level `level`, dealt to the grid's threads; all
-// 64 lanes of a wave call it together.
-template <int W>
-__device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level, uint32_t begin, uint32_t cnt) {
+// A level that one block makes out of LDS (k_collapse_block): its nodes' sources, meshes and
+// ranges, and the next level's with their count.
+constexpr uint32_t kHeadNodes = 256;
+struct HeadList {
+    uint2 src[kHeadNodes];
+    uint32_t seg[kHeadNodes], first[kHeadNodes];
+};
+
+// The binary nodes a mesh's first wide node starts from: its root's children, or the root
+// alone when that is one leaf.  (Every other wide node gets its own binary node's children
+// from the level above, which has loaded that node.)
+__device__ __forceinline__ uint2 root_kids(const float4* __restrict__ bnode, uint32_t root, uint32_t leaf_size) {
+    if (root & kLeafBit) return make_uint2(root, kEmpty);
+    const float4* p = bnode + 3 * (size_t)root;
+    if (__float_as_uint(p[2].x) <= leaf_size) return make_uint2(root, kEmpty);
+    return make_uint2(__float_as_uint(p[0].w), __float_as_uint(p[1].w));
+}
+
+// Collapses nodes [begin, begin + cnt) of a level, dealt to the grid's threads; all threads
+// of a block call it together.  The next level's nodes, counted in *next_count, follow them.
+// HEAD: read from `in`, and the next level's (with its count in LDS) listed in `next` too
+// while they fit.
+template <int W, bool HEAD = false>
+__device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t begin, uint32_t cnt,
+                                               uint32_t* next_count, const HeadList* in = nullptr,
+                                               HeadList* next = nullptr) {
     WNode<W>* nodes = reinterpret_cast<WNode<W>*>(a.nodes);
     // every lane runs every iteration (slot allocation is wave-wide); lanes past the
     // level's end take part with nothing to allocate
@@ -1019,85 +1053,67 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level,
         const uint32_t k = k0 + threadIdx.x;
         const bool act = k < cnt;
         uint32_t wi = begin + (act ? k : 0u);
-        uint32_t bref = a.wsrc[wi];
-        uint32_t seg = a.wseg[wi];
-        uint32_t run = a.wfirst[wi];
+        const uint2 kids = HEAD ? in->src[act ? k : 0u] : a.wsrc[wi];
+        uint32_t seg = HEAD ? in->seg[act ? k : 0u] : a.wseg[wi];
+        uint32_t run = HEAD ? in->first[act ? k : 0u] : a.wfirst[wi];
         float pad = o2f(a.segstat[seg * kStat + 6]) * 0x1p-18f;
         // The wide node's children, kept in registers with their triangle counts and
         // boxes: a child is loaded once, with its own children when it is an internal
-        // node (one 48-byte record), so opening it (the child with the largest area among
-        // those with more than leaf_size triangles, the lowest slot on ties) costs one
-        // round of loads instead of re-reading every child's count and box.  Slots are
-        // addressed with compile-time indices only, so nothing spills to scratch.
-        uint32_t refs[W], rc[W], rf[W], rl[W], rr[W];
-        float4 rlo[W], rhi[W];
-        float rar[W];
-        auto load_child = [&](uint32_t r, uint32_t& ref, uint32_t& c, uint32_t& first, uint32_t& l, uint32_t& rgt,
-                              float4& lo, float4& hi, float& ar) {
-            ref = r;
-            const bool internal = !(r & kLeafBit);
-            if (internal) {
-                const float4* p = a.bnode + 3 * (size_t)r;
-                lo = p[0];
-                hi = p[1];
-                const float4 x = p[2];
-                l = __float_as_uint(lo.w);
-                rgt = __float_as_uint(hi.w);
-                c = __float_as_uint(x.x);
-                first = __float_as_uint(x.z);
-            } else {
-                const size_t p = r & ~kLeafBit;
-                lo = a.saabb[2 * p];
-                hi = a.saabb[2 * p + 1];
-                l = rgt = 0u;
-                c = 1u;
-                first = (uint32_t)p;
-            }
-            ar = c > (uint32_t)a.leaf_size ? box_area(lo, hi) : -1.0f;
+        // node (one 48-byte record).  Opening one (the child with the largest area among
+        // those with more than leaf_size triangles, the lowest slot on ties) loads its two
+        // children side by side, whatever their kind and slot, and then selects: a branch
+        // per slot and kind was a memory latency each, and lanes that open different slots
+        // waited for each other's (6 levels in one block 41 -> 29 us).  Slots are addressed with compile-time
+        // indices only, so nothing spills to scratch.
+        struct Child {
+            uint32_t ref, c, first, l, r;
+            float4 lo, hi;
+            float area;  // < 0: not to be opened
         };
+        auto load_child = [&](uint32_t r) {
+            Child x;
+            const bool internal = !(r & kLeafBit);
+            const uint32_t at = r & ~kLeafBit;
+            const float4* p = internal ? a.bnode + 3 * (size_t)at : a.saabb + 2 * (size_t)at;
+            x.lo = p[0];
+            x.hi = p[1];
+            const float4 w = p[internal ? 2 : 1];
+            x.ref = r;
+            x.l = __float_as_uint(x.lo.w);
+            x.r = __float_as_uint(x.hi.w);
+            x.c = internal ? __float_as_uint(w.x) : 1u;
+            x.first = internal ? __float_as_uint(w.z) : at;
+            x.area = x.c > (uint32_t)a.leaf_size ? box_area(x.lo, x.hi) : -1.0f;
+            return x;
+        };
+        Child ch[W];
         int n = 0;
-        if (!act) {
-            // nothing: n stays 0
-        } else {
-            uint32_t bc, bf, bl, br;
-            float4 blo, bhi;
-            float bar;
-            load_child(bref, refs[0], bc, bf, bl, br, blo, bhi, bar);
-            if (bc <= (uint32_t)a.leaf_size) {
-                rc[0] = bc;
-                rf[0] = bf;
-                rlo[0] = blo;
-                rhi[0] = bhi;
-                n = 1;
-            } else {
-                load_child(bl, refs[0], rc[0], rf[0], rl[0], rr[0], rlo[0], rhi[0], rar[0]);
-                load_child(br, refs[1], rc[1], rf[1], rl[1], rr[1], rlo[1], rhi[1], rar[1]);
+        if (act) {
+            ch[0] = load_child(kids.x);
+            n = 1;
+            if (kids.y != kEmpty) {
+                ch[1] = load_child(kids.y);
                 n = 2;
-                while (n < W) {
+#pragma unroll
+                for (int m = 2; m < W; m++) {
                     int best = -1;
                     float best_area = -1.0f;
-#pragma unroll
-                    for (int j = 0; j < W; j++) {
-                        if (j < n && rar[j] > best_area) {
-                            best_area = rar[j];
-                            best = j;
-                        }
-                    }
-                    if (best < 0) break;
                     uint32_t ol = 0, orr = 0;
 #pragma unroll
-                    for (int j = 0; j < W; j++) {
-                        if (j == best) {
-                            ol = rl[j];
-                            orr = rr[j];
-                        }
+                    for (int j = 0; j < m; j++) {
+                        const bool b = ch[j].area > best_area;
+                        best = b ? j : best;
+                        best_area = b ? ch[j].area : best_area;
+                        ol = b ? ch[j].l : ol;
+                        orr = b ? ch[j].r : orr;
                     }
+                    if (best < 0) break;  // (n == m until here)
+                    const Child x = load_child(ol);
+                    ch[m] = load_child(orr);
 #pragma unroll
-                    for (int j = 0; j < W; j++) {
-                        if (j == best) load_child(ol, refs[j], rc[j], rf[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
-                        if (j == n) load_child(orr, refs[j], rc[j], rf[j], rl[j], rr[j], rlo[j], rhi[j], rar[j]);
-                    }
-                    n++;
+                    for (int j = 0; j < m; j++)
+                        if (j == best) ch[j] = x;
+                    n = m + 1;
                 }
             }
         }
@@ -1105,20 +1121,20 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level,
         uint32_t n_internal = 0;
 #pragma unroll
         for (int j = 0; j < W; j++)
-            if (j < n && rc[j] > (uint32_t)a.leaf_size) n_internal++;
+            if (j < n && ch[j].c > (uint32_t)a.leaf_size) n_internal++;
 #pragma unroll
         for (int j = 0; j < W; j++) {
             if (j < n) {
-                const float4 lo = rlo[j], hi = rhi[j];
+                const float4 lo = ch[j].lo, hi = ch[j].hi;
                 out.lox[j] = lo.x - pad; out.loy[j] = lo.y - pad; out.loz[j] = lo.z - pad;
                 out.hix[j] = hi.x + pad; out.hiy[j] = hi.y + pad; out.hiz[j] = hi.z + pad;
-                const uint32_t c = rc[j];
+                const uint32_t c = ch[j].c;
                 out.aux[j] = c;
-                if (a.repack) rf[j] = run;
+                if (a.repack) ch[j].first = run;
                 run += c;
                 if (c <= (uint32_t)a.leaf_size) {
-                    if (a.repack) list_leaf(a, refs[j], rf[j]);
-                    out.child[j] = make_leaf(rf[j], c);
+                    if (a.repack) list_leaf(a, ch[j].ref, ch[j].first);
+                    out.child[j] = make_leaf(ch[j].first, c);
                 }
             } else {
                 out.lox[j] = out.loy[j] = out.loz[j] = INFINITY;
@@ -1127,9 +1143,9 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level,
                 out.aux[j] = 0;
             }
         }
-        uint32_t wave_total = 0;
-        const uint32_t base = wave_alloc(&a.counters[0], n_internal, wave_total);
-        if ((threadIdx.x & 63u) == 63u && wave_total) gatomic_add(&a.lvl_cnt[level + 1], wave_total);
+        const uint32_t base =
+            begin + cnt + block_alloc([&](uint32_t x) { return HEAD ? atomicAdd(next_count, x) : gatomic_add(next_count, x); },
+                                      n_internal);
         if (n_internal) {
             uint32_t m = 0;
 #pragma unroll
@@ -1137,9 +1153,16 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, int level,
                 if (j < n && out.aux[j] > (uint32_t)a.leaf_size) {
                     uint32_t idx = base + m++;
                     if (idx < a.capacity) {
-                        a.wsrc[idx] = refs[j];
+                        const uint2 kids = make_uint2(ch[j].l, ch[j].r);
+                        a.wsrc[idx] = kids;
                         a.wseg[idx] = seg;
-                        a.wfirst[idx] = rf[j];
+                        a.wfirst[idx] = ch[j].first;
+                        const uint32_t at = idx - (begin + cnt);
+                        if (HEAD && at < kHeadNodes) {
+                            next->src[at] = kids;
+                            next->seg[at] = seg;
+                            next->first[at] = ch[j].first;
+                        }
                         out.child[j] = idx;
                     } else {
                         gatomic_or(&a.counters[1], 2u);
@@ -1162,15 +1185,16 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs a) {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t begin = lane < (uint32_t)a.level ? a.lvl_cnt[lane] : 0u;
     for (int o = 32; o > 0; o >>= 1) begin += __shfl_xor(begin, o);
-    collapse_level<W>(a, a.level, begin, cnt);
+    collapse_level<W>(a, begin, cnt, a.lvl_cnt + a.level + 1);
 }
 static_assert(kMaxLevels <= 64, "k_collapse sums the levels before its own with one wave");
 
 // The levels from a.level on, by one block: the few nodes of levels that trees of ordinary
 // depth do not reach (a launch each would be 40 empty launches per batch replay).  The
 // counts are read past the L1, where the atomics left them.
+
 template <int W>
-__global__ __launch_bounds__(1024) void k_collapse_tail(CollapseArgs a) {
+__global__ __launch_bounds__(kBlockLevelThreads) void k_collapse_tail(CollapseArgs a) {
     auto count = [&](int l) {
         return __hip_atomic_load((global_u32*)(a.lvl_cnt + l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
@@ -1179,10 +1203,42 @@ __global__ __launch_bounds__(1024) void k_collapse_tail(CollapseArgs a) {
     for (int l = a.level; l < kMaxLevels; l++) {
         const uint32_t cnt = count(l);
         if (cnt == 0) break;
-        collapse_level<W>(a, l, begin, cnt);
+        collapse_level<W>(a, begin, cnt, a.lvl_cnt + l + 1);
         begin += cnt;
         __threadfence_block();
         __syncthreads();
+    }
+    if (threadIdx.x == 0) a.counters[0] = begin + count(kMaxLevels);
+}
+
+// Levels [0, last), none of more than kHeadNodes nodes, by one block.  A level of a few
+// nodes is latency alone: 7-12 us as a launch that reads its count and its list and takes its
+// slots through device memory, 5 us with these in LDS (a 5 K triangle build's 5 first levels
+// 45 -> 24 us).  With 1024 nodes (one level more) a 2.3 M triangle build is no faster than
+// with launches: its nodes are cold, and one CU waits for them longer than many.
+template <int W>
+__global__ __launch_bounds__(kBlockLevelThreads) void k_collapse_head(CollapseArgs a, int n_seg, int last,
+                                                                      const SegDesc* __restrict__ segs,
+                                                                      const uint32_t* __restrict__ seg_root) {
+    __shared__ HeadList list[2];
+    __shared__ uint32_t count[2];
+    for (uint32_t i = threadIdx.x; i < (uint32_t)n_seg; i += kBlockLevelThreads) {
+        list[0].src[i] = root_kids(a.bnode, seg_root[i], (uint32_t)a.leaf_size);
+        list[0].seg[i] = i;
+        list[0].first[i] = segs[i].tri_offset;
+        a.wseg[i] = i;
+        a.wfirst[i] = segs[i].tri_offset;
+    }
+    uint32_t begin = 0, cnt = (uint32_t)n_seg;
+    for (int l = 0; l < last && cnt; l++) {
+        uint32_t* const next_count = &count[(l + 1) & 1];
+        if (threadIdx.x == 0) *next_count = 0;
+        __syncthreads();
+        collapse_level<W, true>(a, begin, cnt, next_count, &list[l & 1], &list[(l + 1) & 1]);
+        __syncthreads();
+        begin += cnt;
+        cnt = *next_count;
+        if (threadIdx.x == 0) a.lvl_cnt[l + 1] = cnt;
     }
 }
 
@@ -1223,13 +1279,12 @@ __global__ __launch_bounds__(kBlock) void k_sah_cost(const WNode<W>* __restrict_
 
 // level 0 of the wide tree: one node per mesh root
 __global__ void k_init_levels(int n_seg, const SegDesc* __restrict__ segs, const uint32_t* __restrict__ seg_root,
-                              uint32_t* __restrict__ wsrc, uint32_t* __restrict__ wseg,
-                              uint32_t* __restrict__ wfirst) {
+                              CollapseArgs a) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n_seg) {
-        wsrc[i] = seg_root[i];
-        wseg[i] = (uint32_t)i;
-        wfirst[i] = segs[i].tri_offset;
+        a.wsrc[i] = root_kids(a.bnode, seg_root[i], (uint32_t)a.leaf_size);
+        a.wseg[i] = (uint32_t)i;
+        a.wfirst[i] = segs[i].tri_offset;
     }
 }
 
@@ -1401,23 +1456,27 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
             b.repacked = true;
         }
     }
-    hipLaunchKernelGGL(k_init_levels, dim3(cdiv(n_seg, kBlock)), dim3(kBlock), 0, s, n_seg, b.segs, b.seg_root,
-                       b.wsrc, b.wseg, b.wfirst);
     GPURT_HIP(hipGetLastError());
     return GPURT_OK;
 }
 
 template <int W>
-static void launch_collapse(CollapseArgs a, int levels, unsigned grid, hipStream_t s) {
-    for (int level = 0; level < levels; level++) {
+static void launch_collapse(CollapseArgs a, int n_seg, const SegDesc* segs, const uint32_t* seg_root, int levels,
+                            unsigned grid, hipStream_t s) {
+    int head = 0;  // levels of at most kHeadNodes nodes
+    for (size_t n = (size_t)n_seg; n <= kHeadNodes && head < levels; n *= W) head++;
+    if (head)
+        hipLaunchKernelGGL(k_collapse_head<W>, dim3(1), dim3(kBlockLevelThreads), 0, s, a, n_seg, head, segs, seg_root);
+    else
+        hipLaunchKernelGGL(k_init_levels, dim3(cdiv(n_seg, kBlock)), dim3(kBlock), 0, s, n_seg, segs, seg_root, a);
+    for (int level = head; level < levels; level++) {
         a.level = level;
         hipLaunchKernelGGL(k_collapse<W>, dim3(grid), dim3(kBlock), 0, s, a);
     }
     a.level = levels;
-    hipLaunchKernelGGL(k_collapse_tail<W>, dim3(1), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(k_collapse_tail<W>, dim3(1), dim3(kBlockLevelThreads), 0, s, a);
 }
 
-// Enqueues the wide collapse (every level: no host synchronisation) and the re-pack.
 int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s) {
     CollapseArgs ca{};
     ca.bnode = b.bnode;
@@ -1441,9 +1500,9 @@ int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s) {
     const int per = b.width == 2 ? 10 : (b.width == 4 ? 8 : 5);
     const int levels = std::min(kMaxLevels - 1, 2 + nbits * per / 10);
     const unsigned grid = std::min(cdiv(b.capacity, kBlock), 2048u);
-    if (b.width == 2) launch_collapse<2>(ca, levels, grid, s);
-    else if (b.width == 4) launch_collapse<4>(ca, levels, grid, s);
-    else launch_collapse<8>(ca, levels, grid, s);
+    if (b.width == 2) launch_collapse<2>(ca, b.n_seg, b.segs, b.seg_root, levels, grid, s);
+    else if (b.width == 4) launch_collapse<4>(ca, b.n_seg, b.segs, b.seg_root, levels, grid, s);
+    else launch_collapse<8>(ca, b.n_seg, b.segs, b.seg_root, levels, grid, s);
     if (b.repacked)
         hipLaunchKernelGGL(k_repack, dim3(cdiv(3 * (size_t)b.N, kBlock)), dim3(kBlock), 0, s, b.N, b.perm, b.tris,
                            b.leaf_order, b.tris2, b.leaf_order2);

@@ -328,7 +328,8 @@ struct BuildBufs {
     uint32_t* lvl_begin = nullptr;  // bucket k = lvl_order[lvl_begin[k] .. lvl_begin[k+1])
     uint32_t* lvl_fill = nullptr;
     float4* bnode = nullptr;  // binary node records, 3 float4 each (build_common.h)
-    uint32_t *wsrc = nullptr, *wseg = nullptr;
+    uint2* wsrc = nullptr;       // wide node -> the binary refs it starts from
+    uint32_t* wseg = nullptr;
     uint32_t* wfirst = nullptr;  // wide node -> first packed triangle of its (contiguous) range
     uint32_t* perm = nullptr;    // re-packed slot -> sorted position (treelet builds)
     // What the host reads of a build, in one piece (kReportWords); lvl and counters point
