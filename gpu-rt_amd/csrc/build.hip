@@ -610,56 +610,6 @@ __global__ __launch_bounds__(kBlock) void k_pack(uint32_t N, const uint64_t* __r
 }
 
 // ------------------------------------------------------------------------------------
-// k_karras: binary radix tree (Karras 2012, Algorithm 2) over 64-bit keys
-// ------------------------------------------------------------------------------------
-
-__device__ __forceinline__ int kdelta(const uint64_t* __restrict__ k, int n, int i, int j) {
-    if (j < 0 || j >= n) return -1;
-    uint64_t a = k[i], b = k[j];
-    if (a == b) return 64 + __clz((uint32_t)(i ^ j));
-    return __clzll(a ^ b);
-}
-
-// binary references: internal node i -> i; leaf (sorted primitive p) -> kLeafBit | p
-__global__ __launch_bounds__(kBlock) void k_karras(int N, const uint64_t* __restrict__ keys,
-                                                   const SegDesc* __restrict__ segs,
-                                                   uint2* __restrict__ kids, uint2* __restrict__ range,
-                                                   uint32_t* __restrict__ seg_root,
-                                                   uint8_t* __restrict__ dlev) {
-    int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= N - 1) return;
-    int d = (kdelta(keys, N, i, i + 1) - kdelta(keys, N, i, i - 1)) >= 0 ? 1 : -1;
-    int dmin = kdelta(keys, N, i, i - d);
-    int lmax = 2;
-    while (kdelta(keys, N, i, i + lmax * d) > dmin) lmax *= 2;
-    int l = 0;
-    for (int t = lmax / 2; t >= 1; t /= 2)
-        if (kdelta(keys, N, i, i + (l + t) * d) > dmin) l += t;
-    int j = i + l * d;
-    int dnode = kdelta(keys, N, i, j);
-    int s = 0, t = l;
-    do {
-        t = (t + 1) / 2;
-        if (kdelta(keys, N, i, i + (s + t) * d) > dnode) s += t;
-    } while (t > 1);
-    int split = i + s * d + min(d, 0);
-    int first = min(i, j), last = max(i, j);
-    uint32_t L = (first == split) ? (kLeafBit | (uint32_t)split) : (uint32_t)split;
-    uint32_t R = (last == split + 1) ? (kLeafBit | (uint32_t)(split + 1)) : (uint32_t)(split + 1);
-    kids[i] = make_uint2(L, R);
-    range[i] = make_uint2((uint32_t)first, (uint32_t)last);
-    uint32_t sf = (uint32_t)(keys[first] >> 30), sl = (uint32_t)(keys[last] >> 30);
-    if (sf == sl) {
-        const SegDesc sd = segs[sf];
-        if ((uint32_t)first == sd.tri_offset && (uint32_t)last == sd.tri_offset + sd.n_tris - 1u)
-            seg_root[sf] = (uint32_t)i;
-    }
-    // nodes above the mesh roots (their range spans several meshes) belong to no BVH:
-    // prefix length 0xFF keeps the box and treelet passes away from them
-    dlev[i] = (sf == sl) ? (uint8_t)dnode : (uint8_t)0xFF;
-}
-
-// ------------------------------------------------------------------------------------
 // internal node boxes and SAH costs
 // ------------------------------------------------------------------------------------
 
@@ -746,7 +696,7 @@ __global__ __launch_bounds__(kBlock) void k_level_scatter(int n_int, const uint8
 
 // Node boxes without atomics, fences or an order between launches.
 //
-// k_boxes_local: block c owns internal nodes [256c, 256c + 256).  A node whose leaf range
+// k_tree_local: block c owns internal nodes [256c, 256c + 256).  A node whose leaf range
 // lies in one such chunk has its whole subtree there (a Karras node's index is an end of
 // its range, so the subtree's internal nodes lie inside the range), so the block computes
 // all of these bottom up by itself: rounds in which every node whose children are done
@@ -763,7 +713,7 @@ __global__ __launch_bounds__(kBlock) void k_level_scatter(int n_int, const uint8
 // 61 of them) gave them before: 110 us of GPU time and 40 launches' gaps in a 5 K triangle
 // build, 235 us at 2.3 M, 390 us in a 7 M triangle batch.
 __device__ __forceinline__ bool box_in_chunk(uint2 r) { return (r.x >> 8) == (r.y >> 8); }
-static_assert(kBlock == 256, "k_boxes_local chunks are 256 nodes");
+static_assert(kBlock == 256, "k_tree_local chunks are 256 nodes");
 
 __device__ __forceinline__ void write_bnode(float4* __restrict__ bnode, uint32_t i, float4 lo, float4 hi, uint2 kid,
                                             uint2 range, float cost) {
@@ -774,27 +724,33 @@ __device__ __forceinline__ void write_bnode(float4* __restrict__ bnode, uint32_t
     bnode[3 * (size_t)i + 2] = make_float4(__uint_as_float(range.y - range.x + 1u), cost, __uint_as_float(range.x), 0.0f);
 }
 
-__global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t N, const uint2* __restrict__ range,
-                                                        const uint2* __restrict__ kids,
-                                                        const uint8_t* __restrict__ dlev,
-                                                        const float4* __restrict__ saabb,
-                                                        float4* __restrict__ bnode, float4* __restrict__ rbox,
-                                                        int leaf_size) {
+// Karras' binary radix tree over the sorted 64-bit keys (Karras 2012, Algorithm 2) and the
+// boxes of its in-chunk nodes, thread i of the grid making node i.  The searches compare a
+// node's key with ones mostly near it, so the chunk's keys and a chunk's either side are held
+// in LDS (as a launch of its own that read every key from memory: 76 us on 2.3 M triangles,
+// and 88 us for the boxes; 132 us together).  binary references: internal node i -> i; leaf
+// (sorted primitive p) -> kLeafBit | p
+__global__ __launch_bounds__(kBlock) void k_tree_local(uint32_t N, const uint64_t* __restrict__ keys,
+                                                       const SegDesc* __restrict__ segs,
+                                                       const float4* __restrict__ saabb, uint2* __restrict__ kids,
+                                                       uint2* __restrict__ range, uint32_t* __restrict__ seg_root,
+                                                       uint8_t* __restrict__ dlev, float4* __restrict__ bnode,
+                                                       float4* __restrict__ rbox, int leaf_size) {
     __shared__ float4 slo[kBlock], shi[kBlock];  // the chunk's leaf boxes
-    __shared__ float4 blo[kBlock], bhi[kBlock];
+    __shared__ float4 box[2 * kBlock];           // the keys, then the in-chunk nodes' boxes
     __shared__ float bcost[kBlock];
     __shared__ uint8_t done[kBlock];
+    constexpr uint32_t kWindow = 3 * kBlock;
+    static_assert(sizeof(uint64_t) * kWindow <= sizeof(box), "the keys fit");
+    uint64_t* const skey = reinterpret_cast<uint64_t*>(box);
+    float4 *const blo = box, *const bhi = box + kBlock;
     const uint32_t c0 = blockIdx.x * kBlock, tid = threadIdx.x;
     const uint32_t i = c0 + tid;
-    bool todo = false;
-    uint32_t L = 0, R = 0;
-    uint2 rg = make_uint2(0u, 0u);
-    if (i < n_int && dlev[i] != 0xFF) {
-        rg = range[i];
-        todo = box_in_chunk(rg);
-        const uint2 k = kids[i];
-        L = k.x;
-        R = k.y;
+    const int w0 = (int)c0 - kBlock;
+#pragma unroll
+    for (uint32_t k = tid; k < kWindow; k += kBlock) {
+        const int j = w0 + (int)k;
+        skey[k] = j >= 0 && j < (int)N ? keys[j] : 0ull;
     }
     float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
     if (i < N) {
@@ -804,11 +760,57 @@ __global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t
     slo[tid] = lo;
     shi[tid] = hi;
     done[tid] = 0;
-    if (rbox) write_range_blocks(N, i, lo, hi, rbox, blo);  // (blo is not in use yet)
     __syncthreads();
+    bool todo = false;
+    uint32_t L = 0, R = 0;
+    uint2 rg = make_uint2(0u, 0u);
+    if (i < N - 1) {
+        auto key = [&](int j) { return (uint32_t)(j - w0) < kWindow ? skey[j - w0] : keys[j]; };
+        const uint64_t mine = skey[tid + kBlock];
+        const int n = (int)i;
+        // common prefix of keys n and j (equal keys: of the indices, behind 64 bits)
+        auto delta = [&](int j) {
+            if (j < 0 || j >= (int)N) return -1;
+            const uint64_t x = mine ^ key(j);
+            return x ? __clzll(x) : 64 + __clz((uint32_t)(n ^ j));
+        };
+        const int dir = delta(n + 1) - delta(n - 1) >= 0 ? 1 : -1;
+        const int dmin = delta(n - dir);
+        int lmax = 2;
+        while (delta(n + lmax * dir) > dmin) lmax *= 2;
+        int l = 0;
+        for (int t = lmax / 2; t >= 1; t /= 2)
+            if (delta(n + (l + t) * dir) > dmin) l += t;
+        const int j = n + l * dir;
+        const int dnode = delta(j);
+        int s = 0, t = l;
+        do {
+            t = (t + 1) / 2;
+            if (delta(n + (s + t) * dir) > dnode) s += t;
+        } while (t > 1);
+        const int split = n + s * dir + min(dir, 0);
+        const int first = min(n, j), last = max(n, j);
+        L = first == split ? (kLeafBit | (uint32_t)split) : (uint32_t)split;
+        R = last == split + 1 ? (kLeafBit | (uint32_t)(split + 1)) : (uint32_t)(split + 1);
+        rg = make_uint2((uint32_t)first, (uint32_t)last);
+        kids[i] = make_uint2(L, R);
+        range[i] = rg;
+        const uint32_t sf = (uint32_t)(key(first) >> 30), sl = (uint32_t)(key(last) >> 30);
+        if (sf == sl) {
+            const SegDesc sd = segs[sf];
+            if ((uint32_t)first == sd.tri_offset && (uint32_t)last == sd.tri_offset + sd.n_tris - 1u) seg_root[sf] = i;
+        }
+        // nodes above the mesh roots (their range spans several meshes) belong to no BVH:
+        // prefix length 0xFF keeps the box and treelet passes away from them
+        dlev[i] = sf == sl ? (uint8_t)dnode : (uint8_t)0xFF;
+        todo = sf == sl && box_in_chunk(rg);
+    }
+    __syncthreads();  // the keys have been read
+    if (rbox) write_range_blocks(N, i, lo, hi, rbox, blo);
+    const bool mine_to_write = todo;
+    float cost = 0.f;
     while (__syncthreads_or(todo)) {
         const bool ready = todo && ((L & kLeafBit) || done[L - c0]) && ((R & kLeafBit) || done[R - c0]);
-        float c = 0.f;
         if (ready) {
             // a leaf of an in-chunk node lies in the chunk
             const uint32_t l = (L & ~kLeafBit) - c0, r = (R & ~kLeafBit) - c0;
@@ -818,18 +820,19 @@ __global__ __launch_bounds__(kBlock) void k_boxes_local(uint32_t n_int, uint32_t
             const float cl = ll ? kCt * box_area(al, ah) : bcost[l], cr = rl ? kCt * box_area(bl, bh) : bcost[r];
             lo = min4(al, bl);
             hi = max4(ah, bh);
-            c = sah_node_cost(lo, hi, rg.y - rg.x + 1u, cl, cr, leaf_size);
+            cost = sah_node_cost(lo, hi, rg.y - rg.x + 1u, cl, cr, leaf_size);
         }
         __syncthreads();  // every read of this round before any write
         if (ready) {
             blo[tid] = lo;
             bhi[tid] = hi;
-            bcost[tid] = c;
+            bcost[tid] = cost;
             done[tid] = 1;
-            write_bnode(bnode, i, lo, hi, make_uint2(L, R), rg, c);
             todo = false;
         }
     }
+    // (written together at the end: a store per round had few lanes in it)
+    if (mine_to_write) write_bnode(bnode, i, lo, hi, make_uint2(L, R), rg, cost);
 }
 
 // The aligned blocks above the chunks, level by level: one block of threads for all levels
@@ -919,7 +922,7 @@ __global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t n_int, uint32_t
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n_int || dlev[i] == 0xFF) return;
     const uint2 rg = range[i];
-    if (box_in_chunk(rg)) return;  // done by k_boxes_local
+    if (box_in_chunk(rg)) return;  // done by k_tree_local
     float4 lo, hi;
     range_union(
         rg.x, rg.y + 1u, N, rbox,
@@ -1428,11 +1431,9 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
     if (N > 1) {
         const uint32_t n_int = N - 1;
         const unsigned gI = cdiv(n_int, kBlock);
-        hipLaunchKernelGGL(k_karras, dim3(gI), dim3(kBlock), 0, s, (int)N, kin, b.segs, b.kids, b.range, b.seg_root,
-                           b.dlev);
         const bool cross = N > kBlock;  // more than one chunk
-        hipLaunchKernelGGL(k_boxes_local, dim3(gN), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
-                           b.bnode, cross ? b.rbox : nullptr, b.leaf_size);
+        hipLaunchKernelGGL(k_tree_local, dim3(gN), dim3(kBlock), 0, s, N, kin, b.segs, b.saabb, b.kids, b.range,
+                           b.seg_root, b.dlev, b.bnode, cross ? b.rbox : nullptr, b.leaf_size);
         if (cross) {
             launch_range_top(N, b.rbox, s);
             hipLaunchKernelGGL(k_boxes_cross, dim3(gI), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,

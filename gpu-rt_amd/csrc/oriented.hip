@@ -49,19 +49,6 @@ struct OrientArgs {
     const uint32_t* skip;   // nothing is written when *skip (null: never)
 };
 
-// minimum and maximum as the hardware's instructions, without the quieting of signalling
-// NaNs that fminf and fmaxf put before them (a third of this kernel's instructions; a NaN
-// operand is dropped all the same)
-__device__ __forceinline__ float vmin(float a, float b) {
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmax(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
 __device__ __forceinline__ V3 vmin(V3 a, V3 b) { return v3(vmin(a.x, b.x), vmin(a.y, b.y), vmin(a.z, b.z)); }
 __device__ __forceinline__ V3 vmax(V3 a, V3 b) { return v3(vmax(a.x, b.x), vmax(a.y, b.y), vmax(a.z, b.z)); }
 
