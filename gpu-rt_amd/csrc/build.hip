@@ -735,11 +735,13 @@ __global__ __launch_bounds__(kBlock) void k_tree_local(uint32_t N, const uint64_
                                                        const float4* __restrict__ saabb, uint2* __restrict__ kids,
                                                        uint2* __restrict__ range, uint32_t* __restrict__ seg_root,
                                                        uint8_t* __restrict__ dlev, float4* __restrict__ bnode,
-                                                       float4* __restrict__ rbox, int leaf_size) {
+                                                       float4* __restrict__ rbox, uint8_t* __restrict__ xlist,
+                                                       uint32_t* __restrict__ xcount, int leaf_size) {
     __shared__ float4 slo[kBlock], shi[kBlock];  // the chunk's leaf boxes
     __shared__ float4 box[2 * kBlock];           // the keys, then the in-chunk nodes' boxes
     __shared__ float bcost[kBlock];
     __shared__ uint8_t done[kBlock];
+    __shared__ uint32_t xwave[kBlock / 64];
     constexpr uint32_t kWindow = 3 * kBlock;
     static_assert(sizeof(uint64_t) * kWindow <= sizeof(box), "the keys fit");
     uint64_t* const skey = reinterpret_cast<uint64_t*>(box);
@@ -761,7 +763,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_local(uint32_t N, const uint64_
     shi[tid] = hi;
     done[tid] = 0;
     __syncthreads();
-    bool todo = false;
+    bool todo = false, cross = false;
     uint32_t L = 0, R = 0;
     uint2 rg = make_uint2(0u, 0u);
     if (i < N - 1) {
@@ -804,8 +806,17 @@ __global__ __launch_bounds__(kBlock) void k_tree_local(uint32_t N, const uint64_
         // prefix length 0xFF keeps the box and treelet passes away from them
         dlev[i] = sf == sl ? (uint8_t)dnode : (uint8_t)0xFF;
         todo = sf == sl && box_in_chunk(rg);
+        cross = sf == sl && !todo;
     }
-    __syncthreads();  // the keys have been read
+    const uint64_t xmask = __ballot(cross);
+    if ((tid & 63u) == 0) xwave[tid >> 6] = (uint32_t)__popcll(xmask);
+    __syncthreads();  // (the keys have been read, too)
+    if (rbox) {  // the chunk's other nodes, for k_boxes_cross
+        uint32_t at = (uint32_t)__popcll(xmask & ((1ull << (tid & 63u)) - 1ull));
+        for (uint32_t w = 0; w < tid >> 6; w++) at += xwave[w];
+        if (cross) xlist[c0 + at] = (uint8_t)tid;
+        if (tid == 0) xcount[blockIdx.x] = xwave[0] + xwave[1] + xwave[2] + xwave[3];
+    }
     if (rbox) write_range_blocks(N, i, lo, hi, rbox, blo);
     const bool mine_to_write = todo;
     float cost = 0.f;
@@ -852,9 +863,11 @@ __global__ __launch_bounds__(1024) void k_range_top(uint32_t N, float4* rbox) {
         float4* dst = src + 2 * (size_t)cnt;
         for (uint32_t e = threadIdx.x; e < up; e += 1024) {
             float4 lo = src[8 * (size_t)e], hi = src[8 * (size_t)e + 1];
-            for (uint32_t k = 1; k < 4 && 4 * e + k < cnt; k++) {
-                lo = min4(lo, src[2 * (4 * (size_t)e + k)]);
-                hi = max4(hi, src[2 * (4 * (size_t)e + k) + 1]);
+#pragma unroll
+            for (uint32_t k = 1; k < 4; k++) {  // (past the end: the last one again)
+                const size_t c = min(4 * e + k, cnt - 1);
+                lo = min4(lo, src[2 * c]);
+                hi = max4(hi, src[2 * c + 1]);
             }
             dst[2 * (size_t)e] = lo;
             dst[2 * (size_t)e + 1] = hi;
@@ -913,27 +926,36 @@ __device__ float small_cost(uint32_t root, const uint2* __restrict__ kids, const
     return c;
 }
 
-__global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t n_int, uint32_t N, const uint2* __restrict__ range,
+// kCrossLanes lanes per chunk share its list: ~10 of a chunk's 256 nodes are here, each a
+// chain of dependent loads (a thread per node of the tree, 10 of 256 with work: 48 us on 2.3 M triangles,
+// 137 us on a 6.9 M triangle batch; now 29 and ~60).
+constexpr uint32_t kCrossLanes = 16;
+
+__global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t N, const uint2* __restrict__ range,
                                                         const uint2* __restrict__ kids,
-                                                        const uint8_t* __restrict__ dlev,
+                                                        const uint8_t* __restrict__ xlist,
+                                                        const uint32_t* __restrict__ xcount,
                                                         const float4* __restrict__ saabb,
                                                         const float4* __restrict__ rbox, float4* __restrict__ bnode,
                                                         int leaf_size, int costs) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n_int || dlev[i] == 0xFF) return;
-    const uint2 rg = range[i];
-    if (box_in_chunk(rg)) return;  // done by k_tree_local
-    float4 lo, hi;
-    range_union(
-        rg.x, rg.y + 1u, N, rbox,
-        [&](uint32_t k, float4& l, float4& h) {
-            l = min4(l, saabb[2 * (size_t)k]);
-            h = max4(h, saabb[2 * (size_t)k + 1]);
-        },
-        lo, hi);
-    float c = 0.0f;
-    if (costs && rg.y - rg.x + 1u <= 2u * (uint32_t)leaf_size) c = small_cost(i, kids, range, saabb, leaf_size);
-    write_bnode(bnode, i, lo, hi, kids[i], rg, c);
+    const uint32_t chunk = (blockIdx.x * kBlock + threadIdx.x) / kCrossLanes;
+    if (chunk * kBlock >= N) return;
+    const uint32_t n = xcount[chunk];
+    for (uint32_t k = threadIdx.x % kCrossLanes; k < n; k += kCrossLanes) {
+        const uint32_t i = chunk * kBlock + xlist[chunk * kBlock + k];
+        const uint2 rg = range[i];
+        float4 lo, hi;
+        range_union(
+            rg.x, rg.y + 1u, N, rbox,
+            [&](uint32_t k, float4& l, float4& h) {
+                l = min4(l, saabb[2 * (size_t)k]);
+                h = max4(h, saabb[2 * (size_t)k + 1]);
+            },
+            lo, hi);
+        float c = 0.0f;
+        if (costs && rg.y - rg.x + 1u <= 2u * (uint32_t)leaf_size) c = small_cost(i, kids, range, saabb, leaf_size);
+        write_bnode(bnode, i, lo, hi, kids[i], rg, c);
+    }
 }
 
 // ------------------------------------------------------------------------------------
@@ -1330,6 +1352,8 @@ static void carve_all(BuildBufs& b, Carver& c, size_t NI) {
     c.take(b.range, NI);
     c.take(b.seg_root, n_seg);
     c.take(b.dlev, NI);
+    c.take(b.xlist, N);
+    c.take(b.xcount, cdiv(N, kBlock));
     c.take(b.lvl_order, b.treelets ? NI : 1);
     c.take(b.lvl_hist, kLevelBuckets);
     c.take(b.lvl_begin, kLevelBuckets + 1);
@@ -1433,11 +1457,12 @@ int build_enqueue_binary(BuildBufs& b, int treelet_size, int treelet_rounds, hip
         const unsigned gI = cdiv(n_int, kBlock);
         const bool cross = N > kBlock;  // more than one chunk
         hipLaunchKernelGGL(k_tree_local, dim3(gN), dim3(kBlock), 0, s, N, kin, b.segs, b.saabb, b.kids, b.range,
-                           b.seg_root, b.dlev, b.bnode, cross ? b.rbox : nullptr, b.leaf_size);
+                           b.seg_root, b.dlev, b.bnode, cross ? b.rbox : nullptr, b.xlist, b.xcount, b.leaf_size);
         if (cross) {
             launch_range_top(N, b.rbox, s);
-            hipLaunchKernelGGL(k_boxes_cross, dim3(gI), dim3(kBlock), 0, s, n_int, N, b.range, b.kids, b.dlev, b.saabb,
-                               b.rbox, b.bnode, b.leaf_size, b.treelets ? 1 : 0);
+            hipLaunchKernelGGL(k_boxes_cross, dim3(cdiv((size_t)gN * kCrossLanes, kBlock)), dim3(kBlock), 0, s, N,
+                               b.range, b.kids, b.xlist, b.xcount, b.saabb, b.rbox, b.bnode, b.leaf_size,
+                               b.treelets ? 1 : 0);
         }
         if (treelet_size > 0) {
             // bucket the treelet roots by prefix length; distinct keys give

@@ -320,6 +320,8 @@ struct BuildBufs {
     float4* saabb = nullptr;  // sorted triangle boxes (lo, hi)
     float4* rbox = nullptr;   // boxes of aligned blocks of 4, 16, ... sorted triangles
     uint2 *kids = nullptr, *range = nullptr;  // binary tree: children, leaf range
+    uint8_t* xlist = nullptr;    // per chunk of 256 nodes, the ones whose range crosses chunks
+    uint32_t* xcount = nullptr;  // and their number
     uint32_t* seg_root = nullptr;
     uint8_t* dlev = nullptr;  // common-prefix length (Karras delta) of each internal node
     // treelet roots bucketed by prefix length
