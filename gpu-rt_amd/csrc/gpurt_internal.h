@@ -208,12 +208,11 @@ struct gpurt_ctx_s {
 namespace gpurt_impl {
 // Vertex-gradient sums of the backward passes: the fixed-order sum (sort by vertex, then
 // segmented sums) when the context asks for it, FP32 atomics when it asks for them, and
-// otherwise whichever is faster -- the fixed order from about 2 M vertex terms, where
-// the atomics' device-wide rate (~20 G/s) costs more than the sort's passes (1 M
-// closest-point queries = 3.1 M terms: 0.38 vs 0.48 ms; a 256-mesh batch of 19 M queries
-// and rays: forward + backward 32.3 vs 36.1 ms; 262 K rays = 0.8 M terms: 0.17 vs 0.13
-// ms).
-constexpr size_t kFixedOrderMinTerms = size_t(1) << 21;
+// otherwise whichever is faster -- the fixed order from about 0.6 M vertex terms, where the
+// atomics' device-wide rate (~18 G/s) costs more than the sort's passes (points or rays on a
+// 0.66 M vertex mesh, fixed order / atomics, us: 65 K 72 / 38, 131 K 82 / 69, 262 K 102 /
+// 132, 524 K 150 / 252; fewer vertices favour the fixed order, which has fewer passes).
+constexpr size_t kFixedOrderMinTerms = 600000;
 inline bool fixed_order_sums(const gpurt_ctx_s* c, size_t terms) {
     return c->vertex_sums == GPURT_SUMS_FIXED_ORDER ||
            (c->vertex_sums == GPURT_SUMS_AUTO && terms >= kFixedOrderMinTerms);

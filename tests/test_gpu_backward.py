@@ -283,3 +283,25 @@ def test_fixed_order_sums_at_sort_edges(dev, level, n):
     assert (np.abs(runs[0] - ev) <= ((count + 4) * 2.0**-24 * total)[:, None] + 1e-30).all()
     bvh.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("n,fixed", [(199_999, False), (200_000, True)])
+def test_auto_vertex_sums_change_at_600000_terms(dev, n, fixed):
+    """The default mode adds in the fixed order (the same bits as the fixed mode) from 600,000
+    terms on and with atomics below (bits that then vary from it, within rounding)."""
+    V, F = _sphere(6, 11)
+    Q = W.surface_samples(V.astype(np.float64), F, np.random.default_rng(13), n, 0.01).astype(np.float32)
+    out = {}
+    for mode in ("auto", "fixed"):
+        ctx = gpurt.Context(0, vertex_sums=mode)
+        bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev))
+        tq = _t(Q, dev)
+        prim, pt, dist, bary = bvh.closest_point(tq)
+        gv = torch.zeros((V.shape[0], 3), device=dev)
+        bvh.closest_point_bwd(tq, prim, bary, pt, dist, torch.ones(n, device=dev), None, gv)
+        out[mode] = gv.cpu().numpy()
+        bvh.close()
+        ctx.close()
+    assert not fixed or np.array_equal(out["auto"], out["fixed"])
+    scale = np.abs(out["fixed"]).max()
+    np.testing.assert_allclose(out["auto"], out["fixed"], atol=1e-5 * scale, rtol=1e-4)
