@@ -160,21 +160,29 @@ __device__ __forceinline__ void scatter_terms(const CornerTerms& t, float* g_ver
 // add nothing), are summed per key in two passes with a fixed order (the same bits on
 // every run), and without a serial loop over a long run:
 //   k_wave_segsum  one thread per sorted term: within each 64-term wave, a segmented
-//                  suffix scan over shuffles; the first term of each key in the wave keeps
-//                  the sum of that key's terms in the wave (partial[p])
-//   k_run_sum      the first term of each key's run adds the partials of the waves the
-//                  run spans (one per 64 terms) and hands the total to the sink
-template <int BS, typename K>
+//                  suffix scan over shuffles leaves a key's sum with its first term, which
+//                  hands it to the sink when the key's run lies in the wave
+//   k_run_sum      one thread per wave: the sum of a run that starts in it and goes on (its
+//                  part in the wave, then those of the next waves in turn)
+// Only the parts of runs across waves pass through memory, two per wave (a partial sum per
+// term and a second pass over all terms: the sums of a step on 1.3 M triangles, 3.1 M terms,
+// 75 us, of a 256-mesh batch 353 us; now 55 and 208).
+struct WaveSums {
+    float *first, *last;  // per wave: part of the run it continues, part of the one that goes on
+};
+
+template <int BS, typename K, typename Sink>
 __global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const K* __restrict__ keys,
                                                     const uint32_t* __restrict__ vals, const float* __restrict__ terms,
-                                                    float* __restrict__ partial) {
+                                                    uint64_t none, WaveSums sums, Sink sink) {
     const uint32_t p = blockIdx.x * BS + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t lane = threadIdx.x & 63u, wave = p >> 6;
     const bool in = p < m;
     const K key = in ? keys[p] : ~(K)0;
-    const bool head = in && (lane == 0 || keys[p - 1] != key);
+    const bool goes_on = in && p > 0 && keys[p - 1] == key;  // (at lane 0: the run began before the wave)
+    const bool head = in && (lane == 0 || !goes_on);
     float x = 0.f, y = 0.f, z = 0.f;
-    if (in) {
+    if (in && key < none) {
         const size_t k = vals[p];
         x = terms[3 * k];
         y = terms[3 * k + 1];
@@ -193,27 +201,36 @@ __global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const K* __restr
             z += oz;
         }
     }
-    if (head) {
-        partial[3 * (size_t)p] = x;
-        partial[3 * (size_t)p + 1] = y;
-        partial[3 * (size_t)p + 2] = z;
+    if (!head || key >= none) return;
+    const size_t next = 64 * ((size_t)wave + 1);
+    float* part = goes_on ? sums.first : end == 64u && next < m && keys[next] == key ? sums.last : nullptr;
+    if (part) {
+        part[3 * (size_t)wave] = x;
+        part[3 * (size_t)wave + 1] = y;
+        part[3 * (size_t)wave + 2] = z;
+    } else {
+        sink(key, x, y, z);
     }
 }
 
 template <int BS, typename K, typename Sink>
-__global__ __launch_bounds__(BS) void k_run_sum(uint32_t m, const K* __restrict__ keys,
-                                                const float* __restrict__ partial, uint64_t none, Sink sink) {
-    const uint32_t p = blockIdx.x * BS + threadIdx.x;
-    if (p >= m) return;
-    const K key = keys[p];
-    if (key >= none || (p > 0 && keys[p - 1] == key)) return;
-    float x = partial[3 * (size_t)p], y = partial[3 * (size_t)p + 1], z = partial[3 * (size_t)p + 2];
-    for (uint32_t q = (p | 63u) + 1u; q < m && keys[q] == key; q += 64u) {
-        x += partial[3 * (size_t)q];
-        y += partial[3 * (size_t)q + 1];
-        z += partial[3 * (size_t)q + 2];
+__global__ __launch_bounds__(BS) void k_run_sum(uint32_t m, const K* __restrict__ keys, uint64_t none, WaveSums sums,
+                                                Sink sink) {
+    const uint32_t w = blockIdx.x * BS + threadIdx.x;
+    const size_t b = 64 * (size_t)w, next = b + 64;
+    if (next >= m) return;
+    const K key = keys[next];
+    if (key >= none || keys[next - 1] != key || (keys[b] == key && b > 0 && keys[b - 1] == key)) return;
+    float x = sums.last[3 * (size_t)w], y = sums.last[3 * (size_t)w + 1], z = sums.last[3 * (size_t)w + 2];
+    for (size_t q = next; q < m && keys[q] == key; q += 64) {
+        x += sums.first[3 * (q >> 6)];
+        y += sums.first[3 * (q >> 6) + 1];
+        z += sums.first[3 * (q >> 6) + 2];
     }
     sink(key, x, y, z);
 }
+
+// floats of a WaveSums array for m terms
+inline size_t wave_sum_floats(size_t m) { return 3 * ((m + 63) / 64); }
 
 }  // namespace gpurt_impl

@@ -96,7 +96,8 @@ struct TermScratch {
     void* mem = nullptr;
     CallScratch cs;
     uint32_t *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr, *sort = nullptr;
-    float *terms = nullptr, *partial = nullptr;
+    float* terms = nullptr;
+    WaveSums sums{};
 };
 
 int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
@@ -104,7 +105,7 @@ int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
     const size_t m = 3 * n;
     const size_t words = radix_sort_scratch_words((uint32_t)m);
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t bytes = 4 * up(4 * m) + 2 * up(12 * m) + up(4 * words) + 256;
+    const size_t bytes = 4 * up(4 * m) + up(12 * m) + 2 * up(4 * wave_sum_floats(m)) + up(4 * words) + 256;
     const int rc = ctx_scratch(c, s, bytes, t.cs);
     if (rc) return rc;
     t.mem = t.cs.mem;
@@ -119,8 +120,10 @@ int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
     p += up(4 * m);
     t.terms = reinterpret_cast<float*>(p);
     p += up(12 * m);
-    t.partial = reinterpret_cast<float*>(p);
-    p += up(12 * m);
+    for (float** q : {&t.sums.first, &t.sums.last}) {
+        *q = reinterpret_cast<float*>(p);
+        p += up(4 * wave_sum_floats(m));
+    }
     t.sort = reinterpret_cast<uint32_t*>(p);
     return GPURT_OK;
 }
@@ -140,9 +143,11 @@ void sum_terms(TermScratch& t, size_t n, uint32_t n_verts, float* g_verts, hipSt
         k = t.k1;
         v = t.v1;
     }
-    hipLaunchKernelGGL((k_wave_segsum<kBlock, uint32_t>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, v, t.terms, t.partial);
-    hipLaunchKernelGGL((k_run_sum<kBlock, uint32_t, VertexSink>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, t.partial,
-                       (uint64_t)n_verts, VertexSink{g_verts});
+    const VertexSink sink{g_verts};
+    hipLaunchKernelGGL((k_wave_segsum<kBlock, uint32_t, VertexSink>), dim3(cdiv(m, kBlock)), dim3(kBlock), 0, s, m, k, v,
+                       t.terms, (uint64_t)n_verts, t.sums, sink);
+    hipLaunchKernelGGL((k_run_sum<kBlock, uint32_t, VertexSink>), dim3(cdiv(cdiv(m, 64), kBlock)), dim3(kBlock), 0, s, m,
+                       k, (uint64_t)n_verts, t.sums, sink);
 }
 
 }  // namespace

@@ -430,7 +430,8 @@ namespace {
 struct BatchTerms {
     void *k0, *k1;
     uint32_t *v0, *v1, *sort;
-    float *terms, *partial;
+    float* terms;
+    WaveSums sums;
     const uint64_t* voff;
     uint64_t none;
     uint32_t m;
@@ -452,10 +453,11 @@ void record_batch_bwd(gpurt_batch b, const BatchTerms& t, uint32_t n_meshes) {
     // each (mesh, vertex)'s terms in chunk order, summed in a fixed order
     const bool in1 = radix_sort_pairs(k0, t.v0, k1, t.v1, t.m, t.kbits, t.sort, s);
     const K* k = in1 ? k1 : k0;
-    hipLaunchKernelGGL((k_wave_segsum<kBlock, K>), dim3(cdiv(t.m, kBlock)), dim3(kBlock), 0, s, t.m, k,
-                       in1 ? t.v1 : t.v0, t.terms, t.partial);
-    hipLaunchKernelGGL((k_run_sum<kBlock, K, MeshVertexSink>), dim3(cdiv(t.m, kBlock)), dim3(kBlock), 0, s, t.m, k,
-                       t.partial, t.none, MeshVertexSink{b->grads_d, t.voff, n_meshes});
+    const MeshVertexSink sink{b->grads_d, t.voff, n_meshes};
+    hipLaunchKernelGGL((k_wave_segsum<kBlock, K, MeshVertexSink>), dim3(cdiv(t.m, kBlock)), dim3(kBlock), 0, s, t.m, k,
+                       in1 ? t.v1 : t.v0, t.terms, t.none, t.sums, sink);
+    hipLaunchKernelGGL((k_run_sum<kBlock, K, MeshVertexSink>), dim3(cdiv(cdiv(t.m, 64), kBlock)), dim3(kBlock), 0, s,
+                       t.m, k, t.none, t.sums, sink);
 }
 
 }  // namespace
@@ -678,7 +680,8 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     while (kbits < 64 && (none >> kbits)) kbits++;
     auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t ksize = kbits <= 32 ? 4 : 8;
-    const size_t tbytes = 2 * up(ksize * m) + 2 * up(4 * (size_t)m) + 2 * up(12 * (size_t)m) +
+    const size_t tbytes = 2 * up(ksize * m) + 2 * up(4 * (size_t)m) + up(12 * (size_t)m) +
+                          2 * up(4 * wave_sum_floats(m)) +
                           up(4 * radix_sort_scratch_words(std::max<uint32_t>(m, 1))) + up(8 * (n_meshes + 1));
     DevGuard dg(b->ctx->device);
     if (!dg.ok) return set_error(GPURT_E_DEVICE, "hipSetDevice failed");
@@ -692,20 +695,24 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     }
     void *k0 = nullptr, *k1 = nullptr;
     uint32_t *v0 = nullptr, *v1 = nullptr, *sort_scratch = nullptr;
-    float *terms = nullptr, *partial = nullptr;
+    float* terms = nullptr;
+    WaveSums sums{};
     uint64_t* voff_d = nullptr;
     if (m) {
         char* tp = static_cast<char*>(b->terms_mem);
-        const size_t mk = up(ksize * m), m4 = up(4 * (size_t)m), m12 = up(12 * (size_t)m);
-        k0 = tp;
-        k1 = tp + mk;
-        v0 = reinterpret_cast<uint32_t*>(tp + 2 * mk);
-        v1 = reinterpret_cast<uint32_t*>(tp + 2 * mk + m4);
-        terms = reinterpret_cast<float*>(tp + 2 * mk + 2 * m4);
-        partial = reinterpret_cast<float*>(tp + 2 * mk + 2 * m4 + m12);
-        sort_scratch = reinterpret_cast<uint32_t*>(tp + 2 * mk + 2 * m4 + 2 * m12);
-        voff_d = reinterpret_cast<uint64_t*>(tp + 2 * mk + 2 * m4 + 2 * m12 +
-                                             up(4 * radix_sort_scratch_words(std::max<uint32_t>(m, 1))));
+        auto carve = [&](auto*& p, size_t bytes) {
+            p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(tp);
+            tp += up(bytes);
+        };
+        carve(k0, ksize * m);
+        carve(k1, ksize * m);
+        carve(v0, 4 * (size_t)m);
+        carve(v1, 4 * (size_t)m);
+        carve(terms, 12 * (size_t)m);
+        carve(sums.first, 4 * wave_sum_floats(m));
+        carve(sums.last, 4 * wave_sum_floats(m));
+        carve(sort_scratch, 4 * radix_sort_scratch_words(std::max<uint32_t>(m, 1)));
+        carve(voff_d, 8 * (n_meshes + 1));
     }
     if (hipMemcpy(b->grads_d, gd.data(), sizeof(BatchGradDev) * n_meshes, hipMemcpyHostToDevice) != hipSuccess ||
         (!segs.empty() &&
@@ -723,7 +730,7 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     if (!segs.empty())
         hipLaunchKernelGGL(k_batch_zero_vgrads, dim3((unsigned)segs.size()), dim3(256), 0, b->cap, b->grads_d,
                            b->zero_segs_d);
-    const BatchTerms bt{k0, k1, v0, v1, sort_scratch, terms, partial, voff_d, none, m, kbits};
+    const BatchTerms bt{k0, k1, v0, v1, sort_scratch, terms, sums, voff_d, none, m, kbits};
     if (kbits <= 32)
         record_batch_bwd<uint32_t>(b, bt, (uint32_t)n_meshes);
     else

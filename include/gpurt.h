@@ -153,7 +153,7 @@ GPURT_API int gpurt_ctx_status(gpurt_ctx ctx, uint32_t* flags, int clear);
  * add the per-query vertex terms (three per query or ray) into the vertex gradients:
  *   GPURT_SUMS_FIXED_ORDER  the terms are sorted by vertex (a stable radix sort) and each
  *                           vertex's terms added in a fixed order (a tree over query
- *                           order): the same bits on every run; 120 bytes of
+ *                           order): the same bits on every run; 84 bytes of
  *                           scratch per query (the context's per-stream buffer)
  *   GPURT_SUMS_ATOMIC       FP32 atomic adds, one pass; the summation order, and so the
  *                           last bits, can vary from run to run
@@ -334,9 +334,9 @@ typedef struct gpurt_batch_grad {
  * gpurt_ctx_set_vertex_sums mode when this is called (the default picks it for batches
  * of 600,000 terms and more), sorted by (mesh, vertex) and each vertex's terms added in a
  * fixed order (the same bits on every run).  Vertex gradients of hit t need the
- * forward's r_uv.  The fixed-order sum's term buffers (allocated here) take 120 bytes
- * per query or ray slot (3 terms of 40 bytes; slots are allotted in 64-item chunks per
- * mesh; 48 bytes where 32 bits do not number every vertex): about 2.3 GB for 19 M
+ * forward's r_uv.  The fixed-order sum's term buffers (allocated here) take 84 bytes
+ * per query or ray slot (3 terms of 28 bytes; slots are allotted in 64-item chunks per
+ * mesh; 36 bytes where 32 bits do not number every vertex): about 1.6 GB for 19 M
  * queries and rays.
  * No counterpart in the reference (it has no gradients); it is the batched form of
  * gpurt_closest_point_bwd + gpurt_trace_bwd.  Calling it again replaces the buffers. */
