@@ -842,40 +842,63 @@ __global__ __launch_bounds__(kBlock) void k_tree_local(uint32_t N, const uint64_
             todo = false;
         }
     }
-    // (written together at the end: a store per round had few lanes in it)
+    // (all at once at the end: a store per round had few lanes in it)
     if (mine_to_write) write_bnode(bnode, i, lo, hi, make_uint2(L, R), rg, cost);
 }
 
-// The aligned blocks above the chunks, level by level: one block of threads for all levels
-// (they hold a 768th of the leaf count in all), so no launch per level.  The level below is
-// read back from this block's own writes.
-__global__ __launch_bounds__(1024) void k_range_top(uint32_t N, float4* rbox) {
-    uint32_t cnt = N;
-    size_t off = 0;
-    for (int lvl = 1; lvl < 4; lvl++) {
-        cnt = (cnt + 3) / 4;
-        off += cnt;
+// The aligned blocks above the chunks, five levels per launch: a block of threads reduces 1024
+// boxes by shuffles and a last step through LDS.  (One block for all levels, reading each
+// level back, took 20 us for 9 K chunks and 63 us for 27 K; now 5 and 10 us.)
+constexpr int kRangeTop = 1024, kRangeLevels = 5;  // a block makes 5 levels of 1024 boxes
+
+__global__ __launch_bounds__(kRangeTop) void k_range_top(uint32_t cnt, const float4* __restrict__ src,
+                                                      float4* __restrict__ dst) {
+    __shared__ float4 part[2][kRangeTop / 64];
+    const uint32_t tid = threadIdx.x, i = blockIdx.x * kRangeTop + tid;
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    if (i < cnt) {
+        lo = src[2 * (size_t)i];
+        hi = src[2 * (size_t)i + 1];
     }
-    cnt = (cnt + 3) / 4;  // the chunks
-    while (cnt > 1) {
-        const uint32_t up = (cnt + 3) / 4;
-        float4* src = rbox + 2 * off;
-        float4* dst = src + 2 * (size_t)cnt;
-        for (uint32_t e = threadIdx.x; e < up; e += 1024) {
-            float4 lo = src[8 * (size_t)e], hi = src[8 * (size_t)e + 1];
 #pragma unroll
-            for (uint32_t k = 1; k < 4; k++) {  // (past the end: the last one again)
-                const size_t c = min(4 * e + k, cnt - 1);
-                lo = min4(lo, src[2 * c]);
-                hi = max4(hi, src[2 * c + 1]);
-            }
+    for (int lvl = 1; lvl <= 3; lvl++) {
+        if (cnt == 1) return;
+        const int o = 1 << (2 * (lvl - 1));
+        lo = min4(lo, shfl_xor4(lo, o));
+        hi = max4(hi, shfl_xor4(hi, o));
+        lo = min4(lo, shfl_xor4(lo, 2 * o));
+        hi = max4(hi, shfl_xor4(hi, 2 * o));
+        cnt = (cnt + 3) / 4;
+        const uint32_t e = i >> (2 * lvl);
+        if ((tid & (4u * o - 1u)) == 0 && e < cnt) {
             dst[2 * (size_t)e] = lo;
             dst[2 * (size_t)e + 1] = hi;
         }
-        __threadfence_block();
-        __syncthreads();
-        off += cnt;
-        cnt = up;
+        dst += 2 * (size_t)cnt;
+    }
+    if (cnt == 1) return;
+    if ((tid & 63u) == 0) {
+        part[0][tid >> 6] = lo;
+        part[1][tid >> 6] = hi;
+    }
+    __syncthreads();
+    if (tid >= 16) return;
+    lo = part[0][tid];
+    hi = part[1][tid];
+#pragma unroll
+    for (int o = 1; o <= 4; o *= 4) {  // 16 boxes to 4, then to 1
+        lo = min4(lo, shfl_xor4(lo, o));
+        hi = max4(hi, shfl_xor4(hi, o));
+        lo = min4(lo, shfl_xor4(lo, 2 * o));
+        hi = max4(hi, shfl_xor4(hi, 2 * o));
+        if (cnt == 1) return;
+        cnt = (cnt + 3) / 4;
+        const uint32_t e = (blockIdx.x * 16 + tid) / (4 * o);
+        if (tid % (4 * o) == 0 && e < cnt) {
+            dst[2 * (size_t)e] = lo;
+            dst[2 * (size_t)e + 1] = hi;
+        }
+        dst += 2 * (size_t)cnt;
     }
 }
 
@@ -891,7 +914,19 @@ size_t range_boxes(uint32_t N) {
 }
 
 void launch_range_top(uint32_t N, float4* rbox, hipStream_t s) {
-    hipLaunchKernelGGL(k_range_top, dim3(1), dim3(1024), 0, s, N, rbox);
+    uint32_t cnt = N;
+    for (int lvl = 1; lvl <= 4; lvl++) {  // past the local pass's levels, to the chunks
+        if (lvl > 1) rbox += 2 * (size_t)cnt;
+        cnt = (cnt + 3) / 4;
+    }
+    while (cnt > 1) {
+        float4* dst = rbox + 2 * (size_t)cnt;
+        hipLaunchKernelGGL(k_range_top, dim3(cdiv(cnt, kRangeTop)), dim3(kRangeTop), 0, s, cnt, rbox, dst);
+        for (int lvl = 1; lvl <= kRangeLevels && cnt > 1; lvl++) {
+            rbox += 2 * (size_t)cnt;
+            cnt = (cnt + 3) / 4;
+        }
+    }
 }
 
 // A subtree of at most 2 leaf_size triangles that crosses a chunk: its SAH cost, by a walk
@@ -927,8 +962,8 @@ __device__ float small_cost(uint32_t root, const uint2* __restrict__ kids, const
 }
 
 // kCrossLanes lanes per chunk share its list: ~10 of a chunk's 256 nodes are here, each a
-// chain of dependent loads (a thread per node of the tree, 10 of 256 with work: 48 us on 2.3 M triangles,
-// 137 us on a 6.9 M triangle batch; now 29 and ~60).
+// chain of dependent loads (a thread per node of the tree, 10 of 256 with work: 48 us on
+// 2.3 M triangles, 137 us on a 6.9 M triangle batch; now 29 and ~60).
 constexpr uint32_t kCrossLanes = 16;
 
 __global__ __launch_bounds__(kBlock) void k_boxes_cross(uint32_t N, const uint2* __restrict__ range,

@@ -182,3 +182,12 @@ def test_treelet_of_the_whole_mesh_is_optimal(ctx, dev, n, tsize):
         bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev), node_width=2, leaf_size=1, treelet_size=tsize)
         want = _best_sah(V, F)
         assert abs(bvh.info()["sah_cost"] - want) <= 2e-3 * want, (seed, bvh.info()["sah_cost"], want)
+
+
+@pytest.mark.parametrize("n", [65536, 262143, 262144, 262145, 600_001])
+def test_build_at_range_level_edges(ctx, dev, n):
+    """Sizes at which the boxes above the 256-node chunks take another level (256 and 1,024
+    chunks: a second launch) and the upper nodes' boxes come from them."""
+    print("build", n, flush=True)
+    V, F = _soup(n, n, dup=0.0)
+    _check(gpurt.Bvh(ctx, _t(V, dev), _t(F, dev)), V, F)
