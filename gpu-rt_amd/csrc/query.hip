@@ -135,12 +135,19 @@ static int dispatch_stack(int S, QKind kind, const TravArgs& a, unsigned grid, h
 // CU and a refill at 24 idle lanes 218 us (24 waves, 16 lanes: 230 us), any hit at 28
 // waves and 16 lanes 148-151 us (158 us); 32 waves crowd the L2 (+5%).  (The TLAS
 // passes its own launch options.)
+// waves per CU up to which a small set gets a wave per query (plan_traversal)
+constexpr size_t kWidePoints = 12, kWideRays = 8;
+
 static uint32_t default_leaf_trigger(QKind) { return 32u; }
 static uint32_t default_refill_trigger(QKind kind) { return kind == QKind::Closest ? 24u : 16u; }
-static int default_waves_per_cu(QKind kind) { return kind == QKind::Cpq ? 16 : 28; }
-
-// waves per CU up to which a small set gets a wave per query (plan_traversal)
-constexpr size_t kWidePoints = 16, kWideRays = 8;
+// Closest points: 16 waves per CU, but 12 for a set of at most a query per lane of these
+// (kWidePoints), whose time is its longest searches' and not the lanes': 65,536 points near
+// 252,000 triangles 149 -> 137 us, 200,000 mixed on 1.3 M 568 -> 511, 5,000 near 20,000
+// 52 -> 47; 500,000 mixed 771 -> 835, 1 M near 719 -> 811 with 12.
+static int default_waves_per_cu(QKind kind, size_t n, int n_cu) {
+    if (kind != QKind::Cpq) return 28;
+    return n <= (size_t)n_cu * 16 * 64 ? (int)kWidePoints : 16;
+}
 
 static int block_for_stack(int S) { return S <= 16 ? 256 : (S == 32 ? 128 : 64); }
 
@@ -164,19 +171,19 @@ int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need
     int blocks_per_cu = std::min(ctx->lds_per_cu / ((p.S * 8 + lds_extra) * p.BS), std::min(32, 4 * hint) / waves_per_block);
     if (opts && opts->waves_per_cu > 0)
         blocks_per_cu = std::max(1, opts->waves_per_cu / waves_per_block);
-    else if (default_waves_per_cu(kind) > 0)
-        blocks_per_cu = std::min(blocks_per_cu, std::max(1, default_waves_per_cu(kind) / waves_per_block));
+    else
+        blocks_per_cu = std::min(blocks_per_cu,
+                                 std::max(1, default_waves_per_cu(kind, n, ctx->n_cu) / waves_per_block));
     blocks_per_cu = std::max(blocks_per_cu, 1);
     // A small set is spread over more lanes than it has queries (first_query); the idle
     // ones take work from the busy ones once the queues are empty.  A launch of few queries
-    // is one chain of visits, so it gets a wave per query -- until the launch holds kWide
-    // waves per CU, all that run at once for points; for rays fewer, since a wave with
-    // less than 16 rays starts its donation late (65,536 rays on rays_scene 119 us with 8
-    // waves per CU, 137 us with the 28 a launch may hold) -- and 4 lanes per query beyond
-    // that.  Against 4 lanes for every set, us: 100 points on 1,200 triangles 58 -> 46,
-    // 1,000 near 252,000 triangles 91 -> 57, 20,000 on 1.3 M 261 -> 220; 100 rays on 2.3 M
-    // triangles 70 -> 65, 1,000 on 236,000 66 -> 55, 100 on the same scene as instances
-    // 88 -> 73.
+    // is one chain of visits, so it gets a wave per query -- until the launch holds all waves
+    // of such a set of points, or 8 per CU for rays (a wave with less than 16 rays starts its
+    // donation late: 65,536 rays on rays_scene 119 us with 8 waves per CU, 137 us with the
+    // 28 a launch may hold) -- and 4 lanes per query beyond that.  Against 4 lanes for every
+    // set, us: 100 points on 1,200 triangles 58 -> 46, 1,000 near 252,000 triangles 91 -> 57,
+    // 20,000 on 1.3 M 261 -> 220; 100 rays on 2.3 M triangles 70 -> 65, 1,000 on 236,000
+    // 66 -> 55, 100 on the same scene as instances 88 -> 73.
     p.wide = (size_t)ctx->n_cu * (kind == QKind::Cpq ? kWidePoints : kWideRays) * 64;
     p.grid = (unsigned)std::min<size_t>(cdiv(spread_lanes(n, p.wide), p.BS), (size_t)ctx->n_cu * blocks_per_cu);
     if (p.grid == 0) p.grid = 1;
