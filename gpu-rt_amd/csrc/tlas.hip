@@ -448,11 +448,13 @@ struct TlasArgs {
     float origin_bound;  // |origin| coordinates beyond this are outside the exact domain
 };
 
-template <int W, bool Q, int S, int BS, bool ANY, bool STATS>
+// PAIR: with a second list (a kernel of its own: the choice of the list per ray cost the plain
+// one 0.5%)
+template <int W, bool Q, int S, int BS, bool ANY, bool STATS, bool PAIR = false>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kTlasWaves<W>))) void k_tlas_ray(
     TlasArgs a) {
     const uint32_t n1 = a.n_dev ? min(*a.n_dev, a.n) : a.n;
-    const uint32_t n2 = a.n2_dev ? min(*a.n2_dev, a.n2) : 0u;
+    const uint32_t n2 = PAIR ? min(*a.n2_dev, a.n2) : 0u;
     // A launch sized for a list's capacity takes as many of its blocks as the list's true
     // length would be given (they are fewer than the grid only when every query is some
     // lane's first, so the queues' share by grid stays right): the late bounces of a
@@ -467,11 +469,17 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kTlasWaves<W
     const uint32_t gid = blockIdx.x * BS + threadIdx.x;
     LaneStack<S, BS> st;
     st.init(a.spill, a.spill_slots, gid, total);
-    PairSource src{{a.rays, nullptr, n1 + n2, first_query(gid, total), total, a.counter}, a.rays2, n1};
+    using Source = typename std::conditional<PAIR, PairSource, QueueSource>::type;
+    Source src;
+    const QueueSource all{a.rays, nullptr, n1 + n2, first_query(gid, total), total, a.counter};
+    if constexpr (PAIR)
+        src = Source{all, a.rays2, n1};
+    else
+        src = all;
     auto out = [&](uint32_t ri, uint32_t obj, uint32_t id, float t, float u, float v, bool any) {
         if (ANY) {
             a.occ[ri] = any ? 1 : 0;
-        } else if (ri >= n1) {
+        } else if (PAIR && ri >= n1) {
             a.obj2[ri - n1] = id != 0xFFFFFFFFu ? (int32_t)obj : -1;
         } else {
             const bool hit = id != 0xFFFFFFFFu;
@@ -500,6 +508,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kTlasWaves<W
 
 template <int W, bool Q, int S, int BS, bool STATS>
 static void launch_tlas_kind(bool any, const TlasArgs& a, unsigned grid, hipStream_t s) {
+    if constexpr (!STATS) {
+        if (a.n2_dev) {
+            hipLaunchKernelGGL((k_tlas_ray<W, Q, S, BS, false, STATS, true>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kTlasGroupBytes) * BS, s, a);
+            return;
+        }
+    }
     if (any)
         hipLaunchKernelGGL((k_tlas_ray<W, Q, S, BS, true, STATS>), dim3(grid), dim3(BS), (S * sizeof(uint2) + kTlasGroupBytes) * BS, s, a);
     else
@@ -864,6 +878,8 @@ int tlas_trace_ex(gpurt_tlas T, const gpurt_ray* rays, size_t n, const uint32_t*
     hipStream_t s = stream;
     const int W = T->width;
     TravPlan p;
+    if (second && (any || (opts && opts->stats)))
+        return set_error(GPURT_E_UNSUPPORTED, "a second ray list is for plain closest-hit launches");
     const size_t n2 = second && second->n_dev ? second->n : 0;
     int rc = tlas_plan(T, n + n2, any, opts, p);
     if (rc) return rc;
