@@ -16,6 +16,7 @@
 
 #include "backward.h"
 #include "build_common.h"
+#include "index_math.h"
 #include "traverse.h"
 
 namespace gpurt_impl {
@@ -298,8 +299,8 @@ struct MeshVertexSink {
         // Sorted keys: the first active lane's mesh by a search with one value for the wave,
         // then the few meshes up to this lane's.  (A search per lane is a chain of ~8
         // dependent loads each: k_run_sum of the 256-mesh batch 228 -> 158 us.)
-        const uint64_t key0 = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(key >> 32)) << 32 |
-                              __builtin_amdgcn_readfirstlane((uint32_t)key);
+        const uint64_t key0 = u64_of_halves(__builtin_amdgcn_readfirstlane((uint32_t)(key >> 32)),
+                                            __builtin_amdgcn_readfirstlane((uint32_t)key));
         uint32_t lo = 0, hi = n_meshes;  // voff[lo] <= key0 < voff[hi]
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) / 2;
