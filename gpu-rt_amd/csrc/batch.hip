@@ -288,7 +288,8 @@ __global__ __launch_bounds__(256) void k_batch_bwd(const BatchMeshDev* __restric
 }
 
 // adds a batch-wide vertex's total to its mesh's vertex gradient (cleared by
-// k_batch_zero_vgrads; each key has one run).  voff[0..n_meshes] are the meshes' first
+// k_batch_zero_vgrads; each key has one run, and the add is atomic because meshes may share
+// a gradient buffer).  voff[0..n_meshes] are the meshes' first
 // batch-wide vertices (a mesh without a vertex gradient adds none), so the mesh is the
 // last m with voff[m] <= key.
 struct MeshVertexSink {
@@ -310,9 +311,9 @@ struct MeshVertexSink {
         while (voff[lo + 1] <= key) lo++;  // ends: key < voff[n_meshes]
         float* g = grads[lo].g_verts;
         const size_t v = key - voff[lo];
-        g[3 * v] += x;
-        g[3 * v + 1] += y;
-        g[3 * v + 2] += z;
+        unsafeAtomicAdd(&g[3 * v], x);
+        unsafeAtomicAdd(&g[3 * v + 1], y);
+        unsafeAtomicAdd(&g[3 * v + 2], z);
     }
 };
 

@@ -305,3 +305,62 @@ def test_auto_vertex_sums_change_at_600000_terms(dev, n, fixed):
     assert not fixed or np.array_equal(out["auto"], out["fixed"])
     scale = np.abs(out["fixed"]).max()
     np.testing.assert_allclose(out["auto"], out["fixed"], atol=1e-5 * scale, rtol=1e-4)
+
+
+def test_calls_on_two_streams_add_to_one_vertex_gradient(dev):
+    """Backward calls that run at the same time on two streams may accumulate into one g_verts,
+    in every mode: with one fixed-order call each, a vertex's gradient is the rounded sum of
+    the two calls' own gradients, exactly (each call adds once to it)."""
+    ctx = gpurt.Context(0)
+    V, F = _sphere(7, 11)
+    n = 250_000  # fixed order by default
+    Q = [W.surface_samples(V.astype(np.float64), F, np.random.default_rng(20 + k), n, 0.01).astype(np.float32)
+         for k in range(2)]
+    bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev))
+    q = [_t(x, dev) for x in Q]
+    g = torch.ones(n, device=dev)
+    hits = [bvh.closest_point(x) for x in q]
+    streams = [torch.cuda.Stream(dev) for _ in range(2)]
+
+    def add(k, gv):
+        prim, pt, dist, bary = hits[k]
+        bvh.closest_point_bwd(q[k], prim, bary, pt, dist, g, None, gv)
+
+    own = [torch.zeros((V.shape[0], 3), device=dev) for _ in range(2)]
+    for k in range(2):
+        add(k, own[k])
+    want = own[0] + own[1]
+    for _ in range(20):
+        both = torch.zeros((V.shape[0], 3), device=dev)
+        torch.cuda.synchronize()
+        for k, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                add(k, both)
+        torch.cuda.synchronize()
+        assert torch.equal(both, want)
+    bvh.close()
+    ctx.close()
+
+
+def test_fixed_order_sums_keep_subnormal_gradients(dev):
+    """A vertex gradient below the smallest normal FP32 number arrives whole: within the
+    spacing of the subnormals times the roundings of a term (weight, product, two adds)."""
+    ctx = gpurt.Context(0, vertex_sums="fixed")
+    V, F = _sphere(3, 5)
+    Q = W.surface_samples(V.astype(np.float64), F, np.random.default_rng(6), 64, 0.05).astype(np.float32)
+    bvh = gpurt.Bvh(ctx, _t(V, dev), _t(F, dev))
+    tq = _t(Q, dev)
+    prim, pt, dist, bary = bvh.closest_point(tq)
+    gn = np.float32(2.0**-132)
+    gv = torch.zeros((V.shape[0], 3), device=dev)
+    bvh.closest_point_bwd(tq, prim, bary, pt, dist, torch.full((64,), float(gn), device=dev), None, gv)
+    p, b = prim.cpu().numpy(), bary.cpu().numpy().astype(np.float64)
+    ev, count = np.zeros(V.shape), np.zeros(len(V))
+    gq, _ = O.cpq_grad_f64(V.astype(np.float64), F, Q.astype(np.float64), p)
+    for j in range(3):
+        np.add.at(ev, F[p, j], -(b[:, j] * float(gn))[:, None] * gq)
+        np.add.at(count, F[p, j], 1)
+    assert np.abs(ev).max() > 2.0**-136
+    assert (np.abs(gv.cpu().numpy() - ev) <= (4 * count * 2.0**-149 + 1e-6 * np.abs(ev).max())[:, None]).all()
+    bvh.close()
+    ctx.close()
