@@ -15,4 +15,11 @@ __host__ __device__ constexpr uint64_t u64_of_halves(int hi, int lo) {
     return (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
 }
 
+// f(i) for i = first, first + step, ... below n.  The index is 64 bits wide: n may be any
+// 32-bit count, and a 32-bit index within a step of 2^32 would wrap and never reach it.
+template <typename F>
+__host__ __device__ inline void grid_stride(uint32_t n, uint64_t first, uint64_t step, F f) {
+    for (uint64_t i = first; i < n; i += step) f((uint32_t)i);
+}
+
 }  // namespace gpurt_impl

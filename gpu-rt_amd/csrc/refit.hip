@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "build_common.h"
+#include "index_math.h"
 
 namespace gpurt_impl {
 
@@ -33,12 +34,12 @@ __global__ __launch_bounds__(kBlock) void k_refit_check(uint32_t n_verts, const 
     __shared__ float part[kBlock / 64];
     bool bad = false;
     float amax = 0.0f;
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n_verts; i += gridDim.x * kBlock) {
+    grid_stride(n_verts, blockIdx.x * kBlock + threadIdx.x, gridDim.x * kBlock, [&](uint32_t i) {
         const float* p = v + (size_t)i * stride;
         const float x = p[0], y = p[1], z = p[2];
         bad = bad || !(isfinite(x) && isfinite(y) && isfinite(z));
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)));
-    }
+    });
     if (__any(bad) && (threadIdx.x & 63) == 0) gatomic_or(tmp + 1, 1u);
     for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;

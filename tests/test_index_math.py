@@ -25,3 +25,20 @@ def test_64_bit_keys_from_halves(tmp_path):
                "for (unsigned hi : v) for (unsigned lo : v)\n"
                "    printf(\"%llu\\n\", (unsigned long long)u64_of_halves((int)hi, (int)lo));")
     assert [int(x) for x in out] == [hi << 32 | lo for hi in halves for lo in halves]
+
+
+def test_grid_stride_ends_at_every_32_bit_count(tmp_path):
+    """Counts up to 2^32 - 1 with the step of the refit's vertex check (512 blocks of 256): each
+    thread sees its indices once and stops."""
+    step = 512 * 256
+    cases = [(n, first) for n in (1, step, step + 1, 2**32 - step - 1, 2**32 - step, 2**32 - step + 1, 2**32 - 1)
+             for first in (0, 1, step - 1)]
+    out = _run(tmp_path, "const unsigned c[][2] = {" + ", ".join("{%du, %du}" % c for c in cases) + "};\n"
+               "for (auto& k : c) {\n"
+               "    unsigned long long seen = 0, last = 0;\n"
+               "    grid_stride(k[0], k[1], %d, [&](unsigned i) { seen++; last = i; if (seen > 40000) throw 1; });\n"
+               "    printf(\"%%llu %%llu\\n\", seen, last);\n}" % step)
+    got = list(zip(map(int, out[::2]), map(int, out[1::2])))
+    for (n, first), g in zip(cases, got):
+        r = range(first, n, step)
+        assert g == (len(r), r[-1] if len(r) else 0)
