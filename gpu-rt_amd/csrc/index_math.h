@@ -22,4 +22,21 @@ __host__ __device__ inline void grid_stride(uint32_t n, uint64_t first, uint64_t
     for (uint64_t i = first; i < n; i += step) f((uint32_t)i);
 }
 
+// The last m from lo on with off[m] <= key, for off[lo] <= key < off[n] and off[0..n] in
+// ascending order (equal entries are empty): steps that double, then halve, so the cost is
+// the logarithm of the distance.
+template <typename Offsets>
+__host__ __device__ inline uint32_t last_from(const Offsets& off, uint32_t n, uint32_t lo, uint64_t key) {
+    uint32_t step = 1;
+    while (step < n - lo && off[lo + step] <= key) {
+        lo += step;
+        step *= 2;
+    }
+    while (step > 1) {
+        step /= 2;
+        if (step < n - lo && off[lo + step] <= key) lo += step;
+    }
+    return lo;
+}
+
 }  // namespace gpurt_impl

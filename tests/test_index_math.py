@@ -42,3 +42,37 @@ def test_grid_stride_ends_at_every_32_bit_count(tmp_path):
     for (n, first), g in zip(cases, got):
         r = range(first, n, step)
         assert g == (len(r), r[-1] if len(r) else 0)
+
+
+def test_mesh_of_a_key_in_few_steps(tmp_path):
+    """The mesh that holds a batch-wide vertex, from any earlier mesh, with empty meshes
+    between; and over 100,000 meshes in a logarithmic number of reads."""
+    n_off = [[0, 5], [0, 0, 0, 3], [0, 2, 2, 2, 7, 7], [0, 1, 2, 3, 4, 5, 6, 7, 8, 9], [0, 4, 4, 4, 4, 4, 4, 4, 4, 6, 6, 9]]
+    body = "std::vector<std::vector<uint64_t>> offs = {" + ", ".join(
+        "{" + ", ".join(map(str, o)) + "}" for o in n_off) + "};\n"
+    body += """for (auto& o : offs) {
+        const uint32_t n = (uint32_t)o.size() - 1;
+        for (uint64_t key = 0; key < o[n]; key++)
+            for (uint32_t lo = 0; lo < n && o[lo] <= key; lo++) printf("%u\\n", last_from(o.data(), n, lo, key));
+    }
+    std::vector<uint64_t> big(100001, 1ull << 40);
+    big[0] = 0;
+    big[100000] = (1ull << 40) + 8;
+    int reads = 0;
+    struct Counted {
+        const uint64_t* p;
+        int* reads;
+        uint64_t operator[](uint32_t i) const { return ++*reads, p[i]; }
+    };
+    printf("%u\\n", last_from(Counted{big.data(), &reads}, 100000, 0, (1ull << 40) + 3));
+    printf("%d\\n", reads);
+"""
+    out = [int(x) for x in _run(tmp_path, body)]
+    want = []
+    for o in n_off:
+        n = len(o) - 1
+        for key in range(o[n]):
+            m = max(k for k in range(n) if o[k] <= key)
+            want += [m for lo in range(n) if o[lo] <= key]
+    assert out[:-1] == want + [99999]
+    assert out[-1] <= 2 * 17 + 1
