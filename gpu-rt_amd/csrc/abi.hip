@@ -111,8 +111,17 @@ static void free_bvh_buffers(gpurt_bvh_s* b, hipStream_t s) {
     b->verts = nullptr;
 }
 
-// frees idle pool blocks, the longest idle first, until at most `keep` idle bytes are left
-// (the caller holds pool_mu)
+// returns to the device what has been freed on the release stream (HIP's own pool keeps it
+// otherwise); waits for that stream
+static void give_back_freed(gpurt_ctx_s* c) {
+    hipMemPool_t pool;
+    if (hipStreamSynchronize(c->release) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, c->device) == hipSuccess)
+        (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+}
+
+// frees idle pool blocks, the longest idle first, until at most `keep` idle bytes are left, in
+// order on the release stream and without a host wait (the caller holds pool_mu)
 static void pool_trim(gpurt_ctx_s* c, size_t keep) {
     while (c->pool_idle > keep) {
         size_t k = c->pool.size();
@@ -120,8 +129,8 @@ static void pool_trim(gpurt_ctx_s* c, size_t keep) {
             if (!c->pool[i].used && (k == c->pool.size() || c->pool[i].when < c->pool[k].when)) k = i;
         if (k == c->pool.size()) return;
         gpurt_ctx_s::PoolBlock& e = c->pool[k];
-        (void)hipEventSynchronize(e.freed);
-        (void)hipFree(e.mem);
+        if (hipStreamWaitEvent(c->release, e.freed, 0) != hipSuccess) (void)hipDeviceSynchronize();
+        (void)hipFreeAsync(e.mem, c->release);
         (void)hipEventDestroy(e.freed);
         (void)hipGetLastError();
         c->pool_idle -= e.bytes;
@@ -153,18 +162,21 @@ int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     gpurt_ctx_s::PoolBlock e;
     e.bytes = bytes;
     e.used = true;
-    if (hipMalloc(&e.mem, bytes) != hipSuccess) {
+    // stream-ordered, so that pool_trim can free it without a host wait (hipFree waits for
+    // every stream of the device)
+    if (hipMallocAsync(&e.mem, bytes, s) != hipSuccess) {
         (void)hipGetLastError();
         e.mem = nullptr;
         pool_trim(c, 0);
-        if (hipMalloc(&e.mem, bytes) != hipSuccess) {
+        give_back_freed(c);
+        if (hipMallocAsync(&e.mem, bytes, s) != hipSuccess) {
             (void)hipGetLastError();
             return set_error(GPURT_E_OOM, "allocation of " + std::to_string(bytes) + " bytes failed");
         }
     }
     if (hipEventCreateWithFlags(&e.freed, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
-        (void)hipFree(e.mem);
+        (void)hipFreeAsync(e.mem, s);
         return set_error(GPURT_E_DEVICE, "event creation failed");
     }
     c->pool.push_back(e);
@@ -193,11 +205,12 @@ void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s) {
 void pool_release(gpurt_ctx_s* c) {
     std::lock_guard<std::mutex> lk(c->pool_mu);
     for (auto& e : c->pool) {
-        (void)hipFree(e.mem);
+        (void)hipFreeAsync(e.mem, c->release);
         (void)hipEventDestroy(e.freed);
     }
     c->pool.clear();
     c->pool_idle = 0;
+    give_back_freed(c);
 }
 
 int compact_verts(const float* verts, size_t stride_floats, size_t n, float* out, hipStream_t s) {
@@ -239,9 +252,8 @@ int ctx_scratch(gpurt_ctx_s* c, hipStream_t s, size_t bytes, CallScratch& out) {
             if (e.mem && hipStreamWaitEvent(s, e.last, 0) != hipSuccess)
                 return hip_error(hipGetLastError(), "hipStreamWaitEvent");
             if (e.bytes < bytes) {
-                // Outside the stream-ordered pool, so the builds' own stream-ordered
-                // allocations keep reusing the pool's memory.  Growing waits for the
-                // device (hipFree), once per new largest call on the stream.
+                // Growing waits for the device (hipFree), once per new largest call on
+                // the stream.
                 if (e.mem) (void)hipFree(e.mem);
                 e.mem = nullptr;
                 e.bytes = 0;
@@ -365,8 +377,8 @@ int gpurt_ctx_create(int device, gpurt_ctx* out) {
     }
     size_t mem_free = 0, mem_total = 0;
     if (hipMemGetInfo(&mem_free, &mem_total) == hipSuccess) c->pool_limit = std::max(c->pool_limit, mem_total / 16);
-    // keep freed stream-ordered allocations (scratch of captured or concurrent calls) in
-    // HIP's pool
+    // keep freed stream-ordered allocations (scratch of captured or concurrent calls, blocks
+    // that leave the context's pool) in HIP's pool
     hipMemPool_t pool;
     if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) {
         uint64_t thr = ~0ull;

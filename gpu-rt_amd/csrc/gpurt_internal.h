@@ -266,10 +266,10 @@ void wait_uses(gpurt_bvh_s* b, hipStream_t s);
 // Device memory of builds and BVHs, kept by the context: a block given back on a stream is
 // handed out again after a wait (on the device) for that point of the stream, so any
 // stream and thread may take it.  Idle blocks are bounded (1/16 of the device's memory; the
-// longest idle go first) and all are freed with the context.  hipMallocAsync and
-// hipFreeAsync, used before, cost a small build about 100 us for its ten buffers, and after
-// a hundred builds of 2.3 M triangles each hipFreeAsync took 10 ms (a build 27 ms instead
-// of 8).
+// longest idle go first) and all are freed with the context.  The blocks themselves are
+// stream-ordered allocations.  Taking each buffer of a build as one (hipMallocAsync and
+// hipFreeAsync) cost a small build about 100 us for its ten buffers, and after a hundred
+// builds of 2.3 M triangles each hipFreeAsync took 10 ms (a build 27 ms instead of 8).
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s);
 void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s);
 void pool_release(gpurt_ctx_s* c);  // after the device is idle (context destroy)

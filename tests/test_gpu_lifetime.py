@@ -5,6 +5,7 @@ destroy, and a process that exits with objects still open exits cleanly."""
 import os
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -85,3 +86,78 @@ print("ok", flush=True)
                        capture_output=True, text=True, timeout=240)
     print(r.stdout, r.stderr[-2000:])
     assert r.returncode == 0 and "ok" in r.stdout
+
+
+def _sleep(stream, seconds):
+    """A spinning kernel of about that time on the stream."""
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    cycles = 1_000_000
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(cycles)
+        a.record(stream)
+        torch.cuda._sleep(cycles)
+        b.record(stream)
+        b.synchronize()
+        torch.cuda._sleep(int(cycles * seconds * 1e3 / a.elapsed_time(b)))
+
+
+def _soup(n, dev):
+    g = torch.Generator(device=dev).manual_seed(1)
+    c = torch.rand(n, 1, 3, generator=g, device=dev)
+    v = (c + 0.01 * torch.rand(n, 3, 3, generator=g, device=dev)).reshape(-1, 3).contiguous()
+    return v, torch.arange(3 * n, device=dev, dtype=torch.int32).reshape(-1, 3)
+
+
+@pytest.fixture
+def many_bvhs(dev):
+    """A context and BVHs whose memory together is more than the context keeps idle (a
+    sixteenth of the device's)."""
+    V, F = _soup(2_000_000, dev)
+    ctx = gpurt.Context(0)
+    free0, total = torch.cuda.mem_get_info(dev)
+    bvhs = []
+    while len(bvhs) < 400 and free0 - torch.cuda.mem_get_info(dev)[0] < total / 16 + (4 << 30):
+        bvhs += [gpurt.Bvh(ctx, V, F) for _ in range(8)]
+    yield V[:4096].contiguous(), bvhs
+    ctx.close()
+    torch.cuda.synchronize()
+    # given back with the context
+    assert torch.cuda.mem_get_info(dev)[0] > free0 - (1 << 30)
+
+
+def test_destroy_beyond_the_idle_limit_does_not_wait(dev, many_bvhs):
+    """Destroying them while a query on the first is still to run waits for nothing, and the
+    query's answer is whole."""
+    Q, bvhs = many_bvhs
+    busy, done = torch.cuda.Stream(dev), torch.cuda.Event()
+    want = bvhs[0].closest_point(Q)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        bvhs[0].closest_point(Q)
+        _sleep(busy, 0.5)
+        got = bvhs[0].closest_point(Q)
+        done.record(busy)
+    for b in bvhs:
+        b.close()
+    assert not done.query(), "a destroy waited for the query"
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_destroy_beyond_the_idle_limit_while_another_thread_captures(dev, many_bvhs):
+    """Destroying them while a stream is captured in HIP's global mode leaves the capture whole."""
+    _, bvhs = many_bvhs
+    x = torch.arange(1024, dtype=torch.float32, device=dev)
+    y = torch.zeros_like(x)
+    t = threading.Thread(target=lambda: [b.close() for b in bvhs])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, capture_error_mode="global"):
+        torch.add(x, 1.0, out=y)
+        t.start()
+        t.join(60)
+        torch.mul(y, 2.0, out=y)
+    for _ in range(2):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, (x + 1.0) * 2.0)
