@@ -44,6 +44,14 @@ __global__ void k_compact_verts(uint32_t n, const float* __restrict__ v, uint64_
     out[3 * (size_t)i + 2] = p[2];
 }
 
+EventRef make_event() {
+    auto r = std::make_shared<Event>();
+    if (hipEventCreateWithFlags(&r->e, hipEventDisableTiming) == hipSuccess) return r;
+    (void)hipGetLastError();
+    r->e = nullptr;
+    return nullptr;
+}
+
 void note_use(gpurt_bvh_s* b, hipStream_t s) {
     std::lock_guard<std::mutex> lk(b->use_mu);
     // work recorded into a graph runs when the graph is launched: no event can mark it
@@ -55,20 +63,19 @@ void note_use(gpurt_bvh_s* b, hipStream_t s) {
     }
     for (auto& u : b->uses)
         if (u.first == s) {
-            if (hipEventRecord(u.second, s) != hipSuccess) {
+            if (hipEventRecord(u.second->e, s) != hipSuccess) {
                 (void)hipGetLastError();
                 b->uses_lost = true;
             }
             return;
         }
-    hipEvent_t e = nullptr;
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess || hipEventRecord(e, s) != hipSuccess) {
+    EventRef e = make_event();
+    if (!e || hipEventRecord(e->e, s) != hipSuccess) {
         (void)hipGetLastError();
-        if (e) (void)hipEventDestroy(e);
         b->uses_lost = true;
         return;
     }
-    b->uses.emplace_back(s, e);
+    b->uses.emplace_back(s, std::move(e));
 }
 
 // note_use without creating an event (the no-allocation entry point): a stream not seen
@@ -83,7 +90,7 @@ static void note_use_existing(gpurt_bvh_s* b, hipStream_t s) {
     }
     for (auto& u : b->uses)
         if (u.first == s) {
-            if (hipEventRecord(u.second, s) != hipSuccess) {
+            if (hipEventRecord(u.second->e, s) != hipSuccess) {
                 (void)hipGetLastError();
                 b->uses_lost = true;
             }
@@ -95,47 +102,72 @@ static void note_use_existing(gpurt_bvh_s* b, hipStream_t s) {
 void wait_uses(gpurt_bvh_s* b, hipStream_t s) {
     std::lock_guard<std::mutex> lk(b->use_mu);
     for (auto& u : b->uses)
-        if (hipStreamWaitEvent(s, u.second, 0) != hipSuccess) {
+        if (hipStreamWaitEvent(s, u.second->e, 0) != hipSuccess) {
             (void)hipGetLastError();
             b->uses_lost = true;
         }
 }
 
-// gives a BVH's memory back in order on stream s
-static void free_bvh_buffers(gpurt_bvh_s* b, hipStream_t s) {
+Uses uses_of(gpurt_bvh_s* b) {
+    std::lock_guard<std::mutex> lk(b->use_mu);
+    // uses that no event marks (graph capture, a failed record)
+    if (b->uses_lost) (void)hipDeviceSynchronize();
+    return b->uses_lost ? Uses{} : b->uses;
+}
+
+// gives a BVH's memory back after a point of a stream, or after some uses
+template <typename After>
+static void free_bvh_buffers(gpurt_bvh_s* b, const After& after) {
     for (void* p : {b->mesh_mem, b->node_mem})
-        if (p) pool_free(b->ctx, p, s);
+        if (p) pool_free(b->ctx, p, after);
     b->mesh_mem = b->node_mem = b->nodes = b->qnodes = b->onodes = nullptr;
     b->tris = nullptr;
     b->tri_idx = b->leaf_order = b->refit_tmp = b->node_first = nullptr;
     b->verts = nullptr;
 }
 
-// returns to the device what has been freed on the release stream (HIP's own pool keeps it
-// otherwise); waits for that stream
-static void give_back_freed(gpurt_ctx_s* c) {
-    hipMemPool_t pool;
-    if (hipStreamSynchronize(c->release) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, c->device) == hipSuccess)
-        (void)hipMemPoolTrimTo(pool, 0);
-    (void)hipGetLastError();
+// HIP refuses event queries, host waits and the like (and breaks the capture) while any thread
+// captures a stream in global mode, unless the calling thread says that it knows.
+struct AnyCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// drops the points that are reached from what an idle block waits for (those on stream s may
+// stay); true when no others are left
+static bool ended(gpurt_ctx_s::PoolBlock& e, const hipStream_t* s = nullptr) {
+    for (size_t i = e.after.size(); i-- > 0;) {
+        if (s && e.after[i].first == *s) continue;
+        if (hipEventQuery(e.after[i].second->e) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        e.after.erase(e.after.begin() + (ptrdiff_t)i);
+    }
+    return true;
 }
 
-// frees idle pool blocks, the longest idle first, until at most `keep` idle bytes are left, in
-// order on the release stream and without a host wait (the caller holds pool_mu)
+// Frees idle pool blocks, the longest idle first, until at most `keep` idle bytes are left (the
+// caller holds pool_mu).  A block whose work has not ended stays for a later call: this one
+// does not wait, and memory given to HIP's pool while work on it was still to run has been
+// handed out again before that work.
 static void pool_trim(gpurt_ctx_s* c, size_t keep) {
-    while (c->pool_idle > keep) {
-        size_t k = c->pool.size();
-        for (size_t i = 0; i < c->pool.size(); i++)
-            if (!c->pool[i].used && (k == c->pool.size() || c->pool[i].when < c->pool[k].when)) k = i;
-        if (k == c->pool.size()) return;
-        gpurt_ctx_s::PoolBlock& e = c->pool[k];
-        if (hipStreamWaitEvent(c->release, e.freed, 0) != hipSuccess) (void)hipDeviceSynchronize();
-        (void)hipFreeAsync(e.mem, c->release);
-        (void)hipEventDestroy(e.freed);
+    if (c->pool_idle <= keep) return;
+    AnyCapture mode;
+    std::vector<gpurt_ctx_s::PoolBlock*> idle;
+    for (auto& e : c->pool)
+        if (!e.used) idle.push_back(&e);
+    std::sort(idle.begin(), idle.end(), [](auto* a, auto* b) { return a->when < b->when; });
+    for (auto* e : idle) {
+        if (c->pool_idle <= keep) break;
+        if (!ended(*e)) continue;
+        (void)hipFreeAsync(e->mem, c->release);
         (void)hipGetLastError();
-        c->pool_idle -= e.bytes;
-        c->pool.erase(c->pool.begin() + (ptrdiff_t)k);
+        c->pool_idle -= e->bytes;
+        e->mem = nullptr;
     }
+    c->pool.erase(std::remove_if(c->pool.begin(), c->pool.end(), [](auto& e) { return !e.mem; }), c->pool.end());
 }
 
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
@@ -146,37 +178,58 @@ int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     while (step * 16 <= bytes) step *= 2;
     bytes = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    // the smallest idle block that fits without wasting half of it; of equals the one
-    // given back first
-    gpurt_ctx_s::PoolBlock* best = nullptr;
+    using Block = gpurt_ctx_s::PoolBlock;
+    auto take = [&](Block& e) {
+        for (auto& u : e.after)
+            if (hipStreamWaitEvent(s, u.second->e, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        e.used = true;
+        e.after.clear();
+        c->pool_idle -= e.bytes;
+        *p = e.mem;
+        return true;
+    };
+    auto better = [](const Block& e, const Block* best) {
+        return !best || e.bytes < best->bytes || (e.bytes == best->bytes && e.when < best->when);
+    };
+    // The smallest idle block that fits without wasting half of it, of equals the one given
+    // back first, among those that need no wait.  (Waiting for another stream's work would hold
+    // this stream, and the host with it, until some long query there has ended.)
+    AnyCapture mode;
+    Block* best = nullptr;
     for (auto& e : c->pool)
-        if (!e.used && e.bytes >= bytes && e.bytes <= 2 * bytes &&
-            (!best || e.bytes < best->bytes || (e.bytes == best->bytes && e.when < best->when)))
-            best = &e;
-    if (best && hipStreamWaitEvent(s, best->freed, 0) == hipSuccess) {
-        best->used = true;
-        c->pool_idle -= best->bytes;
-        *p = best->mem;
-        return GPURT_OK;
-    }
+        if (!e.used && e.bytes >= bytes && e.bytes <= 2 * bytes && better(e, best) && ended(e, &s)) best = &e;
+    if (best && take(*best)) return GPURT_OK;
     gpurt_ctx_s::PoolBlock e;
     e.bytes = bytes;
     e.used = true;
-    // stream-ordered, so that pool_trim can free it without a host wait (hipFree waits for
-    // every stream of the device)
-    if (hipMallocAsync(&e.mem, bytes, s) != hipSuccess) {
+    // from a pool of HIP's, so that pool_trim can free it without a host wait (hipFree waits
+    // for every stream of the device)
+    if (hipMallocFromPoolAsync(&e.mem, bytes, c->mem, s) != hipSuccess) {
         (void)hipGetLastError();
         e.mem = nullptr;
+        // memory is short: any block that fits will do, then all idle ones are freed, after
+        // their work, and HIP's pool gives them back
+        best = nullptr;
+        for (auto& x : c->pool)
+            if (!x.used && x.bytes >= bytes && better(x, best)) best = &x;
+        if (best && take(*best)) return GPURT_OK;
+        for (auto& x : c->pool)
+            for (auto& u : x.after) (void)hipEventSynchronize(u.second->e);
         pool_trim(c, 0);
-        give_back_freed(c);
-        if (hipMallocAsync(&e.mem, bytes, s) != hipSuccess) {
+        (void)hipStreamSynchronize(c->release);
+        (void)hipMemPoolTrimTo(c->mem, 0);
+        (void)hipGetLastError();
+        if (hipMallocFromPoolAsync(&e.mem, bytes, c->mem, s) != hipSuccess) {
             (void)hipGetLastError();
             return set_error(GPURT_E_OOM, "allocation of " + std::to_string(bytes) + " bytes failed");
         }
     }
-    if (hipEventCreateWithFlags(&e.freed, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipFreeAsync(e.mem, s);
+    e.own = make_event();
+    if (!e.own) {
+        (void)hipFreeAsync(e.mem, s);  // (nothing uses it)
         return set_error(GPURT_E_DEVICE, "event creation failed");
     }
     c->pool.push_back(e);
@@ -184,16 +237,14 @@ int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     return GPURT_OK;
 }
 
-void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s) {
+// after: what the block's memory still waits for, given the block (the caller holds nothing)
+template <typename After>
+static void give_back(gpurt_ctx_s* c, void* p, After after) {
     if (!p) return;
     std::lock_guard<std::mutex> lk(c->pool_mu);
     for (auto& e : c->pool)
         if (e.mem == p) {
-            if (hipEventRecord(e.freed, s) != hipSuccess) {
-                // the stream cannot say when its work is done: wait for the device
-                (void)hipGetLastError();
-                (void)hipDeviceSynchronize();
-            }
+            e.after = after(e);
             e.used = false;
             e.when = ++c->pool_clock;
             c->pool_idle += e.bytes;
@@ -202,15 +253,28 @@ void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s) {
     pool_trim(c, c->pool_limit);
 }
 
+void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s) {
+    give_back(c, p, [s](gpurt_ctx_s::PoolBlock& e) {
+        if (hipEventRecord(e.own->e, s) == hipSuccess) return Uses{{s, e.own}};
+        // the stream cannot say when its work is done: wait for the device
+        (void)hipGetLastError();
+        (void)hipDeviceSynchronize();
+        return Uses{};
+    });
+}
+
+void pool_free(gpurt_ctx_s* c, void* p, const Uses& after) {
+    give_back(c, p, [&](gpurt_ctx_s::PoolBlock&) { return after; });
+}
+
 void pool_release(gpurt_ctx_s* c) {
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    for (auto& e : c->pool) {
-        (void)hipFreeAsync(e.mem, c->release);
-        (void)hipEventDestroy(e.freed);
-    }
+    for (auto& e : c->pool) (void)hipFreeAsync(e.mem, c->release);
     c->pool.clear();
     c->pool_idle = 0;
-    give_back_freed(c);
+    (void)hipStreamSynchronize(c->release);
+    if (c->mem) (void)hipMemPoolDestroy(c->mem);
+    c->mem = nullptr;
 }
 
 int compact_verts(const float* verts, size_t stride_floats, size_t n, float* out, hipStream_t s) {
@@ -357,9 +421,14 @@ int gpurt_ctx_create(int device, gpurt_ctx* out) {
         delete c;
         return set_error(GPURT_E_OOM, "context allocation failed");
     }
-    if (hipMemset(c->err, 0, 256) != hipSuccess ||
+    hipMemPoolProps props{};
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = device;
+    if (hipMemset(c->err, 0, 256) != hipSuccess || hipMemPoolCreate(&c->mem, &props) != hipSuccess ||
         hipStreamCreateWithFlags(&c->release, hipStreamNonBlocking) != hipSuccess) {
         (void)hipGetLastError();
+        if (c->mem) (void)hipMemPoolDestroy(c->mem);
         (void)hipFree(c->err);
         delete c;
         return set_error(GPURT_E_DEVICE, "context init failed");
@@ -369,6 +438,7 @@ int gpurt_ctx_create(int device, gpurt_ctx* out) {
     {
         const int rc = noalloc_scratch_init(device);
         if (rc) {
+            (void)hipMemPoolDestroy(c->mem);
             (void)hipStreamDestroy(c->release);
             (void)hipFree(c->err);
             delete c;
@@ -377,8 +447,8 @@ int gpurt_ctx_create(int device, gpurt_ctx* out) {
     }
     size_t mem_free = 0, mem_total = 0;
     if (hipMemGetInfo(&mem_free, &mem_total) == hipSuccess) c->pool_limit = std::max(c->pool_limit, mem_total / 16);
-    // keep freed stream-ordered allocations (scratch of captured or concurrent calls, blocks
-    // that leave the context's pool) in HIP's pool
+    // keep freed stream-ordered allocations (scratch of captured or concurrent calls) in
+    // HIP's pool
     hipMemPool_t pool;
     if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) {
         uint64_t thr = ~0ull;
@@ -399,8 +469,7 @@ void gpurt_ctx_destroy(gpurt_ctx ctx) {
         for (gpurt_tlas_s* t : ctx->tlases) tlas_orphan(t);
         ctx->tlases.clear();
         for (gpurt_bvh_s* b : ctx->bvhs) {
-            free_bvh_buffers(b, ctx->release);
-            for (auto& u : b->uses) (void)hipEventDestroy(u.second);
+            free_bvh_buffers(b, Uses{});
             b->uses.clear();
             b->ctx = nullptr;
         }
@@ -530,12 +599,7 @@ void gpurt_bvh_destroy(gpurt_bvh b) {
         b->ctx->bvhs.erase(b);
     }
     DeviceGuard g(b->ctx->device);
-    hipStream_t rs = b->ctx->release;
-    // uses that no event marks (graph capture, a failed record): wait for the device
-    if (b->uses_lost) (void)hipDeviceSynchronize();
-    wait_uses(b, rs);
-    free_bvh_buffers(b, rs);
-    for (auto& u : b->uses) (void)hipEventDestroy(u.second);
+    free_bvh_buffers(b, uses_of(b));
     (void)hipGetLastError();
     delete b;
 }

@@ -21,6 +21,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <string>
@@ -164,6 +165,22 @@ struct DeviceBvh {
     uint32_t n_tris;
 };
 
+// An event, destroyed with its last holder: points of streams that a BVH's memory waits for
+// outlive the BVH.
+struct Event {
+    hipEvent_t e = nullptr;
+    Event() = default;
+    Event(const Event&) = delete;
+    Event& operator=(const Event&) = delete;
+    ~Event() {
+        if (e) (void)hipEventDestroy(e);
+    }
+};
+using EventRef = std::shared_ptr<Event>;
+EventRef make_event();  // without timing; null when HIP cannot create one
+// points of streams, each the last use of something there
+using Uses = std::vector<std::pair<hipStream_t, EventRef>>;
+
 }  // namespace gpurt_impl
 
 struct gpurt_ctx_s {
@@ -173,9 +190,11 @@ struct gpurt_ctx_s {
     uint32_t* err = nullptr;  // sticky device error bits (bit 0: traversal stack overflow)
     // GPURT_SUMS_* mode of the backward passes' vertex-gradient sums
     int vertex_sums = 0;
-    // stream on which destroyed handles release their memory, after waiting for the
-    // recorded uses of the handle (stream-ordered, no host wait)
+    // stream on which memory that leaves the pool is freed, and which stands for the uses of a
+    // destroyed TLAS (stream-ordered, no host wait)
     hipStream_t release = nullptr;
+    hipMemPool_t mem = nullptr;  // HIP's pool under the context's (its freed memory goes back at
+                                 // the next synchronisation)
     // BVHs and TLASes still open on the context: gpurt_ctx_destroy releases their device
     // memory, and destroying such a handle afterwards frees only its host part
     std::mutex live_mu;
@@ -196,8 +215,9 @@ struct gpurt_ctx_s {
         void* mem = nullptr;
         size_t bytes = 0;
         bool used = false;
-        hipEvent_t freed = nullptr;  // recorded where the block was given back
-        uint64_t when = 0;           // order of giving back
+        gpurt_impl::EventRef own;  // recorded where a stream gives the block back
+        gpurt_impl::Uses after;    // the work an idle block waits for
+        uint64_t when = 0;         // order of giving back
     };
     std::mutex pool_mu;
     std::vector<PoolBlock> pool;
@@ -244,10 +264,10 @@ struct gpurt_bvh_s {
     float* verts = nullptr;       // 3 * n_verts compact positions, original order
     uint32_t* leaf_order = nullptr;  // packed position -> original triangle (refit)
     uint32_t* refit_tmp = nullptr;   // two words of a refit
-    // gpurt_bvh_destroy gives the blocks back on ctx->release after waiting for the last
-    // use recorded on each stream that used the handle.
+    // gpurt_bvh_destroy gives the blocks back after the last use recorded on each stream that
+    // used the handle.
     std::mutex use_mu;
-    std::vector<std::pair<hipStream_t, hipEvent_t>> uses;
+    gpurt_impl::Uses uses;
     bool uses_lost = false;  // an event could not be recorded: destroy waits for the device
 };
 
@@ -262,16 +282,19 @@ int hip_error(hipError_t e, const char* what);
 // makes stream `s` wait for every recorded use
 void note_use(gpurt_bvh_s* b, hipStream_t s);
 void wait_uses(gpurt_bvh_s* b, hipStream_t s);
+// the recorded uses; waits for the device first when there may be others
+Uses uses_of(gpurt_bvh_s* b);
 
-// Device memory of builds and BVHs, kept by the context: a block given back on a stream is
-// handed out again after a wait (on the device) for that point of the stream, so any
-// stream and thread may take it.  Idle blocks are bounded (1/16 of the device's memory; the
-// longest idle go first) and all are freed with the context.  The blocks themselves are
-// stream-ordered allocations.  Taking each buffer of a build as one (hipMallocAsync and
+// Device memory of builds and BVHs, kept by the context: a block given back after some points
+// of streams is handed out again once they are reached (or, in order, to the one stream that
+// they are on), so any stream and thread may take it and none waits for another's work.  Idle blocks are bounded (1/16 of the device's memory; the
+// longest idle go first) and all are freed with the context.  Taking each buffer of a build as one (hipMallocAsync and
 // hipFreeAsync) cost a small build about 100 us for its ten buffers, and after a hundred
-// builds of 2.3 M triangles each hipFreeAsync took 10 ms (a build 27 ms instead of 8).
+// builds of 2.3 M triangles each hipFreeAsync took 10 ms (a build 27 ms instead of 8); and
+// memory freed there in order behind a query was handed out before that query had run.
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s);
-void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s);
+void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s);        // after what s holds now
+void pool_free(gpurt_ctx_s* c, void* p, const Uses& after);
 void pool_release(gpurt_ctx_s* c);  // after the device is idle (context destroy)
 
 // Lays buffers out in one allocation, 256-byte aligned: a first pass without a base gives

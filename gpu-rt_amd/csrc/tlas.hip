@@ -569,20 +569,12 @@ struct gpurt_tlas_s {
     float origin_bound = INFINITY;      // 2^8 x the largest |world box coordinate|
     std::vector<uint32_t> custom;       // custom index of every instance (host copy)
     std::vector<gpurt_bvh_s*> blas;     // BLAS of every instance
-    // frees in stream order on the context's release stream (see gpurt_tlas_destroy);
-    // a TLAS whose context is gone (tlas_orphan) holds no device memory
+    // gives its memory back after its uses, which are recorded with the instance BVH (see
+    // gpurt_tlas_destroy); a TLAS whose context is gone (tlas_orphan) holds no device memory
     ~gpurt_tlas_s() {
         if (inst_d && ctx) {
-            if (top) {
-                wait_uses(top, ctx->release);
-                bool lost;
-                {
-                    std::lock_guard<std::mutex> lk(top->use_mu);
-                    lost = top->uses_lost;
-                }
-                if (lost) (void)hipDeviceSynchronize();  // uses that no event marks
-            }
-            pool_free(ctx, inst_d, ctx->release);
+            if (top) pool_free(ctx, inst_d, uses_of(top));
+            else pool_free(ctx, inst_d, ctx->release);
         }
         if (top) gpurt_bvh_destroy(top);
     }
@@ -858,7 +850,7 @@ void tlas_note_use(gpurt_tlas t, hipStream_t s) {
 }
 
 void tlas_orphan(gpurt_tlas t) {
-    pool_free(t->ctx, t->inst_d, t->ctx->release);
+    pool_free(t->ctx, t->inst_d, Uses{});  // (the device is idle)
     t->inst_d = nullptr;
     t->ctx = nullptr;
 }

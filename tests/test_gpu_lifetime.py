@@ -108,6 +108,26 @@ def _soup(n, dev):
     return v, torch.arange(3 * n, device=dev, dtype=torch.int32).reshape(-1, 3)
 
 
+def _two_queues(dev):
+    """Two streams whose work runs side by side (streams share the few hardware queues, and
+    what is behind a running kernel in its queue waits for it)."""
+    busy = torch.cuda.Stream(dev)
+    x = torch.zeros(1, device=dev)
+    for _ in range(16):
+        side = torch.cuda.Stream(dev)
+        torch.cuda.synchronize()
+        _sleep(busy, 0.1)
+        slept = torch.cuda.Event()
+        slept.record(busy)
+        with torch.cuda.stream(side):
+            x.add_(1.0)
+        side.synchronize()
+        if not slept.query():
+            torch.cuda.synchronize()
+            return busy, side
+    pytest.skip("no two streams run side by side")
+
+
 @pytest.fixture
 def many_bvhs(dev):
     """A context and BVHs whose memory together is more than the context keeps idle (a
@@ -127,9 +147,10 @@ def many_bvhs(dev):
 
 def test_destroy_beyond_the_idle_limit_does_not_wait(dev, many_bvhs):
     """Destroying them while a query on the first is still to run waits for nothing, and the
-    query's answer is whole."""
+    query's answer is whole although the next builds take as much memory."""
     Q, bvhs = many_bvhs
-    busy, done = torch.cuda.Stream(dev), torch.cuda.Event()
+    busy, side = _two_queues(dev)
+    done = torch.cuda.Event()
     want = bvhs[0].closest_point(Q)
     torch.cuda.synchronize()
     with torch.cuda.stream(busy):
@@ -140,7 +161,14 @@ def test_destroy_beyond_the_idle_limit_does_not_wait(dev, many_bvhs):
     for b in bvhs:
         b.close()
     assert not done.query(), "a destroy waited for the query"
+    V = Q.repeat(300, 1)
+    F = torch.arange(3 * (len(V) // 3), device=dev, dtype=torch.int32).reshape(-1, 3)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        others = [gpurt.Bvh(bvhs[0].ctx, V, F) for _ in bvhs]
     torch.cuda.synchronize()
+    for b in others:
+        b.close()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
@@ -161,3 +189,57 @@ def test_destroy_beyond_the_idle_limit_while_another_thread_captures(dev, many_b
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, (x + 1.0) * 2.0)
+
+
+@pytest.mark.parametrize("other", [False, True])
+def test_build_does_not_wait_for_another_streams_query(dev, other):
+    """A build and a refit on one stream after a BVH that a query on another stream still reads
+    was destroyed (and, other, after it a BVH that only this stream has used): they take other
+    memory and return while that query is still to run."""
+    w = W.cpq_small(n_queries=4096)
+    V, F, Q = _t(w["verts"], dev), _t(w["tris"], dev), _t(w["queries"], dev)
+    V2, V3 = V * 2.0, V * 3.0
+    ctx = gpurt.Context(0)
+    busy, side = _two_queues(dev)
+    done = torch.cuda.Event()
+    with torch.cuda.stream(side):
+        own, bvh = gpurt.Bvh(ctx, V, F), gpurt.Bvh(ctx, V, F)
+        own.closest_point(Q)
+        want = bvh.closest_point(Q)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        bvh.closest_point(Q)
+        _sleep(busy, 0.5)
+        got = bvh.closest_point(Q)
+        done.record(busy)
+    bvh.close()
+    if other:
+        own.close()
+    with torch.cuda.stream(side):
+        after = gpurt.Bvh(ctx, V2, F)
+        after.refit(V3)
+    assert not done.query(), "the build waited for the other stream"
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    for b in (after, own):
+        b.close()
+    ctx.close()
+
+
+def test_rebuilding_in_a_loop_takes_no_new_memory(dev):
+    """Build, query and destroy on one stream, without waiting: the next build takes the memory
+    of the last, so the device's free memory stays as it is."""
+    V, F = _soup(1_000_000, dev)
+    Q = V[:65536].contiguous()
+    ctx = gpurt.Context(0)
+    out = None
+    for k in range(24):
+        bvh = gpurt.Bvh(ctx, V, F)
+        out = bvh.closest_point(Q, out=out)
+        bvh.close()
+        if k == 3:
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info(dev)[0]
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info(dev)[0] > free - (64 << 20)
+    ctx.close()
