@@ -160,10 +160,13 @@ __device__ __forceinline__ void scatter_terms(const CornerTerms& t, float* g_ver
 // add nothing), are summed per key in two passes with a fixed order (the same bits on
 // every run), and without a serial loop over a long run:
 //   k_wave_segsum  one thread per sorted term: within each 64-term wave, a segmented
-//                  suffix scan over shuffles leaves a key's sum with its first term, which
-//                  hands it to the sink when the key's run lies in the wave
+//                  suffix scan over shuffles leaves a key's sum with its first term, and it
+//                  is added to the gradient when the key's run lies in the wave
 //   k_run_sum      one thread per wave: the sum of a run that starts in it and goes on (its
 //                  part in the wave, then those of the next waves in turn)
+// The gradient of a key is at sink.at(key).  Each key's total is added once, atomically: calls
+// on several streams may add to one gradient buffer at the same time (and meshes of a batch
+// share one), as they may with scatter_terms.
 // Only the parts of runs across waves pass through memory, two per wave (a partial sum per
 // term and a second pass over all terms: the sums of a step on 1.3 M triangles, 3.1 M terms,
 // 75 us, of a 256-mesh batch 353 us; now 55 and 208).
@@ -175,8 +178,10 @@ template <int BS, typename K, typename Sink>
 __global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const K* __restrict__ keys,
                                                     const uint32_t* __restrict__ vals, const float* __restrict__ terms,
                                                     uint64_t none, WaveSums sums, Sink sink) {
+    __shared__ float* at[BS];       // per wave: where its finished totals go
+    __shared__ float total[3 * BS];
     const uint32_t p = blockIdx.x * BS + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63u, wave = p >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = p >> 6, w0 = threadIdx.x & ~63u;
     const bool in = p < m;
     const K key = in ? keys[p] : ~(K)0;
     const bool goes_on = in && p > 0 && keys[p - 1] == key;  // (at lane 0: the run began before the wave)
@@ -201,16 +206,29 @@ __global__ __launch_bounds__(BS) void k_wave_segsum(uint32_t m, const K* __restr
             z += oz;
         }
     }
-    if (!head || key >= none) return;
     const size_t next = 64 * ((size_t)wave + 1);
-    float* part = goes_on ? sums.first : end == 64u && next < m && keys[next] == key ? sums.last : nullptr;
+    const bool sum = head && key < none;
+    float* part = nullptr;
+    if (sum) part = goes_on ? sums.first : end == 64u && next < m && keys[next] == key ? sums.last : nullptr;
     if (part) {
         part[3 * (size_t)wave] = x;
         part[3 * (size_t)wave + 1] = y;
         part[3 * (size_t)wave + 2] = z;
-    } else {
-        sink(key, x, y, z);
     }
+    // the totals of neighbouring vertices leave as one component per lane, so that the atomics
+    // of a wave go to few lines
+    const bool whole = sum && !part;
+    const uint64_t done = __ballot(whole);
+    if (whole) {
+        const uint32_t k = w0 + (uint32_t)__popcll(lane ? done & (~0ull >> (64u - lane)) : 0ull);
+        at[k] = sink.at(key);
+        total[3 * k] = x;
+        total[3 * k + 1] = y;
+        total[3 * k + 2] = z;
+    }
+    __syncthreads();
+    for (uint32_t e = lane; e < 3u * (uint32_t)__popcll(done); e += 64u)
+        unsafeAtomicAdd(at[w0 + e / 3u] + e % 3u, total[3u * w0 + e]);
 }
 
 template <int BS, typename K, typename Sink>
@@ -227,7 +245,10 @@ __global__ __launch_bounds__(BS) void k_run_sum(uint32_t m, const K* __restrict_
         y += sums.first[3 * (q >> 6) + 1];
         z += sums.first[3 * (q >> 6) + 2];
     }
-    sink(key, x, y, z);
+    float* const g = sink.at(key);
+    unsafeAtomicAdd(g, x);
+    unsafeAtomicAdd(g + 1, y);
+    unsafeAtomicAdd(g + 2, z);
 }
 
 // floats of a WaveSums array for m terms

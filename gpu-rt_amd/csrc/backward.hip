@@ -79,16 +79,10 @@ __global__ __launch_bounds__(kBlock) void k_ray_bwd(uint32_t n, const float4* __
     scatter_terms(ray_bwd_terms(i, rays, prim, t, uv, g, tri_idx, n_tris, verts, 3, g_o, g_d), uv ? g_verts : nullptr);
 }
 
-// adds a vertex's total to its gradient: each vertex has one run, so a call adds once to each
-// component (the same bits on every run), but calls on several streams may add to one buffer
-// at the same time, as they may with the atomics below kFixedOrderMinTerms
+// a vertex's gradient
 struct VertexSink {
     float* g_verts;
-    __device__ void operator()(uint64_t v, float x, float y, float z) const {
-        unsafeAtomicAdd(&g_verts[3 * v], x);
-        unsafeAtomicAdd(&g_verts[3 * v + 1], y);
-        unsafeAtomicAdd(&g_verts[3 * v + 2], z);
-    }
+    __device__ float* at(uint64_t v) const { return g_verts + 3 * v; }
 };
 
 namespace {

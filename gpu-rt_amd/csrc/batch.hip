@@ -287,16 +287,14 @@ __global__ __launch_bounds__(256) void k_batch_bwd(const BatchMeshDev* __restric
     }
 }
 
-// adds a batch-wide vertex's total to its mesh's vertex gradient (cleared by
-// k_batch_zero_vgrads; each key has one run, and the add is atomic because meshes may share
-// a gradient buffer).  voff[0..n_meshes] are the meshes' first
-// batch-wide vertices (a mesh without a vertex gradient adds none), so the mesh is the
-// last m with voff[m] <= key.
+// A batch-wide vertex's gradient, in its mesh's buffer (cleared by k_batch_zero_vgrads).
+// voff[0..n_meshes] are the meshes' first batch-wide vertices (a mesh without a vertex
+// gradient adds none), so the mesh is the last m with voff[m] <= key.
 struct MeshVertexSink {
     const BatchGradDev* grads;
     const uint64_t* voff;
     uint32_t n_meshes;
-    __device__ void operator()(uint64_t key, float x, float y, float z) const {
+    __device__ float* at(uint64_t key) const {
         // Sorted keys: the first active lane's mesh by a search with one value for the wave,
         // then on from it, mostly no step or one.  (A search per lane is a chain of ~8
         // dependent loads each: the sums of the 256-mesh batch 228 -> 158 us.  Meshes that
@@ -311,11 +309,7 @@ struct MeshVertexSink {
             else hi = mid;
         }
         lo = last_from(voff, n_meshes, lo, key);
-        float* g = grads[lo].g_verts;
-        const size_t v = key - voff[lo];
-        unsafeAtomicAdd(&g[3 * v], x);
-        unsafeAtomicAdd(&g[3 * v + 1], y);
-        unsafeAtomicAdd(&g[3 * v + 2], z);
+        return grads[lo].g_verts + 3 * (key - voff[lo]);
     }
 };
 
