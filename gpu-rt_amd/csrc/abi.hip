@@ -170,6 +170,30 @@ static void pool_trim(gpurt_ctx_s* c, size_t keep) {
     c->pool.erase(std::remove_if(c->pool.begin(), c->pool.end(), [](auto& e) { return !e.mem; }), c->pool.end());
 }
 
+// memory is short: frees all idle blocks, after their work, and has HIP give them back (the
+// caller holds pool_mu)
+static void pool_empty(gpurt_ctx_s* c) {
+    AnyCapture mode;
+    for (auto& e : c->pool)
+        for (auto& u : e.after) (void)hipEventSynchronize(u.second->e);
+    pool_trim(c, 0);
+    (void)hipStreamSynchronize(c->release);
+    (void)hipMemPoolTrimTo(c->mem, 0);
+    (void)hipGetLastError();
+}
+
+hipError_t ctx_malloc(gpurt_ctx_s* c, void** p, size_t bytes) {
+    *p = nullptr;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lk(c->pool_mu);
+        pool_empty(c);
+    }
+    return hipMalloc(p, bytes);
+}
+
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     *p = nullptr;
     // sizes in steps of an eighth of their power of two (at least 64 KiB), so that the
@@ -210,18 +234,12 @@ int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     if (hipMallocFromPoolAsync(&e.mem, bytes, c->mem, s) != hipSuccess) {
         (void)hipGetLastError();
         e.mem = nullptr;
-        // memory is short: any block that fits will do, then all idle ones are freed, after
-        // their work, and HIP's pool gives them back
+        // any block that fits will do, then none is kept
         best = nullptr;
         for (auto& x : c->pool)
             if (!x.used && x.bytes >= bytes && better(x, best)) best = &x;
         if (best && take(*best)) return GPURT_OK;
-        for (auto& x : c->pool)
-            for (auto& u : x.after) (void)hipEventSynchronize(u.second->e);
-        pool_trim(c, 0);
-        (void)hipStreamSynchronize(c->release);
-        (void)hipMemPoolTrimTo(c->mem, 0);
-        (void)hipGetLastError();
+        pool_empty(c);
         if (hipMallocFromPoolAsync(&e.mem, bytes, c->mem, s) != hipSuccess) {
             (void)hipGetLastError();
             return set_error(GPURT_E_OOM, "allocation of " + std::to_string(bytes) + " bytes failed");
@@ -322,7 +340,7 @@ int ctx_scratch(gpurt_ctx_s* c, hipStream_t s, size_t bytes, CallScratch& out) {
                 e.mem = nullptr;
                 e.bytes = 0;
                 const size_t want = bytes + bytes / 4;  // room for somewhat larger calls
-                if (hipMalloc(&e.mem, want) != hipSuccess) {
+                if (ctx_malloc(c, &e.mem, want) != hipSuccess) {
                     (void)hipGetLastError();
                     e.mem = nullptr;
                     return set_error(GPURT_E_OOM, "query scratch allocation failed");

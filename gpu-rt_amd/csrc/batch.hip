@@ -529,6 +529,7 @@ int gpurt_batch_create(gpurt_ctx ctx, const gpurt_batch_mesh* meshes, size_t n_m
     // bits 8-15: the ray kernel's refill trigger (16 lanes by default, as for single meshes)
     b->leaf_trigger |= (qopts && qopts->refill_trigger ? (uint32_t)qopts->refill_trigger : 16u) << 8;
     b->host_meshes.assign(meshes, meshes + n_meshes);
+    b->build.owner = ctx;
     int rc = build_alloc(segs.data(), (int)n_meshes, W, leaf, tsize, b->build);
     if (rc) {
         delete b;
@@ -574,14 +575,14 @@ int gpurt_batch_create(gpurt_ctx ctx, const gpurt_batch_mesh* meshes, size_t n_m
     // deepest possible wide tree (kMaxLevels levels) bounds the stack: no overflow
     const int need = (W - 1) * kMaxLevels + 1;
     b->spill_slots = need > S ? (uint32_t)(need - S) : 0u;
-    bool fail = hipMalloc((void**)&b->meshes_d, sizeof(BatchMeshDev) * n_meshes) != hipSuccess ||
-                hipMalloc((void**)&b->chunks_d, sizeof(uint2) * std::max<size_t>(1, chunks.size())) != hipSuccess ||
-                hipMalloc((void**)&b->counter_d, sizeof(uint32_t) * 2 * kQueues * kQueueStride) != hipSuccess ||
-                (has_qnodes(bp.format) && hipMalloc(&b->qnodes, qnode_bytes(W) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
+    bool fail = ctx_malloc(ctx, (void**)&b->meshes_d, sizeof(BatchMeshDev) * n_meshes) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&b->chunks_d, sizeof(uint2) * std::max<size_t>(1, chunks.size())) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&b->counter_d, sizeof(uint32_t) * 2 * kQueues * kQueueStride) != hipSuccess ||
+                (has_qnodes(bp.format) && ctx_malloc(ctx, &b->qnodes, qnode_bytes(W) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
                 (oriented &&
-                 hipMalloc(&b->onodes, sizeof(ONode) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
+                 ctx_malloc(ctx, &b->onodes, sizeof(ONode) * std::max<uint32_t>(1u, b->build.capacity)) != hipSuccess) ||
                 (b->spill_slots &&
-                 hipMalloc((void**)&b->spill, (size_t)b->spill_slots * b->grid * BS * sizeof(uint2)) != hipSuccess);
+                 ctx_malloc(ctx, (void**)&b->spill, (size_t)b->spill_slots * b->grid * BS * sizeof(uint2)) != hipSuccess);
     if (fail) {
         (void)hipGetLastError();
         delete b;
@@ -684,9 +685,9 @@ int gpurt_batch_set_grads(gpurt_batch b, const gpurt_batch_grad* grads) {
     DevGuard dg(b->ctx->device);
     if (!dg.ok) return set_error(GPURT_E_DEVICE, "hipSetDevice failed");
     b->drop_backward();
-    if (hipMalloc((void**)&b->grads_d, sizeof(BatchGradDev) * n_meshes) != hipSuccess ||
-        (!segs.empty() && hipMalloc((void**)&b->zero_segs_d, sizeof(uint2) * segs.size()) != hipSuccess) ||
-        (m && hipMalloc(&b->terms_mem, tbytes) != hipSuccess)) {
+    if (ctx_malloc(b->ctx, (void**)&b->grads_d, sizeof(BatchGradDev) * n_meshes) != hipSuccess ||
+        (!segs.empty() && ctx_malloc(b->ctx, (void**)&b->zero_segs_d, sizeof(uint2) * segs.size()) != hipSuccess) ||
+        (m && ctx_malloc(b->ctx, &b->terms_mem, tbytes) != hipSuccess)) {
         (void)hipGetLastError();
         b->drop_backward();
         return set_error(GPURT_E_OOM, "batch gradient allocation failed");

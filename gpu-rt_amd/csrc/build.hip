@@ -1362,7 +1362,7 @@ BuildBufs::~BuildBufs() {
 hipError_t BuildBufs::alloc(void** p, size_t bytes) {
     *p = nullptr;
     const hipError_t e = ctx ? (pool_alloc(ctx, p, bytes, pool_stream) ? hipErrorOutOfMemory : hipSuccess)
-                             : hipMalloc(p, bytes);
+                             : ctx_malloc(owner, p, bytes);
     if (e == hipSuccess) allocs.push_back(*p);
     return e;
 }

@@ -295,6 +295,8 @@ Uses uses_of(gpurt_bvh_s* b);
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s);
 void pool_free(gpurt_ctx_s* c, void* p, hipStream_t s);        // after what s holds now
 void pool_free(gpurt_ctx_s* c, void* p, const Uses& after);
+// hipMalloc; when memory is short the pool's idle blocks are freed and it is tried again
+hipError_t ctx_malloc(gpurt_ctx_s* c, void** p, size_t bytes);
 void pool_release(gpurt_ctx_s* c);  // after the device is idle (context destroy)
 
 // Lays buffers out in one allocation, 256-byte aligned: a first pass without a base gives
@@ -368,9 +370,9 @@ struct BuildBufs {
     float4* final_tris() const { return repacked ? tris2 : tris; }
     uint32_t* final_order() const { return repacked ? leaf_order2 : leaf_order; }
     // Plain builds: scratch from the context's pool, and the BVH's own buffers for the
-    // triangles and their order.  Without a context everything is hipMalloc'ed and kept
-    // (the batch).
-    gpurt_ctx_s* ctx = nullptr;
+    // triangles and their order.  Without a context everything is hipMalloc'ed (for `owner`)
+    // and kept (the batch).
+    gpurt_ctx_s *ctx = nullptr, *owner = nullptr;
     hipStream_t pool_stream = nullptr;
     float4* own_tris = nullptr;
     uint32_t* own_order = nullptr;

@@ -1073,17 +1073,17 @@ int gpurt_scene_create(gpurt_tlas tlas, const gpurt_object* objects, size_t n_ob
         delete S;
         return code;
     };
-    if (hipMalloc((void**)&S->objs, sizeof(ObjDev) * n_objects) != hipSuccess ||
-        hipMalloc((void**)&S->verts, 48 * std::max<uint64_t>(nv, 1)) != hipSuccess ||
-        hipMalloc((void**)&S->idx, 4 * std::max<uint64_t>(ni, 1)) != hipSuccess ||
-        hipMalloc((void**)&S->tally, 2 * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc((void**)&bad, sizeof(uint32_t)) != hipSuccess ||
-        (nl && (hipMalloc((void**)&S->lights, sizeof(LightDev) * lights.size()) != hipSuccess ||
-                hipMalloc((void**)&S->lworld, 48 * nl) != hipSuccess ||
-                hipMalloc((void**)&S->ltri_n, 4 * nl) != hipSuccess ||
-                hipMalloc((void**)&flat, 36 * nl) != hipSuccess ||
-                hipMalloc((void**)&flat_idx, 12 * nl) != hipSuccess ||
-                hipMalloc((void**)&src_d, sizeof(uint2) * nl) != hipSuccess))) {
+    if (ctx_malloc(ctx, (void**)&S->objs, sizeof(ObjDev) * n_objects) != hipSuccess ||
+        ctx_malloc(ctx, (void**)&S->verts, 48 * std::max<uint64_t>(nv, 1)) != hipSuccess ||
+        ctx_malloc(ctx, (void**)&S->idx, 4 * std::max<uint64_t>(ni, 1)) != hipSuccess ||
+        ctx_malloc(ctx, (void**)&S->tally, 2 * sizeof(unsigned long long)) != hipSuccess ||
+        ctx_malloc(ctx, (void**)&bad, sizeof(uint32_t)) != hipSuccess ||
+        (nl && (ctx_malloc(ctx, (void**)&S->lights, sizeof(LightDev) * lights.size()) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&S->lworld, 48 * nl) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&S->ltri_n, 4 * nl) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&flat, 36 * nl) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&flat_idx, 12 * nl) != hipSuccess ||
+                ctx_malloc(ctx, (void**)&src_d, sizeof(uint2) * nl) != hipSuccess))) {
         (void)hipGetLastError();
         return fail(set_error(GPURT_E_OOM, "scene allocation failed"));
     }
@@ -1210,9 +1210,9 @@ int gpurt_render(gpurt_scene S, const gpurt_render_params* prm, float* image, fl
         S->cap = S->lane_cap = 0;
         S->trav_bytes = tlas_scratch_bytes(S->tlas, 2 * (size_t)per);
         if (S->trav_bytes == 0) return set_error(GPURT_E_INVALID, "cannot plan the traversal");
-        bool ok = hipMalloc(&S->wf, carve(nullptr, P, nullptr)) == hipSuccess;
+        bool ok = ctx_malloc(S->ctx, &S->wf, carve(nullptr, P, nullptr)) == hipSuccess;
         for (Lane& l : S->lanes)
-            ok = ok && hipMalloc(&l.trav, S->trav_bytes) == hipSuccess && hipMalloc(&l.trav2, S->trav_bytes) == hipSuccess;
+            ok = ok && ctx_malloc(S->ctx, &l.trav, S->trav_bytes) == hipSuccess && ctx_malloc(S->ctx, &l.trav2, S->trav_bytes) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
             for (Lane& l : S->lanes) l.free_scratch();
@@ -1224,8 +1224,8 @@ int gpurt_render(gpurt_scene S, const gpurt_render_params* prm, float* image, fl
         S->lane_cap = per;
     }
     for (int g = 0; g < G; g++)  // groups created since the last sizing
-        if (!S->lanes[g].trav && (hipMalloc(&S->lanes[g].trav, S->trav_bytes) != hipSuccess ||
-                                  hipMalloc(&S->lanes[g].trav2, S->trav_bytes) != hipSuccess)) {
+        if (!S->lanes[g].trav && (ctx_malloc(S->ctx, &S->lanes[g].trav, S->trav_bytes) != hipSuccess ||
+                                  ctx_malloc(S->ctx, &S->lanes[g].trav2, S->trav_bytes) != hipSuccess)) {
             (void)hipGetLastError();
             return set_error(GPURT_E_OOM, "traversal scratch allocation failed");
         }

@@ -243,3 +243,35 @@ def test_rebuilding_in_a_loop_takes_no_new_memory(dev):
     torch.cuda.synchronize()
     assert torch.cuda.mem_get_info(dev)[0] > free - (64 << 20)
     ctx.close()
+
+
+def test_idle_memory_is_given_up_when_memory_is_short(dev):
+    """Memory that a context keeps idle is freed for its other allocations: with a gigabyte free
+    on the device and several idle, the scratch of a backward call (84 bytes a query, 2.1 GB) and
+    then a build are made."""
+    V, F = _soup(2_000_000, dev)
+    ctx = gpurt.Context(0, vertex_sums="fixed")
+    bvh = gpurt.Bvh(ctx, V, F)
+    n = 20_000_000
+    q = V.repeat(4, 1)[:n].contiguous()
+    prim, pt, dist, bary = bvh.closest_point(q)
+    g, gv = torch.ones(n, device=dev), torch.zeros_like(V)
+    idle = [gpurt.Bvh(ctx, V, F) for _ in range(12)]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free0 = torch.cuda.mem_get_info(dev)[0]
+    for b in idle:
+        b.close()
+    assert torch.cuda.mem_get_info(dev)[0] < free0 + (1 << 30)  # (kept)
+    hog = torch.empty(torch.cuda.mem_get_info(dev)[0] - (1 << 30), dtype=torch.uint8, device=dev)
+    bvh.closest_point_bwd(q, prim, bary, pt, dist, g, None, gv)
+    other = gpurt.Bvh(ctx, V, F)
+    torch.cuda.synchronize()
+    assert torch.isfinite(gv).all()
+    p2 = other.closest_point(q[:4096])[0]
+    assert torch.equal(p2, prim[:4096])
+    del hog, q, pt, bary, g, gv
+    other.close()
+    bvh.close()
+    ctx.close()
+    torch.cuda.empty_cache()
