@@ -469,7 +469,7 @@ constexpr int kGroupKeyBytes = 12;
 // waves_per_simd: what the kernel is compiled for (0: the single-level kernels' WavesHint);
 // lds_extra: LDS bytes per lane beyond the stack slots
 int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need, const gpurt_query_opts* opts,
-                   size_t n, TravPlan& p, int waves_per_simd = 0, int lds_extra = kGroupKeyBytes);
+                   size_t n, TravPlan& p, int waves_per_simd = 0, int lds_extra = kGroupKeyBytes, bool oriented = false);
 int alloc_traversal_scratch(gpurt_ctx_s* c, const TravPlan& p, hipStream_t s, TravScratch& t);
 void free_traversal_scratch(gpurt_ctx_s* c, TravScratch& t);
 // the same scratch in memory the caller holds

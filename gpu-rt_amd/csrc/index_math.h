@@ -1,9 +1,10 @@
-// index_math.h -- index arithmetic of the kernels at sizes that no test on a device reaches,
-// kept apart so that the host can run it over their whole range.
+// index_math.h -- index arithmetic of the kernels at sizes that no test on a device reaches, and
+// rules of launches, kept apart so that the host can run them over their whole range.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 namespace gpurt_impl {
@@ -37,6 +38,17 @@ __host__ __device__ inline uint32_t last_from(const Offsets& off, uint32_t n, ui
         if (step < n - lo && off[lo + step] <= key) lo += step;
     }
     return lo;
+}
+
+// Waves per CU of a set of n closest points: 16, but 12 for up to 256 points per CU (a
+// quarter of 16 waves' lanes) on oriented nodes, where the time is the longest searches' and
+// not the lanes'.  12 against 16, us: 65,536 points near 20,000 / 330,000 / 1.3 M triangles 99 /
+// 106, 159 / 166, 182 / 194, on a soup of 100,000 triangles 119 / 121, on 20,000 overlapping
+// ones 201 / 194; 131,072 on the overlapping ones 319 / 291, 200,000 near 20,000 triangles
+// 160 / 125; on FP32 and 8-bit nodes, whose far queries take long, 65,536 uniform on 1.3 M
+// 2,200 / 1,890 (FP32, W = 4).
+inline int point_waves_per_cu(size_t n, int n_cu, bool oriented) {
+    return oriented && n <= (size_t)n_cu * 256 ? 12 : 16;
 }
 
 }  // namespace gpurt_impl

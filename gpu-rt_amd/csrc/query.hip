@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "index_math.h"
 #include "traverse.h"
 
 namespace gpurt_impl {
@@ -135,24 +136,18 @@ static int dispatch_stack(int S, QKind kind, const TravArgs& a, unsigned grid, h
 // CU and a refill at 24 idle lanes 218 us (24 waves, 16 lanes: 230 us), any hit at 28
 // waves and 16 lanes 148-151 us (158 us); 32 waves crowd the L2 (+5%).  (The TLAS
 // passes its own launch options.)
-// waves per CU up to which a small set gets a wave per query (plan_traversal)
-constexpr size_t kWidePoints = 12, kWideRays = 8;
-
 static uint32_t default_leaf_trigger(QKind) { return 32u; }
 static uint32_t default_refill_trigger(QKind kind) { return kind == QKind::Closest ? 24u : 16u; }
-// Closest points: 16 waves per CU, but 12 for a set of at most a query per lane of these
-// (kWidePoints), whose time is its longest searches' and not the lanes': 65,536 points near
-// 252,000 triangles 149 -> 137 us, 200,000 mixed on 1.3 M 568 -> 511, 5,000 near 20,000
-// 52 -> 47; 500,000 mixed 771 -> 835, 1 M near 719 -> 811 with 12.
-static int default_waves_per_cu(QKind kind, size_t n, int n_cu) {
-    if (kind != QKind::Cpq) return 28;
-    return n <= (size_t)n_cu * 16 * 64 ? (int)kWidePoints : 16;
+static int default_waves_per_cu(QKind kind, size_t n, int n_cu, bool oriented) {
+    return kind == QKind::Cpq ? point_waves_per_cu(n, n_cu, oriented) : 28;
 }
+// waves per CU up to which a small set gets a wave per query (plan_traversal)
+constexpr size_t kWidePoints = 12, kWideRays = 8;
 
 static int block_for_stack(int S) { return S <= 16 ? 256 : (S == 32 ? 128 : 64); }
 
 int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need, const gpurt_query_opts* opts,
-                   size_t n, TravPlan& p, int waves_per_simd, int lds_extra) {
+                   size_t n, TravPlan& p, int waves_per_simd, int lds_extra, bool oriented) {
     if (n > 0xFFFFFFFFull - 1024u) return set_error(GPURT_E_INVALID, "too many queries in one call");
     // default: the smallest LDS stack (most resident waves) for rays; 8-wide nodes push
     // more entries per visit, so they default to 16, and so do closest-point queries,
@@ -173,7 +168,7 @@ int plan_traversal(gpurt_ctx ctx, int width, bool q8, QKind kind, int stack_need
         blocks_per_cu = std::max(1, opts->waves_per_cu / waves_per_block);
     else
         blocks_per_cu = std::min(blocks_per_cu,
-                                 std::max(1, default_waves_per_cu(kind, n, ctx->n_cu) / waves_per_block));
+                                 std::max(1, default_waves_per_cu(kind, n, ctx->n_cu, oriented) / waves_per_block));
     blocks_per_cu = std::max(blocks_per_cu, 1);
     // A small set is spread over more lanes than it has queries (first_query); the idle
     // ones take work from the busy ones once the queues are empty.  A launch of few queries
@@ -292,7 +287,9 @@ static int run_query(gpurt_bvh_s* b, QKind kind, TravArgs a, size_t n, const gpu
     const bool q8 = kind == QKind::Cpq ? cpq_use_q8(b->format) : rays_use_q8(b->format);
     // worst case stack: (W-1) entries per level above the last plus W for the last
     TravPlan p;
-    int rc = plan_traversal(b->ctx, b->width, q8, kind, (b->width - 1) * b->depth + 1, opts, n, p);
+    const bool oriented = kind == QKind::Cpq && cpq_use_oriented(b->format, b->width);
+    int rc = plan_traversal(b->ctx, b->width, q8, kind, (b->width - 1) * b->depth + 1, opts, n, p, 0, kGroupKeyBytes,
+                            oriented);
     if (rc) return rc;
     TravScratch t;
     if (fixed_scratch) {
@@ -314,7 +311,6 @@ static int run_query(gpurt_bvh_s* b, QKind kind, TravArgs a, size_t n, const gpu
     a.leaf_trigger = p.leaf_trigger;
     const bool stats = a.stats != nullptr;
     int bs = 0;
-    const bool oriented = kind == QKind::Cpq && cpq_use_oriented(b->format, b->width);
     a.nodes = oriented ? b->onodes : (q8 ? b->qnodes : b->nodes);
     if (oriented)
         bs = stats ? dispatch_stack<4, kEncOriented, true>(p.S, kind, a, p.grid, s)

@@ -1,5 +1,5 @@
-"""Index arithmetic of the kernels (csrc/index_math.h) on the host, at sizes that no test on
-a device reaches."""
+"""Index arithmetic of the kernels and rules of launches (csrc/index_math.h) on the host, at
+sizes that no test on a device reaches."""
 import os
 import subprocess
 
@@ -76,3 +76,12 @@ def test_mesh_of_a_key_in_few_steps(tmp_path):
             want += [m for lo in range(n) if o[lo] <= key]
     assert out[:-1] == want + [99999]
     assert out[-1] <= 2 * 17 + 1
+
+
+def test_waves_of_closest_point_sets(tmp_path):
+    """12 waves per CU only for small sets on oriented nodes: from 65,537 points of 256 CUs on,
+    and on every other encoding, 16 (12 was up to a half slower there)."""
+    n = [1, 65536, 65537, 131072, 196608, 200000, 262144, 262145, 1 << 40]
+    out = _run(tmp_path, "for (bool o : {true, false}) for (size_t n : {" + ", ".join("%dull" % k for k in n) + "})\n"
+               "    printf(\"%d\\n\", point_waves_per_cu(n, 256, o));")
+    assert [int(x) for x in out] == [12 if k <= 65536 else 16 for k in n] + [16] * len(n)
