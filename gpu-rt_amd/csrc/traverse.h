@@ -914,13 +914,19 @@ __device__ __forceinline__ bool ray_stream(const NodeT* __restrict__ nodes, cons
     return ok;
 }
 
-// Stack entries a lane looks at per iteration for one within its bound.  Most entries of a
-// query near the surface were pushed before its best point was known and are culled when
-// popped; with one a step, each such lane sits out the wave's node step.  1 M queries near
-// 1.3 M triangles: 780 us with 1, 713 us with 2, 709 us with 3 (but queries far from the
-// surface +6%); small sets and uniform queries the same with 1 and 2.  A lane that shares
-// its query takes one, since each read of its group's best may tighten the bound.
-constexpr int kPointPops = 2;
+// Stack entries a lane looks at per iteration for one within its bound.  On oriented nodes
+// most entries of a query near the surface were pushed before its best point was known and
+// are culled when popped; with one a step, each such lane sits out the wave's node step.  1 M
+// queries near 1.3 M triangles: 780 us with 1, 713 us with 2, 709 us with 3 (but queries far
+// from the surface +6%); small sets and uniform queries the same with 1 and 2 (1-2% apart);
+// 300,000 and more near 1,280 to 1.3 M triangles and in soups 4-9% faster with 2, in a soup of
+// overlapping triangles up to 5% slower.  The other encodings open more nodes at a distance
+// and have fewer entries to cull: with 2, 400,000 uniform queries on 20,000 triangles take
+// 1,096 -> 1,200 us (FP32, W = 4), 300,000 mixed ones on 1.3 M 2,291 -> 2,680 (8-bit, W = 4),
+// so they take one.  A lane that shares its query takes one, since each read of its group's
+// best may tighten the bound.
+template <typename NodeT>
+constexpr int kPointPops = std::is_same<NodeT, ONode>::value ? 2 : 1;
 
 template <typename NodeT, int S, int BS, bool STATS, typename Src, typename Out>
 __device__ __forceinline__ bool cpq_stream(const NodeT* __restrict__ nodes, const float4* __restrict__ tris,
@@ -1025,7 +1031,7 @@ __device__ __forceinline__ bool cpq_stream(const NodeT* __restrict__ nodes, cons
         }
         if (!has || wait) continue;
         // up to kPointPops entries, to the first one still within the bound
-        for (int pops = grouped ? 1 : kPointPops; pops > 0 && !have && st.sp > 0; pops--) {
+        for (int pops = grouped ? 1 : kPointPops<NodeT>; pops > 0 && !have && st.sp > 0; pops--) {
             const uint2 e = st.pop();
             if (grouped) {
                 // the group's best so far, read beside the stack entry (a read of its own
