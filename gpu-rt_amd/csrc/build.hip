@@ -1044,7 +1044,8 @@ __global__ __launch_bounds__(kBlock) void k_repack(uint32_t N, const uint32_t* _
     const size_t k = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (k >= 3 * (size_t)N) return;
     const uint32_t out = (uint32_t)(k / 3), v = (uint32_t)(k - 3 * (size_t)out);
-    const uint32_t in = perm[out];
+    // (a tree deeper than kMaxLevels, which is refused, leaves slots without a position)
+    const uint32_t in = min(perm[out], N - 1u);
     tris_out[k] = tris_in[3 * (size_t)in + v];
     if (v == 0) order_out[out] = order_in[in];
 }
@@ -1101,11 +1102,13 @@ __device__ __forceinline__ uint2 root_kids(const float4* __restrict__ bnode, uin
 // Collapses nodes [begin, begin + cnt) of a level, dealt to the grid's threads; all threads
 // of a block call it together.  The next level's nodes, counted in *next_count, follow them.
 // HEAD: read from `in`, and the next level's (with its count in LDS) listed in `next` too
-// while they fit.
+// while they fit.  last: no level follows; *next_count tells that one would have to (the tree
+// is refused then), and the children that it would hold are left out, so that no node of the
+// tree points to one that nothing makes.
 template <int W, bool HEAD = false>
 __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t begin, uint32_t cnt,
                                                uint32_t* next_count, const HeadList* in = nullptr,
-                                               HeadList* next = nullptr) {
+                                               HeadList* next = nullptr, bool last = false) {
     WNode<W>* nodes = reinterpret_cast<WNode<W>*>(a.nodes);
     // every lane runs every iteration (slot allocation is wave-wide); lanes past the
     // level's end take part with nothing to allocate
@@ -1178,6 +1181,12 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t b
             }
         }
         WNode<W> out;
+        auto leave_out = [&](int j) {
+            out.lox[j] = out.loy[j] = out.loz[j] = INFINITY;
+            out.hix[j] = out.hiy[j] = out.hiz[j] = -INFINITY;
+            out.child[j] = kEmpty;
+            out.aux[j] = 0;
+        };
         uint32_t n_internal = 0;
 #pragma unroll
         for (int j = 0; j < W; j++)
@@ -1197,10 +1206,7 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t b
                     out.child[j] = make_leaf(ch[j].first, c);
                 }
             } else {
-                out.lox[j] = out.loy[j] = out.loz[j] = INFINITY;
-                out.hix[j] = out.hiy[j] = out.hiz[j] = -INFINITY;
-                out.child[j] = kEmpty;
-                out.aux[j] = 0;
+                leave_out(j);
             }
         }
         const uint32_t base =
@@ -1212,7 +1218,9 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t b
             for (int j = 0; j < W; j++) {
                 if (j < n && out.aux[j] > (uint32_t)a.leaf_size) {
                     uint32_t idx = base + m++;
-                    if (idx < a.capacity) {
+                    if (last) {
+                        leave_out(j);
+                    } else if (idx < a.capacity) {
                         const uint2 kids = make_uint2(ch[j].l, ch[j].r);
                         a.wsrc[idx] = kids;
                         a.wseg[idx] = seg;
@@ -1226,7 +1234,7 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t b
                         out.child[j] = idx;
                     } else {
                         gatomic_or(&a.counters[1], 2u);
-                        out.child[j] = kEmpty;
+                        leave_out(j);
                     }
                 }
             }
@@ -1263,12 +1271,12 @@ __global__ __launch_bounds__(kBlockLevelThreads) void k_collapse_tail(CollapseAr
     for (int l = a.level; l < kMaxLevels; l++) {
         const uint32_t cnt = count(l);
         if (cnt == 0) break;
-        collapse_level<W>(a, begin, cnt, a.lvl_cnt + l + 1);
+        collapse_level<W>(a, begin, cnt, a.lvl_cnt + l + 1, nullptr, nullptr, l == kMaxLevels - 1);
         begin += cnt;
         __threadfence_block();
         __syncthreads();
     }
-    if (threadIdx.x == 0) a.counters[0] = begin + count(kMaxLevels);
+    if (threadIdx.x == 0) a.counters[0] = begin;
 }
 
 // Levels [0, last), none of more than kHeadNodes nodes, by one block.  A level of a few

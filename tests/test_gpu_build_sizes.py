@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import gpurt
+from gpurt import _lib
 from gpurt import workloads as W
 from oracle import oracle as O
 
@@ -191,3 +192,44 @@ def test_build_at_range_level_edges(ctx, dev, n):
     print("build", n, flush=True)
     V, F = _soup(n, n, dup=0.0)
     _check(gpurt.Bvh(ctx, _t(V, dev), _t(F, dev)), V, F)
+
+
+def _fractal(n):
+    """Soups at 16 halving scales about one point: trees much deeper than their size asks for, of
+    many nodes per level all the way down."""
+    rng = np.random.default_rng(3)
+    c = rng.uniform(-1, 1, (n, 1, 3))
+    v = (c + rng.normal(0, 0.02, (n, 3, 3))) * 0.5 ** rng.integers(0, 16, (n, 1, 1))
+    return v.astype(np.float32).reshape(-1, 3), np.arange(3 * n, dtype=np.int32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("n,width,tsize", [(20_000, 2, 0), (20_000, 2, 5), (20_000, 2, 7), (20_000, 4, 7), (20_000, 8, 7),
+                                           (600_000, 2, 0), (600_000, 2, 7), (600_000, 4, 7), (600_000, 8, 0)])
+def test_deep_trees_are_built_or_refused(ctx, dev, n, width, tsize):
+    """A tree deeper than the supported level count (binary nodes with treelets, 600,000
+    triangles) is refused with GPURT_E_UNSUPPORTED, by a plain build and by a batch; any other
+    answers as the brute force."""
+    print("fractal", n, width, tsize, flush=True)
+    V, F = _fractal(n)
+    tv, tf = _t(V, dev), _t(F, dev)
+    rng = np.random.default_rng(4)
+    q = V[3 * rng.integers(0, n, 64)]
+    q = (q + 0.01 * np.linalg.norm(q, axis=1, keepdims=True) * rng.normal(size=(64, 3))).astype(np.float32)
+    meshes = [{"verts": tv, "tris": tf, "queries": _t(q, dev)}]
+    opts = {"node_width": width, "treelet_size": tsize}
+    if (n, width, tsize) == (600_000, 2, 7):
+        for _ in range(2):
+            for build in (lambda: gpurt.Bvh(ctx, tv, tf, **opts), lambda: gpurt.Batch(ctx, meshes, **opts)):
+                with pytest.raises(gpurt.GpurtError) as e:
+                    build()
+                assert e.value.code == _lib.GPURT_E_UNSUPPORTED
+        return
+    ep, _, ed, _ = O.cpq_brute_f32(V, F, q)
+    bvh = gpurt.Bvh(ctx, tv, tf, **opts)
+    print("depth", bvh.info()["depth"], flush=True)
+    batch = gpurt.Batch(ctx, meshes, **opts)
+    r = batch.run()[0]
+    for prim, dist in (bvh.closest_point(_t(q, dev))[::2], (r["q_prim"], r["q_dist"])):
+        assert np.array_equal(prim.cpu().numpy(), ep) and np.array_equal(dist.cpu().numpy(), ed)
+    batch.close()
+    bvh.close()
