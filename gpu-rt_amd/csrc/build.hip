@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "build_common.h"
+#include "index_math.h"
 
 namespace gpurt_impl {
 
@@ -1561,13 +1562,7 @@ int build_enqueue_collapse(BuildBufs& b, int leaf_size, hipStream_t s) {
     ca.leaf_size = leaf_size;
     ca.repack = b.repacked ? 1 : 0;
     ca.perm = b.perm;
-    // Launches for the depth that trees of this size have (5 K triangles: 8 wide levels at
-    // W = 4, 2.3 M: 16; a W-wide level takes about log2(W) binary ones on the way down the
-    // larger side) and some; a deeper tree's last levels, with few nodes, are the tail's.
-    int nbits = 1;
-    while ((1u << nbits) < b.N) nbits++;
-    const int per = b.width == 2 ? 10 : (b.width == 4 ? 8 : 5);
-    const int levels = std::min(kMaxLevels - 1, 2 + nbits * per / 10);
+    const int levels = std::min(kMaxLevels - 1, collapse_launches(b.N, b.width, b.treelets));
     const unsigned grid = std::min(cdiv(b.capacity, kBlock), 2048u);
     if (b.width == 2) launch_collapse<2>(ca, b.n_seg, b.segs, b.seg_root, levels, grid, s);
     else if (b.width == 4) launch_collapse<4>(ca, b.n_seg, b.segs, b.seg_root, levels, grid, s);

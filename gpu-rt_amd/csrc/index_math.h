@@ -51,4 +51,17 @@ inline int point_waves_per_cu(size_t n, int n_cu, bool oriented) {
     return oriented && n <= (size_t)n_cu * 256 ? 12 : 16;
 }
 
+// Wide levels of a W-wide tree over n triangles that get a launch each: what such trees have (5
+// K triangles: 8 levels at W = 4, 2.3 M: 16; a level takes about log2(W) binary ones on the way
+// down the larger side) and some.  The levels below are one block's, which is no slower for
+// the few nodes that a small mesh has there; a large one's binary nodes, whose trees run 22 to
+// 48 levels (58 with treelets), need more launches for that: a cluster of 1 M triangles in a
+// scene of 64 takes 2,620 us with 22 launches and 570 us with 30; with treelets 7,620 us, with 42 1,370 us.
+inline int collapse_launches(uint32_t n, int width, bool treelets) {
+    int bits = 1;
+    while (bits < 31 && (1u << bits) < n) bits++;
+    const int per = width == 8 ? 5 : width == 4 ? 8 : n <= 65536 ? 10 : treelets ? 20 : 14;
+    return 2 + bits * per / 10;
+}
+
 }  // namespace gpurt_impl

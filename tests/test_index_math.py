@@ -85,3 +85,16 @@ def test_waves_of_closest_point_sets(tmp_path):
     out = _run(tmp_path, "for (bool o : {true, false}) for (size_t n : {" + ", ".join("%dull" % k for k in n) + "})\n"
                "    printf(\"%d\\n\", point_waves_per_cu(n, 256, o));")
     assert [int(x) for x in out] == [12 if k <= 65536 else 16 for k in n] + [16] * len(n)
+
+
+def test_collapse_launches(tmp_path):
+    """Launches per tree: the levels that trees of the size have and some, with room below the
+    64 supported levels; binary trees of large meshes get more, most with treelets."""
+    n = [1, 2, 5000, 65536, 65537, 1_000_000, 2_300_000, (1 << 28) - 9]
+    out = _run(tmp_path, "for (unsigned n : {" + ", ".join("%du" % k for k in n) + "})\n"
+               "    for (int w : {2, 4, 8}) for (bool t : {false, true}) printf(\"%d\\n\", collapse_launches(n, w, t));")
+    got = {(k, w, t): int(out.pop(0)) for k in n for w in (2, 4, 8) for t in (0, 1)}
+    assert max(got.values()) < 64 and min(got.values()) >= 2
+    assert [got[k, 4, t] for k in (5000, 2_300_000) for t in (0, 1)] == [12, 12, 19, 19]
+    assert [got[1_000_000, 2, t] for t in (0, 1)] == [30, 42]
+    assert all(got[k, w, 0] == got[k, w, 1] for k in n for w in (2, 4, 8) if w > 2 or k <= 65536)
