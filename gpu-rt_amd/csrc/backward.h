@@ -158,12 +158,13 @@ __device__ __forceinline__ void scatter_terms(const CornerTerms& t, float* g_ver
 // ---- fixed-order vertex sums ---------------------------------------------------------
 // The terms, sorted by key (a vertex, or (mesh, vertex) in a batch; `none` for terms that
 // add nothing), are summed per key in two passes with a fixed order (the same bits on
-// every run), and without a serial loop over a long run:
+// every run):
 //   k_wave_segsum  one thread per sorted term: within each 64-term wave, a segmented
 //                  suffix scan over shuffles leaves a key's sum with its first term, and it
 //                  is added to the gradient when the key's run lies in the wave
 //   k_run_sum      one thread per wave: the sum of a run that starts in it and goes on (its
-//                  part in the wave, then those of the next waves in turn)
+//                  part in the wave, then those of the next waves in turn: a step per 64
+//                  terms of the longest run, 0.5 us each)
 // The gradient of a key is at sink.at(key).  Each key's total is added once, atomically: calls
 // on several streams may add to one gradient buffer at the same time (and meshes of a batch
 // share one), as they may with scatter_terms.

@@ -124,6 +124,15 @@ int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
     return GPURT_OK;
 }
 
+// Whether the vertex sums of n items are added in the fixed order, and then its scratch.
+int plan_sums(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t, bool& fixed) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool recorded = hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+    if (recorded) (void)hipGetLastError();
+    fixed = fixed_order_sums(c, 3 * n, recorded);
+    return fixed ? alloc_terms(c, n, s, t) : GPURT_OK;
+}
+
 int bits_for(uint32_t n_verts) {
     int b = 1;
     while (b < 32 && (n_verts >> b) != 0) b++;
@@ -151,15 +160,16 @@ void sum_terms(TermScratch& t, size_t n, uint32_t n_verts, float* g_verts, hipSt
 int launch_cpq_bwd(gpurt_bvh_s* b, const float* q, size_t n, const int32_t* prim, const float* g,
                    float* g_q, float* g_verts, hipStream_t s) {
     if (n == 0) return GPURT_OK;
-    if (!g_verts || !fixed_order_sums(b->ctx, 3 * n)) {
+    TermScratch t;
+    bool fixed = false;
+    if (g_verts)
+        if (const int rc = plan_sums(b->ctx, n, s, t, fixed)) return rc;
+    if (!fixed) {
         hipLaunchKernelGGL(k_cpq_bwd, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n, q, prim, g,
                            b->tri_idx, (uint32_t)b->n_tris, b->verts, g_q, g_verts);
         GPURT_HIP(hipGetLastError());
         return GPURT_OK;
     }
-    TermScratch t;
-    int rc = alloc_terms(b->ctx, n, s, t);
-    if (rc) return rc;
     hipLaunchKernelGGL(k_cpq_bwd_terms, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n, q, prim, g,
                        b->tri_idx, (uint32_t)b->n_tris, b->verts, (uint32_t)b->n_verts, g_q, t.k0, t.terms);
     sum_terms(t, n, (uint32_t)b->n_verts, g_verts, s);
@@ -173,17 +183,17 @@ int launch_ray_bwd(gpurt_bvh_s* b, const gpurt_ray* rays, size_t n, const int32_
                    const float* t, const float* uv, const float* g, float* g_o, float* g_d,
                    float* g_verts, hipStream_t s) {
     if (n == 0) return GPURT_OK;
-    const bool vgrad = g_verts && uv;
-    if (!vgrad || !fixed_order_sums(b->ctx, 3 * n)) {
+    TermScratch ts;
+    bool fixed = false;
+    if (g_verts && uv)
+        if (const int rc = plan_sums(b->ctx, n, s, ts, fixed)) return rc;
+    if (!fixed) {
         hipLaunchKernelGGL(k_ray_bwd, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n,
                            reinterpret_cast<const float4*>(rays), prim, t, uv, g, b->tri_idx, (uint32_t)b->n_tris,
                            b->verts, g_o, g_d, g_verts);
         GPURT_HIP(hipGetLastError());
         return GPURT_OK;
     }
-    TermScratch ts;
-    int rc = alloc_terms(b->ctx, n, s, ts);
-    if (rc) return rc;
     hipLaunchKernelGGL(k_ray_bwd_terms, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (uint32_t)n,
                        reinterpret_cast<const float4*>(rays), prim, t, uv, g, b->tri_idx, (uint32_t)b->n_tris,
                        b->verts, (uint32_t)b->n_verts, g_o, g_d, ts.k0, ts.terms);

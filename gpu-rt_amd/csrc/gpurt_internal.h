@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "../../include/gpurt.h"
+#include "index_math.h"
 
 namespace gpurt_impl {
 
@@ -226,16 +227,9 @@ struct gpurt_ctx_s {
 };
 
 namespace gpurt_impl {
-// Vertex-gradient sums of the backward passes: the fixed-order sum (sort by vertex, then
-// segmented sums) when the context asks for it, FP32 atomics when it asks for them, and
-// otherwise whichever is faster -- the fixed order from about 0.6 M vertex terms, where the
-// atomics' device-wide rate (~18 G/s) costs more than the sort's passes (points or rays on a
-// 0.66 M vertex mesh, fixed order / atomics, us: 65 K 72 / 38, 131 K 82 / 69, 262 K 102 /
-// 132, 524 K 150 / 252; fewer vertices favour the fixed order, which has fewer passes).
-constexpr size_t kFixedOrderMinTerms = 600000;
-inline bool fixed_order_sums(const gpurt_ctx_s* c, size_t terms) {
-    return c->vertex_sums == GPURT_SUMS_FIXED_ORDER ||
-           (c->vertex_sums == GPURT_SUMS_AUTO && terms >= kFixedOrderMinTerms);
+// recorded: the call goes into a HIP graph and takes its scratch there
+inline bool fixed_order_sums(const gpurt_ctx_s* c, size_t terms, bool recorded = false) {
+    return fixed_order_rule(c->vertex_sums, terms, recorded);
 }
 }  // namespace gpurt_impl
 

@@ -7,6 +7,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "../../include/gpurt.h"
+
 namespace gpurt_impl {
 
 // A 64-bit value from its halves as __builtin_amdgcn_readfirstlane returns them: ints, so
@@ -38,6 +40,20 @@ __host__ __device__ inline uint32_t last_from(const Offsets& off, uint32_t n, ui
         if (step < n - lo && off[lo + step] <= key) lo += step;
     }
     return lo;
+}
+
+// Vertex-gradient sums of a backward call: the fixed order (sort by vertex, then segmented sums)
+// when the context asks for it, FP32 atomics when it asks for them, and otherwise whichever is
+// faster -- the fixed order from about 0.6 M vertex terms, where the atomics' device-wide rate
+// (~18 G/s) costs more than the sort's passes (points or rays on a 0.66 M vertex mesh, fixed
+// order / atomics, us: 65 K queries 72 / 38, 131 K 82 / 69, 262 K 102 / 132, 524 K 150 / 252).
+// Fewer vertices favour it more, though a run of many terms is added 64 at a time by one thread:
+// 210 K queries on 6, 42, 642 and 10,242 vertices 590 / 12,100, 155 / 3,400, 100 / 370 and 98 /
+// 131 (all on one vertex 1,070 / 13,900).  A call recorded into a HIP graph takes it from 2^21
+// terms only: its scratch is a memory node of the graph then.
+inline bool fixed_order_rule(int mode, size_t terms, bool recorded) {
+    if (mode != GPURT_SUMS_AUTO) return mode == GPURT_SUMS_FIXED_ORDER;
+    return terms >= (recorded ? size_t(1) << 21 : size_t(600000));
 }
 
 // Waves per CU of a set of n closest points: 16, but 12 for up to 256 points per CU (a

@@ -98,3 +98,13 @@ def test_collapse_launches(tmp_path):
     assert [got[k, 4, t] for k in (5000, 2_300_000) for t in (0, 1)] == [12, 12, 19, 19]
     assert [got[1_000_000, 2, t] for t in (0, 1)] == [30, 42]
     assert all(got[k, w, 0] == got[k, w, 1] for k in n for w in (2, 4, 8) if w > 2 or k <= 65536)
+
+
+def test_vertex_sums_rule(tmp_path):
+    """The default mode adds in the fixed order from 600,000 terms (200,000 queries) on, and from
+    2^21 in a call recorded into a graph; the other modes always and never."""
+    n = [0, 3, 3 * 199_999, 3 * 200_000, (1 << 21) - 1, 1 << 21, 1 << 33]
+    out = _run(tmp_path, "for (int m : {GPURT_SUMS_AUTO, GPURT_SUMS_FIXED_ORDER, GPURT_SUMS_ATOMIC}) for (bool r : {false, true})\n"
+               "    for (size_t n : {" + ", ".join("%dull" % k for k in n) + "}) printf(\"%d\\n\", fixed_order_rule(m, n, r));")
+    want = [int(k >= lim) for lim in (600_000, 1 << 21) for k in n] + [1] * 14 + [0] * 14
+    assert [int(x) for x in out] == want
