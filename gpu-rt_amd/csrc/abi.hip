@@ -183,6 +183,7 @@ static void pool_empty(gpurt_ctx_s* c) {
 }
 
 hipError_t ctx_malloc(gpurt_ctx_s* c, void** p, size_t bytes) {
+    AnyCapture mode;
     *p = nullptr;
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory) return e;

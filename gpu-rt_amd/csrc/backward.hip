@@ -124,13 +124,18 @@ int alloc_terms(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t) {
     return GPURT_OK;
 }
 
-// Whether the vertex sums of n items are added in the fixed order, and then its scratch.
+// Whether the vertex sums of n items are added in the fixed order, and then its scratch; with
+// the default mode, whose atomics need none, memory that cannot be had is no error.
 int plan_sums(gpurt_ctx_s* c, size_t n, hipStream_t s, TermScratch& t, bool& fixed) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     const bool recorded = hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
     if (recorded) (void)hipGetLastError();
     fixed = fixed_order_sums(c, 3 * n, recorded);
-    return fixed ? alloc_terms(c, n, s, t) : GPURT_OK;
+    if (!fixed) return GPURT_OK;
+    const int rc = alloc_terms(c, n, s, t);
+    if (rc != GPURT_E_OOM || c->vertex_sums != GPURT_SUMS_AUTO) return rc;
+    fixed = false;
+    return GPURT_OK;
 }
 
 int bits_for(uint32_t n_verts) {

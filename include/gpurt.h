@@ -160,7 +160,8 @@ GPURT_API int gpurt_ctx_status(gpurt_ctx ctx, uint32_t* flags, int clear);
  *   GPURT_SUMS_AUTO         (the default) whichever is faster for the call: the fixed
  *                           order from 600,000 terms (200,000 queries; the atomics' device-
  *                           wide rate then costs more than the sort; from 2^21 terms in a
- *                           call recorded into a HIP graph), atomics below
+ *                           call recorded into a HIP graph), atomics below and where the
+ *                           scratch cannot be had
  * Applies to calls made after it; a batch reads it in gpurt_batch_set_grads.  An unknown
  * mode: GPURT_E_INVALID.  No counterpart in the reference (it has no gradients). */
 #define GPURT_SUMS_AUTO 0

@@ -275,3 +275,33 @@ def test_idle_memory_is_given_up_when_memory_is_short(dev):
     bvh.close()
     ctx.close()
     torch.cuda.empty_cache()
+
+
+def test_default_vertex_sums_without_memory_for_scratch(dev):
+    """The default mode falls back to atomics, which need no scratch, where the fixed order's (84
+    bytes a query) cannot be had: within 2 c^2 2^-24 for vertices of up to c terms of at most 1."""
+    V, F = _soup(2_000_000, dev)
+    n = 20_000_000
+    q = (V.repeat(4, 1)[:n] + 0.002).contiguous()
+    g, got = torch.ones(n, device=dev), []
+    for mode in ("fixed", "auto"):
+        ctx = gpurt.Context(0, vertex_sums=mode)
+        bvh = gpurt.Bvh(ctx, V, F)
+        prim, pt, dist, bary = bvh.closest_point(q)
+        gv = torch.zeros_like(V)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        hog = None
+        if mode == "auto":
+            hog = torch.empty(torch.cuda.mem_get_info(dev)[0] - (1 << 29), dtype=torch.uint8, device=dev)
+        bvh.closest_point_bwd(q, prim, bary, pt, dist, g, None, gv)
+        torch.cuda.synchronize()
+        del hog
+        got.append(gv)
+        bvh.close()
+        ctx.close()
+    c = float(torch.bincount(F.long()[prim.long()].reshape(-1)).max())
+    assert float(got[0].abs().max()) > 0
+    assert float((got[0] - got[1]).abs().max()) <= 2.0 * c * c * 2.0**-24
+    del q, g, pt, bary, got
+    torch.cuda.empty_cache()
