@@ -335,6 +335,7 @@ int ctx_scratch(gpurt_ctx_s* c, hipStream_t s, size_t bytes, CallScratch& out) {
             if (e.mem && hipStreamWaitEvent(s, e.last, 0) != hipSuccess)
                 return hip_error(hipGetLastError(), "hipStreamWaitEvent");
             if (e.bytes < bytes) {
+                AnyCapture mode;
                 // Growing waits for the device (hipFree), once per new largest call on
                 // the stream.
                 if (e.mem) (void)hipFree(e.mem);

@@ -548,9 +548,14 @@ int gpurt_batch_create(gpurt_ctx ctx, const gpurt_batch_mesh* meshes, size_t n_m
         for (uint32_t st = 0; st < md[m].n_r; st += 64) chunks.push_back(make_uint2(m, st));
     b->n_ray_chunks = (uint32_t)chunks.size() - b->n_cpq_chunks;
     // Oriented nodes are remade with every replay's trees, which only enough closest-point
-    // queries pay for: 7.1 M triangles and 3.0 M queries (256 meshes): the nodes cost 500
-    // us and the queries take 1.63 instead of 2.42 ms, so the line lies at a query for
-    // every four triangles; below it the queries use the FP32 nodes.
+    // queries pay for; how many depends on their distance, which is not known here.  Points
+    // near the surface pay from about a query per triangle on meshes of 20,000, far ones much
+    // earlier; the line, a query for every four triangles, lies between.  A replay with FP32 /
+    // oriented nodes, us: 64 meshes of 20,480 triangles, 1/8 query per triangle, near 685 /
+    // 743, a fifth of them far 1,035 / 834; 1/4: 731 / 782, 1,074 / 878; 1: 1,180 / 1,177, 1,929 /
+    // 1,367; one of 1.3 M, 1/8: 1,075 / 949, 3,103 / 1,190; 256 of 1,280, 1/4: 373 / 400, 475 / 453;
+    // 2,000 of 80, 1: 367 / 387, 378 / 399.  (256 uneven ones, 7.1 M triangles and 3.0 M queries:
+    // the nodes cost 500 us and the queries take 1.63 instead of 2.42 ms.)
     uint64_t total_q = 0;
     for (size_t m = 0; m < n_meshes; m++) total_q += md[m].n_q;
     const bool oriented = cpq_use_oriented(bp.format, W) && 4 * total_q >= off;

@@ -12,15 +12,21 @@
 //   radix sort     LSD, 8-bit digits, LDS histograms + LDS ranking by wave ballots
 //                  (stable, so equal codes stay in triangle order); one block up to 8192
 //   k_pack         triangles and boxes gathered into sorted (leaf) order
-//   k_karras       Karras (HPG 2012) binary radix tree over the sorted keys; because the
+//   k_tree_local   Karras (HPG 2012) binary radix tree over the sorted keys; because the
 //                  mesh id is in the high key bits every mesh is one subtree, whose root
-//                  is recorded
-//   k_boxes_*      node boxes: those inside a chunk of 256 leaves bottom-up by one block,
-//                  the others as unions over their leaf range (no atomics, no order)
-//   k_treelet      optional SAH treelet restructuring (treelet.hip)
-//   k_collapse     one launch per wide level: a node opens the child with the largest
-//                  surface area until it has W children; subtrees of <= leaf_size
-//                  triangles become leaves (contiguous ranges of packed triangles)
+//                  is recorded.  With it the boxes of nodes inside a chunk of 256 leaves,
+//                  bottom-up by one block
+//   k_range_top, k_boxes_cross
+//                  the other nodes' boxes, as unions over their leaf range (no atomics, no
+//                  order)
+//   k_treelet      optional SAH treelet restructuring (treelet.hip), roots bucketed by
+//                  k_level_hist / scan / scatter
+//   k_collapse_head, k_collapse, k_collapse_tail
+//                  the first levels in one launch, one launch per wide level, the last
+//                  levels in one: a node opens the child with the largest surface area
+//                  until it has W children; subtrees of <= leaf_size triangles become
+//                  leaves (contiguous ranges of packed triangles, gathered by k_repack
+//                  after treelets)
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -1111,7 +1117,7 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, uint32_t b
                                                uint32_t* next_count, const HeadList* in = nullptr,
                                                HeadList* next = nullptr, bool last = false) {
     WNode<W>* nodes = reinterpret_cast<WNode<W>*>(a.nodes);
-    // every lane runs every iteration (slot allocation is wave-wide); lanes past the
+    // every lane runs every iteration (slot allocation is block-wide); lanes past the
     // level's end take part with nothing to allocate
     for (uint32_t k0 = blockIdx.x * blockDim.x; k0 < cnt; k0 += gridDim.x * blockDim.x) {
         const uint32_t k = k0 + threadIdx.x;

@@ -7,8 +7,9 @@
 namespace gpurt_impl {
 
 // per-mesh statistics: [cmin xyz, cmax xyz, max|coord|, unused] as ordered uints.
-// k_prep accumulates into kRep replicas (block b uses replica b % kRep) so that the
-// atomics of ~N/64 waves do not serialise on 7 addresses; k_reduce_stats folds them.
+// k_prep accumulates into kRep replicas (wave w, of up to 1,024 triangles, uses replica
+// w % kRep) so that the waves' atomics do not serialise on 7 addresses; k_reduce_stats folds
+// them.
 constexpr int kStat = 8;
 constexpr int kRep = 64;
 

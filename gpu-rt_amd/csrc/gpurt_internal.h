@@ -38,7 +38,8 @@ constexpr uint32_t kLeafBit = 0x80000000u;
 constexpr uint32_t kMaxLeafFirst = 0x0FFFFFFFu;  // 2^28 - 1 packed triangles max
 // Wide-node levels the collapse can emit.  A mesh's binary radix tree is at most 58
 // levels deep (30 Morton bits + 28 index tie-break bits) and every wide level consumes
-// at least one binary level, so 64 launches always finish the tree.
+// at least one binary level; treelets can make it deeper, and a tree of more wide levels than
+// these is refused.
 constexpr int kMaxLevels = 64;
 constexpr int kBlock = 256;
 // buckets of the treelet pass, one per prefix length

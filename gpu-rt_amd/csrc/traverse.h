@@ -494,7 +494,8 @@ __device__ __forceinline__ uint32_t first_query(uint32_t g, uint32_t total) {
 // Plain source with load balancing: lane g takes query first_query(g) first; the queries after the
 // first `total` are cut into 64-query chunks dealt round-robin to nq = min(kQueues,
 // blocks) queues (chunk j belongs to queue j % nq), each with its own device counter
-// (zero at launch, 256 bytes apart).  Block b's waves take chunks of queue b % nq, so
+// (256 bytes apart; zero at launch when n > total, and not to be read otherwise: a launch
+// with a lane per query does without the clearing, and `more` is false from the start).  Block b's waves take chunks of queue b % nq, so
 // every queue is served by at least one block: a wave takes a
 // chunk when lanes want work and its pool is empty, and gives the chunk's queries to
 // those lanes in lane order.  Lanes that get cheap queries take more of them, so no

@@ -11,8 +11,8 @@
 //   3. if it is cheaper than the current one, rewrite the treelet's N - 1 internal nodes
 //      (r keeps its index, so ancestors are untouched) with their new children, boxes,
 //      triangle counts and costs.
-// Bottom-up order is the same as the box pass: one launch per Karras prefix length,
-// largest first.  Two roots of one launch have equal prefix length, so neither is an
+// Bottom-up order: one launch per Karras prefix length, largest first (the roots are bucketed
+// by it).  Two roots of one launch have equal prefix length, so neither is an
 // ancestor of the other and their treelets are disjoint; everything below a root was
 // finished by earlier launches.  (That argument holds for the tree as Karras built it,
 // so one round is supported.)  Subtrees of <= leaf_size triangles become single leaves
@@ -329,7 +329,7 @@ static void launch_treelet_levels(BuildBufs& b, int key_bits, int nbits, hipStre
 }
 
 int run_treelets(BuildBufs& b, int treelet_size, int rounds, int key_bits, int nbits, hipStream_t s) {
-    // buckets (b.lvl_begin / b.lvl_order) were filled by the box pass
+    // buckets (b.lvl_begin / b.lvl_order) were filled by k_level_hist, scan and scatter
     if (rounds > 1)
         return set_error(GPURT_E_UNSUPPORTED, "treelet_rounds > 1 is not supported (one bottom-up round)");
     if (b.N < 3) return GPURT_OK;
