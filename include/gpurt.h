@@ -85,8 +85,9 @@ typedef struct gpurt_build_opts {
                                2 = 8-bit child boxes relative to the node's box
                                    (48/64/96 bytes for W = 2/4/8),
                                3 = 8-bit for rays; for closest points 8-bit boxes in a
-                                   frame of each node's own (W = 4, 64 bytes) or FP32
-                                   boxes (W = 2, 8),
+                                   frame of each node's own (W = 4, 64 bytes more a node
+                                   and a pass of the build that a program of rays alone
+                                   saves with 2) or FP32 boxes (W = 2, 8),
                                0 = library default (3)                                */
 } gpurt_build_opts;
 
