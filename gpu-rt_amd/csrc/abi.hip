@@ -44,6 +44,14 @@ __global__ void k_compact_verts(uint32_t n, const float* __restrict__ v, uint64_
     out[3 * (size_t)i + 2] = p[2];
 }
 
+// HIP refuses event queries, host waits and the like (and breaks the capture) while any thread
+// captures a stream in global mode, unless the calling thread says that it knows.
+struct AnyCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 EventRef make_event() {
     auto r = std::make_shared<Event>();
     if (hipEventCreateWithFlags(&r->e, hipEventDisableTiming) == hipSuccess) return r;
@@ -110,9 +118,12 @@ void wait_uses(gpurt_bvh_s* b, hipStream_t s) {
 
 Uses uses_of(gpurt_bvh_s* b) {
     std::lock_guard<std::mutex> lk(b->use_mu);
+    if (!b->uses_lost) return b->uses;
     // uses that no event marks (graph capture, a failed record)
-    if (b->uses_lost) (void)hipDeviceSynchronize();
-    return b->uses_lost ? Uses{} : b->uses;
+    AnyCapture mode;
+    if (hipDeviceSynchronize() == hipSuccess) return Uses{};
+    (void)hipGetLastError();
+    return b->uses;
 }
 
 // gives a BVH's memory back after a point of a stream, or after some uses
@@ -125,14 +136,6 @@ static void free_bvh_buffers(gpurt_bvh_s* b, const After& after) {
     b->tri_idx = b->leaf_order = b->refit_tmp = b->node_first = nullptr;
     b->verts = nullptr;
 }
-
-// HIP refuses event queries, host waits and the like (and breaks the capture) while any thread
-// captures a stream in global mode, unless the calling thread says that it knows.
-struct AnyCapture {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    ~AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-};
 
 // drops the points that are reached from what an idle block waits for (those on stream s may
 // stay); true when no others are left
@@ -197,6 +200,13 @@ hipError_t ctx_malloc(gpurt_ctx_s* c, void** p, size_t bytes) {
 
 int pool_alloc(gpurt_ctx_s* c, void** p, size_t bytes, hipStream_t s) {
     *p = nullptr;
+    // (memory allocated on such a stream would be the graph's, and an event recorded on it a
+    // node of the graph)
+    hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cst) != hipSuccess || cst != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return set_error(GPURT_E_DEVICE, "builds and refits cannot be recorded into a HIP graph");
+    }
     // sizes in steps of an eighth of their power of two (at least 64 KiB), so that the
     // slightly different node counts of similar meshes share blocks
     size_t step = size_t(1) << 16;

@@ -305,3 +305,35 @@ def test_default_vertex_sums_without_memory_for_scratch(dev):
     assert float((got[0] - got[1]).abs().max()) <= 2.0 * c * c * 2.0**-24
     del q, g, pt, bary, got
     torch.cuda.empty_cache()
+
+
+def test_build_on_a_captured_stream_is_refused(dev):
+    """A build on a stream that is being captured is refused (it reads a report back) and takes no
+    memory of the graph into the context's pool: the capture is whole, and later builds on the
+    stream work."""
+    w = W.cpq_small(n_queries=64)
+    V, F, Q = _t(w["verts"], dev), _t(w["tris"], dev), _t(w["queries"], dev)
+    ep, _, ed, _ = O.cpq_brute_f32(w["verts"], w["tris"], w["queries"])
+    ctx = gpurt.Context(0)
+    x = torch.arange(1024, dtype=torch.float32, device=dev)
+    y = torch.zeros_like(x)
+    cap = torch.cuda.Stream(dev)
+    for warm in (False, True):  # with nothing in the pool, and with blocks that would fit
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cap):
+            torch.add(x, 1.0, out=y)
+            with pytest.raises(gpurt.GpurtError):
+                gpurt.Bvh(ctx, V, F)
+            torch.mul(y, 2.0, out=y)
+        for _ in range(2):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, (x + 1.0) * 2.0)
+        with torch.cuda.stream(cap):
+            bvh = gpurt.Bvh(ctx, V, F)
+            prim, _, dist, _ = bvh.closest_point(Q)
+        torch.cuda.synchronize()
+        assert np.array_equal(prim.cpu().numpy(), ep) and np.array_equal(dist.cpu().numpy(), ed)
+        bvh.close()
+    ctx.close()
